@@ -61,16 +61,17 @@ typedef enum
     R355_KERNEL_TILED  = 2, /* LDS-staged 256 x 256 macro tile (m, n multiples of 16; k of 8 for 16-bit, 16 for 8-bit operands)
                                (samples/perf_hgemm.cpp:515-711,
                                 test/gemm/gemm_PGR1_LB2_MP0_MB_CP/device/kernel_device_func.hpp:52-283) */
-    R355_KERNEL_TILED_128 = 3, /* the same kernels with a 128 x 128 macro tile (the only one for f64): what AUTO
+    R355_KERNEL_TILED_128 = 3, /* the same kernels with a 128 x 128 macro tile (f64: this one or the 64 x 64): what AUTO
                                picks when the 256 x 256 tiles of a problem would leave most CUs idle */
     R355_KERNEL_TILED_128_SPLITK = 4, /* 128 x 128 tiles with K split over several workgroups per tile and a reduction
                                (needs `workspace`; what AUTO picks for few tiles and a long K when a workspace is given).
                                No counterpart in the reference. */
-    R355_KERNEL_TILED_DEEP = 5 /* the 256 x 256 macro tile with its K loop on five LDS buffers filled two to three stages ahead.
+    R355_KERNEL_TILED_DEEP = 5, /* the 256 x 256 macro tile with its K loop on five LDS buffers filled two to three stages ahead.
                                8-bit and f32 operands always run that way (the selector then equals R355_KERNEL_TILED); for
                                f16 / bf16 it is what AUTO and R355_KERNEL_TILED take once A and B together exceed the 256 MiB
                                memory-side cache, where the default two-buffer loop no longer hides the HBM latency, and for
                                k <= 1536. */
+    R355_KERNEL_TILED_64 = 7 /* the same kernels with a 64 x 64 macro tile, up to four workgroups per CU (dense GEMM only) */
 } r355_gemm_kernel;
 
 /*
@@ -128,7 +129,9 @@ int r355_gemm(const r355_gemm_args* args, void* stream);
  * (the values the reference computes on the host: samples/perf_hgemm.cpp:807-817).
  * R355_KERNEL_AUTO may split a problem of several rounds of 256 x 256 tiles into two launches on the
  * same stream - whole rounds on that tile, the rest (at most half a round) on 128 x 128 tiles; the
- * plan then describes the first launch. */
+ * plan then describes the first launch.  It may also work a problem of 128 x 128 tiles as 64 x 64 quarters of them
+ * (R355_KERNEL_TILED_64: four workgroups of a quarter of the LDS per tile) and with fewer K splits than planned, where
+ * a timing model prices that as faster; the plan then describes the 128 x 128 tiling and the most workspace a launch uses. */
 typedef struct
 {
     int32_t  kernel;                       /* r355_gemm_kernel actually selected */

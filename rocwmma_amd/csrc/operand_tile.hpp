@@ -2,8 +2,8 @@
 // LDS, and how a wave reads its operand blocks back.  Shared by the dense kernels (gemm_tiled.hip) and the 2:4 sparse one
 // (sparse.hip, dense B).
 //
-// A stage is 128 bytes of K.  An operand tile of 32 WB rows (WB = 8: 256 rows, 32 KiB; WB = 4: 128 rows, 16 KiB) is
-// written by direct loads, chunk L = j * 256 + tid at LDS byte 16 L:
+// A stage is 128 bytes of K.  An operand tile of 32 WB rows (WB = 8: 256 rows, 32 KiB; WB = 4: 128 rows, 16 KiB; WB = 2:
+// 64 rows, 8 KiB) is written by direct loads, chunk L = j * 256 + tid at LDS byte 16 L:
 //   * K-contiguous (A row-major / B col-major): rows x 128 B, chunk c of row r in slot c ^ ((r >> 1) & 7); a lane
 //     reads 16 consecutive K bytes of its row with one ds_read_b128;
 //   * M/N-contiguous (A col-major / B row-major): k-rows x (32 WB ES) B with a swizzle that depends on the element
@@ -38,8 +38,12 @@ namespace r355
                 return ((krow >> 1) & 1u) << 3; // f64: a 32-lane pass reads two k-rows 2 apart, 128 bytes each
             else if constexpr(ES == 4)
                 return ((krow >> 2) & 3u) << 2; // f32: a wave reads k-rows 4 apart, 64 bytes each
+            else if constexpr(ES == 2 && WB == 2)
+                return (krow & 2u) | (((krow >> 3) & 1u) << 2); // 128-byte k-rows, 8 chunks: of k-rows 0..3, 8..11 two share banks with 0 (1)
             else if constexpr(ES == 2)
                 return ((krow & 3u) << 2) | (((krow >> 3) & 1u) << 1); // 16-bit elements: as in gemmTiled16
+            else if constexpr(WB == 2)
+                return ((krow >> 2) & 1u) | ((krow >> 3) & 2u); // 64-byte k-rows, 4 chunks: k-rows 4 and 16 apart share banks
             else if constexpr(WB == 8)
                 return (krow & 7u) | ((krow >> 1) & 8u); // 256-byte k-rows, 16 chunks
             else

@@ -734,6 +734,8 @@ namespace r355
             return fail(R355_ERR_MISALIGNED, "sparse gemm: values, B, C and D need 16-byte alignment (pointers and leading dimensions), metadata 4-byte");
         if(g.kernel == R355_KERNEL_TILED_128_SPLITK)
             return fail(R355_ERR_UNSUPPORTED, "sparse gemm: no split along K (R355_KERNEL_TILED_128 is the 128 x 128 macro tile)");
+        if(g.kernel == R355_KERNEL_TILED_64)
+            return fail(R355_ERR_UNSUPPORTED, "sparse gemm: no 64 x 64 macro tile");
         if((g.kernel == R355_KERNEL_TILED || g.kernel == R355_KERNEL_TILED_DEEP || g.kernel == R355_KERNEL_TILED_128) && !tiledOk(g))
             return fail(R355_ERR_UNSUPPORTED,
                         "sparse gemm (macro tile): C (when beta != 0) and D must share an orientation, metadata 16-byte aligned, ldb below 8 MiB");
