@@ -5,9 +5,9 @@
 // (dlrm_kernel_base_impl.hpp:146-151) - but without their global scratch: the forward kernels take the lower triangle
 // out of an accumulator block through 1 KiB of the wave's LDS instead of a [batch][m][m] f32 buffer, and the backward
 // kernels form each 16 x 16 block of S = T + T^T in LDS from the packed upstream triangle instead of reconstructing
-// [batch][m][m] in memory first.  Each direction has two forms: one 16 x 16 block per wave, as in the reference, for
-// small shapes, and a register-blocked one (several blocks per wave, so that a fragment feeds several matrix
-// instructions) for large ones.
+// [batch][m][m] in memory first.  These kernels run one 16 x 16 block per wave, as in the reference, and serve small
+// shapes; larger ones go to macro tiles (forward: gemm_tiled.hip) or to a register-blocked kernel (backward: several blocks
+// per wave, so that a fragment feeds several matrix instructions).
 #include <rocwmma/rocwmma.hpp>
 
 #include "common.hpp"
@@ -75,86 +75,6 @@ namespace
             if(gj < gi)
                 o[k + gi * (gi - 1u) / 2u + gj] = static_cast<T>(mine[e]);
         }
-    }
-
-    // Forward from 64 features on: a wave owns NB x NB blocks at once - super-block (si, sj), sj <= si, of X X^T; p = si (si +
-    // 1) / 2 + sj - so that every fragment it loads feeds NB matrix instructions instead of one (a quarter of the bytes
-    // from the caches per flop at NB = 4: with a block per wave m = k = 1024 reads every row block of X 64 times over).
-    // BK: the K depth per step, 32 for 16-bit elements where k allows it (64-byte runs of a row per lane group instead of 32).
-    template <typename T, uint32_t NB, uint32_t BK>
-    __global__ void __launch_bounds__(THREADS) dlrmFwdGeneralBlocked(const T* __restrict__ in, T* __restrict__ out, uint32_t m, uint32_t k,
-                                                                    uint32_t pairs)
-    {
-        using FragA   = fragment<matrix_a, BLK, BLK, BK, T, row_major>;
-        using FragB   = fragment<matrix_b, BLK, BLK, BK, T, col_major>;
-        using FragAcc = fragment<accumulator, BLK, BLK, BK, float32_t>;
-        __shared__ float block[WAVES][BLK * BLK];
-
-        const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-        const uint32_t p    = blockIdx.x * WAVES + wave;
-        if(p >= pairs)
-            return;
-        uint32_t si = 0;
-        while((si + 1u) * (si + 2u) / 2u <= p)
-            ++si;
-        const uint32_t sj     = p - si * (si + 1u) / 2u;
-        const uint32_t tiles  = m / BLK;
-        const uint64_t stride = (uint64_t)k + (uint64_t)m * (m - 1u) / 2u;
-        const T*       x      = in + (uint64_t)blockIdx.y * m * k;
-        T*             o      = out + (uint64_t)blockIdx.y * stride;
-
-        if(p == 0u) // the bottom-MLP row
-            for(uint32_t e = lane; e < k; e += 64u)
-                o[e] = x[e];
-
-        // block (i, j) of the super-block is block (ti, tj) = (si NB + i, sj NB + j) of X X^T; wanted when it exists and
-        // touches the strict lower triangle (tj <= ti)
-        auto wanted = [&](uint32_t i, uint32_t j) { return si * NB + i < tiles && sj * NB + j < tiles && sj * NB + j <= si * NB + i; };
-        FragAcc acc[NB][NB];
-#pragma unroll
-        for(uint32_t i = 0; i < NB; ++i)
-#pragma unroll
-            for(uint32_t j = 0; j < NB; ++j)
-                fill_fragment(acc[i][j], 0.0f);
-        for(uint32_t kk = 0; kk < k; kk += BK)
-        {
-            FragA a[NB];
-            FragB b[NB];
-#pragma unroll
-            for(uint32_t i = 0; i < NB; ++i)
-            {
-                // (a row block past the end reads the last one again: its products are not used)
-                const uint32_t ti = si * NB + i < tiles ? si * NB + i : tiles - 1u, tj = sj * NB + i < tiles ? sj * NB + i : tiles - 1u;
-                load_matrix_sync(a[i], x + (uint64_t)ti * BLK * k + kk, k);
-                load_matrix_sync(b[i], x + (uint64_t)tj * BLK * k + kk, k); // X^T as a col-major k x m matrix: column n is row n of X
-            }
-#pragma unroll
-            for(uint32_t i = 0; i < NB; ++i)
-#pragma unroll
-                for(uint32_t j = 0; j < NB; ++j)
-                    if(wanted(i, j))
-                        mma_sync(acc[i][j], a[i], b[j], acc[i][j]);
-        }
-        float* mine = block[wave];
-#pragma unroll
-        for(uint32_t i = 0; i < NB; ++i)
-#pragma unroll
-            for(uint32_t j = 0; j < NB; ++j)
-            {
-                if(!wanted(i, j))
-                    continue;
-                store_matrix_sync(mine, acc[i][j], BLK, mem_row_major);
-                __builtin_amdgcn_wave_barrier(); // (LDS is in order within a wave: the reads below see the block)
-#pragma unroll
-                for(uint32_t q = 0; q < BLK * BLK / 64u; ++q)
-                {
-                    const uint32_t e = q * 64u + lane, r = e / BLK, c = e % BLK;
-                    const uint64_t gi = (uint64_t)(si * NB + i) * BLK + r, gj = (uint64_t)(sj * NB + j) * BLK + c;
-                    if(gj < gi)
-                        o[k + gi * (gi - 1u) / 2u + gj] = static_cast<T>(mine[e]);
-                }
-                __builtin_amdgcn_wave_barrier(); // the block is rewritten by the next one
-            }
     }
 
     // Backward.  Wave (ti, kc) of sample blockIdx.z owns block (ti, kc) of the gradient S X; S(i, j) is the upstream
@@ -393,19 +313,34 @@ namespace
             }
     }
 
+    // Forward: the macro tile's edge (dlrmFwdTiled in gemm_tiled.hip), or 0 for a block per wave.  Measured on one box:
+    //   * up to 16 features a sample is a single block, and a tile of 64 rows would be three quarters padding
+    //     (16 x 96, batch 4096, f16: 5.3 us a block per wave, 15.7 on 64 x 64 tiles);
+    //   * a launch of a few short waves is over before a tile's K loop has filled its five buffers (64 x 96 x 64 f16: 4.05
+    //     against 4.57 us; at k = 256 5.5 against 4.6, and from 128 x 144 x 64 on, 2304 waves, 5.6 against 4.6);
+    //   * 16-bit types take the 128 x 128 tile where every CU gets 16 K stages of such tiles or more (512 x 1024 x 64: 30.5
+    //     against 35.0 us on 64 x 64, 1024 x 1024 x 64: 86 against 118; 1024 x 256 x 16: 16.1 against 14.2); f32, bound by its matrix
+    //     instructions, is faster on 64 x 64 throughout (1024 x 1024 x 64: 565 against 590 us).
+    // Leading dimensions beyond 8 MiB per row do not fit the tile kernels' 32-bit lane offsets.
+    uint32_t forwardTile(int32_t dtype, uint32_t m, uint32_t k, uint32_t batch)
+    {
+#ifdef R355_DLRM_BLOCK_PER_WAVE // measurement build: a block per wave for every shape
+        return 0u;
+#endif
+        const uint64_t es = r355::dtypeBytes(dtype), cus = r355::computeUnits();
+        if(m <= BLK || (uint64_t)k * es > (1u << 23))
+            return 0u;
+        const uint64_t blocks = m / BLK, waves = blocks * (blocks + 1u) / 2u * batch, steps = k / (es == 2u ? 16u : 4u);
+        if(waves <= 5u * cus && steps <= 12u)
+            return 0u;
+        const uint64_t tiles = (m + 127u) / 128u, stages = (k * es + 127u) / 128u;
+        return es == 2u && tiles * (tiles + 1u) / 2u * batch * stages >= 16u * cus ? 128u : 64u;
+    }
+
     template <typename T>
     int fwd(const void* in, void* out, uint32_t m, uint32_t k, uint32_t batch, hipStream_t s)
     {
-        constexpr uint32_t NB = 4;
-#ifdef R355_DLRM_BLOCK_PER_WAVE // measurement build: the block-per-wave kernels for every shape
-        const bool blocked = false;
-#else
-        // NB x NB blocks per wave from 64 features on, where that still leaves every SIMD two waves or so (fewer, and the
-        // many short waves of the block-per-wave kernel hide latency better: 128 x 128 x 64 runs 8 us against 10)
-        const uint32_t supers  = (m / BLK + NB - 1u) / NB;
-        const bool     blocked = m >= NB * BLK && (uint64_t)supers * (supers + 1u) / 2u * batch >= 2ull * r355::computeUnits();
-#endif
-        const uint32_t tiles = blocked ? (m / BLK + NB - 1u) / NB : m / BLK, pairs = tiles * (tiles + 1u) / 2u;
+        const uint32_t tiles = m / BLK, pairs = tiles * (tiles + 1u) / 2u;
         const uint64_t stride = (uint64_t)k + (uint64_t)m * (m - 1u) / 2u;
         // the batch is a grid dimension of at most 65535: a larger one goes out in several launches on the same stream
         for(uint32_t first = 0; first < batch; first += GRID_BATCH)
@@ -414,12 +349,7 @@ namespace
             const dim3     grid((pairs + WAVES - 1u) / WAVES, count);
             const T*       src = static_cast<const T*>(in) + (uint64_t)first * m * k;
             T*             dst = static_cast<T*>(out) + (uint64_t)first * stride;
-            if(!blocked)
-                hipLaunchKernelGGL((dlrmFwdGeneral<T>), grid, dim3(THREADS), 0, s, src, dst, m, k, pairs);
-            else if(sizeof(T) == 2 && k % 32u == 0u)
-                hipLaunchKernelGGL((dlrmFwdGeneralBlocked<T, NB, sizeof(T) == 2 ? 32u : blockK<T>()>), grid, dim3(THREADS), 0, s, src, dst, m, k, pairs);
-            else
-                hipLaunchKernelGGL((dlrmFwdGeneralBlocked<T, NB, blockK<T>()>), grid, dim3(THREADS), 0, s, src, dst, m, k, pairs);
+            hipLaunchKernelGGL((dlrmFwdGeneral<T>), grid, dim3(THREADS), 0, s, src, dst, m, k, pairs);
         }
         return r355::checkLaunch("dlrm_fwd (general)");
     }
@@ -470,6 +400,8 @@ namespace r355
         const int rc = checkGeneral("dlrm_fwd", m, k, batch);
         if(rc != R355_OK)
             return rc;
+        if(const uint32_t tile = forwardTile(dtype, m, k, batch))
+            return dlrmFwdTiled(dtype, in, out, m, k, batch, tile, s);
         switch(dtype)
         {
         case R355_F16: return fwd<float16_t>(in, out, m, k, batch, s);

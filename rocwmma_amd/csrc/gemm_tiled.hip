@@ -129,6 +129,10 @@ namespace r355
     int gemmTiledPart1(const r355_gemm_args& g, bool aK, bool bK, uint32_t tile, const GemmTileParams& p, hipStream_t s);
     int gemmTiledPart2(const r355_gemm_args& g, bool aK, bool bK, uint32_t tile, const GemmTileParams& p, hipStream_t s);
     int gemmTiledPart3(const r355_gemm_args& g, bool aK, bool bK, uint32_t tile, const GemmTileParams& p, hipStream_t s);
+    // DLRM forward on macro tiles of X X^T (dlrmFwdTiled below), one per element type
+    int dlrmFwdTiledPart0(const GemmTileParams& p, uint32_t tile, uint32_t groups, hipStream_t s);
+    int dlrmFwdTiledPart1(const GemmTileParams& p, uint32_t tile, uint32_t groups, hipStream_t s);
+    int dlrmFwdTiledPart3(const GemmTileParams& p, uint32_t tile, uint32_t groups, hipStream_t s);
 } // namespace r355
 
 namespace
@@ -475,6 +479,64 @@ namespace
             storeTileStaged<OutT, false, AccV, OutT, WBM, WBN, SCRATCH>(acc, p, m0, n0, lane, scratch);
         else
             storeTileStaged<AccE, true, AccV, OutT, WBM, WBN, SCRATCH>(acc, p, m0, n0, lane, scratch);
+    }
+
+    // The strict lower triangle of one wave's tile of X X^T, packed row by row: element (gi, gj), gj < gi, goes to
+    // d[gi (gi - 1) / 2 + gj].  The wave tile starts at (m0, n0); rows from m on do not exist.  Staged through the wave's LDS
+    // like storeTileStaged; a row of the wave tile is then one run of 16 WB elements that starts at any element: a lane
+    // stores 16 bytes of it whatever its alignment (the memory pipeline takes unaligned vectors; the L2 puts the partial lines of
+    // neighbouring tiles together), and the wave tiles on the diagonal, whose rows end anywhere, go out element by element.
+    template <typename OutT, uint32_t WB>
+    __device__ __forceinline__ void storeTriangle(f32x4 (&acc)[WB][WB], OutT* d, uint32_t m, uint32_t m0, uint32_t n0, uint32_t lane, char* scratch)
+    {
+        constexpr uint32_t OS = sizeof(OutT), WT = 16u * WB, ROW_BYTES = WT * OS, ROW_CHUNKS = ROW_BYTES / CHUNK;
+        constexpr uint32_t SWZ = ROW_CHUNKS < 16u ? ROW_CHUNKS - 1u : 15u, EPC = CHUNK / OS, RPI = 64u / ROW_CHUNKS;
+        using OutV = OutT __attribute__((ext_vector_type(4)));
+        typedef int i32x4u __attribute__((ext_vector_type(4), aligned(2)));
+        if(n0 > m0 || m0 >= m)
+            return; // (uniform) above the diagonal, or past the last feature
+        const uint32_t r16 = lane & 15u, g = lane >> 4;
+#pragma unroll
+        for(uint32_t i = 0; i < WB; ++i)
+#pragma unroll
+            for(uint32_t j = 0; j < WB; ++j)
+            {
+                OutV out;
+#pragma unroll
+                for(uint32_t e = 0; e < 4; ++e)
+                    out[e] = static_cast<OutT>(acc[i][j][e]);
+                const uint32_t row = 16u * i + r16, byteInRow = (16u * j + 4u * g) * OS;
+                *reinterpret_cast<OutV*>(scratch + row * ROW_BYTES + (((byteInRow / CHUNK) ^ (row & SWZ)) * CHUNK) + byteInRow % CHUNK) = out;
+            }
+        __builtin_amdgcn_wave_barrier(); // the same wave reads back what it wrote (LDS is in order per wave)
+        auto rowStart = [&](uint32_t row) { // element n0 of the row in the packed triangle
+            const uint64_t gi = m0 + row;
+            return d + (gi * (gi - 1u) / 2u + n0);
+        };
+        if(n0 < m0) // (uniform) whole rows
+        {
+            const uint32_t c = lane % ROW_CHUNKS;
+#pragma unroll
+            for(uint32_t it = 0; it < WT / RPI; ++it)
+            {
+                const uint32_t row = it * RPI + lane / ROW_CHUNKS;
+                const i32x4    v   = *reinterpret_cast<const i32x4*>(scratch + row * ROW_BYTES + ((c ^ (row & SWZ)) * CHUNK));
+                if(m0 + row < m)
+                    *reinterpret_cast<i32x4u*>(rowStart(row) + c * EPC) = v;
+            }
+        }
+        else // the diagonal: row r of the wave tile holds r elements
+        {
+            const uint32_t col = lane % WT;
+#pragma unroll 8
+            for(uint32_t it = 0; it < WT / (64u / WT); ++it)
+            {
+                const uint32_t row = it * (64u / WT) + lane / WT, byteInRow = col * OS;
+                const OutT     v   = *reinterpret_cast<const OutT*>(scratch + row * ROW_BYTES + (((byteInRow / CHUNK) ^ (row & SWZ)) * CHUNK) + byteInRow % CHUNK);
+                if(col < row && m0 + row < m)
+                    rowStart(row)[col] = v;
+            }
+        }
     }
 
     //
@@ -878,7 +940,25 @@ namespace
         }
     }
 
-    template <Elem E, typename OutT, bool A_KCONTIG, bool B_KCONTIG, uint32_t WB>
+    // Which sample of a DLRM batch a workgroup works on and which tile (tm, tn), tn <= tm, of its X X^T; false: none.  All
+    // workgroups of an XCD walk one contiguous run of (sample, tile), so that the tiles of a sample share its X in one L2.
+    __device__ __forceinline__ bool triangleCoord(uint32_t bid, uint32_t tiles, uint32_t total, uint32_t& sample, uint32_t& tm, uint32_t& tn)
+    {
+        const uint32_t perXcd = (total + 7u) / 8u, slot = bid / 8u, local = (bid % 8u) * perXcd + slot;
+        if(slot >= perXcd || local >= total)
+            return false;
+        const uint32_t pairs = tiles * (tiles + 1u) / 2u;
+        sample               = local / pairs;
+        uint32_t rest        = local % pairs;
+        for(tm = 0; rest > tm; ++tm)
+            rest -= tm + 1u;
+        tn = rest;
+        return true;
+    }
+
+    // TRIANGLE: not a GEMM but the DLRM dot interaction, X X^T of every sample of a batch (p.a: [batch][m][k], lda = k) with its
+    // strict lower triangle packed behind the sample's first row (p.d: [batch][k + m (m - 1) / 2]); tileCount = batch x tiles.
+    template <Elem E, typename OutT, bool A_KCONTIG, bool B_KCONTIG, uint32_t WB, bool TRIANGLE = false>
     __device__ __forceinline__ void gemmTiled5(const Params& whole)
     {
         static_assert(WB == 8 || WB == 4 || WB == 2, "wave tile of 8 x 8, 4 x 4 or 2 x 2 blocks");
@@ -888,8 +968,8 @@ namespace
         R355_STAMP_ID();
         constexpr uint32_t ES = ElemTraits<E>::Bytes;
         // split-K: this workgroup row's share of K (the whole problem when splitStages is 0)
-        const Params p = splitShare<ES>(whole, A_KCONTIG ? (uint64_t)STAGE_KB : (uint64_t)STAGE_KB * whole.lda,
-                                        B_KCONTIG ? (uint64_t)STAGE_KB : (uint64_t)STAGE_KB * whole.ldb);
+        Params p = splitShare<ES>(whole, A_KCONTIG ? (uint64_t)STAGE_KB : (uint64_t)STAGE_KB * whole.lda,
+                                  B_KCONTIG ? (uint64_t)STAGE_KB : (uint64_t)STAGE_KB * whole.ldb);
         using AccV            = std::conditional_t<E == Elem::I8, i32x4v, std::conditional_t<E == Elem::F64, f64x4, f32x4>>;
         constexpr uint32_t TILE = 32u * WB, WT = 16u * WB; // macro tile and wave tile edge
         constexpr uint32_t OPER = TILE * STAGE_KB; // bytes of one operand per stage: 32 or 16 KiB
@@ -901,10 +981,25 @@ namespace
         __shared__ __attribute__((aligned(1024))) char lds[5u * OPER];
 
         uint32_t tm, tn;
-        if(!r355::tileCoordRange(blockIdx.x, p.tilesM, p.tilesN, p.tileFirst, p.tileCount, p.tileQuad != 0u, tm, tn))
-            return;
-        if(p.tileQuad && (tm * TILE >= p.m || tn * TILE >= p.n))
-            return; // a quarter of a partial edge tile that lies outside the matrix
+        if constexpr(TRIANGLE)
+        {
+            uint32_t sample;
+            if(!triangleCoord(blockIdx.x, p.tilesM, p.tileCount, sample, tm, tn))
+                return;
+            const uint64_t x = (uint64_t)sample * p.m * p.k * ES;
+            p.d += (uint64_t)sample * ((uint64_t)p.k + (uint64_t)p.m * (p.m - 1u) / 2u) * ES;
+            if(tm == 0u) // the bottom-MLP row (k is a multiple of 16: whole 16-byte pieces)
+                for(uint32_t at = threadIdx.x * CHUNK; at < p.k * ES; at += THREADS * CHUNK)
+                    *reinterpret_cast<i32x4*>(p.d + at) = *reinterpret_cast<const i32x4*>(p.a + x + at);
+            p.a += x, p.b += x, p.d += p.k * ES;
+        }
+        else
+        {
+            if(!r355::tileCoordRange(blockIdx.x, p.tilesM, p.tilesN, p.tileFirst, p.tileCount, p.tileQuad != 0u, tm, tn))
+                return;
+            if(p.tileQuad && (tm * TILE >= p.m || tn * TILE >= p.n))
+                return; // a quarter of a partial edge tile that lies outside the matrix
+        }
         staggeredStart(p);
 
         const uint32_t tid  = threadIdx.x;
@@ -1138,7 +1233,10 @@ namespace
         asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
         waitVmcnt<0>();
         ldsBarrier();
-        storeTile16<AccV, OutT, WB, WB>(acc, p, tm * TILE + wm * WT, tn * TILE + wn * WT, lane, lds + wave * (WB * 4096u));
+        if constexpr(TRIANGLE)
+            storeTriangle<OutT, WB>(acc, reinterpret_cast<OutT*>(p.d), p.m, tm * TILE + wm * WT, tn * TILE + wn * WT, lane, lds + wave * (WB * 4096u));
+        else
+            storeTile16<AccV, OutT, WB, WB>(acc, p, tm * TILE + wm * WT, tn * TILE + wn * WT, lane, lds + wave * (WB * 4096u));
         R355_STAMP_END();
     }
 
@@ -1449,6 +1547,20 @@ namespace
     __global__ void __launch_bounds__(THREADS) gemmTiledKernelF64Small(Params p)
     {
         gemmTiled5<Elem::F64, double, A_KCONTIG, B_KCONTIG, 4>(p);
+    }
+    template <Elem E, typename T, uint32_t WB>
+    __global__ void __launch_bounds__(THREADS) dlrmFwdTiled(Params p)
+    {
+        gemmTiled5<E, T, true, true, WB, true>(p);
+    }
+    template <Elem E, typename T>
+    int launchTriangle(const Params& p, uint32_t tile, uint32_t groups, hipStream_t stream)
+    {
+        if(tile == 128u)
+            hipLaunchKernelGGL((dlrmFwdTiled<E, T, 4>), dim3(groups), dim3(THREADS), 0, stream, p);
+        else
+            hipLaunchKernelGGL((dlrmFwdTiled<E, T, 2>), dim3(groups), dim3(THREADS), 0, stream, p);
+        return r355::checkLaunch("dlrm_fwd (macro tile)");
     }
     // The 128 x 128 tile of f16 / bf16 runs the five-buffer body as well: with a stage lasting a quarter as
     // long, the two-buffer scheme of gemmTiled16 keeps too little in flight (2048^3 f16: 710 TFLOP/s against 887
@@ -2090,6 +2202,30 @@ namespace r355
         return checkLaunch("gemm (split-K reduction)");
     }
 
+    int dlrmFwdTiled(int32_t dtype, const void* in, void* out, uint32_t m, uint32_t k, uint32_t batch, uint32_t tile, hipStream_t stream)
+    {
+        GemmTileParams p{};
+        p.m = p.n = m, p.k = p.lda = p.ldb = k;
+        p.tilesM = p.tilesN = (m + tile - 1u) / tile;
+        const uint32_t pairs = p.tilesM * (p.tilesM + 1u) / 2u;
+        const uint64_t es = dtypeBytes(dtype), stride = (uint64_t)k + (uint64_t)m * (m - 1u) / 2u;
+        const uint32_t most = (1u << 30) / pairs; // samples per launch: a grid dimension holds 2^31 workgroups
+        for(uint32_t first = 0; first < batch; first += most)
+        {
+            const uint32_t count = batch - first < most ? batch - first : most;
+            p.a = p.b   = static_cast<const char*>(in) + (uint64_t)first * m * k * es;
+            p.d         = static_cast<char*>(out) + (uint64_t)first * stride * es;
+            p.tileCount = count * pairs;
+            const uint32_t groups = (p.tileCount + 7u) / 8u * 8u;
+            const int      rc     = dtype == R355_F16    ? dlrmFwdTiledPart0(p, tile, groups, stream)
+                                    : dtype == R355_BF16 ? dlrmFwdTiledPart1(p, tile, groups, stream)
+                                                         : dlrmFwdTiledPart3(p, tile, groups, stream);
+            if(rc != R355_OK)
+                return rc;
+        }
+        return R355_OK;
+    }
+
     int gemmTiledCheck(const r355_gemm_args& g, r355_gemm_plan* plan)
     {
         const bool pairOk = (g.in_type == R355_F16 && (g.out_type == R355_F16 || g.out_type == R355_F32))
@@ -2234,6 +2370,10 @@ namespace r355
 #endif // part 0
 
 #if R355_TILED_HAS(0)
+    int dlrmFwdTiledPart0(const GemmTileParams& p, uint32_t tile, uint32_t groups, hipStream_t stream)
+    {
+        return launchTriangle<Elem::F16, _Float16>(p, tile, groups, stream);
+    }
     int gemmTiledPart0(const r355_gemm_args& g, bool aK, bool bK, uint32_t tile, const GemmTileParams& p, hipStream_t stream)
     {
         return g.out_type == R355_F16 ? launchLayouts<Elem::F16, _Float16>(aK, bK, tile, p, stream)
@@ -2241,6 +2381,10 @@ namespace r355
     }
 #endif
 #if R355_TILED_HAS(1)
+    int dlrmFwdTiledPart1(const GemmTileParams& p, uint32_t tile, uint32_t groups, hipStream_t stream)
+    {
+        return launchTriangle<Elem::BF16, __bf16>(p, tile, groups, stream);
+    }
     int gemmTiledPart1(const r355_gemm_args& g, bool aK, bool bK, uint32_t tile, const GemmTileParams& p, hipStream_t stream)
     {
         return g.out_type == R355_BF16 ? launchLayouts<Elem::BF16, __bf16>(aK, bK, tile, p, stream)
@@ -2259,6 +2403,10 @@ namespace r355
     }
 #endif
 #if R355_TILED_HAS(3)
+    int dlrmFwdTiledPart3(const GemmTileParams& p, uint32_t tile, uint32_t groups, hipStream_t stream)
+    {
+        return launchTriangle<Elem::F32, float>(p, tile, groups, stream);
+    }
     int gemmTiledPart3(const r355_gemm_args& g, bool aK, bool bK, uint32_t tile, const GemmTileParams& p, hipStream_t stream)
     {
         return g.in_type == R355_F32 ? launchLayouts<Elem::F32, float>(aK, bK, tile, p, stream)
