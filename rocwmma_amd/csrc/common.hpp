@@ -88,6 +88,9 @@ namespace r355
     int gemmSparseLaunch(const r355_gemm_args& g, hipStream_t stream);
     // DLRM forward on macro tiles of 128 or 64 features (gemm_tiled.hip): m, k multiples of 16, in and out 16-byte aligned
     int dlrmFwdTiled(int32_t dtype, const void* in, void* out, uint32_t m, uint32_t k, uint32_t batch, uint32_t tile, hipStream_t stream);
+    // DLRM backward on macro tiles of 128 or 64 features (gemm_tiled.hip): m, k multiples of 16, every pointer 16-byte aligned
+    int dlrmBwdTiled(int32_t dtype, const void* in, const void* upstream, void* mlpGrad, void* inGrad, uint32_t m, uint32_t k, uint32_t batch,
+                     uint32_t tile, hipStream_t stream);
     // DLRM shapes beyond the specialised kernels (dlrm_general.hip): m, k multiples of 16
     int dlrmGeneralFwd(int32_t dtype, const void* in, void* out, uint32_t m, uint32_t k, uint32_t batch, hipStream_t stream);
     int dlrmGeneralBwd(int32_t dtype, const void* in, const void* upstream, void* mlpGrad, void* inGrad, uint32_t m, uint32_t k,

@@ -6,8 +6,9 @@
 // out of an accumulator block through 1 KiB of the wave's LDS instead of a [batch][m][m] f32 buffer, and the backward
 // kernels form each 16 x 16 block of S = T + T^T in LDS from the packed upstream triangle instead of reconstructing
 // [batch][m][m] in memory first.  These kernels run one 16 x 16 block per wave, as in the reference, and serve small
-// shapes; larger ones go to macro tiles (forward: gemm_tiled.hip) or to a register-blocked kernel (backward: several blocks
-// per wave, so that a fragment feeds several matrix instructions).
+// shapes; larger ones go to macro tiles (gemm_tiled.hip).  Backward launches of many blocks that the macro tiles do not take (up
+// to 16 features, pointers off 16-byte alignment) go to a register-blocked kernel: several blocks per wave, so that a fragment
+// feeds several matrix instructions.
 #include <rocwmma/rocwmma.hpp>
 
 #include "common.hpp"
@@ -337,6 +338,25 @@ namespace
         return es == 2u && tiles * (tiles + 1u) / 2u * batch * stages >= 16u * cus ? 128u : 64u;
     }
 
+    // Backward: the macro tile's edge (dlrmBwdTiled in gemm_tiled.hip), or 0 for the fragment-API kernels below.  Measured on one
+    // box, 45 shapes (m 48 ... 1024, k 64 ... 1024), against those kernels' 16 x 16 blocks per wave: the 64 x 64 tile is ahead by 1.05
+    // (112 x 800 x 436 bf16: 70.5 -> 61.8 us) to 10 times (1024 x 256 x 4 f16: 96 -> 10.5), and level only where the call itself
+    // is the time (48 x 1024 x 4) and at 80 x 256 x 537 (20.3 / 20.6).  The 128 x 128 tile loads half the bytes per product and is
+    // ahead from 768 features on where it fills the chip (1024 x 1024 x 64 f16: 295 -> 214 us, f32 1024 x 1024 x 16: 295 -> 271;
+    // 880 x 240 x 21: level; 512 x 480 x 41 f32: 107 against 113).  Up to 16 features a tile would be three quarters padding.
+    // The kernel reads upstream and writes mlpGrad in 16-byte pieces; rows beyond 8 MiB do not fit its 32-bit lane offsets.
+    uint32_t backwardTile(int32_t dtype, const void* upstream, const void* mlpGrad, uint32_t m, uint32_t k, uint32_t batch)
+    {
+#ifdef R355_DLRM_BLOCK_PER_WAVE
+        return 0u;
+#endif
+        const uint64_t es = r355::dtypeBytes(dtype);
+        if(m <= BLK || (uint64_t)k * es > (1u << 23) || !r355::aligned(upstream, 16) || !r355::aligned(mlpGrad, 16))
+            return 0u;
+        const uint64_t tiles = (uint64_t)((m + 127u) / 128u) * ((k + 127u) / 128u);
+        return m >= 768u && tiles * batch >= 2u * r355::computeUnits() ? 128u : 64u;
+    }
+
     template <typename T>
     int fwd(const void* in, void* out, uint32_t m, uint32_t k, uint32_t batch, hipStream_t s)
     {
@@ -415,6 +435,8 @@ namespace r355
         const int rc = checkGeneral("dlrm_bwd", m, k, batch);
         if(rc != R355_OK)
             return rc;
+        if(const uint32_t tile = backwardTile(dtype, upstream, mlpGrad, m, k, batch))
+            return dlrmBwdTiled(dtype, in, upstream, mlpGrad, inGrad, m, k, batch, tile, s);
         switch(dtype)
         {
         case R355_F16: return bwd<float16_t>(in, upstream, mlpGrad, inGrad, m, k, batch, s);

@@ -133,6 +133,16 @@ namespace r355
     int dlrmFwdTiledPart0(const GemmTileParams& p, uint32_t tile, uint32_t groups, hipStream_t s);
     int dlrmFwdTiledPart1(const GemmTileParams& p, uint32_t tile, uint32_t groups, hipStream_t s);
     int dlrmFwdTiledPart3(const GemmTileParams& p, uint32_t tile, uint32_t groups, hipStream_t s);
+    // DLRM backward on macro tiles of S X (dlrmBwdTile below), one per element type
+    struct DlrmBwdParams
+    {
+        uint32_t    m, k, tilesM, tilesN, total; // total: tiles of all samples of the launch
+        const char *x, *up;
+        char *      mlp, *grad;
+    };
+    int dlrmBwdTiledPart0(const DlrmBwdParams& p, uint32_t tile, hipStream_t s);
+    int dlrmBwdTiledPart1(const DlrmBwdParams& p, uint32_t tile, hipStream_t s);
+    int dlrmBwdTiledPart3(const DlrmBwdParams& p, uint32_t tile, hipStream_t s);
 } // namespace r355
 
 namespace
@@ -1562,6 +1572,229 @@ namespace
             hipLaunchKernelGGL((dlrmFwdTiled<E, T, 2>), dim3(groups), dim3(THREADS), 0, stream, p);
         return r355::checkLaunch("dlrm_fwd (macro tile)");
     }
+    // ------------------------------------------------------------------------------------------
+    // DLRM backward on macro tiles: the gradient S X of every sample of a batch, S = T + T^T formed from the packed strict lower
+    // triangle T (upstream gradient), X [m][k] row-major.  A workgroup owns TILE x TILE of one sample's gradient.
+    //   * B = X is the macro-tile GEMM's N-contiguous operand: direct loads, transposing reads.
+    //   * A = S lies in memory as rows of T that start at any element.  Left of the diagonal tile a stage is TILE rows x 128 bytes
+    //     of T (the K-contiguous image); right of it S(i, j) = T(j, i), so a stage is 128 bytes' worth of rows of T, TILE
+    //     elements each (the M-contiguous image, transposing reads): the same 16-byte pieces at unaligned addresses either way,
+    //     through registers into the image.  The stages of the diagonal tile itself are gathered element by element.
+    //   * two buffers per operand; the loads of stage kt + 1 are in flight under the matrix instructions of stage kt, and what
+    //     that leaves exposed other workgroups of the CU cover (two of the 128 x 128 tile, four of the 64 x 64 one).
+    // S holds zeros only on its diagonal and beyond row or column m, as the products of the [m][m] matrix have them.  Few stages bound
+    // the small shapes (latency of one stage's loads each), the matrix instructions and the loads' distance the large ones:
+    // f16 1024 x 1024 x 64 473 -> 214 us (640 TFLOP/s), bf16 320 x 192 x 96 26.7 -> 15.0, f32 224 x 384 x 213 141 -> 95.
+    using BwdParams = r355::DlrmBwdParams;
+
+    template <Elem E, typename T, uint32_t WB>
+    __device__ __forceinline__ void dlrmBwdTile(const BwdParams& p)
+    {
+        constexpr uint32_t ES = ElemTraits<E>::Bytes, TILE = 32u * WB, WT = 16u * WB, OPER = TILE * STAGE_KB;
+        constexpr uint32_t TK = STAGE_KB / ES, EPC = CHUNK / ES; // K elements per stage, elements per 16-byte piece
+        using Word            = std::conditional_t<ES == 2, uint16_t, uint32_t>;
+        typedef int i32x4u __attribute__((ext_vector_type(4), aligned(2)));
+        __shared__ __attribute__((aligned(1024))) char lds[4u * OPER];
+        constexpr uint32_t B_AT = 2u * OPER; // two buffers of A, then two of B
+
+        // all workgroups of an XCD walk one contiguous run of (sample, tile): the tiles of a sample share its X and T in one L2
+        const uint32_t perXcd = (p.total + 7u) / 8u, slotX = blockIdx.x / 8u, local = (blockIdx.x % 8u) * perXcd + slotX;
+        if(slotX >= perXcd || local >= p.total)
+            return;
+        const uint32_t tiles = p.tilesM * p.tilesN, sample = local / tiles, rest = local % tiles;
+        const uint32_t tm = rest / p.tilesN, tn = rest % p.tilesN;
+        const uint64_t xAt = (uint64_t)sample * p.m * p.k * ES;
+        const char*    up  = p.up + (uint64_t)sample * ((uint64_t)p.k + (uint64_t)p.m * (p.m - 1u) / 2u) * ES;
+        const uint32_t tid = threadIdx.x, lane = tid & 63u;
+        const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1u;
+        const uint32_t row0 = tm * TILE, col0 = tn * TILE;
+        if(tm == 0u) // bottom-MLP gradient: the first k values of the upstream row, this tile's columns of them
+        {
+            const uint32_t bytes = (p.k - col0 < TILE ? p.k - col0 : TILE) * ES, at = tid * CHUNK;
+            if(at < bytes)
+                *reinterpret_cast<i32x4*>(p.mlp + ((uint64_t)sample * p.k + col0) * ES + at)
+                    = *reinterpret_cast<const i32x4*>(up + (uint64_t)col0 * ES + at);
+        }
+        const Word* tril = reinterpret_cast<const Word*>(up + (uint64_t)p.k * ES);
+
+        const uint32_t ldsBase = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds));
+        const uint32_t dmaDst  = ldsBase + wave * 64u * CHUNK;
+        uint32_t       gOffB[WB], gStepB, kByteB;
+        uint64_t       gStageB;
+        laneOffsets8<false, WB, ES>(tid, p.k, p.k - col0 < TILE ? p.k - col0 : TILE, gOffB, gStepB, gStageB, kByteB);
+        const uint64_t gB        = r355::uniformAddress(p.x + xAt + (uint64_t)col0 * ES);
+        const uint32_t numStages = (p.m + TK - 1u) / TK;
+        auto           issueB    = [&](uint32_t st, uint32_t at) { // rows of X past the last one arrive as zeros
+            const uint32_t left = (p.m - st * TK) * ES;
+            const i32x4    rsrc = stageRsrc8(false, gB + st * gStageB, left < STAGE_KB ? left : STAGE_KB, p.k);
+#pragma unroll
+            for(uint32_t j = 0; j < WB; ++j)
+                loadToLds(rsrc, gOffB[j], j * gStepB, dmaDst + at + j * THREADS * CHUNK);
+        };
+
+        // A: stages [0, diagFirst) left of the diagonal tile, [diagFirst, diagEnd) in it, [diagEnd, numStages) right of it
+        const uint32_t diagFirst = row0 / TK, diagEnd = diagFirst + TILE / TK < numStages ? diagFirst + TILE / TK : numStages;
+        const uint32_t rK = tid >> 3, cK = ((tid & 7u) ^ swzK8(tid >> 3)) * EPC; // K-contiguous image: row rK + 32 j, first column of the piece
+        i32x4          aNext[WB];
+        auto           loadRight = [&](uint32_t st) {
+            constexpr uint32_t SLOTS = 2u * WB * ES, KROWS = THREADS / SLOTS;
+#pragma unroll
+            for(uint32_t j = 0; j < WB; ++j)
+            {
+                const uint32_t kr = KROWS * j + tid / SLOTS, c = ((tid % SLOTS) ^ swzMN8<WB, ES>(kr)) * EPC;
+                const uint64_t gj = st * TK + kr;
+                aNext[j]          = i32x4{0, 0, 0, 0};
+                if(gj < p.m) // (then columns up to the end of the diagonal tile lie left of T's diagonal: inside the row)
+                    aNext[j] = *reinterpret_cast<const i32x4u*>(tril + (gj * (gj - 1u) / 2u + row0 + c));
+            }
+        };
+        auto loadA = [&](uint32_t st) {
+            const uint32_t k0 = st * TK;
+            if(st < diagFirst)
+            {
+#pragma unroll
+                for(uint32_t j = 0; j < WB; ++j) // (a row past the last one reads the last: its products are not stored)
+                {
+                    const uint64_t gi = row0 + rK + 32u * j < p.m ? row0 + rK + 32u * j : p.m - 1u;
+                    aNext[j]          = *reinterpret_cast<const i32x4u*>(tril + (gi * (gi - 1u) / 2u + k0 + cK));
+                }
+            }
+            else if(st >= diagEnd)
+                loadRight(st);
+            else
+            {
+#pragma unroll
+                for(uint32_t j = 0; j < WB; ++j)
+                {
+                    const uint32_t gi = row0 + rK + 32u * j;
+                    Word           w[EPC];
+#pragma unroll
+                    for(uint32_t e = 0; e < EPC; ++e)
+                    {
+                        const uint32_t gj = k0 + cK + e;
+                        const uint64_t hi = gi > gj ? gi : gj, lo = gi > gj ? gj : gi;
+                        w[e]              = hi < p.m && gi != gj ? tril[hi * (hi - 1u) / 2u + lo] : Word(0);
+                    }
+                    if constexpr(ES == 2)
+                    {
+#pragma unroll
+                        for(uint32_t e = 0; e < 4; ++e)
+                            aNext[j][e] = static_cast<int>(w[2u * e] | (static_cast<uint32_t>(w[2u * e + 1u]) << 16));
+                    }
+                    else
+                    {
+#pragma unroll
+                        for(uint32_t e = 0; e < 4; ++e)
+                            aNext[j][e] = static_cast<int>(w[e]);
+                    }
+                }
+            }
+        };
+        auto writeA = [&](uint32_t at) { // (both images take piece j * 256 + tid at byte 16 of that)
+#pragma unroll
+            for(uint32_t j = 0; j < WB; ++j)
+                *reinterpret_cast<i32x4*>(lds + at + (j * THREADS + tid) * CHUNK) = aNext[j];
+        };
+
+        uint32_t rdAK[8], rdAM[8], rdB[8];
+        readOffsets8<true, WB, ES>(wm, lane, rdAK);
+        readOffsets8<false, WB, ES>(wm, lane, rdAM);
+        readOffsets8<false, WB, ES>(wn, lane, rdB);
+        f32x4 acc[WB][WB];
+#pragma unroll
+        for(uint32_t i = 0; i < WB; ++i)
+#pragma unroll
+            for(uint32_t j = 0; j < WB; ++j)
+                acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        // Builtins, not inline assembly: between its loops the compiler may copy accumulators, and it has to know that the last
+        // instructions' results are late.
+        auto multiply = [](f32x4& c, i32x4 x, i32x4 y) {
+            if constexpr(E == Elem::F16)
+                c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, x), __builtin_bit_cast(f16x8, y), c, 0, 0, 0);
+            else if constexpr(E == Elem::BF16)
+                c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x), __builtin_bit_cast(bf16x8, y), c, 0, 0, 0);
+            else
+            {
+#pragma unroll
+                for(uint32_t e = 0; e < 4; ++e)
+                {
+                    const int xe = x[e], ye = y[e]; // (a bit cast of the vector element itself takes element 0)
+                    c = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, xe), __builtin_bit_cast(float, ye), c, 0, 0, 0);
+                }
+            }
+        };
+        auto compute = [&](auto aK, uint32_t aAt, uint32_t bAt) {
+            constexpr bool AK = decltype(aK)::value;
+            i32x4          fa[2][WB], fb[2][WB];
+#pragma unroll
+            for(uint32_t s = 0; s < 2; ++s)
+#pragma unroll
+                for(uint32_t i = 0; i < WB; ++i)
+#pragma unroll
+                    for(uint32_t part = 0; part < 2; ++part)
+                    {
+                        readBlock8<AK, WB, ES>(lds + aAt, AK ? rdAK : rdAM, i, s, part, fa[s][i], 0u);
+                        readBlock8<false, WB, ES>(lds + bAt, rdB, i, s, part, fb[s][i], 0u);
+                    }
+#pragma unroll
+            for(uint32_t s = 0; s < 2; ++s)
+#pragma unroll
+                for(uint32_t i = 0; i < WB; ++i)
+#pragma unroll
+                    for(uint32_t j = 0; j < WB; ++j)
+                        multiply(acc[i][j], fb[s][j], fa[s][i]); // (operands swapped, as everywhere here)
+        };
+
+        issueB(0u, B_AT);
+        loadA(0u);
+        writeA(0u);
+        waitVmcnt<0>();
+        ldsBarrier();
+        auto stageBody = [&](auto aK, uint32_t st) {
+            const uint32_t cur = (st & 1u) * OPER, nxt = OPER - cur;
+            const bool     more = st + 1u < numStages; // (uniform)
+            if(more)
+            {
+                issueB(st + 1u, B_AT + nxt);
+                if constexpr(decltype(aK)::value)
+                    loadA(st + 1u);
+                else
+                    loadRight(st + 1u);
+            }
+            compute(aK, cur, B_AT + cur);
+            if(more)
+                writeA(nxt);
+            // the direct loads of the next stage have landed, and every wave has read this one
+            waitVmcnt<0>();
+            ldsBarrier();
+        };
+        uint32_t st = 0;
+        for(; st < diagEnd; ++st)
+            stageBody(std::true_type{}, st);
+        for(; st < numStages; ++st)
+            stageBody(std::false_type{}, st);
+        Params d{};
+        d.m = p.m, d.n = p.k, d.ldd = p.k;
+        d.d     = p.grad + xAt;
+        d.alpha = 1.0;
+        storeTileStaged<T, false, f32x4, T, WB, WB, WB * 4096u>(acc, d, row0 + wm * WT, col0 + wn * WT, lane, lds + wave * (WB * 4096u));
+    }
+    template <Elem E, typename T, uint32_t WB>
+    __global__ void __launch_bounds__(THREADS, 2) dlrmBwdTiled(BwdParams p)
+    {
+        dlrmBwdTile<E, T, WB>(p);
+    }
+    template <Elem E, typename T>
+    int launchBwdTiled(const BwdParams& p, uint32_t tile, hipStream_t stream)
+    {
+        const uint32_t groups = (p.total + 7u) / 8u * 8u;
+        if(tile == 128u)
+            hipLaunchKernelGGL((dlrmBwdTiled<E, T, 4>), dim3(groups), dim3(THREADS), 0, stream, p);
+        else
+            hipLaunchKernelGGL((dlrmBwdTiled<E, T, 2>), dim3(groups), dim3(THREADS), 0, stream, p);
+        return r355::checkLaunch("dlrm_bwd (macro tiles)");
+    }
+
     // The 128 x 128 tile of f16 / bf16 runs the five-buffer body as well: with a stage lasting a quarter as
     // long, the two-buffer scheme of gemmTiled16 keeps too little in flight (2048^3 f16: 710 TFLOP/s against 887
     // here).  For the 256 x 256 tile the two-buffer kernel stays 1-2 % ahead (it is power-bound, not latency-bound).
@@ -2226,6 +2459,36 @@ namespace r355
         return R355_OK;
     }
 
+    int dlrmBwdTiled(int32_t dtype, const void* in, const void* upstream, void* mlpGrad, void* inGrad, uint32_t m, uint32_t k, uint32_t batch,
+                     uint32_t tile, hipStream_t stream)
+    {
+        DlrmBwdParams p{};
+        p.m = m, p.k = k;
+        p.tilesM = (m + tile - 1u) / tile, p.tilesN = (k + tile - 1u) / tile;
+        const uint64_t es = dtypeBytes(dtype), stride = (uint64_t)k + (uint64_t)m * (m - 1u) / 2u;
+        const uint64_t tiles = (uint64_t)p.tilesM * p.tilesN;
+        if(tiles > 1u << 30)
+            return fail(R355_ERR_BAD_SIZE, "dlrm_bwd: m=%u, k=%u: too many tiles of a sample", m, k);
+        const uint32_t most = (1u << 30) / static_cast<uint32_t>(tiles); // samples per launch: a grid dimension holds 2^31 workgroups
+        for(uint32_t first = 0; first < batch; first += most)
+        {
+            const uint32_t count = batch - first < most ? batch - first : most;
+            p.x     = static_cast<const char*>(in) + (uint64_t)first * m * k * es;
+            p.up    = static_cast<const char*>(upstream) + (uint64_t)first * stride * es;
+            p.mlp   = static_cast<char*>(mlpGrad) + (uint64_t)first * k * es;
+            p.grad  = static_cast<char*>(inGrad) + (uint64_t)first * m * k * es;
+            p.total = count * static_cast<uint32_t>(tiles);
+            const int rc = dtype == R355_F16    ? dlrmBwdTiledPart0(p, tile, stream)
+                           : dtype == R355_BF16 ? dlrmBwdTiledPart1(p, tile, stream)
+                                                : dlrmBwdTiledPart3(p, tile, stream);
+            if(rc != R355_OK)
+                return rc;
+            if(batch - first <= most)
+                break; // (first + most may pass 2^32)
+        }
+        return R355_OK;
+    }
+
     int gemmTiledCheck(const r355_gemm_args& g, r355_gemm_plan* plan)
     {
         const bool pairOk = (g.in_type == R355_F16 && (g.out_type == R355_F16 || g.out_type == R355_F32))
@@ -2374,6 +2637,10 @@ namespace r355
     {
         return launchTriangle<Elem::F16, _Float16>(p, tile, groups, stream);
     }
+    int dlrmBwdTiledPart0(const DlrmBwdParams& p, uint32_t tile, hipStream_t stream)
+    {
+        return launchBwdTiled<Elem::F16, _Float16>(p, tile, stream);
+    }
     int gemmTiledPart0(const r355_gemm_args& g, bool aK, bool bK, uint32_t tile, const GemmTileParams& p, hipStream_t stream)
     {
         return g.out_type == R355_F16 ? launchLayouts<Elem::F16, _Float16>(aK, bK, tile, p, stream)
@@ -2384,6 +2651,10 @@ namespace r355
     int dlrmFwdTiledPart1(const GemmTileParams& p, uint32_t tile, uint32_t groups, hipStream_t stream)
     {
         return launchTriangle<Elem::BF16, __bf16>(p, tile, groups, stream);
+    }
+    int dlrmBwdTiledPart1(const DlrmBwdParams& p, uint32_t tile, hipStream_t stream)
+    {
+        return launchBwdTiled<Elem::BF16, __bf16>(p, tile, stream);
     }
     int gemmTiledPart1(const r355_gemm_args& g, bool aK, bool bK, uint32_t tile, const GemmTileParams& p, hipStream_t stream)
     {
@@ -2406,6 +2677,10 @@ namespace r355
     int dlrmFwdTiledPart3(const GemmTileParams& p, uint32_t tile, uint32_t groups, hipStream_t stream)
     {
         return launchTriangle<Elem::F32, float>(p, tile, groups, stream);
+    }
+    int dlrmBwdTiledPart3(const DlrmBwdParams& p, uint32_t tile, hipStream_t stream)
+    {
+        return launchBwdTiled<Elem::F32, float>(p, tile, stream);
     }
     int gemmTiledPart3(const r355_gemm_args& g, bool aK, bool bK, uint32_t tile, const GemmTileParams& p, hipStream_t stream)
     {

@@ -29,3 +29,36 @@ def test_forward_on_macro_tiles(dtype, m, k, batch):
     out = to_host(dout, store)
     assert np.all(out[batch * stride:].view(np.uint8) == 0xEE)  # nothing behind the last row
     assert np.array_equal(out[:batch * stride].view(np.uint8), O.dlrm_fwd(dtype, x, m, k, batch).ravel().view(np.uint8))
+
+
+# backward: one tile and several, so that stages left of, in and right of the diagonal tile all occur, partial tiles and K stages,
+# widths off the tile's edge, samples spread unevenly over the XCDs; shapes for both macro tiles and for the kernels below them
+@pytest.mark.parametrize("dtype", [O.F16, O.BF16, O.F32])
+@pytest.mark.parametrize("m,k,batch", [(16, 80, 9), (32, 176, 5), (48, 272, 3), (64, 16, 700), (80, 80, 41), (128, 384, 2), (144, 448, 17), (272, 96, 33),
+                                       (336, 272, 40), (400, 144, 3), (528, 272, 24)])
+def test_backward_on_macro_tiles(dtype, m, k, batch):
+    store, stride = O.NP_STORAGE[dtype], k + m * (m - 1) // 2
+    x, up = _small_integers(21 + m, batch * m * k, dtype), _small_integers(22 + m, batch * stride, dtype)
+    dmlp, dgrad = device_filled(batch * k + 8, store, 0xEE), device_filled(batch * m * k + 8, store, 0xEE)
+    R.dlrm_bwd(dtype, to_device(x), to_device(up), dmlp, dgrad, m, k, batch)
+    mlp, grad = to_host(dmlp, store), to_host(dgrad, store)
+    assert np.all(mlp[batch * k:].view(np.uint8) == 0xEE) and np.all(grad[batch * m * k:].view(np.uint8) == 0xEE)
+    want_mlp, want_grad = O.dlrm_bwd(dtype, x, up, m, k, batch)
+    assert np.array_equal(mlp[:batch * k].view(np.uint8), want_mlp.ravel().view(np.uint8))
+    g, w = grad[:batch * m * k], want_grad.ravel()  # (values: -0.0 and +0.0 are the same gradient)
+    if dtype != O.F32:
+        g, w = O.storage_to_f32(g, dtype), O.storage_to_f32(w, dtype)
+    assert np.array_equal(g, w)
+
+
+def test_backward_with_an_upstream_off_16_bytes():
+    """upstream at 2 bytes past a 16-byte boundary: taken by the kernels that read single elements, as ever."""
+    m, k, batch, dtype = 80, 80, 3, O.F16
+    store, stride = O.NP_STORAGE[dtype], k + m * (m - 1) // 2
+    x, up = _small_integers(1, batch * m * k, dtype), _small_integers(2, batch * stride, dtype)
+    held = to_device(np.concatenate([np.zeros(1, store), up]))
+    dmlp, dgrad = device_filled(batch * k, store, 0xEE), device_filled(batch * m * k, store, 0xEE)
+    R.dlrm_bwd(dtype, to_device(x), held.data_ptr() + 2, dmlp, dgrad, m, k, batch)
+    want_mlp, want_grad = O.dlrm_bwd(dtype, x, up, m, k, batch)
+    assert np.array_equal(to_host(dmlp, store).view(np.uint8), want_mlp.ravel().view(np.uint8))
+    assert np.array_equal(O.storage_to_f32(to_host(dgrad, store), dtype), O.storage_to_f32(want_grad.ravel(), dtype))
