@@ -129,7 +129,8 @@ int r355_gemm(const r355_gemm_args* args, void* stream);
  * (the values the reference computes on the host: samples/perf_hgemm.cpp:807-817).
  * R355_KERNEL_AUTO may split a problem of several rounds of 256 x 256 tiles into two launches on the
  * same stream - whole rounds on that tile, the rest (at most half a round) on 128 x 128 tiles; the
- * plan then describes the first launch.  It may also work a problem of 128 x 128 tiles as 64 x 64 quarters of them
+ * plan then describes the first launch.  16-bit and int8 problems may run as one launch of tiles of 224 or 192 rows (columns
+ * of a col-major D) by 256 instead, where a timing model prices that as faster.  It may also work a problem of 128 x 128 tiles as 64 x 64 quarters of them
  * (R355_KERNEL_TILED_64: four workgroups of a quarter of the LDS per tile) and with fewer K splits than planned, where
  * a timing model prices that as faster; the plan then describes the 128 x 128 tiling and the most workspace a launch uses. */
 typedef struct

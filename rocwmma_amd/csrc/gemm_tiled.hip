@@ -7,7 +7,8 @@
 // and eight matrix instructions per wave between barriers; this one is shaped for
 // MI355X's 160 KB LDS and 256 CUs:
 //
-//   macro tile   256 x 256, K stage of 128 bytes (64 f16/bf16, 128 int8/fp8 elements); 128 x 128 (wave tile
+//   macro tile   256 x 256 (16-bit, int8: also 224 x 256 and 192 x 256), K stage of 128 bytes (64 f16/bf16, 128 int8/fp8
+//                elements); 128 x 128 (wave tile
 //                64 x 64, five 16 KiB LDS buffers, two workgroups per CU) for problems with too few large tiles
 //   workgroup    256 threads = 4 waves in a 2 x 2 grid, wave tile 128 x 128
 //                = 8 x 8 accumulators of the 16 x 16 matrix-instruction shapes (256 registers):
@@ -124,7 +125,7 @@ namespace r355
     };
     // sum of `splits` partial results (accumulator type: f32, i32 or f64) + the alpha / beta epilogue into the output type
     int splitKReduce(const r355_gemm_args& g, const GemmTileParams& p, uint32_t splits, hipStream_t stream);
-    // launch of one kernel family; aK / bK: operand is K-contiguous; tile: 256 or 128
+    // launch of one kernel family; aK / bK: operand is K-contiguous; tile: 256, 128 or 64, or the rows of a tile of 256 columns (224, 192)
     int gemmTiledPart0(const r355_gemm_args& g, bool aK, bool bK, uint32_t tile, const GemmTileParams& p, hipStream_t s);
     int gemmTiledPart1(const r355_gemm_args& g, bool aK, bool bK, uint32_t tile, const GemmTileParams& p, hipStream_t s);
     int gemmTiledPart2(const r355_gemm_args& g, bool aK, bool bK, uint32_t tile, const GemmTileParams& p, hipStream_t s);
@@ -292,6 +293,15 @@ namespace
         return kContig && kByte >= valid ? 0x80000000u : laneOffset;
     }
 
+    // the largest divisor of n that is at most `most`
+    constexpr uint32_t divisorUpTo(uint32_t n, uint32_t most)
+    {
+        uint32_t d = most < n ? most : n;
+        while(n % d)
+            --d;
+        return d;
+    }
+
     // D = alpha * acc + beta * C for one wave's tile of WB x WB accumulator blocks (16 x 16 each), row-major;
     // the wave tile starts at (m0, n0).  `scratch` is WB * 4 KiB of LDS owned by this wave.
     //
@@ -323,10 +333,10 @@ namespace
         // rows per pass: what the scratch holds, halved where a pass's part of C would take 128 registers
         constexpr uint32_t FIT_ALL    = SCRATCH / ROW_BYTES;
         constexpr uint32_t FIT        = FIT_ALL / ((WITH_C && FIT_ALL * ROW_CHUNKS / 64u * OUT_WORDS >= 128u) ? 2u : 1u);
-        constexpr uint32_t ROWS_PASS  = FIT < 16u * WBM ? FIT : 16u * WBM;
-        constexpr uint32_t BLOCKS_I   = ROWS_PASS / 16u; // row blocks per pass
+        constexpr uint32_t BLOCKS_I   = divisorUpTo(WBM, FIT / 16u); // row blocks per pass
+        constexpr uint32_t ROWS_PASS  = 16u * BLOCKS_I;
         constexpr uint32_t ITERS      = ROWS_PASS * ROW_CHUNKS / 64u; // chunks per lane and pass
-        constexpr uint32_t BATCH      = ITERS < 8u ? ITERS : 8u;
+        constexpr uint32_t BATCH      = divisorUpTo(ITERS, 8u);
         constexpr int      NT         = 2; // cache policy of the raw buffer accesses: nontemporal (C is read, D written, once)
         static_assert(EPC * OS % 4u == 0u && ITERS % BATCH == 0u, "whole words per lane, whole batches per pass");
 
@@ -968,11 +978,12 @@ namespace
 
     // TRIANGLE: not a GEMM but the DLRM dot interaction, X X^T of every sample of a batch (p.a: [batch][m][k], lda = k) with its
     // strict lower triangle packed behind the sample's first row (p.d: [batch][k + m (m - 1) / 2]); tileCount = batch x tiles.
-    template <Elem E, typename OutT, bool A_KCONTIG, bool B_KCONTIG, uint32_t WB, bool TRIANGLE = false>
+    template <Elem E, typename OutT, bool A_KCONTIG, bool B_KCONTIG, uint32_t WB, bool TRIANGLE = false, uint32_t WM = WB>
     __device__ __forceinline__ void gemmTiled5(const Params& whole)
     {
         static_assert(WB == 8 || WB == 4 || WB == 2, "wave tile of 8 x 8, 4 x 4 or 2 x 2 blocks");
         static_assert(E != Elem::F64 || WB <= 4, "f64 accumulators of an 8 x 8 wave tile would need 512 registers");
+        static_assert(WM == WB || (WB == 8 && !TRIANGLE && (WM == 7 || WM == 6) && ElemTraits<E>::Bytes <= 2), "narrower tiles of 8- and 16-bit operands");
         static_assert(E != Elem::E4M3 && E != Elem::E5M2, "fp8 has its own stage structure");
         R355_STAMP(0);
         R355_STAMP_ID();
@@ -981,9 +992,11 @@ namespace
         Params p = splitShare<ES>(whole, A_KCONTIG ? (uint64_t)STAGE_KB : (uint64_t)STAGE_KB * whole.lda,
                                   B_KCONTIG ? (uint64_t)STAGE_KB : (uint64_t)STAGE_KB * whole.ldb);
         using AccV            = std::conditional_t<E == Elem::I8, i32x4v, std::conditional_t<E == Elem::F64, f64x4, f32x4>>;
-        constexpr uint32_t TILE = 32u * WB, WT = 16u * WB; // macro tile and wave tile edge
-        constexpr uint32_t OPER = TILE * STAGE_KB; // bytes of one operand per stage: 32 or 16 KiB
-        constexpr uint32_t XS = 2u * WB, QS = WB / 2u; // operand blocks per K step, matrix instructions per block
+        constexpr uint32_t TILE_R = 32u * WM, TILE = 32u * WB, WTR = 16u * WM, WT = 16u * WB; // rows and columns of macro and wave tile
+        constexpr uint32_t OPER = TILE * STAGE_KB; // bytes of one operand's buffer: 32, 16 or 8 KiB
+        constexpr uint32_t LA = A_KCONTIG ? WM : WB, LB = WB; // direct loads per stage (32 rows of a K-contiguous tile each)
+        constexpr uint32_t XS = WM + WB, NS = WM * WB; // operand blocks and matrix instructions per K step
+        constexpr uint32_t QS = WB / 2u;
         constexpr uint32_t LOAD_Q = QS > 2u ? 2u : QS - 1u;
         // LDS map: A buffers at 0 and OPER, B buffers at 2, 3 and 4 OPER
         constexpr uint32_t A_AT[2] = {0u, OPER};
@@ -1007,7 +1020,7 @@ namespace
         {
             if(!r355::tileCoordRange(blockIdx.x, p.tilesM, p.tilesN, p.tileFirst, p.tileCount, p.tileQuad != 0u, tm, tn))
                 return;
-            if(p.tileQuad && (tm * TILE >= p.m || tn * TILE >= p.n))
+            if(p.tileQuad && (tm * TILE_R >= p.m || tn * TILE >= p.n))
                 return; // a quarter of a partial edge tile that lies outside the matrix
         }
         staggeredStart(p);
@@ -1019,9 +1032,9 @@ namespace
         const uint32_t ldsBase
             = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds));
 
-        uint32_t       gOffA[WB], gOffB[WB], gStepA, gStepB, kByteA, kByteB; // WB direct loads per operand per stage
+        uint32_t       gOffA[WB], gOffB[WB], gStepA, gStepB, kByteA, kByteB; // LA and LB direct loads per stage
         uint64_t       gStageA, gStageB;
-        const uint32_t validM = p.m - tm * TILE < TILE ? p.m - tm * TILE : TILE;
+        const uint32_t validM = p.m - tm * TILE_R < TILE_R ? p.m - tm * TILE_R : TILE_R;
         const uint32_t validN = p.n - tn * TILE < TILE ? p.n - tn * TILE : TILE;
         laneOffsets8<A_KCONTIG, WB, ES>(tid, p.lda, validM, gOffA, gStepA, gStageA, kByteA);
         laneOffsets8<B_KCONTIG, WB, ES>(tid, p.ldb, validN, gOffB, gStepB, gStageB, kByteB);
@@ -1039,38 +1052,39 @@ namespace
             const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
             return (static_cast<uint64_t>(hi) << 32) | lo;
         };
-        const uint64_t gA = uniform64(p.a + (A_KCONTIG ? (uint64_t)tm * TILE * p.lda : (uint64_t)tm * TILE) * ES);
+        const uint64_t gA = uniform64(p.a + (A_KCONTIG ? (uint64_t)tm * TILE_R * p.lda : (uint64_t)tm * TILE_R) * ES);
         const uint64_t gB = uniform64(p.b + (B_KCONTIG ? (uint64_t)tn * TILE * p.ldb : (uint64_t)tn * TILE) * ES);
         auto stageAddr = [&](uint64_t panel, uint64_t perStage, uint32_t stage) { // clamped to the last stage
             return panel + (uint64_t)(stage < numStages ? stage : numStages - 1u) * perStage;
         };
-        auto issueHalf = [&](bool kContig, uint64_t addr, const uint32_t (&gOff)[WB], uint32_t step, uint32_t kByte, uint32_t ld,
+        auto issueHalf = [&](uint32_t loads, bool kContig, uint64_t addr, const uint32_t (&gOff)[WB], uint32_t step, uint32_t kByte, uint32_t ld,
                              uint32_t valid, uint32_t at) {
             const i32x4 rsrc = stageRsrc8(kContig, addr, valid, ld);
 #pragma unroll
-            for(uint32_t j = 0; j < WB; ++j)
+            for(uint32_t j = 0; j < loads; ++j)
                 loadToLds(rsrc, tailOffset(kContig, gOff[j], kByte, valid), j * step, dmaDst + at + j * THREADS * CHUNK);
         };
 
         uint32_t rdA[8], rdB[8];
-        readOffsets8<A_KCONTIG, WB, ES>(wm, lane, rdA);
+        readOffsets8<A_KCONTIG, WB, ES, WM>(wm, lane, rdA);
         readOffsets8<B_KCONTIG, WB, ES>(wn, lane, rdB);
 
-        AccV acc[WB][WB];
+        AccV acc[WM][WB];
 #pragma unroll
-        for(uint32_t i = 0; i < WB; ++i)
+        for(uint32_t i = 0; i < WM; ++i)
 #pragma unroll
             for(uint32_t j = 0; j < WB; ++j)
                 acc[i][j] = AccV{0, 0, 0, 0};
 
-        i32x4 fa[2][WB], fb[2][WB];
+        i32x4 fa[2][WM], fb[2][WB];
         // matrix instruction n of a K step: L-shaped shells, as in gemmTiledKernel16
         auto mfmaAt = [&](uint32_t s, uint32_t n) {
             uint32_t d = 0;
             while((d + 1u) * (d + 1u) <= n)
                 ++d;
-            const uint32_t r = n - d * d;
-            const uint32_t i = r <= d ? d : r - d - 1u, j = r <= d ? r : d;
+            const uint32_t r = n - d * d, past = n - WM * WM; // (columns beyond the square: one after the other)
+            const uint32_t i = n >= WM * WM ? past % WM : r <= d ? d : r - d - 1u;
+            const uint32_t j = n >= WM * WM ? WM + past / WM : r <= d ? r : d;
             if constexpr(E == Elem::I8)
                 mfma16i8(acc[i][j], fb[s][j], fa[s][i]);
             else if constexpr(E == Elem::F32)
@@ -1080,10 +1094,11 @@ namespace
             else
                 mfma16<E>(acc[i][j], fb[s][j], fa[s][i]);
         };
-        // operand block x of K step s: x = 2 i is A block i, x = 2 i + 1 is B block i
+        // operand block x of K step s: x = 2 i is A block i, x = 2 i + 1 is B block i; past the last A block the rest of B
         auto readAt = [&](uint32_t aAt, uint32_t bAt, uint32_t s, uint32_t x, uint32_t part) {
-            if(x & 1u)
-                readBlock8<B_KCONTIG, WB, ES>(lds + bAt, rdB, x >> 1, s, part, fb[s][x >> 1], 0u);
+            const uint32_t bBlock = x < 2u * WM ? x >> 1 : x - WM;
+            if((x & 1u) || x >= 2u * WM)
+                readBlock8<B_KCONTIG, WB, ES>(lds + bAt, rdB, bBlock, s, part, fb[s][bBlock], 0u);
             else
                 readBlock8<A_KCONTIG, WB, ES>(lds + aAt, rdA, x >> 1, s, part, fa[s][x >> 1], 0u);
         };
@@ -1102,7 +1117,9 @@ namespace
         //       late (f16 2048^2 x 8192: 0.0745 ms this way, 0.0770 the other).
         constexpr bool     SPREAD = WB == 8;
         constexpr uint32_t B_AHEAD = SPREAD ? 2u : 3u;
-        uint64_t           refillA, refillB; // stage kt + 2 of A, stage kt + B_AHEAD of B (clamped)
+        // matrix instructions firstOf(x) .. firstOf(x + 1) - 1 of a K step go with operand block x: as many each as the tile allows
+        auto     firstOf = [](uint32_t x) { return x * NS / XS; };
+        uint64_t refillA, refillB; // stage kt + 2 of A, stage kt + B_AHEAD of B (clamped)
         // `full` (compile-time tag): every stage this one requests is a whole stage inside K - the main part of the K
         // loop, whose loads carry no tail select and whose refill pointers always advance
         auto stageBody = [&](auto full, uint32_t kt, uint32_t aCur, uint32_t aNxt, uint32_t bCur, uint32_t bNxt, uint32_t bFree) {
@@ -1116,19 +1133,20 @@ namespace
 #pragma unroll
             for(uint32_t x = 0; x < XS; ++x)
 #pragma unroll
-                for(uint32_t q = 0; q < QS; ++q)
+                for(uint32_t n = firstOf(x); n < firstOf(x + 1u); ++n)
                 {
-                    mfmaAt(0, QS * x + q);
+                    const uint32_t q = n - firstOf(x);
+                    mfmaAt(0, n);
                     if(q < 2u)
                         readAt(aCur, bCur, 1, x, q);
                     if constexpr(QS == 1u)
                         readAt(aCur, bCur, 1, x, 1);
                     if constexpr(SPREAD)
-                        if(q == LOAD_Q && (x & 1u))
-                            loadToLds(rsrcB, offB(x >> 1, vB), (x >> 1) * gStepB, dmaDst + bFree + (x >> 1) * THREADS * CHUNK);
+                        if(const uint32_t l = x * LB / XS; q == LOAD_Q && (x + 1u) * LB / XS > l)
+                            loadToLds(rsrcB, offB(l, vB), l * gStepB, dmaDst + bFree + l * THREADS * CHUNK);
                     __builtin_amdgcn_sched_barrier(0);
                 }
-            waitVmcnt<WB>(); // this wave's part of stage kt + 1 has landed (the youngest WB loads are B of kt + 2)
+            waitVmcnt<LB>(); // this wave's part of stage kt + 1 has landed (the youngest LB loads are B of kt + 2)
             ldsBarrier();
             const uint32_t vA    = FULL ? STAGE_KB : validOf(kt + 2u);
             const i32x4    rsrcA = stageRsrc8(A_KCONTIG, refillA, vA, p.lda);
@@ -1137,17 +1155,18 @@ namespace
 #pragma unroll
             for(uint32_t x = 0; x < XS; ++x)
 #pragma unroll
-                for(uint32_t q = 0; q < QS; ++q)
+                for(uint32_t n = firstOf(x); n < firstOf(x + 1u); ++n)
                 {
-                    mfmaAt(1, QS * x + q);
+                    const uint32_t q = n - firstOf(x);
+                    mfmaAt(1, n);
                     if(q < 2u)
                         readAt(aNxt, bNxt, 0, x, q);
                     if constexpr(QS == 1u)
                         readAt(aNxt, bNxt, 0, x, 1);
                     if constexpr(SPREAD)
                     {
-                        if(q == LOAD_Q && (x & 1u))
-                            loadToLds(rsrcA, offA(x >> 1, vA), (x >> 1) * gStepA, dmaDst + aCur + (x >> 1) * THREADS * CHUNK);
+                        if(const uint32_t l = x * LA / XS; q == LOAD_Q && (x + 1u) * LA / XS > l)
+                            loadToLds(rsrcA, offA(l, vA), l * gStepA, dmaDst + aCur + l * THREADS * CHUNK);
                     }
                     else if(q == LOAD_Q)
                     {
@@ -1164,19 +1183,19 @@ namespace
         // loop keeps; stage 0 published
         if constexpr(SPREAD)
         {
-            issueHalf(B_KCONTIG, stageAddr(gB, gStageB, 0u), gOffB, gStepB, kByteB, p.ldb, validOf(0u), B_AT[0]);
-            issueHalf(A_KCONTIG, stageAddr(gA, gStageA, 0u), gOffA, gStepA, kByteA, p.lda, validOf(0u), A_AT[0]);
-            issueHalf(B_KCONTIG, stageAddr(gB, gStageB, 1u), gOffB, gStepB, kByteB, p.ldb, validOf(1u), B_AT[1]);
-            issueHalf(A_KCONTIG, stageAddr(gA, gStageA, 1u), gOffA, gStepA, kByteA, p.lda, validOf(1u), A_AT[1]);
-            waitVmcnt<2u * WB>();
+            issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, 0u), gOffB, gStepB, kByteB, p.ldb, validOf(0u), B_AT[0]);
+            issueHalf(LA, A_KCONTIG, stageAddr(gA, gStageA, 0u), gOffA, gStepA, kByteA, p.lda, validOf(0u), A_AT[0]);
+            issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, 1u), gOffB, gStepB, kByteB, p.ldb, validOf(1u), B_AT[1]);
+            issueHalf(LA, A_KCONTIG, stageAddr(gA, gStageA, 1u), gOffA, gStepA, kByteA, p.lda, validOf(1u), A_AT[1]);
+            waitVmcnt<LA + LB>();
         }
         else
         {
-            issueHalf(A_KCONTIG, stageAddr(gA, gStageA, 0u), gOffA, gStepA, kByteA, p.lda, validOf(0u), A_AT[0]);
-            issueHalf(B_KCONTIG, stageAddr(gB, gStageB, 0u), gOffB, gStepB, kByteB, p.ldb, validOf(0u), B_AT[0]);
-            issueHalf(A_KCONTIG, stageAddr(gA, gStageA, 1u), gOffA, gStepA, kByteA, p.lda, validOf(1u), A_AT[1]);
-            issueHalf(B_KCONTIG, stageAddr(gB, gStageB, 1u), gOffB, gStepB, kByteB, p.ldb, validOf(1u), B_AT[1]);
-            issueHalf(B_KCONTIG, stageAddr(gB, gStageB, 2u), gOffB, gStepB, kByteB, p.ldb, validOf(2u), B_AT[2]);
+            issueHalf(LA, A_KCONTIG, stageAddr(gA, gStageA, 0u), gOffA, gStepA, kByteA, p.lda, validOf(0u), A_AT[0]);
+            issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, 0u), gOffB, gStepB, kByteB, p.ldb, validOf(0u), B_AT[0]);
+            issueHalf(LA, A_KCONTIG, stageAddr(gA, gStageA, 1u), gOffA, gStepA, kByteA, p.lda, validOf(1u), A_AT[1]);
+            issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, 1u), gOffB, gStepB, kByteB, p.ldb, validOf(1u), B_AT[1]);
+            issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, 2u), gOffB, gStepB, kByteB, p.ldb, validOf(2u), B_AT[2]);
             waitVmcnt<3u * WB>();
         }
         refillA = stageAddr(gA, gStageA, 2u), refillB = stageAddr(gB, gStageB, B_AHEAD);
@@ -1246,7 +1265,7 @@ namespace
         if constexpr(TRIANGLE)
             storeTriangle<OutT, WB>(acc, reinterpret_cast<OutT*>(p.d), p.m, tm * TILE + wm * WT, tn * TILE + wn * WT, lane, lds + wave * (WB * 4096u));
         else
-            storeTile16<AccV, OutT, WB, WB>(acc, p, tm * TILE + wm * WT, tn * TILE + wn * WT, lane, lds + wave * (WB * 4096u));
+            storeTile16<AccV, OutT, WM, WB, WB * 4096u>(acc, p, tm * TILE_R + wm * WTR, tn * TILE + wn * WT, lane, lds + wave * (WB * 4096u));
         R355_STAMP_END();
     }
 
@@ -1517,6 +1536,13 @@ namespace
     __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) gemmTiledKernelI8(Params p)
     {
         gemmTiled5<Elem::I8, OutT, A_KCONTIG, B_KCONTIG, 8>(p);
+    }
+    // macro tiles of 32 WM = 224 or 192 rows (tileRows, which has the figures): the image of A keeps the 256 x 256 tile's pitch, so
+    // that its swizzles and the loop's schedule stay; a stage brings fewer rows and has fewer matrix instructions
+    template <typename OutT, bool A_KCONTIG, bool B_KCONTIG, uint32_t WM>
+    __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) gemmTiledKernelI8Rows(Params p)
+    {
+        gemmTiled5<Elem::I8, OutT, A_KCONTIG, B_KCONTIG, 8, false, WM>(p);
     }
     template <typename OutT, bool A_KCONTIG, bool B_KCONTIG>
     __global__ void __launch_bounds__(THREADS) gemmTiledKernelI8Small(Params p)
@@ -1808,6 +1834,11 @@ namespace
     // exceed it, panels are re-fetched from HBM and one stage of lookahead no longer covers the latency
     // (8192^2 x 16384 TN: 1268 against 1435 TFLOP/s here; 8192 x 12288 x 8192 NN: 1317 against 1474; this body within
     // 1430 - 1490 over every size and orientation tried).
+    template <Elem E, typename OutT, bool A_KCONTIG, bool B_KCONTIG, uint32_t WM>
+    __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) gemmTiledKernel16Rows(Params p)
+    {
+        gemmTiled5<E, OutT, A_KCONTIG, B_KCONTIG, 8, false, WM>(p);
+    }
     template <Elem E, typename OutT, bool A_KCONTIG, bool B_KCONTIG>
     __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) gemmTiledKernel16Deep(Params p)
     {
@@ -2103,6 +2134,10 @@ namespace
                     hipLaunchKernelGGL((gemmTiledKernelI8Tiny<OutT, AK, BK>), grid, block, 0, stream, p);
                 else if(tile == 128u)
                     hipLaunchKernelGGL((gemmTiledKernelI8Small<OutT, AK, BK>), grid, block, 0, stream, p);
+                else if(tile == 224u)
+                    hipLaunchKernelGGL((gemmTiledKernelI8Rows<OutT, AK, BK, 7>), grid, block, 0, stream, p);
+                else if(tile == 192u)
+                    hipLaunchKernelGGL((gemmTiledKernelI8Rows<OutT, AK, BK, 6>), grid, block, 0, stream, p);
                 else if(wideI8())
                     hipLaunchKernelGGL((gemmTiledKernelI8Wide<OutT, AK, BK>), grid, dim3(THREADS_WIDE), 0, stream, p);
                 else
@@ -2137,6 +2172,10 @@ namespace
                 hipLaunchKernelGGL((gemmTiledKernel16Tiny<E, OutT, AK, BK>), grid, block, 0, stream, p);
             else if(tile == 128u)
                 hipLaunchKernelGGL((gemmTiledKernel16Small<E, OutT, AK, BK>), grid, block, 0, stream, p);
+            else if(tile == 224u)
+                hipLaunchKernelGGL((gemmTiledKernel16Rows<E, OutT, AK, BK, 7>), grid, block, 0, stream, p);
+            else if(tile == 192u)
+                hipLaunchKernelGGL((gemmTiledKernel16Rows<E, OutT, AK, BK, 6>), grid, block, 0, stream, p);
             else if(p.deepPipeline)
                 hipLaunchKernelGGL((gemmTiledKernel16Deep<E, OutT, AK, BK>), grid, block, 0, stream, p);
             else
@@ -2405,6 +2444,45 @@ namespace
         const uint32_t rest  = total % cus;
         return (total > cus && rest != 0u && rest <= cus / 2u) ? rest : 0u;
     }
+
+    // Rows of the large macro tile (R355_KERNEL_AUTO, 16-bit and int8 operands): 256, or 224 or 192 where tiles of that height
+    // share the work out better - a last round of 256 x 256 tiles that leaves many CUs idle, or 13 x 19 tiles of 224 rows in one
+    // round instead of 12 x 19 of 256.  (Rows of the problem as the kernel sees it: columns of a col-major D.)  The choice is
+    // the cheapest by a timing model: with `rounds` the most work any CU gets, in tiles (a mixed tiling's second launch counts
+    // as 0.55 of a tile up to a quarter of the CUs, 0.75 beyond), and `mean` what a CU gets on average, a launch takes
+    //     rounds (fixed + out h) + stages stage h (spread mean + (1 - spread) rounds) microseconds,    h = rows / 256,
+    // because the board's power limit lets CUs that share the chip with idle ones run faster.  Fitted to 117 (16-bit) and 75
+    // (int8) random shapes from 1500 x 1500 x 700 to 8192^3, all orientations: fixed 8.32 / 7.76, out (results of 32 bits) 2.72 / 3.89,
+    // stage 1.41 / 1.50, spread 0.52 / 0.58.  On these shapes the model's choices run 1.08 (16-bit) and 1.045 (int8) times as fast as
+    // 256 x 256 with its remainder launch - the best of the three for each shape would be 1.081 and 1.046 - and none of them is slower
+    // by more than the runs differ: bf16 2832 x 4624 x 3080 72.8 -> 65.4 us, int8 5120^3 112 -> 109.6, bf16 4880 x 4624 x 4528 194 -> 166.
+    uint32_t tileRows(const r355_gemm_args& g)
+    {
+        const bool eight = g.in_type == R355_I8;
+        if(g.kernel != R355_KERNEL_AUTO || (!eight && g.in_type != R355_F16 && g.in_type != R355_BF16) || macroTile(g) != 256u)
+            return 256u;
+        const bool     dRow = g.layout_d == R355_ROW_MAJOR;
+        const uint64_t m = dRow ? g.m : g.n, n = dRow ? g.n : g.m, cus = computeUnits();
+        const double   stages = static_cast<double>(((uint64_t)g.k * r355::dtypeBytes(g.in_type) + STAGE_KB - 1u) / STAGE_KB);
+        const double   fixed = eight ? 7.76 : 8.32, stage = eight ? 1.50 : 1.41, spread = eight ? 0.58 : 0.52;
+        const double   out = r355::dtypeBytes(g.out_type) < 4u ? 0.0 : eight ? 3.89 : 2.72;
+        auto           time = [&](uint32_t rows) {
+            const uint64_t tiles = ((m + rows - 1u) / rows) * ((n + 255u) / 256u), full = tiles / cus, rest = tiles % cus;
+            const double   h = rows / 256.0, mean = static_cast<double>(tiles) / static_cast<double>(cus);
+            double         rounds = static_cast<double>(full), launch = 0.0;
+            if(rows == 256u && full > 0u && rest != 0u && rest <= cus / 2u) // mixedRemainder
+                rounds += rest <= cus / 4u ? 0.55 : 0.75, launch = SECOND_LAUNCH;
+            else if(rest != 0u)
+                rounds += 1.0;
+            return rounds * (fixed + out * h) + stages * stage * h * (spread * mean + (1.0 - spread) * rounds) + launch;
+        };
+        uint32_t best     = 256u;
+        double   bestTime = 0.99 * time(256u);
+        for(const uint32_t rows : {224u, 192u})
+            if(const double t = time(rows); t < bestTime)
+                best = rows, bestTime = t;
+        return best;
+    }
 #endif // part 0
 } // namespace
 
@@ -2522,7 +2600,7 @@ namespace r355
         if(plan)
         {
             plan->kernel       = R355_KERNEL_TILED;
-            plan->macro_tile_m = tile;
+            plan->macro_tile_m = tile; // (the nominal plan: tileRows may narrow the tiles that a launch takes)
             plan->macro_tile_n = tile;
             plan->macro_tile_k = tk;
             // with mixed tiling: the first launch (the second covers mixedRemainder(g) tile indices on 128 x 128 tiles)
@@ -2620,6 +2698,12 @@ namespace r355
             }();
             return rc != R355_OK ? rc : splitKReduce(g, p, splits, stream);
         }
+        if(tile == 256u)
+            if(const uint32_t rows = tileRows(g); rows != 256u)
+            {
+                p.tilesM = (p.m + rows - 1u) / rows, p.tileCount = p.tilesM * p.tilesN;
+                return part(rows, p);
+            }
         const uint32_t rest = mixedRemainder(g);
         if(rest == 0u)
             return part(tile, p);

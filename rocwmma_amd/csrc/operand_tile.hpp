@@ -89,19 +89,21 @@ namespace r355
             }
         }
 
-        // LDS -> register lane offsets of one operand for the wave whose tile starts at row 16 WB w.
+        // LDS -> register lane offsets of one operand for the wave whose tile starts at row 16 WT w (WT <= WB blocks per wave;
+        // the image keeps the pitch of 32 WB rows).
         // K-contiguous: rd[q] is 64-byte K step q of block 0 (block i is 16 rows further);
         // M/N-contiguous: rd[i] is block i, the first 8 k-rows of the lane's 16 of K step 0.
-        template <bool KCONTIG, uint32_t WB, uint32_t ES = 1>
+        template <bool KCONTIG, uint32_t WB, uint32_t ES = 1, uint32_t WT = WB>
         __device__ __forceinline__ void readOffsets8(uint32_t w, uint32_t lane, uint32_t (&rd)[8])
         {
+            static_assert(WT == WB || ES <= 2, "narrower wave tiles: 8- and 16-bit operands");
             const uint32_t t = lane & 15u, g = lane >> 4;
     #pragma unroll
             for(uint32_t i = 0; i < 8; ++i)
                 rd[i] = 0u;
             if constexpr(KCONTIG)
             {
-                const uint32_t r = w * 16u * WB + t;
+                const uint32_t r = w * 16u * WT + t;
                 rd[0]            = r * STAGE_KB + ((g ^ swzK8(r)) * CHUNK);
                 rd[1]            = r * STAGE_KB + (((4u + g) ^ swzK8(r)) * CHUNK);
             }
@@ -109,8 +111,8 @@ namespace r355
             {
                 const uint32_t kr = 16u * g + (t >> 1);
     #pragma unroll
-                for(uint32_t i = 0; i < WB; ++i)
-                    rd[i] = kr * 32u * WB + (((w * WB + i) ^ swzMN8<WB>(kr)) * CHUNK) + (t & 1u) * 8u;
+                for(uint32_t i = 0; i < WT; ++i)
+                    rd[i] = kr * 32u * WB + (((w * WT + i) ^ swzMN8<WB>(kr)) * CHUNK) + (t & 1u) * 8u;
             }
             else if constexpr(ES == 8)
             {
@@ -134,9 +136,9 @@ namespace r355
                 // 16-bit: k-row 8 (lane / 16) + (lane % 16) / 4 of the K step's first half, 8-byte piece 4 i + lane % 4
                 const uint32_t kr = 8u * g + (t >> 2);
     #pragma unroll
-                for(uint32_t i = 0; i < WB; ++i)
+                for(uint32_t i = 0; i < WT; ++i)
                 {
-                    const uint32_t piece = w * 4u * WB + 4u * i + (t & 3u);
+                    const uint32_t piece = w * 4u * WT + 4u * i + (t & 3u);
                     rd[i] = kr * 64u * WB + (((piece >> 1) ^ swzMN8<WB, 2>(kr)) * CHUNK) + (piece & 1u) * 8u;
                 }
             }
