@@ -319,9 +319,12 @@ namespace
     //     (16 x 96, batch 4096, f16: 5.3 us a block per wave, 15.7 on 64 x 64 tiles);
     //   * a launch of a few short waves is over before a tile's K loop has filled its five buffers (64 x 96 x 64 f16: 4.05
     //     against 4.57 us; at k = 256 5.5 against 4.6, and from 128 x 144 x 64 on, 2304 waves, 5.6 against 4.6);
-    //   * 16-bit types take the 128 x 128 tile where every CU gets 16 K stages of such tiles or more (512 x 1024 x 64: 30.5
-    //     against 35.0 us on 64 x 64, 1024 x 1024 x 64: 86 against 118; 1024 x 256 x 16: 16.1 against 14.2); f32, bound by its matrix
-    //     instructions, is faster on 64 x 64 throughout (1024 x 1024 x 64: 565 against 590 us).
+    //   * 16-bit types, beyond 192 features (40 shapes of 256 ... 1024 features, f16): the 128 x 128 tile where its launch has 0.6 tiles a CU
+    //     or more and it pads little - at most 0.38 times as many tiles as of 64 x 64 (352 x 928 x 41: 12.7 against 16.5 us; 688 x 816 x 9 10.4
+    //     against 12.3; with fewer tiles 592 x 368 x 6 6.3 against 5.4, 560 x 144 x 7 5.3 against 4.5; padded, 272 x 528 x 96 18.3 against
+    //     16.7) - or where every CU gets 32 K stages (272 x 1024 x 128: 26.8 against 28.3).  Up to 192 features, where every CU gets 16 K
+    //     stages of such tiles.  A 256 x 256 tile gains 2 - 5 % at 768 and 1024 features and loses up to half below: not built in.
+    //   * f32, bound by its matrix instructions, is faster on 64 x 64 throughout (1024 x 1024 x 64: 565 against 590 us).
     // Leading dimensions beyond 8 MiB per row do not fit the tile kernels' 32-bit lane offsets.
     uint32_t forwardTile(int32_t dtype, uint32_t m, uint32_t k, uint32_t batch)
     {
@@ -334,8 +337,16 @@ namespace
         const uint64_t blocks = m / BLK, waves = blocks * (blocks + 1u) / 2u * batch, steps = k / (es == 2u ? 16u : 4u);
         if(waves <= 5u * cus && steps <= 12u)
             return 0u;
-        const uint64_t tiles = (m + 127u) / 128u, stages = (k * es + 127u) / 128u;
-        return es == 2u && tiles * (tiles + 1u) / 2u * batch * stages >= 16u * cus ? 128u : 64u;
+        if(es != 2u)
+            return 64u;
+        auto pairs = [&](uint64_t edge) {
+            const uint64_t tiles = (m + edge - 1u) / edge;
+            return tiles * (tiles + 1u) / 2u * batch;
+        };
+        const uint64_t large = pairs(128u), small = pairs(64u), stages = (k * es + 127u) / 128u;
+        if(m <= 192u)
+            return large * stages >= 16u * cus ? 128u : 64u;
+        return 5u * large >= 3u * cus && (50u * large <= 19u * small || large * stages >= 32u * cus) ? 128u : 64u;
     }
 
     // Backward: the macro tile's edge (dlrmBwdTiled in gemm_tiled.hip), or 0 for the fragment-API kernels below.  Measured on one

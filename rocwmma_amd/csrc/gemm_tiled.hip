@@ -505,7 +505,9 @@ namespace
     // d[gi (gi - 1) / 2 + gj].  The wave tile starts at (m0, n0); rows from m on do not exist.  Staged through the wave's LDS
     // like storeTileStaged; a row of the wave tile is then one run of 16 WB elements that starts at any element: a lane
     // stores 16 bytes of it whatever its alignment (the memory pipeline takes unaligned vectors; the L2 puts the partial lines of
-    // neighbouring tiles together), and the wave tiles on the diagonal, whose rows end anywhere, go out element by element.
+    // neighbouring tiles together); the wave tiles on the diagonal, whose rows end anywhere, add the last few elements of each row.
+    // (Element by element, as 2-byte stores of a row at a time, the diagonal tiles took as long as three others: f16 272 x 1024 x 128 35.3 -> 27.0
+    // us, 320 x 368 x 124 23.3 -> 16.9, 512 x 1024 x 64 31.7 -> 27.3.)
     template <typename OutT, uint32_t WB>
     __device__ __forceinline__ void storeTriangle(f32x4 (&acc)[WB][WB], OutT* d, uint32_t m, uint32_t m0, uint32_t n0, uint32_t lane, char* scratch)
     {
@@ -533,9 +535,9 @@ namespace
             const uint64_t gi = m0 + row;
             return d + (gi * (gi - 1u) / 2u + n0);
         };
+        const uint32_t c = lane % ROW_CHUNKS;
         if(n0 < m0) // (uniform) whole rows
         {
-            const uint32_t c = lane % ROW_CHUNKS;
 #pragma unroll
             for(uint32_t it = 0; it < WT / RPI; ++it)
             {
@@ -545,16 +547,28 @@ namespace
                     *reinterpret_cast<i32x4u*>(rowStart(row) + c * EPC) = v;
             }
         }
-        else // the diagonal: row r of the wave tile holds r elements
+        else // the diagonal: row r of the wave tile holds r elements, whole 16-byte pieces and, a row per lane, what is left of them
         {
-            const uint32_t col = lane % WT;
 #pragma unroll 8
-            for(uint32_t it = 0; it < WT / (64u / WT); ++it)
+            for(uint32_t it = 0; it < WT / RPI; ++it)
             {
-                const uint32_t row = it * (64u / WT) + lane / WT, byteInRow = col * OS;
-                const OutT     v   = *reinterpret_cast<const OutT*>(scratch + row * ROW_BYTES + (((byteInRow / CHUNK) ^ (row & SWZ)) * CHUNK) + byteInRow % CHUNK);
-                if(col < row && m0 + row < m)
-                    rowStart(row)[col] = v;
+                const uint32_t row = it * RPI + lane / ROW_CHUNKS;
+                const i32x4    v   = *reinterpret_cast<const i32x4*>(scratch + row * ROW_BYTES + ((c ^ (row & SWZ)) * CHUNK));
+                if((c + 1u) * EPC <= row && m0 + row < m)
+                    *reinterpret_cast<i32x4u*>(rowStart(row) + c * EPC) = v;
+            }
+#pragma unroll
+            for(uint32_t row0 = 0; row0 < WT; row0 += 64u)
+            {
+                const uint32_t row = row0 + lane, last = row / EPC; // (a wave tile of 32 rows: half of the lanes)
+                if(row >= WT || m0 + row >= m)
+                    continue;
+                const OutT* from = reinterpret_cast<const OutT*>(scratch + row * ROW_BYTES + ((last ^ (row & SWZ)) * CHUNK));
+                OutT*       to   = rowStart(row) + last * EPC;
+#pragma unroll
+                for(uint32_t e = 0; e + 1u < EPC; ++e)
+                    if(e < row % EPC)
+                        to[e] = from[e];
             }
         }
     }

@@ -31,6 +31,14 @@ def test_forward_on_macro_tiles(dtype, m, k, batch):
     assert np.array_equal(out[:batch * stride].view(np.uint8), O.dlrm_fwd(dtype, x, m, k, batch).ravel().view(np.uint8))
 
 
+
+# the 128 x 128 tile of the 16-bit types beyond 192 features: just enough tiles for it and one sample fewer, whole and partial last tiles
+@pytest.mark.parametrize("dtype", [O.F16, O.BF16])
+@pytest.mark.parametrize("m,k,batch", [(256, 80, 52), (256, 80, 51), (352, 208, 26), (496, 64, 16), (1008, 32, 5)])
+def test_forward_on_the_large_tile(dtype, m, k, batch):
+    test_forward_on_macro_tiles(dtype, m, k, batch)
+
+
 # backward: one tile and several, so that stages left of, in and right of the diagonal tile all occur, partial tiles and K stages,
 # widths off the tile's edge, samples spread unevenly over the XCDs; shapes for both macro tiles and for the kernels below them
 @pytest.mark.parametrize("dtype", [O.F16, O.BF16, O.F32])
