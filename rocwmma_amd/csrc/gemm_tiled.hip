@@ -2372,6 +2372,8 @@ namespace
                 const uint32_t share = (stages + s - 1u) / s;
                 if((stages + share - 1u) / share != s)
                     continue; // a share would be empty
+                if(edge == 64u && tiles * s > (1u << 24) - 8u)
+                    continue; // a launch's threads are counted in 32 bits
                 const uint64_t perCu = (tiles * s + cus - 1u) / cus, rest = perCu % together;
                 auto           round = [&](uint64_t count) {
                     const double each = t.each * static_cast<double>(count);
@@ -2527,6 +2529,9 @@ namespace r355
         return checkLaunch("gemm (split-K reduction)");
     }
 
+    // workgroups of a launch: its threads (256 each) are counted in 32 bits; a multiple of the eight XCDs
+    constexpr uint32_t MAX_GROUPS = (1u << 24) - 8u;
+
     int dlrmFwdTiled(int32_t dtype, const void* in, void* out, uint32_t m, uint32_t k, uint32_t batch, uint32_t tile, hipStream_t stream)
     {
         GemmTileParams p{};
@@ -2534,8 +2539,10 @@ namespace r355
         p.tilesM = p.tilesN = (m + tile - 1u) / tile;
         const uint32_t pairs = p.tilesM * (p.tilesM + 1u) / 2u;
         const uint64_t es = dtypeBytes(dtype), stride = (uint64_t)k + (uint64_t)m * (m - 1u) / 2u;
-        const uint32_t most = (1u << 30) / pairs; // samples per launch: a grid dimension holds 2^31 workgroups
-        for(uint32_t first = 0; first < batch; first += most)
+        if(pairs > MAX_GROUPS)
+            return fail(R355_ERR_BAD_SIZE, "dlrm_fwd: m=%u: too many tiles of a sample", m);
+        const uint32_t most = MAX_GROUPS / pairs; // samples per launch
+        for(uint32_t first = 0;; first += most)
         {
             const uint32_t count = batch - first < most ? batch - first : most;
             p.a = p.b   = static_cast<const char*>(in) + (uint64_t)first * m * k * es;
@@ -2545,10 +2552,9 @@ namespace r355
             const int      rc     = dtype == R355_F16    ? dlrmFwdTiledPart0(p, tile, groups, stream)
                                     : dtype == R355_BF16 ? dlrmFwdTiledPart1(p, tile, groups, stream)
                                                          : dlrmFwdTiledPart3(p, tile, groups, stream);
-            if(rc != R355_OK)
+            if(rc != R355_OK || batch - first <= most) // (first + most may pass 2^32)
                 return rc;
         }
-        return R355_OK;
     }
 
     int dlrmBwdTiled(int32_t dtype, const void* in, const void* upstream, void* mlpGrad, void* inGrad, uint32_t m, uint32_t k, uint32_t batch,
@@ -2559,10 +2565,10 @@ namespace r355
         p.tilesM = (m + tile - 1u) / tile, p.tilesN = (k + tile - 1u) / tile;
         const uint64_t es = dtypeBytes(dtype), stride = (uint64_t)k + (uint64_t)m * (m - 1u) / 2u;
         const uint64_t tiles = (uint64_t)p.tilesM * p.tilesN;
-        if(tiles > 1u << 30)
+        if(tiles > MAX_GROUPS)
             return fail(R355_ERR_BAD_SIZE, "dlrm_bwd: m=%u, k=%u: too many tiles of a sample", m, k);
-        const uint32_t most = (1u << 30) / static_cast<uint32_t>(tiles); // samples per launch: a grid dimension holds 2^31 workgroups
-        for(uint32_t first = 0; first < batch; first += most)
+        const uint32_t most = MAX_GROUPS / static_cast<uint32_t>(tiles); // samples per launch
+        for(uint32_t first = 0;; first += most)
         {
             const uint32_t count = batch - first < most ? batch - first : most;
             p.x     = static_cast<const char*>(in) + (uint64_t)first * m * k * es;
@@ -2573,12 +2579,9 @@ namespace r355
             const int rc = dtype == R355_F16    ? dlrmBwdTiledPart0(p, tile, stream)
                            : dtype == R355_BF16 ? dlrmBwdTiledPart1(p, tile, stream)
                                                 : dlrmBwdTiledPart3(p, tile, stream);
-            if(rc != R355_OK)
+            if(rc != R355_OK || batch - first <= most) // (first + most may pass 2^32)
                 return rc;
-            if(batch - first <= most)
-                break; // (first + most may pass 2^32)
         }
-        return R355_OK;
     }
 
     int gemmTiledCheck(const r355_gemm_args& g, r355_gemm_plan* plan)

@@ -3,6 +3,7 @@ kernel) against the CPU oracle.  Integer-valued features: every f32 sum is exact
 after the one rounding to the result type."""
 import numpy as np
 import pytest
+import torch
 
 import oraclelib as O
 import rocwmma_amd as R
@@ -29,7 +30,6 @@ def test_forward_on_macro_tiles(dtype, m, k, batch):
     out = to_host(dout, store)
     assert np.all(out[batch * stride:].view(np.uint8) == 0xEE)  # nothing behind the last row
     assert np.array_equal(out[:batch * stride].view(np.uint8), O.dlrm_fwd(dtype, x, m, k, batch).ravel().view(np.uint8))
-
 
 
 # the 128 x 128 tile of the 16-bit types beyond 192 features: just enough tiles for it and one sample fewer, whole and partial last tiles
@@ -70,3 +70,20 @@ def test_backward_with_an_upstream_off_16_bytes():
     want_mlp, want_grad = O.dlrm_bwd(dtype, x, up, m, k, batch)
     assert np.array_equal(to_host(dmlp, store).view(np.uint8), want_mlp.ravel().view(np.uint8))
     assert np.array_equal(O.storage_to_f32(to_host(dgrad, store), dtype), O.storage_to_f32(want_grad.ravel(), dtype))
+
+
+def test_more_samples_than_a_launch_holds():
+    """2^24 + 4096 samples of one tile each: a launch's 256-thread workgroups are counted in 32 bits of threads, so the batch goes
+    out in two launches.  The batch repeats 4096 samples; each repetition has to give the same bits (18 GB, 18 GB and 18 GB)."""
+    m, k, part, copies = 32, 16, 4096, 4097
+    stride = k + m * (m - 1) // 2
+    x = torch.randn(part, m * k, device="cuda").half().repeat(copies, 1)
+    out = torch.zeros(copies, part * stride, device="cuda", dtype=torch.float16)
+    R.dlrm_fwd(O.F16, x, out, m, k, part * copies)
+    want = torch.zeros(part * stride, device="cuda", dtype=torch.float16)
+    R.dlrm_fwd(O.F16, x, want, m, k, part)
+    assert bool(want.any()) and all(torch.equal(row, want) for row in out)
+    grad, mlp = x.clone().view(copies, -1), torch.zeros(copies, part * k, device="cuda", dtype=torch.float16)
+    R.dlrm_bwd(O.F16, x, out, mlp, grad, m, k, part * copies)
+    assert not torch.equal(grad[0], x[:part].view(-1))
+    assert all(torch.equal(row, grad[0]) for row in grad) and all(torch.equal(row, mlp[0]) for row in mlp)
