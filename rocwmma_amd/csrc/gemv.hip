@@ -26,13 +26,8 @@ namespace
     // (256-byte runs) is taken when the rows suffice for that.  Every lane sums its columns in increasing order; the
     // COL_WAVES * 64 / RL partial sums of a row meet in LDS and are added in a fixed order, so the result does not depend
     // on scheduling.  STREAM as in the row-major kernel.
-    // SPLIT: workgroup (b, s) sums columns [s kPer, (s + 1) kPer) only and leaves its rows' sums, unscaled, in an array of
-    // partial sums (yOut; element (row, s) at row * partRow + s * partSplit) for gemvAddSplits.  The grid counts (b, s) with b
-    // fastest.  Where columns do not start on a 128-byte boundary, the runs of neighbouring blocks of rows share cache lines:
-    // there an XCD takes a contiguous part of that count, so that neighbours walk the same columns on one L2 and the line
-    // they share comes from memory once (f32 6152 x 11012 51.8 -> 49.1 us, 1028 x 65536 53.2 -> 47.5, 2052 x 16384 26.0 -> 22.9,
-    // 14600 x 9004 93.4 -> 87.3; bound: HBM).  Aligned columns share nothing and are better off with neighbours spread over the
-    // XCDs (16640 x 16384 160 us, 168 in contiguous parts; 12288 x 8192 60.1 / 61.6).
+    // SPLIT: workgroup (b, s) of a two-dimensional grid sums columns [s kPer, (s + 1) kPer) only and leaves its rows' sums,
+    // unscaled, in an array of partial sums (yOut; element (row, s) at row * partRow + s * partSplit) for gemvAddSplits.
     template <typename T, uint32_t RL, uint32_t COL_WAVES, bool STREAM, bool SPLIT = false>
     __global__ void __launch_bounds__(COL_WAVES * 64) gemvColMajor(uint32_t m,
                                                                   uint32_t k,
@@ -50,19 +45,9 @@ namespace
         constexpr uint32_t V = 16u / sizeof(T), ROWS = RL * V, CL = 64u / RL, COLS = COL_WAVES * CL, DEPTH = 8;
         using VecT = T __attribute__((ext_vector_type(V)));
         __shared__ T   partial[COLS][ROWS];
-        uint32_t blk = blockIdx.x, spl = 0u;
-        if constexpr(SPLIT)
-        {
-            const uint32_t blocks = (m + ROWS - 1u) / ROWS, total = blocks * ((k - 1u) / kPer + 1u), perXcd = (total + 7u) / 8u;
-            const bool     askew  = ((uint64_t)lda * sizeof(T)) % 128u != 0u;
-            const uint32_t local  = askew ? (blockIdx.x % 8u) * perXcd + blockIdx.x / 8u : blockIdx.x;
-            if(local >= total)
-                return; // the whole workgroup: the grid is rounded up to a multiple of the XCDs
-            blk = local % blocks, spl = local / blocks;
-        }
         const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
         const uint32_t r = lane % RL, c = lane / RL;
-        const uint32_t row0 = blk * ROWS + r * V; // (m is a multiple of V: a lane's rows are inside or outside together)
+        const uint32_t row0 = blockIdx.x * ROWS + r * V; // (m is a multiple of V: a lane's rows are inside or outside together)
         T              acc[V];
 #pragma unroll
         for(uint32_t e = 0; e < V; ++e)
@@ -76,8 +61,8 @@ namespace
                 else
                     return *reinterpret_cast<const VecT*>(at);
             };
-            const uint32_t kEnd = SPLIT ? (k - spl * kPer < kPer ? k : (spl + 1u) * kPer) : k;
-            uint32_t       kk   = (SPLIT ? spl * kPer : 0u) + wave * CL + c;
+            const uint32_t kEnd = SPLIT ? (k - blockIdx.y * kPer < kPer ? k : (blockIdx.y + 1u) * kPer) : k;
+            uint32_t       kk   = (SPLIT ? blockIdx.y * kPer : 0u) + wave * CL + c;
             for(; kk + (DEPTH - 1u) * COLS < kEnd; kk += DEPTH * COLS)
             {
                 VecT v[DEPTH];
@@ -109,7 +94,7 @@ namespace
         __syncthreads();
         if(threadIdx.x < ROWS)
         {
-            const uint32_t row = blk * ROWS + threadIdx.x;
+            const uint32_t row = blockIdx.x * ROWS + threadIdx.x;
             if(row < m)
             {
                 T sum = T(0);
@@ -117,7 +102,7 @@ namespace
                 for(uint32_t w = 0; w < COLS; ++w)
                     sum += partial[w][threadIdx.x];
                 if constexpr(SPLIT)
-                    yOut[(uint64_t)row * partRow + (uint64_t)spl * partSplit] = sum;
+                    yOut[(uint64_t)row * partRow + (uint64_t)blockIdx.y * partSplit] = sum;
                 else
                     yOut[row] = beta != T(0) ? alpha * sum + beta * yIn[row] : alpha * sum;
             }
@@ -546,8 +531,7 @@ namespace
             const bool stream = (uint64_t)k * lda * sizeof(T) > (256ull << 20);
             auto       go     = [&](auto rl, auto waves) {
                 constexpr uint32_t RL = decltype(rl)::value, ROWS = RL * V, WAVES = decltype(waves)::value;
-                const uint32_t     blocks = (m + ROWS - 1u) / ROWS;
-                const dim3         grid(split ? (blocks * splits + 7u) / 8u * 8u : blocks), block(WAVES * 64);
+                const dim3         grid((m + ROWS - 1u) / ROWS, split ? splits : 1u), block(WAVES * 64);
                 if(split && stream)
                     hipLaunchKernelGGL((gemvColMajor<T, RL, WAVES, true, true>), grid, block, 0, s, m, k, a, lda, x, y_in, parts, alpha, beta, kPer, partRow, partSplit);
                 else if(split)
