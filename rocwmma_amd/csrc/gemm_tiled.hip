@@ -123,6 +123,11 @@ namespace r355
         // the rounds' epilogues do not all store at once
         uint32_t stagger, staggerBlocks;
     };
+    // K stages of 128 bytes of a problem.  k in bytes need not fit 32 bits: 16 rows of 2^29 doubles are 64 GiB
+    inline uint32_t stagesOfK(uint32_t k, uint32_t elemBytes)
+    {
+        return static_cast<uint32_t>(((uint64_t)k * elemBytes + 127u) / 128u);
+    }
     // sum of `splits` partial results (accumulator type: f32, i32 or f64) + the alpha / beta epilogue into the output type
     int splitKReduce(const r355_gemm_args& g, const GemmTileParams& p, uint32_t splits, hipStream_t stream);
     // launch of one kernel family; aK / bK: operand is K-contiguous; tile: 256, 128 or 64, or the rows of a tile of 256 columns (224, 192)
@@ -737,10 +742,10 @@ namespace
         };
         // K stages come in pairs; K need not fill the last pair: stage st holds validOf(st) = 0 .. 128 valid
         // bytes per row and the loads fill the rest with zeros
-        const uint32_t kBytes    = p.k * ES;
-        const uint32_t numStages = (kBytes + 2u * STAGE_KB - 1u) / (2u * STAGE_KB) * 2u;
+        const uint32_t kWhole = p.k / TK, kTail = p.k % TK * ES; // (k in bytes need not fit 32 bits)
+        const uint32_t numStages = (kWhole + (kTail != 0u) + 1u) / 2u * 2u;
         auto           validOf   = [&](uint32_t st) { // 0 for the padding stage and for refills past the end: no traffic
-            return st * STAGE_KB >= kBytes ? 0u : (kBytes - st * STAGE_KB < STAGE_KB ? kBytes - st * STAGE_KB : STAGE_KB);
+            return st < kWhole ? STAGE_KB : (st == kWhole ? kTail : 0u);
         };
         auto rsrcAt = [](uint64_t addr, uint32_t records) { // raw buffer, 32-bit data format, no swizzle
             return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char*>(addr), 0, static_cast<int>(records), 0x00020000);
@@ -868,7 +873,7 @@ namespace
 
         // main part: every stage a pair refills (up to kt + 3) is a whole stage of K; then the pairs around the end of K
         // (only a K-contiguous operand has a select to lose: with none, the main part is empty and compiles away)
-        const uint32_t wholeStages = (A_KCONTIG || B_KCONTIG) ? kBytes / STAGE_KB : 0u;
+        const uint32_t wholeStages = (A_KCONTIG || B_KCONTIG) ? kWhole : 0u;
         uint32_t       kt          = 0;
         for(; kt + 3u < wholeStages; kt += 2)
         {
@@ -1054,9 +1059,9 @@ namespace
         laneOffsets8<B_KCONTIG, WB, ES>(tid, p.ldb, validN, gOffB, gStepB, gStageB, kByteB);
         // K need not fill the last stage: its lastBytes (16 .. 128) valid bytes per row are followed by zeros
         // the loads produce themselves (see tailOffset)
-        const uint32_t kBytes    = p.k * ES;
-        const uint32_t numStages = (kBytes + STAGE_KB - 1u) / STAGE_KB;
-        const uint32_t lastBytes = kBytes - (numStages - 1u) * STAGE_KB;
+        constexpr uint32_t TK    = STAGE_KB / ES; // (counted in elements: k in bytes need not fit 32 bits)
+        const uint32_t numStages = (p.k - 1u) / TK + 1u;
+        const uint32_t lastBytes = (p.k - (numStages - 1u) * TK) * ES;
         // (refills past the last stage are issued like all others but with nothing in range: they cost no memory traffic)
         auto validOf = [&](uint32_t stage) { return stage + 1u < numStages ? STAGE_KB : (stage + 1u == numStages ? lastBytes : 0u); };
         const uint32_t dmaDst    = ldsBase + wave * 64u * CHUNK; // + buffer + j * 4 KiB
@@ -1226,7 +1231,7 @@ namespace
         // runs the trips whose requests (up to stage kt + 5 + B_AHEAD) all are whole stages inside K without the tail
         // handling; the trips around the end of K and the remainder carry it.
         // (Only a K-contiguous operand has a select to lose: with none, the main part is empty and compiles away.)
-        const uint32_t     wholeStages = (A_KCONTIG || B_KCONTIG) ? kBytes / STAGE_KB : 0u;
+        const uint32_t     wholeStages = (A_KCONTIG || B_KCONTIG) ? p.k / TK : 0u;
         constexpr uint32_t REACH       = 5u + B_AHEAD;
         const uint32_t     mainTrips   = wholeStages > REACH ? (wholeStages - REACH + 5u) / 6u : 0u;
         using Main = std::true_type;
@@ -1350,7 +1355,7 @@ namespace
         const uint32_t validN = p.n - tn * TILE < TILE ? p.n - tn * TILE : TILE;
         laneOffsetsWide<A_KCONTIG>(tid, p.lda, validM, gOffA, gStepA, gStageA, kByteA);
         laneOffsetsWide<B_KCONTIG>(tid, p.ldb, validN, gOffB, gStepB, gStageB, kByteB);
-        const uint32_t numStages = (p.k + STAGE_KB - 1u) / STAGE_KB;
+        const uint32_t numStages = (p.k - 1u) / STAGE_KB + 1u;
         const uint32_t lastBytes = p.k - (numStages - 1u) * STAGE_KB;
         auto validOf = [&](uint32_t stage) { return stage + 1u < numStages ? STAGE_KB : (stage + 1u == numStages ? lastBytes : 0u); };
         const uint32_t dmaDst = ldsBase + wave * 64u * CHUNK; // + buffer + j * 8 KiB
@@ -1919,7 +1924,7 @@ namespace
         laneOffsets8<B_KCONTIG, WB>(tid, p.ldb, validN, gOffB, gStepB, gStageB, kByteB);
         // K need not fill the last stage: its lastBytes (16 .. 128) valid bytes per row are followed by zeros
         // the loads produce themselves (see tailOffset)
-        const uint32_t numStages = (p.k + STAGE_KB - 1u) / STAGE_KB;
+        const uint32_t numStages = (p.k - 1u) / STAGE_KB + 1u;
         const uint32_t lastBytes = p.k - (numStages - 1u) * STAGE_KB;
         // (refills past the last stage are issued like all others but with nothing in range: they cost no memory traffic)
         auto validOf = [&](uint32_t stage) { return stage + 1u < numStages ? STAGE_KB : (stage + 1u == numStages ? lastBytes : 0u); };
@@ -2138,7 +2143,7 @@ namespace
     int launchLayouts(bool aK, bool bK, uint32_t tile, const Params& p, hipStream_t stream)
     {
         // every XCD gets ceil(count / 8) tile indices (four workgroups each in a quad launch)
-        const uint32_t splits = p.splitStages ? ((p.k * ElemTraits<E>::Bytes + STAGE_KB - 1u) / STAGE_KB + p.splitStages - 1u) / p.splitStages : 1u;
+        const uint32_t splits = p.splitStages ? (r355::stagesOfK(p.k, ElemTraits<E>::Bytes) + p.splitStages - 1u) / p.splitStages : 1u;
         const dim3     grid(((p.tileCount + 7u) / 8u) * 8u * (p.tileQuad ? 4u : 1u), splits), block(THREADS);
         auto launch = [&](auto aKc, auto bKc) {
             constexpr bool AK = decltype(aKc)::value, BK = decltype(bKc)::value;
@@ -2249,7 +2254,7 @@ namespace
         const uint64_t t128 = (uint64_t)((g.m + 127u) / 128u) * ((g.n + 127u) / 128u);
         if(((t128 + cus - 1u) / cus) * 5u < ((t256 + cus - 1u) / cus) * 11u)
             return 128u;
-        const uint64_t stages = ((uint64_t)g.k * r355::dtypeBytes(g.in_type) + STAGE_KB - 1u) / STAGE_KB;
+        const uint32_t stages = r355::stagesOfK(g.k, r355::dtypeBytes(g.in_type));
         if(stages > 8u)
             return 256u; // (at 16 stages the model still picks the small tile now and then where the large one is 3 - 9 % faster)
         const TileCosts c       = tileCosts(g.in_type);
@@ -2299,7 +2304,7 @@ namespace
             return 1u;
         const uint32_t cus = computeUnits();
         const uint64_t tiles = (uint64_t)((g.m + 127u) / 128u) * ((g.n + 127u) / 128u);
-        const uint32_t stages = (g.k * r355::dtypeBytes(g.in_type) + STAGE_KB - 1u) / STAGE_KB;
+        const uint32_t stages = r355::stagesOfK(g.k, r355::dtypeBytes(g.in_type));
         if(tiles * 2u > cus || stages < 16u)
             return 1u;
         // one workgroup per CU (two per CU, which the 80 KiB of LDS allow, measured 5 - 20 % slower), at least 8 stages per share
@@ -2317,7 +2322,7 @@ namespace
     }
     uint32_t splitStagesOf(const r355_gemm_args& g, uint32_t splits)
     {
-        const uint32_t stages = (g.k * r355::dtypeBytes(g.in_type) + STAGE_KB - 1u) / STAGE_KB;
+        const uint32_t stages = r355::stagesOfK(g.k, r355::dtypeBytes(g.in_type));
         return (stages + splits - 1u) / splits;
     }
 
@@ -2358,7 +2363,7 @@ namespace
         if(g.kernel != R355_KERNEL_AUTO || tile != 128u)
             return {tile, splits};
         const uint32_t es     = r355::dtypeBytes(g.in_type), cls = es == 1u ? 0u : es == 2u ? 1u : es == 4u ? 2u : 3u;
-        const uint32_t stages = (g.k * es + STAGE_KB - 1u) / STAGE_KB;
+        const uint32_t stages = r355::stagesOfK(g.k, es);
         const uint64_t cus    = computeUnits();
         TileWork       best{128u, splits};
         double         bestTime = 0.0, plannedTime = 0.0;
@@ -2479,7 +2484,7 @@ namespace
             return 256u;
         const bool     dRow = g.layout_d == R355_ROW_MAJOR;
         const uint64_t m = dRow ? g.m : g.n, n = dRow ? g.n : g.m, cus = computeUnits();
-        const double   stages = static_cast<double>(((uint64_t)g.k * r355::dtypeBytes(g.in_type) + STAGE_KB - 1u) / STAGE_KB);
+        const double   stages = r355::stagesOfK(g.k, r355::dtypeBytes(g.in_type));
         const double   fixed = eight ? 7.76 : 8.32, stage = eight ? 1.50 : 1.41, spread = eight ? 0.58 : 0.52;
         const double   out = r355::dtypeBytes(g.out_type) < 4u ? 0.0 : eight ? 3.89 : 2.72;
         auto           time = [&](uint32_t rows) {
