@@ -128,6 +128,17 @@ namespace r355
     {
         return static_cast<uint32_t>(((uint64_t)k * elemBytes + 127u) / 128u);
     }
+    // tiles of `edge` that cover n > 0 rows or columns
+    constexpr uint32_t tilesOf(uint32_t n, uint32_t edge)
+    {
+        return (n - 1u) / edge + 1u;
+    }
+    // Workgroups of a launch: its threads (256 each) are counted in 32 bits, and a launch of more runs what is left modulo 2^32
+    // and reports success.  A multiple of the eight XCDs.
+    constexpr uint32_t MAX_GROUPS = (1u << 24) - 8u;
+    // Tile indices of a GEMM launch, a multiple of eight: four workgroups of 256 threads each (tileQuad) stay within that.  What a
+    // problem has more goes out in further launches.
+    constexpr uint32_t MAX_TILES = MAX_GROUPS / 32u * 8u;
     // sum of `splits` partial results (accumulator type: f32, i32 or f64) + the alpha / beta epilogue into the output type
     int splitKReduce(const r355_gemm_args& g, const GemmTileParams& p, uint32_t splits, hipStream_t stream);
     // launch of one kernel family; aK / bK: operand is K-contiguous; tile: 256, 128 or 64, or the rows of a tile of 256 columns (224, 192)
@@ -2140,12 +2151,14 @@ namespace
     }
 
     template <Elem E, typename OutT>
-    int launchLayouts(bool aK, bool bK, uint32_t tile, const Params& p, hipStream_t stream)
+    int launchLayouts(bool aK, bool bK, uint32_t tile, const Params& whole, hipStream_t stream)
     {
-        // every XCD gets ceil(count / 8) tile indices (four workgroups each in a quad launch)
+        Params         p      = whole;
         const uint32_t splits = p.splitStages ? (r355::stagesOfK(p.k, ElemTraits<E>::Bytes) + p.splitStages - 1u) / p.splitStages : 1u;
-        const dim3     grid(((p.tileCount + 7u) / 8u) * 8u * (p.tileQuad ? 4u : 1u), splits), block(THREADS);
+        const dim3     block(THREADS);
         auto launch = [&](auto aKc, auto bKc) {
+            // every XCD gets ceil(count / 8) tile indices (four workgroups each in a quad launch)
+            const dim3 grid(((p.tileCount + 7u) / 8u) * 8u * (p.tileQuad ? 4u : 1u), splits);
             constexpr bool AK = decltype(aKc)::value, BK = decltype(bKc)::value;
             if constexpr(E == Elem::I8)
             {
@@ -2202,14 +2215,19 @@ namespace
         };
         using T = std::true_type;
         using F = std::false_type;
-        if(aK && bK)
-            launch(T{}, T{});
-        else if(aK)
-            launch(T{}, F{});
-        else if(bK)
-            launch(F{}, T{});
-        else
-            launch(F{}, F{});
+        for(uint32_t done = 0; done < whole.tileCount; done += p.tileCount)
+        {
+            p.tileFirst = whole.tileFirst + done;
+            p.tileCount = whole.tileCount - done < r355::MAX_TILES ? whole.tileCount - done : r355::MAX_TILES;
+            if(aK && bK)
+                launch(T{}, T{});
+            else if(aK)
+                launch(T{}, F{});
+            else if(bK)
+                launch(F{}, T{});
+            else
+                launch(F{}, F{});
+        }
         return r355::checkLaunch("gemm (macro tile)");
     }
 
@@ -2250,8 +2268,8 @@ namespace
             return 128u; // bound by the matrix-instruction rate either way (146 TFLOP/s at 4096^2 x 2048 with both
                          // tiles), and four times finer rounds: 6144^2 x 2048 runs at 148 TFLOP/s against 111
         const uint64_t cus  = computeUnits();
-        const uint64_t t256 = (uint64_t)((g.m + 255u) / 256u) * ((g.n + 255u) / 256u);
-        const uint64_t t128 = (uint64_t)((g.m + 127u) / 128u) * ((g.n + 127u) / 128u);
+        const uint64_t t256 = (uint64_t)r355::tilesOf(g.m, 256u) * r355::tilesOf(g.n, 256u);
+        const uint64_t t128 = (uint64_t)r355::tilesOf(g.m, 128u) * r355::tilesOf(g.n, 128u);
         if(((t128 + cus - 1u) / cus) * 5u < ((t256 + cus - 1u) / cus) * 11u)
             return 128u;
         const uint32_t stages = r355::stagesOfK(g.k, r355::dtypeBytes(g.in_type));
@@ -2303,7 +2321,7 @@ namespace
         if(g.workspace ? !r355::aligned(g.workspace, 16) : !sizing)
             return 1u;
         const uint32_t cus = computeUnits();
-        const uint64_t tiles = (uint64_t)((g.m + 127u) / 128u) * ((g.n + 127u) / 128u);
+        const uint64_t tiles = (uint64_t)r355::tilesOf(g.m, 128u) * r355::tilesOf(g.n, 128u);
         const uint32_t stages = r355::stagesOfK(g.k, r355::dtypeBytes(g.in_type));
         if(tiles * 2u > cus || stages < 16u)
             return 1u;
@@ -2371,14 +2389,12 @@ namespace
         {
             const TileTimes& t        = edge == 128u ? TIMES_128[cls] : TIMES_64[cls];
             const uint64_t   together = edge == 128u ? 2u : 4u;
-            const uint64_t   tiles    = (uint64_t)((g.m + edge - 1u) / edge) * ((g.n + edge - 1u) / edge);
+            const uint64_t   tiles    = (uint64_t)r355::tilesOf(g.m, edge) * r355::tilesOf(g.n, edge);
             for(uint32_t s = 1u; s <= splits; ++s)
             {
                 const uint32_t share = (stages + s - 1u) / s;
                 if((stages + share - 1u) / share != s)
                     continue; // a share would be empty
-                if(edge == 64u && tiles * s > (1u << 24) - 8u)
-                    continue; // a launch's threads are counted in 32 bits
                 const uint64_t perCu = (tiles * s + cus - 1u) / cus, rest = perCu % together;
                 auto           round = [&](uint64_t count) {
                     const double each = t.each * static_cast<double>(count);
@@ -2461,7 +2477,7 @@ namespace
         if(g.kernel != R355_KERNEL_AUTO || g.in_type == R355_F32 || g.in_type == R355_F64 || macroTile(g) != 256u)
             return 0u;
         const uint32_t cus   = computeUnits();
-        const uint32_t total = ((g.m + 255u) / 256u) * ((g.n + 255u) / 256u);
+        const uint32_t total = r355::tilesOf(g.m, 256u) * r355::tilesOf(g.n, 256u);
         const uint32_t rest  = total % cus;
         return (total > cus && rest != 0u && rest <= cus / 2u) ? rest : 0u;
     }
@@ -2534,14 +2550,11 @@ namespace r355
         return checkLaunch("gemm (split-K reduction)");
     }
 
-    // workgroups of a launch: its threads (256 each) are counted in 32 bits; a multiple of the eight XCDs
-    constexpr uint32_t MAX_GROUPS = (1u << 24) - 8u;
-
     int dlrmFwdTiled(int32_t dtype, const void* in, void* out, uint32_t m, uint32_t k, uint32_t batch, uint32_t tile, hipStream_t stream)
     {
         GemmTileParams p{};
         p.m = p.n = m, p.k = p.lda = p.ldb = k;
-        p.tilesM = p.tilesN = (m + tile - 1u) / tile;
+        p.tilesM = p.tilesN = tilesOf(m, tile);
         const uint32_t pairs = p.tilesM * (p.tilesM + 1u) / 2u;
         const uint64_t es = dtypeBytes(dtype), stride = (uint64_t)k + (uint64_t)m * (m - 1u) / 2u;
         if(pairs > MAX_GROUPS)
@@ -2567,7 +2580,7 @@ namespace r355
     {
         DlrmBwdParams p{};
         p.m = m, p.k = k;
-        p.tilesM = (m + tile - 1u) / tile, p.tilesN = (k + tile - 1u) / tile;
+        p.tilesM = tilesOf(m, tile), p.tilesN = tilesOf(k, tile);
         const uint64_t es = dtypeBytes(dtype), stride = (uint64_t)k + (uint64_t)m * (m - 1u) / 2u;
         const uint64_t tiles = (uint64_t)p.tilesM * p.tilesN;
         if(tiles > MAX_GROUPS)
@@ -2625,8 +2638,9 @@ namespace r355
             plan->macro_tile_m = tile; // (the nominal plan: tileRows may narrow the tiles that a launch takes)
             plan->macro_tile_n = tile;
             plan->macro_tile_k = tk;
-            // with mixed tiling: the first launch (the second covers mixedRemainder(g) tile indices on 128 x 128 tiles)
-            plan->grid_x       = ((((g.m + tile - 1) / tile) * ((g.n + tile - 1) / tile) - mixedRemainder(g) + 7u) / 8u) * 8u;
+            // the first launch: with mixed tiling the second covers mixedRemainder(g) tile indices on 128 x 128 tiles
+            const uint32_t tiles = tilesOf(g.m, tile) * tilesOf(g.n, tile) - mixedRemainder(g);
+            plan->grid_x         = ((tiles < MAX_TILES ? tiles : MAX_TILES) + 7u) / 8u * 8u;
             plan->grid_y       = 1;
             plan->block_x      = THREADS;
             plan->block_y      = 1;
@@ -2671,7 +2685,7 @@ namespace r355
         }
         const TileWork work = tileWork(g);
         const uint32_t tile = work.tile;
-        p.tilesM = (p.m + tile - 1) / tile, p.tilesN = (p.n + tile - 1) / tile;
+        p.tilesM = tilesOf(p.m, tile), p.tilesN = tilesOf(p.n, tile);
         p.tileFirst = 0u, p.tileCount = p.tilesM * p.tilesN, p.tileQuad = 0u;
         auto part = [&](uint32_t t, const Params& q) {
             switch(g.in_type)
@@ -2723,7 +2737,7 @@ namespace r355
         if(tile == 256u)
             if(const uint32_t rows = tileRows(g); rows != 256u)
             {
-                p.tilesM = (p.m + rows - 1u) / rows, p.tileCount = p.tilesM * p.tilesN;
+                p.tilesM = tilesOf(p.m, rows), p.tileCount = p.tilesM * p.tilesN;
                 return part(rows, p);
             }
         const uint32_t rest = mixedRemainder(g);

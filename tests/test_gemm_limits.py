@@ -1,4 +1,4 @@
-"""Problems at the edge of 32-bit counts: a K of 2^32 bytes and more."""
+"""Problems at the edge of 32-bit counts: a K of 2^32 bytes and more, more tiles than a launch's threads can be counted for."""
 import os
 import subprocess
 import sys
@@ -67,4 +67,38 @@ def test_a_k_beyond_32_bits_of_bytes_is_summed_to_its_end(in_t, out_t, k):
     R.gemm(in_t, out_t, 16, 16, k, a, b, None, d, layout_a=R.COL_MAJOR, layout_b=R.ROW_MAJOR, workspace=ws)
     assert torch.equal(d.double(), want)
     del a, b
+    torch.cuda.empty_cache()
+
+
+# one tile more than 2^24: with 256 threads each, 256 threads more than 32 bits count
+MANY_TILES = [(R.KERNEL_TILED_64, 64), (R.KERNEL_AUTO, 64), (R.KERNEL_TILED_128, 128), (R.KERNEL_AUTO, 128)]
+
+
+@pytest.mark.parametrize("kernel,edge", MANY_TILES)
+def test_a_launch_holds_threads_that_32_bits_count(kernel, edge):
+    plan = R.gemm_query(R.gemm_args(R.F16, R.F16, 16, edge * (2 ** 24 + 1), 8, 0x1000, 0x2000, None, 0x3000, 1.0, 0.0, R.ROW_MAJOR,
+                                    R.COL_MAJOR, R.COL_MAJOR, R.COL_MAJOR, kernel=kernel))
+    assert plan.kernel == R.KERNEL_TILED and 0 < plan.grid_x * plan.block_x < 2 ** 32
+    # the widest problem there is: its tiles are not counted from a rounded-up n that wraps to zero
+    plan = R.gemm_query(R.gemm_args(R.F16, R.F16, 16, 2 ** 32 - 16, 8, 0x1000, 0x2000, None, 0x3000, 1.0, 0.0, R.ROW_MAJOR,
+                                    R.COL_MAJOR, R.COL_MAJOR, R.COL_MAJOR, kernel=kernel))
+    assert 0 < plan.grid_x * plan.block_x < 2 ** 32
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kernel,edge", MANY_TILES)
+def test_more_tiles_than_a_launch_holds(kernel, edge):
+    """The columns of B repeat 24929 tiles' worth, so each of the 673 repetitions has to give the same bits (edge 64: 17 and 34 GB)."""
+    part, copies = edge * 97 * 257, 673  # 97 * 257 * 673 = 2^24 + 1
+    torch.cuda.empty_cache()
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    a = torch.randint(-3, 4, (16, 8), device="cuda", generator=gen).half()
+    b = torch.randint(-3, 4, (part, 8), device="cuda", generator=gen).half()  # col-major 8 x part
+    want = (b.float() @ a.float().t().contiguous()).half()  # col-major 16 x part; sums of 8 products of up to 9: exact
+    b = b.repeat(copies, 1)
+    d = torch.full((copies, part, 16), 77, dtype=torch.float16, device="cuda")
+    R.gemm(R.F16, R.F16, 16, part * copies, 8, a, b, None, d, layout_a=R.ROW_MAJOR, layout_b=R.COL_MAJOR, layout_c=R.COL_MAJOR,
+           layout_d=R.COL_MAJOR, kernel=kernel)
+    assert all(torch.equal(d[i], want) for i in range(copies))
+    del b, d
     torch.cuda.empty_cache()
