@@ -18,7 +18,7 @@ def _small_integers(seed, n, dtype):
 
 
 # (features, width, batch): partial tiles of 64 and 128, one and several tiles, K tails and stage counts around the six-stage
-# loop, batches that leave XCDs unevenly loaded; the last two are large enough for the 128 x 128 tile of the 16-bit types
+# loop, batches that leave XCDs unevenly loaded; the last is large enough for the 128 x 128 tile of the 16-bit types
 @pytest.mark.parametrize("dtype", [O.F16, O.BF16, O.F32])
 @pytest.mark.parametrize("m,k,batch", [(32, 176, 5), (48, 272, 3), (64, 16, 1500), (80, 336, 9), (128, 384, 2), (144, 448, 17), (272, 96, 33), (272, 512, 86),
                                        (144, 1040, 81)])
@@ -40,7 +40,7 @@ def test_forward_on_the_large_tile(dtype, m, k, batch):
 
 
 # backward: one tile and several, so that stages left of, in and right of the diagonal tile all occur, partial tiles and K stages,
-# widths off the tile's edge, samples spread unevenly over the XCDs; shapes for both macro tiles and for the kernels below them
+# widths off the tile's edge, samples spread unevenly over the XCDs; all but the first, which runs a block per wave, on the 64 x 64 tile
 @pytest.mark.parametrize("dtype", [O.F16, O.BF16, O.F32])
 @pytest.mark.parametrize("m,k,batch", [(16, 80, 9), (32, 176, 5), (48, 272, 3), (64, 16, 700), (80, 80, 41), (128, 384, 2), (144, 448, 17), (272, 96, 33),
                                        (336, 272, 40), (400, 144, 3), (528, 272, 24)])
@@ -57,6 +57,56 @@ def test_backward_on_macro_tiles(dtype, m, k, batch):
     if dtype != O.F32:
         g, w = O.storage_to_f32(g, dtype), O.storage_to_f32(w, dtype)
     assert np.array_equal(g, w)
+
+
+def _backward_of_repeated_samples(dtype, m, k, batch, off=0, distinct=3):
+    """A batch that goes round `distinct` samples, so that the oracle has only those to do; every sample of the batch against its own.
+    off: upstream and mlp_grad start that many elements behind a 16-byte boundary."""
+    store, stride = O.NP_STORAGE[dtype], k + m * (m - 1) // 2
+    es = np.dtype(store).itemsize
+    x, up = _small_integers(31 + m, distinct * m * k, dtype), _small_integers(32 + m, distinct * stride, dtype)
+    want_mlp, want_grad = O.dlrm_bwd(dtype, x, up, m, k, distinct)
+    turn = np.arange(batch) % distinct
+    held = to_device(np.concatenate([np.zeros(off, store), up.reshape(distinct, stride)[turn].ravel()]))
+    dmlp, dgrad = device_filled(off + batch * k + 8, store, 0xEE), device_filled(batch * m * k + 8, store, 0xEE)
+    R.dlrm_bwd(dtype, to_device(x.reshape(distinct, m * k)[turn]), held.data_ptr() + off * es, dmlp.data_ptr() + off * es, dgrad, m, k, batch)
+    mlp, grad = to_host(dmlp, store), to_host(dgrad, store)
+    assert np.all(mlp[:off].view(np.uint8) == 0xEE) and np.all(mlp[off + batch * k:].view(np.uint8) == 0xEE)
+    assert np.all(grad[batch * m * k:].view(np.uint8) == 0xEE)
+    assert np.array_equal(mlp[off:off + batch * k].reshape(batch, k).view(np.uint8), want_mlp.reshape(distinct, k)[turn].view(np.uint8))
+    g, w = grad[:batch * m * k], want_grad.ravel()  # (values: -0.0 and +0.0 are the same gradient)
+    if dtype != O.F32:
+        g, w = O.storage_to_f32(g, dtype), O.storage_to_f32(w, dtype)
+    assert np.array_equal(g.reshape(batch, m * k), w.reshape(distinct, m * k)[turn])
+
+
+# the 128 x 128 tile of the backward: from 768 features on with two tiles a CU (512).  Stages left of, in and right of the diagonal tile; a partial
+# last row tile, column tile and K stage; whole tiles; a single narrow column tile
+@pytest.mark.parametrize("dtype", [O.F16, O.BF16, O.F32])
+@pytest.mark.parametrize("m,k,batch", [(784, 144, 37), (768, 128, 86), (784, 16, 74), (912, 272, 22)])
+def test_backward_on_the_large_tile(dtype, m, k, batch):
+    _backward_of_repeated_samples(dtype, m, k, batch)
+
+
+# what is left for the register-blocked fragment-API kernel, launches of 2048 of its waves or more: up to 16 features, and upstream and
+# mlp_grad off 16-byte boundaries.  Whole and partial blocks of 2 x 4; (16, 80, 65576) is also more than one launch's grid holds
+@pytest.mark.parametrize("dtype", [O.F16, O.BF16, O.F32])
+@pytest.mark.parametrize("m,k,batch,off", [(16, 80, 1100, 0), (16, 272, 500, 0), (16, 80, 65576, 0), (80, 96, 700, 1), (112, 48, 600, 1), (256, 256, 64, 1)])
+def test_backward_on_the_register_blocked_kernel(dtype, m, k, batch, off):
+    _backward_of_repeated_samples(dtype, m, k, batch, off)
+
+
+def test_forward_of_16_features_beyond_one_grid_dimension():
+    """A block per wave, the batch a grid dimension of at most 65535: two launches."""
+    m, k, batch, distinct = 16, 80, 65576, 3
+    stride = k + m * (m - 1) // 2
+    x, turn = _small_integers(41, distinct * m * k, O.F16), np.arange(batch) % distinct
+    dout = device_filled(batch * stride + 8, np.uint16, 0xEE)
+    R.dlrm_fwd(O.F16, to_device(x.reshape(distinct, m * k)[turn]), dout, m, k, batch)
+    out = to_host(dout, np.uint16)
+    assert np.all(out[batch * stride:] == 0xEEEE)
+    want = O.dlrm_fwd(O.F16, x, m, k, distinct).reshape(distinct, stride)
+    assert np.array_equal(out[:batch * stride].reshape(batch, stride), want[turn])
 
 
 def test_backward_with_an_upstream_off_16_bytes():
