@@ -129,13 +129,14 @@ int r355_gemm(const r355_gemm_args* args, void* stream);
  * (the values the reference computes on the host: samples/perf_hgemm.cpp:807-817).
  * R355_KERNEL_AUTO may split a problem of several rounds of 256 x 256 tiles into two launches on the
  * same stream - whole rounds on that tile, the rest (at most half a round) on 128 x 128 tiles; the
- * plan then describes the first launch.  16-bit and int8 problems may run as one launch of tiles of 224 or 192 rows (columns
- * of a col-major D) by 256 instead, where a timing model prices that as faster.  It may also work a problem of 128 x 128 tiles as 64 x 64 quarters of them
- * (R355_KERNEL_TILED_64: four workgroups of a quarter of the LDS per tile) and with fewer K splits than planned, where
- * a timing model prices that as faster; the plan then describes the 128 x 128 tiling and the most workspace a launch uses. */
+ * plan then describes the first launch.
+ * This is the nominal plan: the kernel family, a tiling by 256 x 256 or 128 x 128 tiles and the most workspace that a call
+ * uses.  Where a timing model prices it as faster R355_KERNEL_AUTO runs 16-bit and int8 problems of 256 x 256 tiles in one
+ * launch of tiles of 224 or 192 rows (columns of a col-major D) by 256, and problems of 128 x 128 tiles on 64 x 64 ones
+ * (R355_KERNEL_TILED_64) and with fewer K splits: r355_gemm_launch_plan reports what a call launches. */
 typedef struct
 {
-    int32_t  kernel;                       /* r355_gemm_kernel actually selected */
+    int32_t  kernel;                       /* the family: R355_KERNEL_TILED or R355_KERNEL_SIMPLE */
     uint32_t macro_tile_m, macro_tile_n, macro_tile_k;
     uint32_t grid_x, grid_y, block_x, block_y;
     uint32_t lds_bytes;
@@ -143,6 +144,10 @@ typedef struct
     uint64_t workspace_bytes; /* bytes of `workspace` the plan uses (0 without split-K) */
 } r355_gemm_plan;
 int r355_gemm_query(const r355_gemm_args* args, r355_gemm_plan* plan);
+
+/* What r355_gemm launches for exactly these arguments, the workspace that they name included: the macro tile that runs, the grid
+ * of the (first) launch, the K splits and the bytes of workspace that they write.  No counterpart in the reference. */
+int r355_gemm_launch_plan(const r355_gemm_args* args, r355_gemm_plan* plan);
 
 /* r355_gemm for callers that cannot allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc) and have no workspace to pass.  No counterpart in the reference.

@@ -25,7 +25,7 @@ KERNEL_TILED_64 = 7
 DTYPE_BYTES = {F16: 2, BF16: 2, E4M3: 1, I8: 1, F32: 4, I32: 4, F64: 8, E5M2: 1}
 
 EXPORTS = [
-    "r355_gemm", "r355_gemm_noalloc", "r355_gemm_query", "r355_gemm_timed", "r355_dlrm_fwd", "r355_dlrm_fwd_timed",
+    "r355_gemm", "r355_gemm_noalloc", "r355_gemm_query", "r355_gemm_launch_plan", "r355_gemm_timed", "r355_dlrm_fwd", "r355_dlrm_fwd_timed",
     "r355_dlrm_bwd", "r355_gemv", "r355_gemv_timed", "r355_dgemv", "r355_gemv_workspace_bytes", "r355_gemv_ws", "r355_dgemv_ws", "r355_compress_24", "r355_decompress_24", "r355_compress_24_16", "r355_decompress_24_16",
     "r355_get_device_info", "r355_last_error", "r355_version",
 ]
@@ -89,6 +89,7 @@ def lib():
         L.r355_gemm.argtypes = [ctypes.POINTER(GemmArgs), vp]
         L.r355_gemm_noalloc.argtypes = [ctypes.POINTER(GemmArgs), vp]
         L.r355_gemm_query.argtypes = [ctypes.POINTER(GemmArgs), ctypes.POINTER(GemmPlan)]
+        L.r355_gemm_launch_plan.argtypes = [ctypes.POINTER(GemmArgs), ctypes.POINTER(GemmPlan)]
         L.r355_gemm_timed.argtypes = [ctypes.POINTER(GemmArgs), vp, ctypes.c_int, ctypes.c_int, fp]
         L.r355_dlrm_fwd.argtypes = [i32, vp, vp, u32, u32, u32, vp]
         L.r355_dlrm_fwd_timed.argtypes = [i32, vp, vp, u32, u32, u32, vp, ctypes.c_int, ctypes.c_int, fp]
@@ -205,6 +206,13 @@ def gemm_noalloc(g, stream=None):
 def gemm_query(g):
     plan = GemmPlan()
     _check(lib().r355_gemm_query(ctypes.byref(g), ctypes.byref(plan)))
+    return plan
+
+
+def gemm_launch_plan(g):
+    """What r355_gemm launches for exactly these GemmArgs: tile, grid, K splits, workspace (gemm_query: the nominal plan)."""
+    plan = GemmPlan()
+    _check(lib().r355_gemm_launch_plan(ctypes.byref(g), ctypes.byref(plan)))
     return plan
 
 

@@ -225,6 +225,23 @@ int r355_gemm_query(const r355_gemm_args* args, r355_gemm_plan* out)
     return plan(args, out, &family);
 }
 
+int r355_gemm_launch_plan(const r355_gemm_args* args, r355_gemm_plan* out)
+{
+    if(!out)
+        return r355::fail(R355_ERR_BAD_ARG, "gemm_launch_plan: plan is null");
+    int32_t family = 0;
+    int     rc     = plan(args, nullptr, &family); // (the checks of r355_gemm itself)
+    if(rc != R355_OK)
+        return rc;
+    out->split_k = 1u, out->workspace_bytes = 0u;
+    if(family == -1)
+        return r355::gemmSparseCheck(*args, out);
+    if(family == R355_KERNEL_SIMPLE)
+        return r355::gemmSimpleCheck(*args, out);
+    r355::gemmTiledLaunchPlan(*args, out);
+    return R355_OK;
+}
+
 int r355_gemm_timed(const r355_gemm_args* args, void* stream, int warmup, int iters, float* avg_ms)
 {
     int32_t family = 0;

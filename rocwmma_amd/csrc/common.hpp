@@ -83,6 +83,7 @@ namespace r355
     int gemmSimpleCheck(const r355_gemm_args& g, r355_gemm_plan* plan);
     int gemmSimpleLaunch(const r355_gemm_args& g, hipStream_t stream);
     int gemmTiledCheck(const r355_gemm_args& g, r355_gemm_plan* plan);
+    void gemmTiledLaunchPlan(const r355_gemm_args& g, r355_gemm_plan* plan); // of a problem that gemmTiledCheck takes
     int gemmTiledLaunch(const r355_gemm_args& g, hipStream_t stream);
     int gemmSparseCheck(const r355_gemm_args& g, r355_gemm_plan* plan);
     int gemmSparseLaunch(const r355_gemm_args& g, hipStream_t stream);

@@ -2520,6 +2520,20 @@ namespace
                 best = rows, bestTime = t;
         return best;
     }
+
+    // What a call launches, as r355_gemm_launch_plan reports it and gemmTiledLaunch runs it
+    struct LaunchShape
+    {
+        uint32_t tile, rows; // macro tile: rows x tile (rows of D as the kernel sees it: columns of a col-major one)
+        uint32_t splits; // shares of K
+        uint32_t rest; // tile indices left to a second launch on 128 x 128 tiles
+    };
+    LaunchShape launchShape(const r355_gemm_args& g)
+    {
+        const TileWork work = tileWork(g);
+        const uint32_t rows = work.tile == 256u ? tileRows(g) : work.tile;
+        return {work.tile, rows, work.splits, rows == 256u ? mixedRemainder(g) : 0u};
+    }
 #endif // part 0
 } // namespace
 
@@ -2635,7 +2649,7 @@ namespace r355
         if(plan)
         {
             plan->kernel       = R355_KERNEL_TILED;
-            plan->macro_tile_m = tile; // (the nominal plan: tileRows may narrow the tiles that a launch takes)
+            plan->macro_tile_m = tile; // (the nominal plan: tileWork and tileRows may choose smaller tiles, gemmTiledLaunchPlan has them)
             plan->macro_tile_n = tile;
             plan->macro_tile_k = tk;
             // the first launch: with mixed tiling the second covers mixedRemainder(g) tile indices on 128 x 128 tiles
@@ -2655,6 +2669,25 @@ namespace r355
                         "tiled gemm (split-K): needs a workspace of splits x m x n accumulator elements (r355_gemm_query with a large "
                         "workspace_bytes reports the size), at most half as many 128 x 128 tiles as CUs and k of at least 16 stages of 128 bytes");
         return R355_OK;
+    }
+
+    void gemmTiledLaunchPlan(const r355_gemm_args& g, r355_gemm_plan* plan)
+    {
+        const LaunchShape shape = launchShape(g);
+        const uint32_t    es    = dtypeBytes(g.in_type), tile = shape.tile;
+        const bool        dRow  = g.layout_d == R355_ROW_MAJOR, fiveBuffers = es != 2u || tile != 256u || shape.rows != 256u || deepPipeline(g);
+        const uint32_t    tiles = tilesOf(dRow ? g.m : g.n, shape.rows) * tilesOf(dRow ? g.n : g.m, tile) - shape.rest;
+        plan->kernel            = R355_KERNEL_TILED;
+        plan->macro_tile_m      = dRow ? shape.rows : tile;
+        plan->macro_tile_n      = dRow ? tile : shape.rows;
+        plan->macro_tile_k      = STAGE_KB / es;
+        plan->grid_x            = ((tiles < MAX_TILES ? tiles : MAX_TILES) + 7u) / 8u * 8u;
+        plan->grid_y            = shape.splits;
+        plan->block_x           = THREADS;
+        plan->block_y           = 1;
+        plan->lds_bytes         = (fiveBuffers ? 5u * OPER_BYTES : NUM_STAGES * STAGE_BYTES) * tile / 256u;
+        plan->split_k           = shape.splits;
+        plan->workspace_bytes   = shape.splits > 1u ? (uint64_t)shape.splits * g.m * g.n * accBytes(g.in_type) : 0u;
     }
 
     int gemmTiledLaunch(const r355_gemm_args& g, hipStream_t stream)
@@ -2683,9 +2716,9 @@ namespace r355
             p.lda = g.ldb, p.ldb = g.lda;
             aK = g.layout_b == R355_COL_MAJOR, bK = g.layout_a == R355_ROW_MAJOR;
         }
-        const TileWork work = tileWork(g);
-        const uint32_t tile = work.tile;
-        p.tilesM = tilesOf(p.m, tile), p.tilesN = tilesOf(p.n, tile);
+        const LaunchShape shape = launchShape(g);
+        const uint32_t    tile  = shape.tile;
+        p.tilesM = tilesOf(p.m, shape.rows), p.tilesN = tilesOf(p.n, tile);
         p.tileFirst = 0u, p.tileCount = p.tilesM * p.tilesN, p.tileQuad = 0u;
         auto part = [&](uint32_t t, const Params& q) {
             switch(g.in_type)
@@ -2707,7 +2740,7 @@ namespace r355
             return v ? static_cast<uint32_t>(atoi(v)) : 0u;
         }();
         p.stagger = staggerTicks, p.staggerBlocks = computeUnits();
-        const uint32_t splits = work.splits;
+        const uint32_t splits = shape.splits;
         if(splits > 1u)
         {
             // partial results in the accumulator type, row-major with leading dimension n, alpha = 1 and beta = 0; the
@@ -2734,15 +2767,9 @@ namespace r355
             }();
             return rc != R355_OK ? rc : splitKReduce(g, p, splits, stream);
         }
-        if(tile == 256u)
-            if(const uint32_t rows = tileRows(g); rows != 256u)
-            {
-                p.tilesM = tilesOf(p.m, rows), p.tileCount = p.tilesM * p.tilesN;
-                return part(rows, p);
-            }
-        const uint32_t rest = mixedRemainder(g);
+        const uint32_t rest = shape.rest;
         if(rest == 0u)
-            return part(tile, p);
+            return part(shape.rows, p);
         // whole rounds on 256 x 256 tiles, then the rest of the walk on 128 x 128 tiles, four per index
         Params big = p, small = p;
         big.tileCount   = p.tileCount - rest;

@@ -50,10 +50,12 @@ def test_tile_64_random_inputs(in_t, out_t, la, lb):
     _check(in_t, out_t, _run(in_t, out_t, la, lb, O.ROW, O.ROW, m, n, k, a, b, c, 2.0, -1.0, R.KERNEL_TILED_64), want, w32)
 
 
-@pytest.mark.parametrize("in_t,out_t,m,n,kbytes", [(O.F64, O.F64, 192, 160, 3200), (O.F32, O.F32, 720, 832, 3136), (O.F16, O.F16, 64, 1024, 16384),
-                                                   (O.E4M3, O.F32, 96, 4912, 4400), (O.I8, O.I32, 48, 2048, 5104)])
+# ... and the tile's edge and the number of K splits that it runs on 256 CUs
+@pytest.mark.parametrize("in_t,out_t,m,n,kbytes,edge,splits", [(O.F64, O.F64, 192, 160, 3200, 64, 3), (O.F32, O.F32, 720, 832, 3136, 64, 1),
+                                                               (O.F16, O.F16, 64, 1024, 16384, 64, 16), (O.E4M3, O.F32, 96, 4912, 4400, 128, 4),
+                                                               (O.I8, O.I32, 48, 2048, 5104, 64, 5)])
 @pytest.mark.parametrize("la,lb", [(O.ROW, O.COL), (O.COL, O.ROW)])
-def test_auto_with_a_workspace_whatever_tile_and_split_it_takes(in_t, out_t, m, n, kbytes, la, lb):
+def test_auto_with_a_workspace_whatever_tile_and_split_it_takes(in_t, out_t, m, n, kbytes, edge, splits, la, lb):
     k = kbytes // np.dtype(O.NP_STORAGE[in_t]).itemsize
     if in_t == O.I8:
         a, b, c = O.uniform_int8(4, m * k), O.uniform_int8(5, k * n), O.uniform_int8(6, m * n).astype(np.int32)
@@ -66,6 +68,8 @@ def test_auto_with_a_workspace_whatever_tile_and_split_it_takes(in_t, out_t, m, 
     assert need > 0
     ws = device_filled(need + 4096, np.uint8, 0xFF)
     g = R.gemm_args(*args, workspace=ws, workspace_bytes=need)
+    plan = R.gemm_launch_plan(g)
+    assert (plan.macro_tile_m, plan.macro_tile_n, plan.split_k) == (edge, edge, splits)
     R._check(R.lib().r355_gemm(R.ctypes.byref(g), None))
     assert np.array_equal(to_host(dd, O.NP_STORAGE[out_t]), want)
     assert np.all(to_host(ws, np.uint8)[need:] == 0xFF)  # nothing behind the bytes that the plan reports
