@@ -79,6 +79,10 @@ namespace r355
         return cus;
     }
 
+    // Workgroups of a launch: its threads (256 each) are counted in 32 bits, and a launch of more runs what is left modulo 2^32
+    // and reports success.  A multiple of the eight XCDs.
+    constexpr uint32_t MAX_GROUPS = (1u << 24) - 8u;
+
     // Kernel families (defined in their own translation units)
     int gemmSimpleCheck(const r355_gemm_args& g, r355_gemm_plan* plan);
     int gemmSimpleLaunch(const r355_gemm_args& g, hipStream_t stream);

@@ -324,7 +324,8 @@ namespace
     //     against 12.3; with fewer tiles 592 x 368 x 6 6.3 against 5.4, 560 x 144 x 7 5.3 against 4.5; padded, 272 x 528 x 96 18.3 against
     //     16.7) - or where every CU gets 32 K stages (272 x 1024 x 128: 26.8 against 28.3).  Up to 192 features, where every CU gets 16 K
     //     stages of such tiles.  A 256 x 256 tile gains 2 - 5 % at 768 and 1024 features and loses up to half below: not built in.
-    //   * f32, bound by its matrix instructions, is faster on 64 x 64 throughout (1024 x 1024 x 64: 565 against 590 us).
+    //   * f32, bound by its matrix instructions, is faster on 64 x 64 throughout (1024 x 1024 x 64: 565 against 590 us); a sample of more
+    //     such tiles than a launch holds (370704 features and more: a result of 256 GiB) takes the 128 x 128 ones.
     // Leading dimensions beyond 8 MiB per row do not fit the tile kernels' 32-bit lane offsets.
     uint32_t forwardTile(int32_t dtype, uint32_t m, uint32_t k, uint32_t batch)
     {
@@ -337,13 +338,13 @@ namespace
         const uint64_t blocks = m / BLK, waves = blocks * (blocks + 1u) / 2u * batch, steps = k / (es == 2u ? 16u : 4u);
         if(waves <= 5u * cus && steps <= 12u)
             return 0u;
-        if(es != 2u)
-            return 64u;
         auto pairs = [&](uint64_t edge) {
             const uint64_t tiles = (m + edge - 1u) / edge;
-            return tiles * (tiles + 1u) / 2u * batch;
+            return tiles * (tiles + 1u) / 2u;
         };
-        const uint64_t large = pairs(128u), small = pairs(64u), stages = (k * es + 127u) / 128u;
+        if(es != 2u)
+            return pairs(64u) <= r355::MAX_GROUPS ? 64u : 128u;
+        const uint64_t large = pairs(128u) * batch, small = pairs(64u) * batch, stages = (k * es + 127u) / 128u;
         if(m <= 192u)
             return large * stages >= 16u * cus ? 128u : 64u;
         return 5u * large >= 3u * cus && (50u * large <= 19u * small || large * stages >= 32u * cus) ? 128u : 64u;

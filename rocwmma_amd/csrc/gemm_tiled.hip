@@ -133,9 +133,6 @@ namespace r355
     {
         return (n - 1u) / edge + 1u;
     }
-    // Workgroups of a launch: its threads (256 each) are counted in 32 bits, and a launch of more runs what is left modulo 2^32
-    // and reports success.  A multiple of the eight XCDs.
-    constexpr uint32_t MAX_GROUPS = (1u << 24) - 8u;
     // Tile indices of a GEMM launch, a multiple of eight: four workgroups of 256 threads each (tileQuad) stay within that.  What a
     // problem has more goes out in further launches.
     constexpr uint32_t MAX_TILES = MAX_GROUPS / 32u * 8u;
