@@ -2349,7 +2349,8 @@ namespace
     // CUs that few 128 x 128 tiles leave idle, and its stages are shorter.  The choice is the cheapest by a timing model of
     // a launch: a CU takes its workgroups `together` (2 or 4) at a time; such a round costs `fixed` plus, per K stage, the
     // longer of one stage's latency and what its workgroups need one after the other.  Microseconds, fitted to 250 random
-    // shapes per class (m, n from 16 to 8192, all orientations; root mean square of the error 5 % for f32 / f64, 13 % for 8- and 16-bit):
+    // shapes per class (m, n from 16 to 8192, all orientations; root mean square of the error 5 % for f32 / f64, 13 % for 8- and 16-bit;
+    // profiles/tile_choice_survey.md has what the choices give on further ones):
     //                        128 x 128                        64 x 64
     //            fixed   latency   per workgroup    fixed   latency   per workgroup
     //   8-bit     3.9     0.46        0.46           2.6     0.28        0.27
@@ -2392,7 +2393,8 @@ namespace
                 const uint32_t share = (stages + s - 1u) / s;
                 if((stages + share - 1u) / share != s)
                     continue; // a share would be empty
-                const uint64_t perCu = (tiles * s + cus - 1u) / cus, rest = perCu % together;
+                // (an XCD's share of the tiles, times the splits, over its CUs: 84 tiles x 3 are 33 on the first seven XCDs of 32 CUs)
+                const uint64_t perXcd = (tiles + 7u) / 8u * s, perCu = (perXcd * 8u + cus - 1u) / cus, rest = perCu % together;
                 auto           round = [&](uint64_t count) {
                     const double each = t.each * static_cast<double>(count);
                     return t.fixed + share * (each > t.latency ? each : t.latency);
@@ -2406,9 +2408,13 @@ namespace
                     best = {edge, s}, bestTime = time;
             }
         }
-        // 8- and 16-bit: within the model's error the plan stays (of 430 shapes 8 are then slower than planned, by 3 - 10 %; 24
-        // without the margin, by up to 19 %)
-        if(es <= 2u && bestTime > 0.88 * plannedTime)
+        // 8- and 16-bit: where the model's lead is within its error the plan stays.  That is most where three or more splits are given up
+        // (e4m3 96 x 8000 x 4672 14.9 -> 17.9 us at a lead of 0.83, bf16 2080 x 432 x 2208 15.0 -> 15.6 at 0.82) and for a K of up to 8
+        // stages (f16 1120 x 1856 x 256 6.5 -> 7.0 at 0.85).  f32 and f64 need none.  Of 2000 further random shapes one is slower than
+        // as planned by more than 3 % (e4m3 1712 x 80 x 4384 14.6 -> 15.4); 8-bit ones run 1.29 times, 16-bit ones 1.27 times and f32 and
+        // f64 ones 2.2 times as fast as planned in the geometric mean.
+        const double margin = splits >= 3u && best.splits == 1u ? 0.70 : stages <= 8u ? 0.80 : 0.86;
+        if(es <= 2u && bestTime > margin * plannedTime)
             return {tile, splits};
         return best;
     }
@@ -2487,9 +2493,10 @@ namespace
     //     rounds (fixed + out h) + stages stage h (spread mean + (1 - spread) rounds) microseconds,    h = rows / 256,
     // because the board's power limit lets CUs that share the chip with idle ones run faster.  Fitted to 117 (16-bit) and 75
     // (int8) random shapes from 1500 x 1500 x 700 to 8192^3, all orientations: fixed 8.32 / 7.76, out (results of 32 bits) 2.72 / 3.89,
-    // stage 1.41 / 1.50, spread 0.52 / 0.58.  On these shapes the model's choices run 1.08 (16-bit) and 1.045 (int8) times as fast as
-    // 256 x 256 with its remainder launch - the best of the three for each shape would be 1.081 and 1.046 - and none of them is slower
-    // by more than the runs differ: bf16 2832 x 4624 x 3080 72.8 -> 65.4 us, int8 5120^3 112 -> 109.6, bf16 4880 x 4624 x 4528 194 -> 166.
+    // stage 1.41 / 1.50, spread 0.52 / 0.58.  Of 300 further shapes none is slower than 256 x 256 with its remainder launch by more than
+    // 3 %, and in the geometric mean they run 1.05 times as fast (1.10 where another tile is taken): bf16 2832 x 4624 x 3080 72.8 -> 65.4 us,
+    // int8 5120^3 112 -> 109.6, bf16 4880 x 4624 x 4528 194 -> 166.  (fp8 operands stay on 256 rows: their K loop works the quadrants of an
+    // 8 x 8 wave tile, see gemmTiledF8, and has no narrower form.)
     uint32_t tileRows(const r355_gemm_args& g)
     {
         const bool eight = g.in_type == R355_I8;
@@ -2510,10 +2517,12 @@ namespace
                 rounds += 1.0;
             return rounds * (fixed + out * h) + stages * stage * h * (spread * mean + (1.0 - spread) * rounds) + launch;
         };
-        uint32_t best     = 256u;
-        double   bestTime = 0.99 * time(256u);
+        const double planned  = time(256u);
+        uint32_t     best     = 256u;
+        double       bestTime = planned;
+        // (192 rows within 3 % of 256 were up to 5 % slower: int8 2160 x 7984 x 7504 133 -> 139 us, bf16 3584 x 4960 x 7488 215 -> 223)
         for(const uint32_t rows : {224u, 192u})
-            if(const double t = time(rows); t < bestTime)
+            if(const double t = time(rows); t < (rows == 224u ? 0.99 : 0.97) * planned && t < bestTime)
                 best = rows, bestTime = t;
         return best;
     }
