@@ -174,8 +174,8 @@ int r355_gemm_timed(const r355_gemm_args* args, void* stream, int warmup, int it
  * order, f32 accumulation, rounded to dtype (R355_F16, R355_BF16 or R355_F32).  Bandwidth-bound kernels for
  * 2 <= m <= 32 with k in {32, 64, 128, 256} (R355_F32: up to 128); any other m and k that are multiples of 16 - the
  * reference's own constraint, test/dlrm/dlrm_kernel_base_impl.hpp:146-151; its tests run m = 128, k = 128 and m = k = 1024 -
- * run kernels written on the fragment API (a 16 x 16 block per wave for small launches, several blocks per wave otherwise;
- * any batch).  No scratch buffer either way (the reference's `acc` argument is gone).
+ * run on the GEMM's macro tiles or with a 16 x 16 block per wave on the fragment API, whichever a timing model prices as faster
+ * (r355_dlrm_kernel; any batch).  No scratch buffer either way (the reference's `acc` argument is gone).
  * Replaces: dlrmDotFwd launch, test/dlrm/dlrm_kernel_base_impl.hpp:78-96,
  * test/dlrm/device/dlrm_dot_fwd.hpp:35-138, samples/simple_dlrm.cpp:184-284.
  */
@@ -186,12 +186,24 @@ int r355_dlrm_fwd_timed(int32_t dtype, const void* in, void* out, uint32_t m, ui
 /*
  * DLRM dot-interaction backward.  upstream: [batch][k + m(m-1)/2]; mlp_grad: [batch][k];
  * in_grad: [batch][m][k].  dtype R355_F16, R355_BF16 (all four pointers 16-byte aligned) or R355_F32
- * (in / in_grad 16-byte, upstream / mlp_grad 4-byte aligned).  Shapes as for the forward call; the general kernels form S = T + T^T
- * block by block from the packed triangle instead of reconstructing it in memory.  Replaces: dlrmDotBwd +
+ * (in / in_grad 16-byte, upstream / mlp_grad 4-byte aligned).  Shapes as for the forward call; the general kernels (macro tiles, one
+ * or several blocks per wave) form S = T + T^T block by block from the packed triangle instead of reconstructing it in memory.  Replaces: dlrmDotBwd +
  * trilReconstruct launches, test/dlrm/device/dlrm_dot_bwd.hpp:35-176.
  */
 int r355_dlrm_bwd(int32_t dtype, const void* in, const void* upstream, void* mlp_grad, void* in_grad,
                   uint32_t m, uint32_t k, uint32_t batch, void* stream);
+
+/* Which kernel r355_dlrm_fwd (backward = 0) or r355_dlrm_bwd runs for a shape on the current device: an r355_dlrm_kernel_id, or the
+ * negative status with which the call is refused.  aligned16: upstream and mlp_grad both keep 16-byte alignment (backward only). */
+typedef enum
+{
+    R355_DLRM_KERNEL_SPECIALISED      = 1, /* the bandwidth-bound kernels */
+    R355_DLRM_KERNEL_BLOCK_PER_WAVE   = 2, /* fragment API, a 16 x 16 block per wave */
+    R355_DLRM_KERNEL_REGISTER_BLOCKED = 3, /* fragment API, several blocks per wave (backward) */
+    R355_DLRM_KERNEL_TILED_64         = 64, /* macro tiles of 64 x 64 */
+    R355_DLRM_KERNEL_TILED_128        = 128 /* macro tiles of 128 x 128 */
+} r355_dlrm_kernel_id;
+int r355_dlrm_kernel(int32_t dtype, int32_t backward, uint32_t m, uint32_t k, uint32_t batch, int32_t aligned16);
 
 /*
  * y_out = alpha * A * x + beta * y_in.  A is m x k f32 (layout_a), x has k elements, y m.

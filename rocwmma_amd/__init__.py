@@ -21,12 +21,14 @@ ROW_MAJOR, COL_MAJOR = 0, 1
 # r355_gemm_kernel
 KERNEL_AUTO, KERNEL_SIMPLE, KERNEL_TILED, KERNEL_TILED_128, KERNEL_TILED_128_SPLITK, KERNEL_TILED_DEEP = range(6)
 KERNEL_TILED_64 = 7
+# r355_dlrm_kernel_id
+DLRM_KERNEL_SPECIALISED, DLRM_KERNEL_BLOCK_PER_WAVE, DLRM_KERNEL_REGISTER_BLOCKED, DLRM_KERNEL_TILED_64, DLRM_KERNEL_TILED_128 = 1, 2, 3, 64, 128
 
 DTYPE_BYTES = {F16: 2, BF16: 2, E4M3: 1, I8: 1, F32: 4, I32: 4, F64: 8, E5M2: 1}
 
 EXPORTS = [
     "r355_gemm", "r355_gemm_noalloc", "r355_gemm_query", "r355_gemm_launch_plan", "r355_gemm_timed", "r355_dlrm_fwd", "r355_dlrm_fwd_timed",
-    "r355_dlrm_bwd", "r355_gemv", "r355_gemv_timed", "r355_dgemv", "r355_gemv_workspace_bytes", "r355_gemv_ws", "r355_dgemv_ws", "r355_compress_24", "r355_decompress_24", "r355_compress_24_16", "r355_decompress_24_16",
+    "r355_dlrm_bwd", "r355_dlrm_kernel", "r355_gemv", "r355_gemv_timed", "r355_dgemv", "r355_gemv_workspace_bytes", "r355_gemv_ws", "r355_dgemv_ws", "r355_compress_24", "r355_decompress_24", "r355_compress_24_16", "r355_decompress_24_16",
     "r355_get_device_info", "r355_last_error", "r355_version",
 ]
 
@@ -94,6 +96,7 @@ def lib():
         L.r355_dlrm_fwd.argtypes = [i32, vp, vp, u32, u32, u32, vp]
         L.r355_dlrm_fwd_timed.argtypes = [i32, vp, vp, u32, u32, u32, vp, ctypes.c_int, ctypes.c_int, fp]
         L.r355_dlrm_bwd.argtypes = [i32, vp, vp, vp, vp, u32, u32, u32, vp]
+        L.r355_dlrm_kernel.argtypes = [i32, i32, u32, u32, u32, i32]
         L.r355_gemv.argtypes = [i32, u32, u32, vp, u32, vp, vp, vp, f32, f32, vp]
         L.r355_gemv_timed.argtypes = [i32, u32, u32, vp, u32, vp, vp, vp, f32, f32, vp, ctypes.c_int, ctypes.c_int, fp]
         L.r355_dgemv.argtypes = [i32, u32, u32, vp, u32, vp, vp, vp, ctypes.c_double, ctypes.c_double, vp]
@@ -237,6 +240,13 @@ def dlrm_fwd_timed(dtype, x, out, m, k, batch, warmup, iters, stream=None):
 def dlrm_bwd(dtype, x, upstream, mlp_grad, in_grad, m, k, batch, stream=None):
     _check(lib().r355_dlrm_bwd(dtype, _ptr(x), _ptr(upstream), _ptr(mlp_grad), _ptr(in_grad), m, k, batch,
                                _stream_handle(stream)))
+
+
+def dlrm_kernel(dtype, m, k, batch, backward=False, aligned16=True):
+    """Which kernel dlrm_fwd or dlrm_bwd runs for a shape (DLRM_KERNEL_*); aligned16: upstream and mlp_grad keep 16-byte alignment."""
+    kernel = lib().r355_dlrm_kernel(dtype, int(backward), m, k, batch, int(aligned16))
+    _check(min(kernel, 0))
+    return kernel
 
 
 def gemv_workspace_bytes(layout_a, m, k, elem_bytes=4):

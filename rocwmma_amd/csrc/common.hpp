@@ -100,6 +100,7 @@ namespace r355
     int dlrmGeneralFwd(int32_t dtype, const void* in, void* out, uint32_t m, uint32_t k, uint32_t batch, hipStream_t stream);
     int dlrmGeneralBwd(int32_t dtype, const void* in, const void* upstream, void* mlpGrad, void* inGrad, uint32_t m, uint32_t k,
                        uint32_t batch, hipStream_t stream);
+    int dlrmGeneralKernel(int32_t dtype, bool backward, uint32_t m, uint32_t k, uint32_t batch, bool aligned16); // r355_dlrm_kernel_id, or an error
 } // namespace r355
 
 #endif // R355_COMMON_HPP

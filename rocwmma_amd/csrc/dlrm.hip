@@ -1287,3 +1287,11 @@ extern "C" int r355_dlrm_bwd(int32_t dtype, const void* in, const void* upstream
 #undef R355_BWD
     return r355::checkLaunch("dlrm_bwd");
 }
+
+extern "C" int r355_dlrm_kernel(int32_t dtype, int32_t backward, uint32_t m, uint32_t k, uint32_t batch, int32_t aligned16)
+{
+    const int rc = checkArgs(backward ? "dlrm_bwd" : "dlrm_fwd", dtype, reinterpret_cast<const void*>(16), reinterpret_cast<const void*>(16), m, k, batch, true);
+    if(rc != R355_OK)
+        return rc;
+    return specialised(dtype, m, k) ? R355_DLRM_KERNEL_SPECIALISED : r355::dlrmGeneralKernel(dtype, backward != 0, m, k, batch, aligned16 != 0);
+}

@@ -5,10 +5,9 @@
 // (dlrm_kernel_base_impl.hpp:146-151) - but without their global scratch: the forward kernels take the lower triangle
 // out of an accumulator block through 1 KiB of the wave's LDS instead of a [batch][m][m] f32 buffer, and the backward
 // kernels form each 16 x 16 block of S = T + T^T in LDS from the packed upstream triangle instead of reconstructing
-// [batch][m][m] in memory first.  These kernels run one 16 x 16 block per wave, as in the reference, and serve small
-// shapes; larger ones go to macro tiles (gemm_tiled.hip).  Backward launches of many blocks that the macro tiles do not take (up
-// to 16 features, pointers off 16-byte alignment) go to a register-blocked kernel: several blocks per wave, so that a fragment
-// feeds several matrix instructions.
+// [batch][m][m] in memory first.  These kernels run one 16 x 16 block per wave, as in the reference, and the backward also several
+// (register-blocked, so that a fragment feeds several matrix instructions); macro tiles (gemm_tiled.hip) take the shapes that
+// they are faster on, by the timing models below.
 #include <rocwmma/rocwmma.hpp>
 
 #include "common.hpp"
@@ -314,59 +313,113 @@ namespace
             }
     }
 
-    // Forward: the macro tile's edge (dlrmFwdTiled in gemm_tiled.hip), or 0 for a block per wave.  Measured on one box:
-    //   * up to 16 features a sample is a single block, and a tile of 64 rows would be three quarters padding
-    //     (16 x 96, batch 4096, f16: 5.3 us a block per wave, 15.7 on 64 x 64 tiles);
-    //   * a launch of a few short waves is over before a tile's K loop has filled its five buffers (64 x 96 x 64 f16: 4.05
-    //     against 4.57 us; at k = 256 5.5 against 4.6, and from 128 x 144 x 64 on, 2304 waves, 5.6 against 4.6);
-    //   * 16-bit types, beyond 192 features (40 shapes of 256 ... 1024 features, f16): the 128 x 128 tile where its launch has 0.6 tiles a CU
-    //     or more and it pads little - at most 0.38 times as many tiles as of 64 x 64 (352 x 928 x 41: 12.7 against 16.5 us; 688 x 816 x 9 10.4
-    //     against 12.3; with fewer tiles 592 x 368 x 6 6.3 against 5.4, 560 x 144 x 7 5.3 against 4.5; padded, 272 x 528 x 96 18.3 against
-    //     16.7) - or where every CU gets 32 K stages (272 x 1024 x 128: 26.8 against 28.3).  Up to 192 features, where every CU gets 16 K
-    //     stages of such tiles.  A 256 x 256 tile gains 2 - 5 % at 768 and 1024 features and loses up to half below: not built in.
-    //   * f32, bound by its matrix instructions, is faster on 64 x 64 throughout (1024 x 1024 x 64: 565 against 590 us); a sample of more
-    //     such tiles than a launch holds (370704 features and more: a result of 256 GiB) takes the 128 x 128 ones.
+#ifdef R355_DLRM_BLOCK_PER_WAVE // measurement build: the block-per-wave kernels for every shape
+    constexpr bool ONLY_BLOCK_PER_WAVE = true;
+#else
+    constexpr bool ONLY_BLOCK_PER_WAVE = false;
+#endif
+
+    // Which kernel a launch runs is the cheapest by a timing model: microseconds as a linear function of the launch's workgroups
+    // (or waves; `groups` in thousands on 256 CUs), their steps along K and one more term.  Fitted by least squares of the relative
+    // error to launches of every kernel on the same random shapes, m from 32 to 1024, k from 16 to 1024, up to 12000 samples
+    // (profiles/tile_choice_survey.md: how well the models do, and what the choices give on further shapes).
+    struct LaunchTime
+    {
+        double fixed, step, group, groupStep, more;
+        double operator()(double steps, double groups, double term) const
+        {
+            return fixed + step * steps + groups * (group + groupStep * steps) + more * term;
+        }
+    };
+    double thousands(uint64_t groups)
+    {
+        return static_cast<double>(groups) / (4.0 * r355::computeUnits());
+    }
+    uint64_t tilesOf(uint32_t n, uint32_t edge)
+    {
+        return (n - 1u) / edge + 1u;
+    }
+    uint64_t triangle(uint64_t rows) // blocks or tiles on and below the diagonal
+    {
+        return rows * (rows + 1u) / 2u;
+    }
+
+    // Forward.  A block per wave (steps of one matrix instruction) has the shortest launch, pads nothing, and re-reads every row of X for
+    // each block of the sample, from lines that collide in the caches where rows are multiples of 128 bytes (the last term: waves times
+    // steps again).  Macro tiles (steps: stages of 128 bytes; the last term: megabytes of input and output) read a row once per 64 or 128
+    // others but pad m to the tile's edge: with few features or a short K most of a tile is padding and fixed cost.  bf16 32 x 48 x 7174: 9.4 us a block
+    // per wave, 22 on 64 x 64 tiles, 51 on 128 x 128 ones; f16 64 x 112 x 2687: 28, 15 and 27; bf16 176 x 576 x 428: 227, 25 and 30; f16
+    // 1024 x 1024 x 64: 96 on 128 x 128 tiles.  Beyond 320 features the model of the block per wave does not reach, and only small launches run it.
+    constexpr LaunchTime FWD_WAVE[2]  = {{2.70, 0.0415, 0.104, 0.124, 0.104}, {2.48, 0.0954, 0.135, 0.225, 0.00649}}; // 16-bit, f32
+    constexpr LaunchTime FWD_64[2]    = {{3.38, 0.00367, 2.13, 0.564, 0.0370}, {3.49, 0.227, 1.95, 1.62, 0.0517}};
+    constexpr LaunchTime FWD_128      = {3.88, 0.124, 5.27, 0.804, 0.0816}; // 16-bit: f32, bound by its matrix instructions, is faster on 64 x 64 throughout
+    constexpr double     FWD_MARGIN   = 0.97; // of the tiles' time that the block per wave may take and still run
+    // The macro tile's edge (dlrmFwdTiled in gemm_tiled.hip), or 0 for a block per wave.  Up to 16 features a sample is a single block.
     // Leading dimensions beyond 8 MiB per row do not fit the tile kernels' 32-bit lane offsets.
     uint32_t forwardTile(int32_t dtype, uint32_t m, uint32_t k, uint32_t batch)
     {
-#ifdef R355_DLRM_BLOCK_PER_WAVE // measurement build: a block per wave for every shape
-        return 0u;
-#endif
-        const uint64_t es = r355::dtypeBytes(dtype), cus = r355::computeUnits();
-        if(m <= BLK || (uint64_t)k * es > (1u << 23))
+        const uint64_t rowBytes = (uint64_t)k * r355::dtypeBytes(dtype);
+        if(ONLY_BLOCK_PER_WAVE || m <= BLK || rowBytes > (1u << 23))
             return 0u;
-        const uint64_t blocks = m / BLK, waves = blocks * (blocks + 1u) / 2u * batch, steps = k / (es == 2u ? 16u : 4u);
-        if(waves <= 5u * cus && steps <= 12u)
-            return 0u;
-        auto pairs = [&](uint64_t edge) {
-            const uint64_t tiles = (m + edge - 1u) / edge;
-            return tiles * (tiles + 1u) / 2u;
-        };
-        if(es != 2u)
-            return pairs(64u) <= r355::MAX_GROUPS ? 64u : 128u;
-        const uint64_t large = pairs(128u) * batch, small = pairs(64u) * batch, stages = (k * es + 127u) / 128u;
-        if(m <= 192u)
-            return large * stages >= 16u * cus ? 128u : 64u;
-        return 5u * large >= 3u * cus && (50u * large <= 19u * small || large * stages >= 32u * cus) ? 128u : 64u;
+        const bool     wide  = dtype == R355_F32;
+        const uint64_t waves = triangle(m / BLK) * batch, steps = k / (wide ? 4u : 16u), stages = (rowBytes + 127u) / 128u;
+        const double   megabytes
+            = 1e-6 * r355::dtypeBytes(dtype) * batch * (static_cast<double>(m) * k + 0.5 * m * (m - 1.0) + static_cast<double>(k));
+        const double small = FWD_64[wide](stages, thousands(triangle(tilesOf(m, 64u)) * batch), megabytes);
+        const double large = FWD_128(stages, thousands(triangle(tilesOf(m, 128u)) * batch), megabytes);
+        const double tiles = wide || small < large ? small : large;
+        if(m <= 320u || waves <= 5u * r355::computeUnits())
+            if(FWD_WAVE[wide](steps, thousands(waves), rowBytes % 128u == 0u ? thousands(waves) * steps : 0.0) <= tiles / FWD_MARGIN)
+                return 0u;
+        // (a sample of more 64 x 64 tiles than a launch holds: f32, 370704 features and more, a result of 256 GiB)
+        return tiles == small && triangle(tilesOf(m, 64u)) <= r355::MAX_GROUPS ? 64u : 128u;
     }
 
-    // Backward: the macro tile's edge (dlrmBwdTiled in gemm_tiled.hip), or 0 for the fragment-API kernels below.  Measured on one
-    // box, 45 shapes (m 48 ... 1024, k 64 ... 1024), against those kernels' 16 x 16 blocks per wave: the 64 x 64 tile is ahead by 1.05
-    // (112 x 800 x 436 bf16: 70.5 -> 61.8 us) to 10 times (1024 x 256 x 4 f16: 96 -> 10.5), and level only where the call itself
-    // is the time (48 x 1024 x 4) and at 80 x 256 x 537 (20.3 / 20.6).  The 128 x 128 tile loads half the bytes per product and is
-    // ahead from 768 features on where it fills the chip (1024 x 1024 x 64 f16: 295 -> 214 us, f32 1024 x 1024 x 16: 295 -> 271;
-    // 880 x 240 x 21: level; 512 x 480 x 41 f32: 107 against 113).  Up to 16 features a tile would be three quarters padding.
-    // The kernel reads upstream and writes mlpGrad in 16-byte pieces; rows beyond 8 MiB do not fit its 32-bit lane offsets.
-    uint32_t backwardTile(int32_t dtype, const void* upstream, const void* mlpGrad, uint32_t m, uint32_t k, uint32_t batch)
+    // Backward.  The fragment-API kernels are a block per wave for launches of few waves and 2 x 4 blocks per wave (the register-blocked
+    // kernel; waves of 32 x 64 of the gradient, workgroups of 32 x 256 that form S once) from eight waves a CU on; macro tiles pad m and the K of
+    // the product, which is m again, to 64 or 128.  f16 32 x 208 x 4021: 23 us register-blocked, 56 on 64 x 64 tiles; f16 80 x 208 x 1410: 34 and 57;
+    // f16 112 x 48 x 1612: 44 and 22; f16 1024 x 256 x 4: 96 a block per wave, 10.5 on 64 x 64; f16 992 x 464 x 27: 117 register-blocked, 72 on 64 x 64,
+    // 58 on 128 x 128 tiles; f16 1024 x 1024 x 64: 473, 295 and 214.
+    // By f16, bf16, f32.  Steps: blocks of 16 rows (fragments), stages of 128 bytes of K (tiles); the last term: megabytes, for the
+    // register-blocked kernel thousands of block products.
+    constexpr LaunchTime BWD_WAVE[3]    = {{1.83, 0.546, 0.0, 0.243, 0.0478}, {2.06, 0.548, 0.0, 0.220, 0.0950}, {1.19, 0.860, 0.0, 0.291, 0.163}};
+    constexpr LaunchTime BWD_BLOCKED[3] = {{2.98, 0.280, 0.977, 0.606, 0.0229}, {4.32, 0.223, 1.20, 0.612, 0.0225}, {2.98, 0.646, 1.38, 0.753, 0.148}};
+    constexpr LaunchTime BWD_64[3]      = {{3.36, 0.257, 1.46, 0.787, 0.122}, {3.45, 0.236, 1.55, 0.790, 0.113}, {2.98, 0.490, 1.24, 2.09, 0.0608}};
+    constexpr LaunchTime BWD_128[3]     = {{3.90, 0.997, 2.80, 1.53, 0.253}, {3.79, 1.11, 2.91, 1.85, 0.210}, {3.34, 1.81, 4.30, 6.64, 0.104}};
+    constexpr uint32_t   NBI = 2, NBK = 4; // blocks per wave of the register-blocked kernel
+    bool backwardBlocked(uint32_t m, uint32_t k, uint32_t count)
     {
-#ifdef R355_DLRM_BLOCK_PER_WAVE
-        return 0u;
-#endif
-        const uint64_t es = r355::dtypeBytes(dtype);
-        if(m <= BLK || (uint64_t)k * es > (1u << 23) || !r355::aligned(upstream, 16) || !r355::aligned(mlpGrad, 16))
+        const uint64_t waves = (uint64_t)((k / BLK + NBK - 1u) / NBK) * ((m / BLK + NBI - 1u) / NBI) * count;
+        return !ONLY_BLOCK_PER_WAVE && waves >= 8ull * r355::computeUnits(); // where that still leaves every SIMD two waves
+    }
+    // The macro tile's edge (dlrmBwdTiled in gemm_tiled.hip), or 0 for the fragment-API kernels: where the tiles' lead is less than the
+    // models' error (at up to 48 features, a tile of 64 mostly padded, 22 %, else 12 %) those stay.  The tile kernel reads upstream and writes
+    // mlpGrad in 16-byte pieces (`aligned`); rows beyond 8 MiB do not fit its 32-bit lane offsets.
+    uint32_t backwardTile(int32_t dtype, bool aligned, uint32_t m, uint32_t k, uint32_t batch)
+    {
+        const uint32_t es = r355::dtypeBytes(dtype);
+        if(ONLY_BLOCK_PER_WAVE || m <= BLK || (uint64_t)k * es > (1u << 23) || !aligned)
             return 0u;
-        const uint64_t tiles = (uint64_t)((m + 127u) / 128u) * ((k + 127u) / 128u);
-        return m >= 768u && tiles * batch >= 2u * r355::computeUnits() ? 128u : 64u;
+        const uint32_t type = dtype == R355_F16 ? 0u : dtype == R355_BF16 ? 1u : 2u, blocks = m / BLK;
+        const uint64_t stages = ((uint64_t)m * es + 127u) / 128u;
+        const double   megabytes
+            = 1e-6 * es * batch * (2.0 * m * k + 0.5 * m * (m - 1.0) + static_cast<double>(k));
+        double fragments;
+        if(backwardBlocked(m, k, batch < GRID_BATCH ? batch : GRID_BATCH))
+        {
+            const LaunchTime& t = BWD_BLOCKED[type];
+            const uint64_t    rows = tilesOf(m, 32u) * batch;
+            fragments = t.fixed + t.step * blocks + t.group * thousands(rows * tilesOf(k, 64u)) + t.groupStep * blocks * thousands(rows * tilesOf(k, 256u))
+                        + t.more * blocks * thousands(rows * (k / BLK));
+        }
+        else
+            fragments = BWD_WAVE[type](blocks, thousands((uint64_t)blocks * (k / BLK) * batch), megabytes);
+        const double small = BWD_64[type](stages, thousands(tilesOf(m, 64u) * tilesOf(k, 64u) * batch), megabytes);
+        const double large = BWD_128[type](stages, thousands(tilesOf(m, 128u) * tilesOf(k, 128u) * batch), megabytes);
+        const double tiles = m < 128u || small < large ? small : large;
+        if(tiles >= (m <= 48u ? 0.78 : 0.88) * fragments)
+            return 0u;
+        return tiles == small && tilesOf(m, 64u) * tilesOf(k, 64u) <= r355::MAX_GROUPS ? 64u : 128u;
     }
 
     template <typename T>
@@ -392,18 +445,11 @@ namespace
         for(uint32_t first = 0; first < batch; first += GRID_BATCH)
         {
             const uint32_t count = batch - first < GRID_BATCH ? batch - first : GRID_BATCH;
-            constexpr uint32_t NBI = 2, NBK = 4;
             const T*           src = static_cast<const T*>(in) + (uint64_t)first * m * k;
             const T*           ups = static_cast<const T*>(up) + (uint64_t)first * stride;
             T*                 dm  = static_cast<T*>(mlp) + (uint64_t)first * k;
             T*                 dg  = static_cast<T*>(grad) + (uint64_t)first * m * k;
-            const uint64_t waves = (uint64_t)((k / BLK + NBK - 1u) / NBK) * ((m / BLK + NBI - 1u) / NBI) * count;
-#ifdef R355_DLRM_BLOCK_PER_WAVE
-            const bool blocked = false;
-#else
-            const bool blocked = waves >= 8ull * r355::computeUnits(); // where that still leaves every SIMD two waves
-#endif
-            if(blocked) // NBI x NBK blocks per wave
+            if(backwardBlocked(m, k, count)) // NBI x NBK blocks per wave
                 hipLaunchKernelGGL((dlrmBwdGeneralBlocked<T, NBI, NBK>),
                                    dim3(((k / BLK + NBK - 1u) / NBK + WAVES - 1u) / WAVES, (m / BLK + NBI - 1u) / NBI, count), dim3(THREADS), 0,
                                    s, src, ups, dm, dg, m, k);
@@ -441,13 +487,23 @@ namespace r355
         default: return fwd<float32_t>(in, out, m, k, batch, s);
         }
     }
+    int dlrmGeneralKernel(int32_t dtype, bool backward, uint32_t m, uint32_t k, uint32_t batch, bool aligned16)
+    {
+        const int rc = checkGeneral(backward ? "dlrm_bwd" : "dlrm_fwd", m, k, batch);
+        if(rc != R355_OK)
+            return rc;
+        if(const uint32_t tile = backward ? backwardTile(dtype, aligned16, m, k, batch) : forwardTile(dtype, m, k, batch))
+            return tile == 64u ? R355_DLRM_KERNEL_TILED_64 : R355_DLRM_KERNEL_TILED_128;
+        return backward && backwardBlocked(m, k, batch < GRID_BATCH ? batch : GRID_BATCH) ? R355_DLRM_KERNEL_REGISTER_BLOCKED
+                                                                                                    : R355_DLRM_KERNEL_BLOCK_PER_WAVE;
+    }
     int dlrmGeneralBwd(int32_t dtype, const void* in, const void* upstream, void* mlpGrad, void* inGrad, uint32_t m, uint32_t k,
                        uint32_t batch, hipStream_t s)
     {
         const int rc = checkGeneral("dlrm_bwd", m, k, batch);
         if(rc != R355_OK)
             return rc;
-        if(const uint32_t tile = backwardTile(dtype, upstream, mlpGrad, m, k, batch))
+        if(const uint32_t tile = backwardTile(dtype, aligned(upstream, 16) && aligned(mlpGrad, 16), m, k, batch))
             return dlrmBwdTiled(dtype, in, upstream, mlpGrad, inGrad, m, k, batch, tile, s);
         switch(dtype)
         {

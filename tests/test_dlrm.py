@@ -390,14 +390,14 @@ def test_bwd_integer_inputs_exact():
 @pytest.mark.parametrize("m,k,batch", [(128, 128, 64),   # the reference's own test sizes: test/dlrm/test/dlrm_test_params.hpp:57
                                        (1024, 1024, 2),  # (its fourth size with a smaller batch: the oracle's time)
                                        (48, 80, 9),      # 3 x 5 blocks of 16: neither a power of two
-                                       (256, 256, 64),   # whole macro tiles
-                                       (80, 96, 700),    # partial macro tiles in both directions
-                                       (112, 48, 600),   # partial macro tiles, k less than a tile's edge
+                                       (256, 256, 64),   # (tests/test_dlrm_tiles.py names the kernels that shapes run)
+                                       (80, 96, 700),    # 5 x 6 blocks
+                                       (112, 48, 600),   # 7 x 3 blocks; k not a multiple of 32
                                        (32, 512, 5),     # few features, an embedding width the specialised kernels have no instance for
                                        (16, 256, 7)])    # (f32: k = 256 is beyond the specialised f32 kernels)
 def test_general_shapes_fwd_and_bwd(dtype, m, k, batch):
-    """More than 32 features, or an embedding width other than 32 / 64 / 128 / 256: macro tiles, and a block per wave on the
-    fragment API.  Forward and backward against the oracle on the reference's metric (10 eps of the type); integer-valued inputs
+    """More than 32 features, or an embedding width other than 32 / 64 / 128 / 256: macro tiles, or one or several blocks per wave on
+    the fragment API.  Forward and backward against the oracle on the reference's metric (10 eps of the type); integer-valued inputs
     must come out exactly."""
     if dtype != O.F32 and (m, k) == (16, 256):
         pytest.skip("the specialised 16-bit kernels take this shape")
@@ -440,8 +440,8 @@ def test_general_shapes_fwd_and_bwd(dtype, m, k, batch):
 
 
 def test_general_shapes_take_a_batch_beyond_one_grid_dimension():
-    """More samples than a grid's second or third dimension holds (65535), on macro tiles, whose grid has one: samples either
-    side of that against the oracle."""
+    """More samples than a grid's second or third dimension holds (65535), which the forward puts the batch of a block per wave into: two
+    launches; the backward's macro tiles have one dimension.  Samples either side of that against the oracle."""
     m, k, batch = 48, 16, 65536 + 40
     stride = k + m * (m - 1) // 2
     x = O.f32_to_storage(np.round(O.uniform_pm1(95, batch * m * k) * 2.0), O.F16)

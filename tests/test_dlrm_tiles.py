@@ -17,12 +17,22 @@ def _small_integers(seed, n, dtype):
     return x if dtype == O.F32 else O.f32_to_storage(x, dtype)
 
 
-# (features, width, batch): partial tiles of 64 and 128, one and several tiles, K tails and stage counts around the six-stage
-# loop, batches that leave XCDs unevenly loaded; the last is large enough for the 128 x 128 tile of the 16-bit types
+# The kernels of 256 CUs (tests/test_dlrm_kernel_choice.py holds the choice itself)
+WAVE, BLOCKED, T64, T128 = R.DLRM_KERNEL_BLOCK_PER_WAVE, R.DLRM_KERNEL_REGISTER_BLOCKED, R.DLRM_KERNEL_TILED_64, R.DLRM_KERNEL_TILED_128
+
+
+# (features, width, batch): partial tiles of 64, one and several tiles, K tails and stage counts around the six-stage loop, batches that leave
+# XCDs unevenly loaded.  f32 runs 64 x 64 tiles throughout, the 16-bit types a block per wave in three of them and 64 x 64 tiles else
 @pytest.mark.parametrize("dtype", [O.F16, O.BF16, O.F32])
 @pytest.mark.parametrize("m,k,batch", [(32, 176, 5), (48, 272, 3), (64, 16, 1500), (80, 336, 9), (128, 384, 2), (144, 448, 17), (272, 96, 33), (272, 512, 86),
                                        (144, 1040, 81)])
 def test_forward_on_macro_tiles(dtype, m, k, batch):
+    waves = dtype != O.F32 and (m, k) in ((32, 176), (48, 272), (64, 16))
+    assert R.dlrm_kernel(dtype, m, k, batch) == (WAVE if waves else T64)
+    _forward(dtype, m, k, batch)
+
+
+def _forward(dtype, m, k, batch):
     store, stride = O.NP_STORAGE[dtype], k + m * (m - 1) // 2
     x = _small_integers(11 + m, batch * m * k, dtype)
     dout = device_filled(batch * stride + 8, store, 0xEE)
@@ -32,19 +42,28 @@ def test_forward_on_macro_tiles(dtype, m, k, batch):
     assert np.array_equal(out[:batch * stride].view(np.uint8), O.dlrm_fwd(dtype, x, m, k, batch).ravel().view(np.uint8))
 
 
-# the 128 x 128 tile of the 16-bit types beyond 192 features: just enough tiles for it and one sample fewer, whole and partial last tiles
+# the 128 x 128 tile of the 16-bit types: whole and partial last tiles, a single tile a sample, one K stage and several
 @pytest.mark.parametrize("dtype", [O.F16, O.BF16])
-@pytest.mark.parametrize("m,k,batch", [(256, 80, 52), (256, 80, 51), (352, 208, 26), (496, 64, 16), (1008, 32, 5)])
+@pytest.mark.parametrize("m,k,batch", [(256, 80, 110), (80, 96, 410), (208, 80, 95), (352, 208, 36), (336, 16, 45), (496, 64, 30), (1008, 32, 8)])
 def test_forward_on_the_large_tile(dtype, m, k, batch):
-    test_forward_on_macro_tiles(dtype, m, k, batch)
+    assert R.dlrm_kernel(dtype, m, k, batch) == T128
+    _forward(dtype, m, k, batch)
+
+
+# small launches, and those around the shapes above, on whatever they run
+@pytest.mark.parametrize("dtype", [O.F16, O.BF16, O.F32])
+@pytest.mark.parametrize("m,k,batch", [(256, 80, 52), (256, 80, 51), (352, 208, 26), (496, 64, 16), (1008, 32, 5), (48, 400, 6), (64, 64, 300), (48, 64, 100)])
+def test_forward_on_other_shapes(dtype, m, k, batch):
+    _forward(dtype, m, k, batch)
 
 
 # backward: one tile and several, so that stages left of, in and right of the diagonal tile all occur, partial tiles and K stages,
-# widths off the tile's edge, samples spread unevenly over the XCDs; all but the first, which runs a block per wave, on the 64 x 64 tile
+# widths off the tile's edge, samples spread unevenly over the XCDs; the first three run a block per wave, the others 64 x 64 tiles
 @pytest.mark.parametrize("dtype", [O.F16, O.BF16, O.F32])
 @pytest.mark.parametrize("m,k,batch", [(16, 80, 9), (32, 176, 5), (48, 272, 3), (64, 16, 700), (80, 80, 41), (128, 384, 2), (144, 448, 17), (272, 96, 33),
-                                       (336, 272, 40), (400, 144, 3), (528, 272, 24)])
+                                       (336, 272, 40), (400, 144, 3), (528, 272, 24), (48, 400, 60), (112, 48, 600)])
 def test_backward_on_macro_tiles(dtype, m, k, batch):
+    assert R.dlrm_kernel(dtype, m, k, batch, backward=True) == (WAVE if (m, k) in ((16, 80), (32, 176), (48, 272)) else T64)
     store, stride = O.NP_STORAGE[dtype], k + m * (m - 1) // 2
     x, up = _small_integers(21 + m, batch * m * k, dtype), _small_integers(22 + m, batch * stride, dtype)
     dmlp, dgrad = device_filled(batch * k + 8, store, 0xEE), device_filled(batch * m * k + 8, store, 0xEE)
@@ -59,9 +78,10 @@ def test_backward_on_macro_tiles(dtype, m, k, batch):
     assert np.array_equal(g, w)
 
 
-def _backward_of_repeated_samples(dtype, m, k, batch, off=0, distinct=3):
+def _backward_of_repeated_samples(dtype, m, k, batch, kernel, off=0, distinct=3):
     """A batch that goes round `distinct` samples, so that the oracle has only those to do; every sample of the batch against its own.
     off: upstream and mlp_grad start that many elements behind a 16-byte boundary."""
+    assert R.dlrm_kernel(dtype, m, k, batch, backward=True, aligned16=off == 0) == kernel
     store, stride = O.NP_STORAGE[dtype], k + m * (m - 1) // 2
     es = np.dtype(store).itemsize
     x, up = _small_integers(31 + m, distinct * m * k, dtype), _small_integers(32 + m, distinct * stride, dtype)
@@ -80,25 +100,33 @@ def _backward_of_repeated_samples(dtype, m, k, batch, off=0, distinct=3):
     assert np.array_equal(g.reshape(batch, m * k), w.reshape(distinct, m * k)[turn])
 
 
-# the 128 x 128 tile of the backward: from 768 features on with two tiles a CU (512).  Stages left of, in and right of the diagonal tile; a partial
-# last row tile, column tile and K stage; whole tiles; a single narrow column tile
+# the 128 x 128 tile of the backward: stages left of, in and right of the diagonal tile; a partial last row tile, column tile and K stage; whole tiles
+@pytest.mark.parametrize("dtype,m,k,batch", [(O.F16, 784, 400, 60), (O.F16, 768, 256, 120), (O.F16, 528, 400, 140), (O.BF16, 784, 400, 90),
+                                             (O.BF16, 768, 256, 125), (O.F32, 976, 560, 52), (O.F32, 768, 256, 90)])
+def test_backward_on_the_large_tile(dtype, m, k, batch):
+    _backward_of_repeated_samples(dtype, m, k, batch, T128, distinct=2)
+
+
+# the same shapes with fewer samples, and narrow ones, run 64 x 64 tiles
 @pytest.mark.parametrize("dtype", [O.F16, O.BF16, O.F32])
 @pytest.mark.parametrize("m,k,batch", [(784, 144, 37), (768, 128, 86), (784, 16, 74), (912, 272, 22)])
-def test_backward_on_the_large_tile(dtype, m, k, batch):
-    _backward_of_repeated_samples(dtype, m, k, batch)
+def test_backward_of_many_features_on_the_small_tile(dtype, m, k, batch):
+    _backward_of_repeated_samples(dtype, m, k, batch, T64)
 
 
-# what is left for the register-blocked fragment-API kernel, launches of 2048 of its waves or more: up to 16 features, and upstream and
-# mlp_grad off 16-byte boundaries.  Whole and partial blocks of 2 x 4; (16, 80, 65576) is also more than one launch's grid holds
+# the register-blocked fragment-API kernel, launches of 2048 of its waves or more: few features, rows that a tile of 64 mostly pads, and
+# upstream and mlp_grad off 16-byte boundaries.  Whole and partial blocks of 2 x 4; (16, 80, 65576) is also more than one launch's grid holds
 @pytest.mark.parametrize("dtype", [O.F16, O.BF16, O.F32])
-@pytest.mark.parametrize("m,k,batch,off", [(16, 80, 1100, 0), (16, 272, 500, 0), (16, 80, 65576, 0), (80, 96, 700, 1), (112, 48, 600, 1), (256, 256, 64, 1)])
+@pytest.mark.parametrize("m,k,batch,off", [(16, 80, 1100, 0), (16, 272, 500, 0), (16, 80, 65576, 0), (80, 96, 700, 1), (112, 48, 600, 1), (256, 256, 64, 1),
+                                           (48, 752, 300, 0), (80, 208, 1000, 0), (32, 16, 3000, 0)])
 def test_backward_on_the_register_blocked_kernel(dtype, m, k, batch, off):
-    _backward_of_repeated_samples(dtype, m, k, batch, off)
+    _backward_of_repeated_samples(dtype, m, k, batch, BLOCKED, off)
 
 
 def test_forward_of_16_features_beyond_one_grid_dimension():
     """A block per wave, the batch a grid dimension of at most 65535: two launches."""
     m, k, batch, distinct = 16, 80, 65576, 3
+    assert R.dlrm_kernel(O.F16, m, k, batch) == WAVE
     stride = k + m * (m - 1) // 2
     x, turn = _small_integers(41, distinct * m * k, O.F16), np.arange(batch) % distinct
     dout = device_filled(batch * stride + 8, np.uint16, 0xEE)
@@ -122,18 +150,34 @@ def test_backward_with_an_upstream_off_16_bytes():
     assert np.array_equal(O.storage_to_f32(to_host(dgrad, store), dtype), O.storage_to_f32(want_grad.ravel(), dtype))
 
 
-def test_more_samples_than_a_launch_holds():
+def test_more_samples_than_a_forward_launch_holds():
     """2^24 + 4096 samples of one tile each: a launch's 256-thread workgroups are counted in 32 bits of threads, so the batch goes
-    out in two launches.  The batch repeats 4096 samples; each repetition has to give the same bits (18 GB, 18 GB and 18 GB)."""
-    m, k, part, copies = 32, 16, 4096, 4097
+    out in two launches.  The batch repeats 4096 samples; each repetition has to give the same bits (52 and 77 GB)."""
+    m, k, part, copies = 48, 16, 4096, 4097
     stride = k + m * (m - 1) // 2
-    x = torch.randn(part, m * k, device="cuda").half().repeat(copies, 1)
-    out = torch.zeros(copies, part * stride, device="cuda", dtype=torch.float16)
-    R.dlrm_fwd(O.F16, x, out, m, k, part * copies)
-    want = torch.zeros(part * stride, device="cuda", dtype=torch.float16)
-    R.dlrm_fwd(O.F16, x, want, m, k, part)
+    assert R.dlrm_kernel(O.F32, m, k, part) == R.dlrm_kernel(O.F32, m, k, part * copies) == T64
+    torch.cuda.empty_cache()
+    x = torch.randn(part, m * k, device="cuda").repeat(copies, 1)
+    out = torch.zeros(copies, part * stride, device="cuda")
+    R.dlrm_fwd(O.F32, x, out, m, k, part * copies)
+    want = torch.zeros(part * stride, device="cuda")
+    R.dlrm_fwd(O.F32, x, want, m, k, part)
     assert bool(want.any()) and all(torch.equal(row, want) for row in out)
-    grad, mlp = x.clone().view(copies, -1), torch.zeros(copies, part * k, device="cuda", dtype=torch.float16)
-    R.dlrm_bwd(O.F16, x, out, mlp, grad, m, k, part * copies)
-    assert not torch.equal(grad[0], x[:part].view(-1))
-    assert all(torch.equal(row, grad[0]) for row in grad) and all(torch.equal(row, mlp[0]) for row in mlp)
+    del x, out
+    torch.cuda.empty_cache()
+
+
+def test_more_samples_than_a_backward_launch_holds():
+    """The same of the backward (34, 68 and 34 GB)."""
+    m, k, part, copies = 64, 16, 4096, 4097
+    stride = k + m * (m - 1) // 2
+    assert R.dlrm_kernel(O.F16, m, k, part, backward=True) == R.dlrm_kernel(O.F16, m, k, part * copies, backward=True) == T64
+    torch.cuda.empty_cache()
+    x, up = (torch.randn(part, width, device="cuda").half().repeat(copies, 1) for width in (m * k, stride))
+    grad, mlp = torch.zeros(copies, part * m * k, device="cuda", dtype=torch.float16), torch.zeros(copies, part * k, device="cuda", dtype=torch.float16)
+    R.dlrm_bwd(O.F16, x, up, mlp, grad, m, k, part * copies)
+    want_grad, want_mlp = torch.zeros(part * m * k, device="cuda", dtype=torch.float16), torch.zeros(part * k, device="cuda", dtype=torch.float16)
+    R.dlrm_bwd(O.F16, x, up, want_mlp, want_grad, m, k, part)
+    assert bool(want_grad.any()) and all(torch.equal(row, want_grad) for row in grad) and all(torch.equal(row, want_mlp) for row in mlp)
+    del x, up, grad, mlp
+    torch.cuda.empty_cache()
