@@ -349,18 +349,19 @@ namespace
     // steps again).  Macro tiles (steps: stages of 128 bytes; the last term: megabytes of input and output) read a row once per 64 or 128
     // others but pad m to the tile's edge: with few features or a short K most of a tile is padding and fixed cost.  bf16 32 x 48 x 7174: 9.4 us a block
     // per wave, 22 on 64 x 64 tiles, 51 on 128 x 128 ones; f16 64 x 112 x 2687: 28, 15 and 27; bf16 176 x 576 x 428: 227, 25 and 30; f16
-    // 1024 x 1024 x 64: 96 on 128 x 128 tiles.  Beyond 320 features the model of the block per wave does not reach, and only small launches run it.
+    // 1024 x 1024 x 64: 96 on 128 x 128 tiles.  Beyond 160 features only small launches run a block per wave: its reads of the
+    // rows of X then cost more than the model says (bf16 192 x 16 x 505: 15.6 us, modelled 11, 13.1 on 64 x 64 tiles).
     constexpr LaunchTime FWD_WAVE[2]  = {{2.70, 0.0415, 0.104, 0.124, 0.104}, {2.48, 0.0954, 0.135, 0.225, 0.00649}}; // 16-bit, f32
     constexpr LaunchTime FWD_64[2]    = {{3.38, 0.00367, 2.13, 0.564, 0.0370}, {3.49, 0.227, 1.95, 1.62, 0.0517}};
     constexpr LaunchTime FWD_128      = {3.88, 0.124, 5.27, 0.804, 0.0816}; // 16-bit: f32, bound by its matrix instructions, is faster on 64 x 64 throughout
-    constexpr double     FWD_MARGIN   = 0.97; // of the tiles' time that the block per wave may take and still run
-    // The macro tile's edge (dlrmFwdTiled in gemm_tiled.hip), or 0 for a block per wave.  Up to 16 features a sample is a single block.
-    // Leading dimensions beyond 8 MiB per row do not fit the tile kernels' 32-bit lane offsets.
-    uint32_t forwardTile(int32_t dtype, uint32_t m, uint32_t k, uint32_t batch)
+    constexpr double     FWD_MARGIN   = 0.97; // a tile has to be ahead of the block per wave by that
+    // The kernel of a launch, an r355_dlrm_kernel_id.  Up to 16 features a sample is a single block.  Leading dimensions beyond 8 MiB per row do not
+    // fit the tile kernels' (dlrmFwdTiled in gemm_tiled.hip) 32-bit lane offsets.
+    int forwardKernel(int32_t dtype, uint32_t m, uint32_t k, uint32_t batch)
     {
         const uint64_t rowBytes = (uint64_t)k * r355::dtypeBytes(dtype);
         if(ONLY_BLOCK_PER_WAVE || m <= BLK || rowBytes > (1u << 23))
-            return 0u;
+            return R355_DLRM_KERNEL_BLOCK_PER_WAVE;
         const bool     wide  = dtype == R355_F32;
         const uint64_t waves = triangle(m / BLK) * batch, steps = k / (wide ? 4u : 16u), stages = (rowBytes + 127u) / 128u;
         const double   megabytes
@@ -368,58 +369,49 @@ namespace
         const double small = FWD_64[wide](stages, thousands(triangle(tilesOf(m, 64u)) * batch), megabytes);
         const double large = FWD_128(stages, thousands(triangle(tilesOf(m, 128u)) * batch), megabytes);
         const double tiles = wide || small < large ? small : large;
-        if(m <= 320u || waves <= 5u * r355::computeUnits())
-            if(FWD_WAVE[wide](steps, thousands(waves), rowBytes % 128u == 0u ? thousands(waves) * steps : 0.0) <= tiles / FWD_MARGIN)
-                return 0u;
+        if(m <= 160u || waves <= 5u * r355::computeUnits())
+            if(FWD_WAVE[wide](steps, thousands(waves), rowBytes % 128u == 0u ? thousands(waves) * steps : 0.0) * FWD_MARGIN <= tiles)
+                return R355_DLRM_KERNEL_BLOCK_PER_WAVE;
         // (a sample of more 64 x 64 tiles than a launch holds: f32, 370704 features and more, a result of 256 GiB)
-        return tiles == small && triangle(tilesOf(m, 64u)) <= r355::MAX_GROUPS ? 64u : 128u;
+        return tiles == small && triangle(tilesOf(m, 64u)) <= r355::MAX_GROUPS ? R355_DLRM_KERNEL_TILED_64 : R355_DLRM_KERNEL_TILED_128;
     }
 
-    // Backward.  The fragment-API kernels are a block per wave for launches of few waves and 2 x 4 blocks per wave (the register-blocked
-    // kernel; waves of 32 x 64 of the gradient, workgroups of 32 x 256 that form S once) from eight waves a CU on; macro tiles pad m and the K of
-    // the product, which is m again, to 64 or 128.  f16 32 x 208 x 4021: 23 us register-blocked, 56 on 64 x 64 tiles; f16 80 x 208 x 1410: 34 and 57;
+    // Backward.  The fragment-API kernels are a block per wave and 2 x 4 blocks per wave (the register-blocked kernel; waves of 32 x 64 of the
+    // gradient, workgroups of 32 x 256 that form S once); macro tiles pad m and the K of the product, which is m again, to 64 or 128.  f16 32 x 208 x 4021: 23 us register-blocked, 56 on 64 x 64 tiles; f16 80 x 208 x 1410: 34 and 57;
     // f16 112 x 48 x 1612: 44 and 22; f16 1024 x 256 x 4: 96 a block per wave, 10.5 on 64 x 64; f16 992 x 464 x 27: 117 register-blocked, 72 on 64 x 64,
     // 58 on 128 x 128 tiles; f16 1024 x 1024 x 64: 473, 295 and 214.
     // By f16, bf16, f32.  Steps: blocks of 16 rows (fragments), stages of 128 bytes of K (tiles); the last term: megabytes, for the
     // register-blocked kernel thousands of block products.
-    constexpr LaunchTime BWD_WAVE[3]    = {{1.83, 0.546, 0.0, 0.243, 0.0478}, {2.06, 0.548, 0.0, 0.220, 0.0950}, {1.19, 0.860, 0.0, 0.291, 0.163}};
-    constexpr LaunchTime BWD_BLOCKED[3] = {{2.98, 0.280, 0.977, 0.606, 0.0229}, {4.32, 0.223, 1.20, 0.612, 0.0225}, {2.98, 0.646, 1.38, 0.753, 0.148}};
-    constexpr LaunchTime BWD_64[3]      = {{3.36, 0.257, 1.46, 0.787, 0.122}, {3.45, 0.236, 1.55, 0.790, 0.113}, {2.98, 0.490, 1.24, 2.09, 0.0608}};
-    constexpr LaunchTime BWD_128[3]     = {{3.90, 0.997, 2.80, 1.53, 0.253}, {3.79, 1.11, 2.91, 1.85, 0.210}, {3.34, 1.81, 4.30, 6.64, 0.104}};
+    constexpr LaunchTime BWD_WAVE[3]    = {{1.71, 0.538, 0.0, 0.195, 0.305}, {1.97, 0.543, 0.0, 0.187, 0.296}, {1.77, 0.735, 0.0, 0.303, 0.124}};
+    constexpr LaunchTime BWD_BLOCKED[3] = {{2.87, 0.531, 1.02, 0.552, 0.0157}, {4.33, 0.481, 1.23, 0.551, 0.0171}, {3.27, 0.916, 1.28, 0.691, 0.142}};
+    constexpr LaunchTime BWD_64[3]      = {{3.39, 0.247, 1.27, 0.827, 0.132}, {3.48, 0.221, 1.33, 0.808, 0.128}, {2.91, 0.5, 1.24, 2.11, 0.0614}};
+    constexpr LaunchTime BWD_128[3]     = {{3.77, 0.998, 2.94, 1.81, 0.251}, {3.38, 1.31, 2.52, 1.69, 0.238}, {3.27, 1.83, 4.09, 7.22, 0.0915}};
+    constexpr double     BWD_MARGIN[3]  = {0.96, 0.92, 0.98}; // a tile has to be ahead of the fragment kernels by that: the models' error there
     constexpr uint32_t   NBI = 2, NBK = 4; // blocks per wave of the register-blocked kernel
-    bool backwardBlocked(uint32_t m, uint32_t k, uint32_t count)
+    // The kernel of a launch, an r355_dlrm_kernel_id.  The tile kernel (dlrmBwdTiled in gemm_tiled.hip) reads upstream and writes mlpGrad in 16-byte
+    // pieces (`aligned`), and rows beyond 8 MiB do not fit its 32-bit lane offsets.  Where it cannot run, and up to 16 features, for which
+    // the models are not fitted, the register-blocked kernel takes launches that leave every SIMD two of its waves.
+    int backwardKernel(int32_t dtype, bool aligned, uint32_t m, uint32_t k, uint32_t batch)
     {
-        const uint64_t waves = (uint64_t)((k / BLK + NBK - 1u) / NBK) * ((m / BLK + NBI - 1u) / NBI) * count;
-        return !ONLY_BLOCK_PER_WAVE && waves >= 8ull * r355::computeUnits(); // where that still leaves every SIMD two waves
-    }
-    // The macro tile's edge (dlrmBwdTiled in gemm_tiled.hip), or 0 for the fragment-API kernels: where the tiles' lead is less than the
-    // models' error (at up to 48 features, a tile of 64 mostly padded, 22 %, else 12 %) those stay.  The tile kernel reads upstream and writes
-    // mlpGrad in 16-byte pieces (`aligned`); rows beyond 8 MiB do not fit its 32-bit lane offsets.
-    uint32_t backwardTile(int32_t dtype, bool aligned, uint32_t m, uint32_t k, uint32_t batch)
-    {
-        const uint32_t es = r355::dtypeBytes(dtype);
-        if(ONLY_BLOCK_PER_WAVE || m <= BLK || (uint64_t)k * es > (1u << 23) || !aligned)
-            return 0u;
-        const uint32_t type = dtype == R355_F16 ? 0u : dtype == R355_BF16 ? 1u : 2u, blocks = m / BLK;
-        const uint64_t stages = ((uint64_t)m * es + 127u) / 128u;
-        const double   megabytes
-            = 1e-6 * es * batch * (2.0 * m * k + 0.5 * m * (m - 1.0) + static_cast<double>(k));
-        double fragments;
-        if(backwardBlocked(m, k, batch < GRID_BATCH ? batch : GRID_BATCH))
-        {
-            const LaunchTime& t = BWD_BLOCKED[type];
-            const uint64_t    rows = tilesOf(m, 32u) * batch;
-            fragments = t.fixed + t.step * blocks + t.group * thousands(rows * tilesOf(k, 64u)) + t.groupStep * blocks * thousands(rows * tilesOf(k, 256u))
-                        + t.more * blocks * thousands(rows * (k / BLK));
-        }
-        else
-            fragments = BWD_WAVE[type](blocks, thousands((uint64_t)blocks * (k / BLK) * batch), megabytes);
-        const double small = BWD_64[type](stages, thousands(tilesOf(m, 64u) * tilesOf(k, 64u) * batch), megabytes);
-        const double large = BWD_128[type](stages, thousands(tilesOf(m, 128u) * tilesOf(k, 128u) * batch), megabytes);
-        const double tiles = m < 128u || small < large ? small : large;
-        if(tiles >= (m <= 48u ? 0.78 : 0.88) * fragments)
-            return 0u;
-        return tiles == small && tilesOf(m, 64u) * tilesOf(k, 64u) <= r355::MAX_GROUPS ? 64u : 128u;
+        const uint32_t es = r355::dtypeBytes(dtype), blocks = m / BLK, samples = batch < GRID_BATCH ? batch : GRID_BATCH;
+        const uint64_t waves = tilesOf(k, NBK * BLK) * tilesOf(m, NBI * BLK); // of a sample, register-blocked
+        if(ONLY_BLOCK_PER_WAVE)
+            return R355_DLRM_KERNEL_BLOCK_PER_WAVE;
+        if(m <= BLK || (uint64_t)k * es > (1u << 23) || !aligned)
+            return waves * samples >= 8ull * r355::computeUnits() ? R355_DLRM_KERNEL_REGISTER_BLOCKED : R355_DLRM_KERNEL_BLOCK_PER_WAVE;
+        const uint32_t type   = dtype == R355_F16 ? 0u : dtype == R355_BF16 ? 1u : 2u;
+        const uint64_t stages = ((uint64_t)m * es + 127u) / 128u, rows = tilesOf(m, NBI * BLK) * batch;
+        const double   megabytes = 1e-6 * es * batch * (2.0 * m * k + 0.5 * m * (m - 1.0) + static_cast<double>(k));
+        const double   wave      = BWD_WAVE[type](blocks, thousands((uint64_t)blocks * (k / BLK) * batch), megabytes);
+        const LaunchTime& t      = BWD_BLOCKED[type];
+        const double   blocked   = t.fixed + t.step * blocks + t.group * thousands(waves * batch) + t.groupStep * blocks * thousands(rows * tilesOf(k, 256u))
+                               + t.more * blocks * thousands(rows * (k / BLK));
+        const double fragments = wave < blocked ? wave : blocked;
+        const double small     = BWD_64[type](stages, thousands(tilesOf(m, 64u) * tilesOf(k, 64u) * batch), megabytes);
+        const double large     = BWD_128[type](stages, thousands(tilesOf(m, 128u) * tilesOf(k, 128u) * batch), megabytes);
+        if(fragments * BWD_MARGIN[type] <= (small < large ? small : large))
+            return wave < blocked ? R355_DLRM_KERNEL_BLOCK_PER_WAVE : R355_DLRM_KERNEL_REGISTER_BLOCKED;
+        return small <= large && tilesOf(m, 64u) * tilesOf(k, 64u) <= r355::MAX_GROUPS ? R355_DLRM_KERNEL_TILED_64 : R355_DLRM_KERNEL_TILED_128;
     }
 
     template <typename T>
@@ -439,7 +431,7 @@ namespace
         return r355::checkLaunch("dlrm_fwd (general)");
     }
     template <typename T>
-    int bwd(const void* in, const void* up, void* mlp, void* grad, uint32_t m, uint32_t k, uint32_t batch, hipStream_t s)
+    int bwd(const void* in, const void* up, void* mlp, void* grad, uint32_t m, uint32_t k, uint32_t batch, bool blocked, hipStream_t s)
     {
         const uint64_t stride = (uint64_t)k + (uint64_t)m * (m - 1u) / 2u;
         for(uint32_t first = 0; first < batch; first += GRID_BATCH)
@@ -449,7 +441,7 @@ namespace
             const T*           ups = static_cast<const T*>(up) + (uint64_t)first * stride;
             T*                 dm  = static_cast<T*>(mlp) + (uint64_t)first * k;
             T*                 dg  = static_cast<T*>(grad) + (uint64_t)first * m * k;
-            if(backwardBlocked(m, k, count)) // NBI x NBK blocks per wave
+            if(blocked) // NBI x NBK blocks per wave
                 hipLaunchKernelGGL((dlrmBwdGeneralBlocked<T, NBI, NBK>),
                                    dim3(((k / BLK + NBK - 1u) / NBK + WAVES - 1u) / WAVES, (m / BLK + NBI - 1u) / NBI, count), dim3(THREADS), 0,
                                    s, src, ups, dm, dg, m, k);
@@ -478,8 +470,9 @@ namespace r355
         const int rc = checkGeneral("dlrm_fwd", m, k, batch);
         if(rc != R355_OK)
             return rc;
-        if(const uint32_t tile = forwardTile(dtype, m, k, batch))
-            return dlrmFwdTiled(dtype, in, out, m, k, batch, tile, s);
+        const int kernel = forwardKernel(dtype, m, k, batch);
+        if(kernel != R355_DLRM_KERNEL_BLOCK_PER_WAVE)
+            return dlrmFwdTiled(dtype, in, out, m, k, batch, kernel == R355_DLRM_KERNEL_TILED_64 ? 64u : 128u, s);
         switch(dtype)
         {
         case R355_F16: return fwd<float16_t>(in, out, m, k, batch, s);
@@ -492,10 +485,7 @@ namespace r355
         const int rc = checkGeneral(backward ? "dlrm_bwd" : "dlrm_fwd", m, k, batch);
         if(rc != R355_OK)
             return rc;
-        if(const uint32_t tile = backward ? backwardTile(dtype, aligned16, m, k, batch) : forwardTile(dtype, m, k, batch))
-            return tile == 64u ? R355_DLRM_KERNEL_TILED_64 : R355_DLRM_KERNEL_TILED_128;
-        return backward && backwardBlocked(m, k, batch < GRID_BATCH ? batch : GRID_BATCH) ? R355_DLRM_KERNEL_REGISTER_BLOCKED
-                                                                                                    : R355_DLRM_KERNEL_BLOCK_PER_WAVE;
+        return backward ? backwardKernel(dtype, aligned16, m, k, batch) : forwardKernel(dtype, m, k, batch);
     }
     int dlrmGeneralBwd(int32_t dtype, const void* in, const void* upstream, void* mlpGrad, void* inGrad, uint32_t m, uint32_t k,
                        uint32_t batch, hipStream_t s)
@@ -503,13 +493,15 @@ namespace r355
         const int rc = checkGeneral("dlrm_bwd", m, k, batch);
         if(rc != R355_OK)
             return rc;
-        if(const uint32_t tile = backwardTile(dtype, aligned(upstream, 16) && aligned(mlpGrad, 16), m, k, batch))
-            return dlrmBwdTiled(dtype, in, upstream, mlpGrad, inGrad, m, k, batch, tile, s);
+        const int kernel = backwardKernel(dtype, aligned(upstream, 16) && aligned(mlpGrad, 16), m, k, batch);
+        if(kernel == R355_DLRM_KERNEL_TILED_64 || kernel == R355_DLRM_KERNEL_TILED_128)
+            return dlrmBwdTiled(dtype, in, upstream, mlpGrad, inGrad, m, k, batch, kernel == R355_DLRM_KERNEL_TILED_64 ? 64u : 128u, s);
+        const bool blocked = kernel == R355_DLRM_KERNEL_REGISTER_BLOCKED;
         switch(dtype)
         {
-        case R355_F16: return bwd<float16_t>(in, upstream, mlpGrad, inGrad, m, k, batch, s);
-        case R355_BF16: return bwd<bfloat16_t>(in, upstream, mlpGrad, inGrad, m, k, batch, s);
-        default: return bwd<float32_t>(in, upstream, mlpGrad, inGrad, m, k, batch, s);
+        case R355_F16: return bwd<float16_t>(in, upstream, mlpGrad, inGrad, m, k, batch, blocked, s);
+        case R355_BF16: return bwd<bfloat16_t>(in, upstream, mlpGrad, inGrad, m, k, batch, blocked, s);
+        default: return bwd<float32_t>(in, upstream, mlpGrad, inGrad, m, k, batch, blocked, s);
         }
     }
 } // namespace r355

@@ -36,7 +36,7 @@ def test_backward_register_blocked(dtype, m, k, batch):
 
 @pytest.mark.parametrize("dtype", [R.F16, R.BF16, R.F32])
 @pytest.mark.parametrize("m,k,batch,kernel", [(112, 48, 847, T64), (320, 192, 96, T64), (1024, 256, 4, T64), (784, 16, 100, T64), (1024, 1024, 64, T128),
-                                              (48, 80, 9, WAVE), (32, 400, 44, WAVE)])
+                                              (32, 16, 100, WAVE)])
 def test_backward_on_tiles_and_with_a_block_per_wave(dtype, m, k, batch, kernel):
     assert R.dlrm_kernel(dtype, m, k, batch, backward=True) == kernel
 
