@@ -58,16 +58,12 @@ def test_other_kernel_families():
         R.gemm_launch_plan(_args(R.F16, R.F16, 256, 256, 250))  # what r355_gemm refuses
 
 
-# measured slower on the smaller tile (or with other splits) although the timing models price that as a little faster
+# measured slower on the smaller tile (or with other splits) although the timing model prices that as a little faster
 @pytest.mark.parametrize("in_t,out_t,m,n,k,tile,splits", [
-    (R.E4M3, R.F32, 96, 8000, 4672, (128, 128), 4),
-    (R.I8, R.I32, 1584, 400, 3952, (128, 128), 3),
-    (R.BF16, R.BF16, 2080, 432, 2208, (128, 128), 3),
+    (R.BF16, R.BF16, 704, 976, 2176, (128, 128), 4),
     (R.F16, R.F16, 1120, 1856, 256, (128, 128), 1),
-    (R.I8, R.I32, 736, 2256, 768, (128, 128), 1),
+    (R.BF16, R.BF16, 1744, 1696, 256, (128, 128), 1),
     (R.F32, R.F32, 1792, 176, 2240, (64, 64), 5),
-    (R.I8, R.I32, 2160, 7984, 7504, (256, 256), 1),
-    (R.BF16, R.BF16, 3584, 4960, 7488, (256, 256), 1),
 ])
 def test_a_lead_within_the_models_error_does_not_move_a_call(in_t, out_t, m, n, k, tile, splits):
     plan = R.gemm_launch_plan(_args(in_t, out_t, m, n, k, need=R.gemm_query(_args(in_t, out_t, m, n, k, need=2 ** 64 - 1)).workspace_bytes))
