@@ -319,7 +319,7 @@ namespace
     // the wave tile starts at (m0, n0).  `scratch` is WB * 4 KiB of LDS owned by this wave.
     //
     // A lane holds four consecutive columns of one row of every block.  The tile is transposed through the wave's own LDS,
-    // 128 to 16 rows at a time, so that an access to C or D covers whole rows of the wave tile (128 to 512 bytes) with up
+    // 128 to 16 rows at a time, so that an access to C or D covers whole rows of the wave tile (128 to 512 bytes; the 64 x 64 tile's 32 to 256) with up
     // to 128 bits per lane.  What is staged: alpha * acc in the output type when beta is zero; in the compute type
     // otherwise, so that alpha * acc + beta * C is rounded once, as the reference's epilogue rounds it
     // (test/reference_impl.hpp:71-77).  C and D are reached through raw buffers that end with the tile's last valid row,
@@ -339,7 +339,7 @@ namespace
         const uint32_t r16 = lane & 15u, g = lane >> 4;
         constexpr uint32_t SS = sizeof(StageT), OS = sizeof(OutT);
         constexpr uint32_t ROW_BYTES  = 16u * WBN * SS;
-        constexpr uint32_t ROW_CHUNKS = ROW_BYTES / CHUNK; // 8, 16 or 32
+        constexpr uint32_t ROW_CHUNKS = ROW_BYTES / CHUNK; // 2 (64 x 64 tile, 8-bit result) to 32
         constexpr uint32_t SWZ        = ROW_CHUNKS < 16u ? ROW_CHUNKS - 1u : 15u;
         constexpr uint32_t EPC        = CHUNK / SS; // elements of a staged 16-byte chunk
         constexpr uint32_t OUT_WORDS  = EPC * OS / 4u; // 32-bit words of C and of D per lane and chunk: 4, 2 or 1
@@ -597,7 +597,7 @@ namespace
         constexpr uint32_t ES = ElemTraits<E>::Bytes;
         constexpr uint32_t TK = STAGE_KB / ES; // 64 K elements per stage = two K steps of 32
         static_assert(ES == 2, "16-bit element types only");
-        static_assert(WB == 8 || WB == 4 || WB == 2, "wave tile of 8 x 8, 4 x 4 or 2 x 2 blocks");
+        static_assert(WB == 8 || WB == 4, "wave tile of 8 x 8 or 4 x 4 blocks"); // (2 x 2: 8 chunks per k-row, which swzMN's 16 would leave)
         R355_STAMP(0);
         R355_STAMP_ID();
         constexpr uint32_t TILE  = 32u * WB; // macro tile edge
@@ -1637,7 +1637,7 @@ namespace
     //     that leaves exposed other workgroups of the CU cover (two of the 128 x 128 tile, four of the 64 x 64 one).
     // S holds zeros only on its diagonal and beyond row or column m, as the products of the [m][m] matrix have them.  Few stages bound
     // the small shapes (latency of one stage's loads each), the matrix instructions and the loads' distance the large ones:
-    // f16 1024 x 1024 x 64 473 -> 214 us (640 TFLOP/s), bf16 320 x 192 x 96 26.7 -> 15.0, f32 224 x 384 x 213 141 -> 95.
+    // f16 1024 x 1024 x 64 473 -> 214 us (640 TFLOP/s), bf16 320 x 192 x 96 26.7 -> 16.7, f32 224 x 384 x 213 141 -> 95.
     using BwdParams = r355::DlrmBwdParams;
 
     template <Elem E, typename T, uint32_t WB>
@@ -1861,15 +1861,16 @@ namespace
     // exceed it, panels are re-fetched from HBM and one stage of lookahead no longer covers the latency
     // (8192^2 x 16384 TN: 1268 against 1435 TFLOP/s here; 8192 x 12288 x 8192 NN: 1317 against 1474; this body within
     // 1430 - 1490 over every size and orientation tried).
-    template <Elem E, typename OutT, bool A_KCONTIG, bool B_KCONTIG, uint32_t WM>
-    __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) gemmTiledKernel16Rows(Params p)
-    {
-        gemmTiled5<E, OutT, A_KCONTIG, B_KCONTIG, 8, false, WM>(p);
-    }
     template <Elem E, typename OutT, bool A_KCONTIG, bool B_KCONTIG>
     __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) gemmTiledKernel16Deep(Params p)
     {
         gemmTiled5<E, OutT, A_KCONTIG, B_KCONTIG, 8>(p);
+    }
+    // 224 or 192 rows (tileRows, gemmTiledKernelI8Rows)
+    template <Elem E, typename OutT, bool A_KCONTIG, bool B_KCONTIG, uint32_t WM>
+    __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) gemmTiledKernel16Rows(Params p)
+    {
+        gemmTiled5<E, OutT, A_KCONTIG, B_KCONTIG, 8, false, WM>(p);
     }
 
     // ------------------------------------------------------------------------------------------
