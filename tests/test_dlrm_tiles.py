@@ -151,6 +151,24 @@ def test_backward_with_an_upstream_off_16_bytes():
     assert np.array_equal(O.storage_to_f32(to_host(dgrad, store), dtype), O.storage_to_f32(want_grad.ravel(), dtype))
 
 
+# (32 features run a block per wave, 257 launches of up to 65535 samples; the two tests below it run macro tiles)
+def test_more_samples_than_a_launch_holds():
+    """2^24 + 4096 samples of one tile each: a launch's 256-thread workgroups are counted in 32 bits of threads, so the batch goes
+    out in two launches.  The batch repeats 4096 samples; each repetition has to give the same bits (18 GB, 18 GB and 18 GB)."""
+    m, k, part, copies = 32, 16, 4096, 4097
+    stride = k + m * (m - 1) // 2
+    x = torch.randn(part, m * k, device="cuda").half().repeat(copies, 1)
+    out = torch.zeros(copies, part * stride, device="cuda", dtype=torch.float16)
+    R.dlrm_fwd(O.F16, x, out, m, k, part * copies)
+    want = torch.zeros(part * stride, device="cuda", dtype=torch.float16)
+    R.dlrm_fwd(O.F16, x, want, m, k, part)
+    assert bool(want.any()) and all(torch.equal(row, want) for row in out)
+    grad, mlp = x.clone().view(copies, -1), torch.zeros(copies, part * k, device="cuda", dtype=torch.float16)
+    R.dlrm_bwd(O.F16, x, out, mlp, grad, m, k, part * copies)
+    assert not torch.equal(grad[0], x[:part].view(-1))
+    assert all(torch.equal(row, grad[0]) for row in grad) and all(torch.equal(row, mlp[0]) for row in mlp)
+
+
 def test_more_samples_than_a_forward_launch_holds():
     """2^24 + 4096 samples of one tile each: a launch's 256-thread workgroups are counted in 32 bits of threads, so the batch goes
     out in two launches.  The batch repeats 4096 samples; each repetition has to give the same bits (52 and 77 GB)."""
