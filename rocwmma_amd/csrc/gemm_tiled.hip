@@ -1632,12 +1632,15 @@ namespace
     //   * A = S lies in memory as rows of T that start at any element.  Left of the diagonal tile a stage is TILE rows x 128 bytes
     //     of T (the K-contiguous image); right of it S(i, j) = T(j, i), so a stage is 128 bytes' worth of rows of T, TILE
     //     elements each (the M-contiguous image, transposing reads): the same 16-byte pieces at unaligned addresses either way,
-    //     through registers into the image.  The stages of the diagonal tile itself are gathered element by element.
+    //     through registers into the image.  A stage of the diagonal tile is both images of its pieces left of the diagonal (16-bit;
+    //     f32 gathers it element by element).
     //   * two buffers per operand; the loads of stage kt + 1 are in flight under the matrix instructions of stage kt, and what
-    //     that leaves exposed other workgroups of the CU cover (two of the 128 x 128 tile, four of the 64 x 64 one).
+    //     that leaves exposed other workgroups of the CU cover (two of the 128 x 128 tile, four of the 64 x 64 one: 80 and 40 KiB of LDS).
     // S holds zeros only on its diagonal and beyond row or column m, as the products of the [m][m] matrix have them.  Few stages bound
     // the small shapes (latency of one stage's loads each), the matrix instructions and the loads' distance the large ones:
-    // f16 1024 x 1024 x 64 473 -> 214 us (640 TFLOP/s), bf16 320 x 192 x 96 26.7 -> 16.7, f32 224 x 384 x 213 141 -> 95.
+    // f16 1024 x 1024 x 64 232 us, bf16 320 x 192 x 96 13.6, bf16 64 x 400 x 1011 25.9, f32 224 x 384 x 213 97.  (Gathered element by element,
+    // eight 2-byte loads for each 16 bytes, the diagonal stages took the 16-bit ones to 250, 16.7 and 39.5; without the matrix instructions the
+    // times do not change, so multiplying by a diagonal stage twice costs nothing there.)
     using BwdParams = r355::DlrmBwdParams;
 
     template <Elem E, typename T, uint32_t WB>
@@ -1647,8 +1650,9 @@ namespace
         constexpr uint32_t TK = STAGE_KB / ES, EPC = CHUNK / ES; // K elements per stage, elements per 16-byte piece
         using Word            = std::conditional_t<ES == 2, uint16_t, uint32_t>;
         typedef int i32x4u __attribute__((ext_vector_type(4), aligned(2)));
-        __shared__ __attribute__((aligned(1024))) char lds[4u * OPER];
-        constexpr uint32_t B_AT = 2u * OPER; // two buffers of A, then two of B
+        constexpr bool     ACROSS = ES == 2; // a diagonal stage's mirrored elements are an image of their own (f32: gathered)
+        constexpr uint32_t B_AT = 2u * OPER, ACROSS_AT = 4u * OPER; // two buffers of A, two of B, that image
+        __shared__ __attribute__((aligned(1024))) char lds[(ACROSS ? 5u : 4u) * OPER];
 
         // all workgroups of an XCD walk one contiguous run of (sample, tile): the tiles of a sample share its X and T in one L2
         const uint32_t perXcd = (p.total + 7u) / 8u, slotX = blockIdx.x / 8u, local = (blockIdx.x % 8u) * perXcd + slotX;
@@ -1688,20 +1692,44 @@ namespace
         // A: stages [0, diagFirst) left of the diagonal tile, [diagFirst, diagEnd) in it, [diagEnd, numStages) right of it
         const uint32_t diagFirst = row0 / TK, diagEnd = diagFirst + TILE / TK < numStages ? diagFirst + TILE / TK : numStages;
         const uint32_t rK = tid >> 3, cK = ((tid & 7u) ^ swzK8(tid >> 3)) * EPC; // K-contiguous image: row rK + 32 j, first column of the piece
-        i32x4          aNext[WB];
-        auto           loadRight = [&](uint32_t st) {
-            constexpr uint32_t SLOTS = 2u * WB * ES, KROWS = THREADS / SLOTS;
+        // A stage of the diagonal tile.  16-bit: two images, T's rows left of the diagonal (K-contiguous), and the stage's rows of T within
+        // the tile's columns (M-contiguous, in a buffer of its own), multiplied one after the other.  A piece that the diagonal cuts is
+        // read as the row's last EPC elements and moved down, which puts zeros in the place of the rest (a row shorter than that
+        // reads into the k elements before the triangle).  f32: gathered element by element, a quarter as many loads per byte, where the
+        // second multiplication would cost more (224 x 384 x 213 96 us gathered, 113 as two images).
+        i32x4 aNext[WB], aAcross[WB];
+        auto  cutBy   = [](uint32_t row, uint32_t col) { return row < col + EPC ? col + EPC - row : 0u; }; // elements from the diagonal on
+        auto  loadCut = [&](uint32_t row, uint32_t col) {
+            const uint64_t gi = row;
+            i32x4          v{0, 0, 0, 0};
+            if(row < p.m && row > col)
+                v = *reinterpret_cast<const i32x4u*>(tril + (static_cast<int64_t>(gi * (gi - 1u) / 2u + col) - cutBy(row, col)));
+            return v;
+        };
+        auto shiftDown = [](i32x4 v, uint32_t elems) { // (elems < EPC, or v is zero)
+            const uint32_t words = elems * ES / 4u, bits = elems * ES % 4u * 8u;
+            uint32_t       w0 = static_cast<uint32_t>(v[0]), w1 = static_cast<uint32_t>(v[1]), w2 = static_cast<uint32_t>(v[2]), w3 = static_cast<uint32_t>(v[3]);
+            w0 = words & 1u ? w1 : w0, w1 = words & 1u ? w2 : w1, w2 = words & 1u ? w3 : w2, w3 = words & 1u ? 0u : w3;
+            w0 = words & 2u ? w2 : w0, w1 = words & 2u ? w3 : w1, w2 = words & 2u ? 0u : w2, w3 = words & 2u ? 0u : w3;
+            return i32x4{static_cast<int>(__builtin_amdgcn_alignbit(w1, w0, bits)), static_cast<int>(__builtin_amdgcn_alignbit(w2, w1, bits)),
+                         static_cast<int>(__builtin_amdgcn_alignbit(w3, w2, bits)), static_cast<int>(__builtin_amdgcn_alignbit(0u, w3, bits))};
+        };
+        constexpr uint32_t SLOTS_M = 2u * WB * ES, KROWS_M = THREADS / SLOTS_M; // M-contiguous image: pieces per k-row, k-rows per 256 pieces
+        auto rowM = [&](uint32_t j) { return KROWS_M * j + tid / SLOTS_M; };
+        auto colM = [&](uint32_t j) { return ((tid % SLOTS_M) ^ swzMN8<WB, ES>(rowM(j))) * EPC; };
+        auto inDiag = [&](uint32_t st) { return st >= diagFirst && st < diagEnd; };
+        // f32
+        auto loadRight = [&](uint32_t st) {
 #pragma unroll
             for(uint32_t j = 0; j < WB; ++j)
             {
-                const uint32_t kr = KROWS * j + tid / SLOTS, c = ((tid % SLOTS) ^ swzMN8<WB, ES>(kr)) * EPC;
-                const uint64_t gj = st * TK + kr;
+                const uint64_t gj = st * TK + rowM(j);
                 aNext[j]          = i32x4{0, 0, 0, 0};
                 if(gj < p.m) // (then columns up to the end of the diagonal tile lie left of T's diagonal: inside the row)
-                    aNext[j] = *reinterpret_cast<const i32x4u*>(tril + (gj * (gj - 1u) / 2u + row0 + c));
+                    aNext[j] = *reinterpret_cast<const i32x4u*>(tril + (gj * (gj - 1u) / 2u + row0 + colM(j)));
             }
         };
-        auto loadA = [&](uint32_t st) {
+        auto loadGathered = [&](uint32_t st) {
             const uint32_t k0 = st * TK;
             if(st < diagFirst)
             {
@@ -1718,35 +1746,44 @@ namespace
             {
 #pragma unroll
                 for(uint32_t j = 0; j < WB; ++j)
-                {
-                    const uint32_t gi = row0 + rK + 32u * j;
-                    Word           w[EPC];
 #pragma unroll
                     for(uint32_t e = 0; e < EPC; ++e)
                     {
-                        const uint32_t gj = k0 + cK + e;
+                        const uint32_t gi = row0 + rK + 32u * j, gj = k0 + cK + e;
                         const uint64_t hi = gi > gj ? gi : gj, lo = gi > gj ? gj : gi;
-                        w[e]              = hi < p.m && gi != gj ? tril[hi * (hi - 1u) / 2u + lo] : Word(0);
+                        aNext[j][e]       = hi < p.m && gi != gj ? static_cast<int>(tril[hi * (hi - 1u) / 2u + lo]) : 0;
                     }
-                    if constexpr(ES == 2)
-                    {
-#pragma unroll
-                        for(uint32_t e = 0; e < 4; ++e)
-                            aNext[j][e] = static_cast<int>(w[2u * e] | (static_cast<uint32_t>(w[2u * e + 1u]) << 16));
-                    }
-                    else
-                    {
-#pragma unroll
-                        for(uint32_t e = 0; e < 4; ++e)
-                            aNext[j][e] = static_cast<int>(w[e]);
-                    }
-                }
             }
         };
-        auto writeA = [&](uint32_t at) { // (both images take piece j * 256 + tid at byte 16 of that)
+        // 16-bit (one place for every kind of stage: with a loop for each the compiler kept the pieces in scratch memory)
+        auto loadA = [&](uint32_t st) {
+            const bool     right = st >= diagEnd; // (uniform)
+            const uint32_t k0    = st * TK;
+            if constexpr(!ACROSS)
+            {
+                loadGathered(st);
+                return;
+            }
 #pragma unroll
             for(uint32_t j = 0; j < WB; ++j)
-                *reinterpret_cast<i32x4*>(lds + at + (j * THREADS + tid) * CHUNK) = aNext[j];
+                aNext[j] = right ? loadCut(k0 + rowM(j), row0 + colM(j)) : loadCut(row0 + rK + 32u * j, k0 + cK);
+            if(inDiag(st))
+#pragma unroll
+                for(uint32_t j = 0; j < WB; ++j)
+                    aAcross[j] = loadCut(k0 + rowM(j), row0 + colM(j));
+        };
+        auto writeA = [&](uint32_t at, uint32_t st) { // (every image takes piece j * 256 + tid at byte 16 of that)
+#pragma unroll
+            for(uint32_t j = 0; j < WB; ++j)
+            {
+                const i32x4 v = ACROSS && inDiag(st) ? shiftDown(aNext[j], cutBy(row0 + rK + 32u * j, st * TK + cK)) : aNext[j];
+                *reinterpret_cast<i32x4*>(lds + at + (j * THREADS + tid) * CHUNK) = v;
+            }
+            if(ACROSS && inDiag(st))
+#pragma unroll
+                for(uint32_t j = 0; j < WB; ++j)
+                    *reinterpret_cast<i32x4*>(lds + ACROSS_AT + (j * THREADS + tid) * CHUNK)
+                        = shiftDown(aAcross[j], cutBy(st * TK + rowM(j), row0 + colM(j)));
         };
 
         uint32_t rdAK[8], rdAM[8], rdB[8];
@@ -1800,7 +1837,7 @@ namespace
 
         issueB(0u, B_AT);
         loadA(0u);
-        writeA(0u);
+        writeA(0u, 0u);
         waitVmcnt<0>();
         ldsBarrier();
         auto stageBody = [&](auto aK, uint32_t st) {
@@ -1809,14 +1846,21 @@ namespace
             if(more)
             {
                 issueB(st + 1u, B_AT + nxt);
-                if constexpr(decltype(aK)::value)
-                    loadA(st + 1u);
-                else
+                if constexpr(!ACROSS && !decltype(aK)::value)
                     loadRight(st + 1u);
+                else
+                    loadA(st + 1u);
             }
             compute(aK, cur, B_AT + cur);
+            if constexpr(ACROSS && decltype(aK)::value)
+                if(inDiag(st))
+                    compute(std::false_type{}, ACROSS_AT, B_AT + cur);
             if(more)
-                writeA(nxt);
+            {
+                if(ACROSS && decltype(aK)::value && inDiag(st) && inDiag(st + 1u))
+                    ldsBarrier(); // the mirrored image is being read until every wave has multiplied by it
+                writeA(nxt, st + 1u);
+            }
             // the direct loads of the next stage have landed, and every wave has read this one
             waitVmcnt<0>();
             ldsBarrier();
@@ -1832,19 +1876,24 @@ namespace
         d.alpha = 1.0;
         storeTileStaged<T, false, f32x4, T, WB, WB, WB * 4096u>(acc, d, row0 + wm * WT, col0 + wn * WT, lane, lds + wave * (WB * 4096u));
     }
-    template <Elem E, typename T, uint32_t WB>
-    __global__ void __launch_bounds__(THREADS, 2) dlrmBwdTiled(BwdParams p)
+    template <Elem E, typename T>
+    __global__ void __launch_bounds__(THREADS, 2) dlrmBwdTiled128(BwdParams p)
     {
-        dlrmBwdTile<E, T, WB>(p);
+        dlrmBwdTile<E, T, 4>(p);
+    }
+    template <Elem E, typename T>
+    __global__ void __launch_bounds__(THREADS, 4) dlrmBwdTiled64(BwdParams p)
+    {
+        dlrmBwdTile<E, T, 2>(p);
     }
     template <Elem E, typename T>
     int launchBwdTiled(const BwdParams& p, uint32_t tile, hipStream_t stream)
     {
         const uint32_t groups = (p.total + 7u) / 8u * 8u;
         if(tile == 128u)
-            hipLaunchKernelGGL((dlrmBwdTiled<E, T, 4>), dim3(groups), dim3(THREADS), 0, stream, p);
+            hipLaunchKernelGGL((dlrmBwdTiled128<E, T>), dim3(groups), dim3(THREADS), 0, stream, p);
         else
-            hipLaunchKernelGGL((dlrmBwdTiled<E, T, 2>), dim3(groups), dim3(THREADS), 0, stream, p);
+            hipLaunchKernelGGL((dlrmBwdTiled64<E, T>), dim3(groups), dim3(THREADS), 0, stream, p);
         return r355::checkLaunch("dlrm_bwd (macro tiles)");
     }
 
