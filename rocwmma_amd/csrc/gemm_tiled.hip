@@ -1005,6 +1005,11 @@ namespace
 
     // TRIANGLE: not a GEMM but the DLRM dot interaction, X X^T of every sample of a batch (p.a: [batch][m][k], lda = k) with its
     // strict lower triangle packed behind the sample's first row (p.d: [batch][k + m (m - 1) / 2]); tileCount = batch x tiles.
+    // Bound by the direct loads: two workgroups of the 128 x 128 tile a CU take 0.95 us a stage, of which 0.6 is the L2's rate for
+    // their 64 KiB and 0.43 the matrix instructions'.  A diagonal tile therefore loads its rows once, into the buffers that run three
+    // stages ahead, and its wave tile above the diagonal is left out: f16 1024 x 1024 x 64 (8 of a sample's 36 tiles) 96.3 -> 87 - 91 us,
+    // 96 x 576 x 1116 (all of them) 41.4 -> 36.8, 64 x 1024 x 200 on 64 x 64 tiles 7.5 -> 6.9.  (Into A's two buffers, two
+    // stages ahead: 94, 37.6 and 9.1.)
     template <Elem E, typename OutT, bool A_KCONTIG, bool B_KCONTIG, uint32_t WB, bool TRIANGLE = false, uint32_t WM = WB>
     __device__ __forceinline__ void gemmTiled5(const Params& whole)
     {
@@ -1149,8 +1154,12 @@ namespace
         uint64_t refillA, refillB; // stage kt + 2 of A, stage kt + B_AHEAD of B (clamped)
         // `full` (compile-time tag): every stage this one requests is a whole stage inside K - the main part of the K
         // loop, whose loads carry no tail select and whose refill pointers always advance
-        auto stageBody = [&](auto full, uint32_t kt, uint32_t aCur, uint32_t aNxt, uint32_t bCur, uint32_t bNxt, uint32_t bFree) {
-            constexpr bool FULL  = decltype(full)::value;
+        // `one`: a diagonal tile of X X^T.  Both operands are the same rows: A's blocks are read from B's image, three stages ahead,
+        // and A is not loaded.
+        auto stageBody = [&](auto full, auto one, uint32_t kt, uint32_t aCur, uint32_t aNxt, uint32_t bCur, uint32_t bNxt, uint32_t bFree) {
+            constexpr bool FULL = decltype(full)::value, ONE = decltype(one)::value;
+            if constexpr(ONE)
+                aCur = bCur, aNxt = bNxt;
             const uint32_t vB    = FULL ? STAGE_KB : validOf(kt + B_AHEAD);
             const i32x4    rsrcB = stageRsrc8(B_KCONTIG, refillB, vB, p.ldb);
             if(FULL || kt + B_AHEAD + 1u < numStages)
@@ -1197,91 +1206,116 @@ namespace
                     }
                     else if(q == LOAD_Q)
                     {
-                        if(x < WB)
+                        if(!ONE && x < WB)
                             loadToLds(rsrcA, offA(x, vA), x * gStepA, dmaDst + aCur + x * THREADS * CHUNK);
-                        else
+                        else if(x >= WB)
                             loadToLds(rsrcB, offB(x - WB, vB), (x - WB) * gStepB, dmaDst + bCur + (x - WB) * THREADS * CHUNK);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
         };
 
-        // prologue: stages 0 and 1 (and, where B runs three stages ahead, B of stage 2) requested in the order the
-        // loop keeps; stage 0 published
-        if constexpr(SPREAD)
-        {
-            issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, 0u), gOffB, gStepB, kByteB, p.ldb, validOf(0u), B_AT[0]);
-            issueHalf(LA, A_KCONTIG, stageAddr(gA, gStageA, 0u), gOffA, gStepA, kByteA, p.lda, validOf(0u), A_AT[0]);
-            issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, 1u), gOffB, gStepB, kByteB, p.ldb, validOf(1u), B_AT[1]);
-            issueHalf(LA, A_KCONTIG, stageAddr(gA, gStageA, 1u), gOffA, gStepA, kByteA, p.lda, validOf(1u), A_AT[1]);
-            waitVmcnt<LA + LB>();
-        }
-        else
-        {
-            issueHalf(LA, A_KCONTIG, stageAddr(gA, gStageA, 0u), gOffA, gStepA, kByteA, p.lda, validOf(0u), A_AT[0]);
-            issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, 0u), gOffB, gStepB, kByteB, p.ldb, validOf(0u), B_AT[0]);
-            issueHalf(LA, A_KCONTIG, stageAddr(gA, gStageA, 1u), gOffA, gStepA, kByteA, p.lda, validOf(1u), A_AT[1]);
-            issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, 1u), gOffB, gStepB, kByteB, p.ldb, validOf(1u), B_AT[1]);
-            issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, 2u), gOffB, gStepB, kByteB, p.ldb, validOf(2u), B_AT[2]);
-            waitVmcnt<3u * WB>();
-        }
-        refillA = stageAddr(gA, gStageA, 2u), refillB = stageAddr(gB, gStageB, B_AHEAD);
-        ldsBarrier();
-        R355_STAMP(1);
-#pragma unroll
-        for(uint32_t x = 0; x < XS; ++x)
-        {
-            readAt(A_AT[0], B_AT[0], 0, x, 0);
-            readAt(A_AT[0], B_AT[0], 0, x, 1);
-        }
-
-        // six stages per trip bring every buffer back to its role; single-exit loops, then the remainder.  The main part
-        // runs the trips whose requests (up to stage kt + 5 + B_AHEAD) all are whole stages inside K without the tail
-        // handling; the trips around the end of K and the remainder carry it.
-        // (Only a K-contiguous operand has a select to lose: with none, the main part is empty and compiles away.)
-        const uint32_t     wholeStages = (A_KCONTIG || B_KCONTIG) ? p.k / TK : 0u;
-        constexpr uint32_t REACH       = 5u + B_AHEAD;
-        const uint32_t     mainTrips   = wholeStages > REACH ? (wholeStages - REACH + 5u) / 6u : 0u;
-        using Main = std::true_type;
-        using Tail = std::false_type;
-        uint32_t kt = 0;
-        for(uint32_t trips = mainTrips; trips > 0; --trips, kt += 6u)
-        {
-            stageBody(Main{}, kt, A_AT[0], A_AT[1], B_AT[0], B_AT[1], B_AT[2]);
-            stageBody(Main{}, kt + 1u, A_AT[1], A_AT[0], B_AT[1], B_AT[2], B_AT[0]);
-            stageBody(Main{}, kt + 2u, A_AT[0], A_AT[1], B_AT[2], B_AT[0], B_AT[1]);
-            stageBody(Main{}, kt + 3u, A_AT[1], A_AT[0], B_AT[0], B_AT[1], B_AT[2]);
-            stageBody(Main{}, kt + 4u, A_AT[0], A_AT[1], B_AT[1], B_AT[2], B_AT[0]);
-            stageBody(Main{}, kt + 5u, A_AT[1], A_AT[0], B_AT[2], B_AT[0], B_AT[1]);
-        }
-        for(uint32_t trips = numStages / 6u - mainTrips; trips > 0; --trips, kt += 6u)
-        {
-            stageBody(Tail{}, kt, A_AT[0], A_AT[1], B_AT[0], B_AT[1], B_AT[2]);
-            stageBody(Tail{}, kt + 1u, A_AT[1], A_AT[0], B_AT[1], B_AT[2], B_AT[0]);
-            stageBody(Tail{}, kt + 2u, A_AT[0], A_AT[1], B_AT[2], B_AT[0], B_AT[1]);
-            stageBody(Tail{}, kt + 3u, A_AT[1], A_AT[0], B_AT[0], B_AT[1], B_AT[2]);
-            stageBody(Tail{}, kt + 4u, A_AT[0], A_AT[1], B_AT[1], B_AT[2], B_AT[0]);
-            stageBody(Tail{}, kt + 5u, A_AT[1], A_AT[0], B_AT[2], B_AT[0], B_AT[1]);
-        }
-        const uint32_t rem = numStages - kt;
-        if(rem > 0u)
-        {
-            stageBody(Tail{}, kt, A_AT[0], A_AT[1], B_AT[0], B_AT[1], B_AT[2]);
-            if(rem > 1u)
+        auto multiply = [&](auto one) {
+            constexpr bool ONE = decltype(one)::value;
+            // prologue: stages 0 and 1 (and, where B runs three stages ahead, B of stage 2) requested in the order the
+            // loop keeps; stage 0 published
+            if constexpr(SPREAD)
             {
-                stageBody(Tail{}, kt + 1u, A_AT[1], A_AT[0], B_AT[1], B_AT[2], B_AT[0]);
-                if(rem > 2u)
+                issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, 0u), gOffB, gStepB, kByteB, p.ldb, validOf(0u), B_AT[0]);
+                issueHalf(LA, A_KCONTIG, stageAddr(gA, gStageA, 0u), gOffA, gStepA, kByteA, p.lda, validOf(0u), A_AT[0]);
+                issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, 1u), gOffB, gStepB, kByteB, p.ldb, validOf(1u), B_AT[1]);
+                issueHalf(LA, A_KCONTIG, stageAddr(gA, gStageA, 1u), gOffA, gStepA, kByteA, p.lda, validOf(1u), A_AT[1]);
+                waitVmcnt<LA + LB>();
+            }
+            else if constexpr(ONE)
+            {
+#pragma unroll
+                for(uint32_t stage = 0; stage < 3u; ++stage)
+                    issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, stage), gOffB, gStepB, kByteB, p.ldb, validOf(stage), B_AT[stage]);
+                waitVmcnt<2u * WB>();
+            }
+            else
+            {
+                issueHalf(LA, A_KCONTIG, stageAddr(gA, gStageA, 0u), gOffA, gStepA, kByteA, p.lda, validOf(0u), A_AT[0]);
+                issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, 0u), gOffB, gStepB, kByteB, p.ldb, validOf(0u), B_AT[0]);
+                issueHalf(LA, A_KCONTIG, stageAddr(gA, gStageA, 1u), gOffA, gStepA, kByteA, p.lda, validOf(1u), A_AT[1]);
+                issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, 1u), gOffB, gStepB, kByteB, p.ldb, validOf(1u), B_AT[1]);
+                issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, 2u), gOffB, gStepB, kByteB, p.ldb, validOf(2u), B_AT[2]);
+                waitVmcnt<3u * WB>();
+            }
+            refillA = stageAddr(gA, gStageA, 2u), refillB = stageAddr(gB, gStageB, B_AHEAD);
+            ldsBarrier();
+            R355_STAMP(1);
+            if constexpr(ONE)
+                if(wm < wn) // (uniform) the wave tile above the diagonal: nothing to multiply, its share of the loads
                 {
-                    stageBody(Tail{}, kt + 2u, A_AT[0], A_AT[1], B_AT[2], B_AT[0], B_AT[1]);
-                    if(rem > 3u)
+                    for(uint32_t kt = 0, at = B_AT[0]; kt < numStages; ++kt, at = at == B_AT[2] ? B_AT[0] : at + OPER)
                     {
-                        stageBody(Tail{}, kt + 3u, A_AT[1], A_AT[0], B_AT[0], B_AT[1], B_AT[2]);
-                        if(rem > 4u)
-                            stageBody(Tail{}, kt + 4u, A_AT[0], A_AT[1], B_AT[1], B_AT[2], B_AT[0]);
+                        waitVmcnt<LB>();
+                        ldsBarrier();
+                        issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, kt + 3u), gOffB, gStepB, kByteB, p.ldb, validOf(kt + 3u), at);
+                    }
+                    return;
+                }
+#pragma unroll
+            for(uint32_t x = 0; x < XS; ++x)
+            {
+                readAt(ONE ? B_AT[0] : A_AT[0], B_AT[0], 0, x, 0);
+                readAt(ONE ? B_AT[0] : A_AT[0], B_AT[0], 0, x, 1);
+            }
+
+            // six stages per trip bring every buffer back to its role; single-exit loops, then the remainder.  The main part
+            // runs the trips whose requests (up to stage kt + 5 + B_AHEAD) all are whole stages inside K without the tail
+            // handling; the trips around the end of K and the remainder carry it.
+            // (Only a K-contiguous operand has a select to lose: with none, the main part is empty and compiles away.)
+            const uint32_t     wholeStages = (A_KCONTIG || B_KCONTIG) ? p.k / TK : 0u;
+            constexpr uint32_t REACH       = 5u + B_AHEAD;
+            const uint32_t     mainTrips   = wholeStages > REACH ? (wholeStages - REACH + 5u) / 6u : 0u;
+            using Main = std::true_type;
+            using Tail = std::false_type;
+            uint32_t kt = 0;
+            for(uint32_t trips = mainTrips; trips > 0; --trips, kt += 6u)
+            {
+                stageBody(Main{}, one, kt, A_AT[0], A_AT[1], B_AT[0], B_AT[1], B_AT[2]);
+                stageBody(Main{}, one, kt + 1u, A_AT[1], A_AT[0], B_AT[1], B_AT[2], B_AT[0]);
+                stageBody(Main{}, one, kt + 2u, A_AT[0], A_AT[1], B_AT[2], B_AT[0], B_AT[1]);
+                stageBody(Main{}, one, kt + 3u, A_AT[1], A_AT[0], B_AT[0], B_AT[1], B_AT[2]);
+                stageBody(Main{}, one, kt + 4u, A_AT[0], A_AT[1], B_AT[1], B_AT[2], B_AT[0]);
+                stageBody(Main{}, one, kt + 5u, A_AT[1], A_AT[0], B_AT[2], B_AT[0], B_AT[1]);
+            }
+            for(uint32_t trips = numStages / 6u - mainTrips; trips > 0; --trips, kt += 6u)
+            {
+                stageBody(Tail{}, one, kt, A_AT[0], A_AT[1], B_AT[0], B_AT[1], B_AT[2]);
+                stageBody(Tail{}, one, kt + 1u, A_AT[1], A_AT[0], B_AT[1], B_AT[2], B_AT[0]);
+                stageBody(Tail{}, one, kt + 2u, A_AT[0], A_AT[1], B_AT[2], B_AT[0], B_AT[1]);
+                stageBody(Tail{}, one, kt + 3u, A_AT[1], A_AT[0], B_AT[0], B_AT[1], B_AT[2]);
+                stageBody(Tail{}, one, kt + 4u, A_AT[0], A_AT[1], B_AT[1], B_AT[2], B_AT[0]);
+                stageBody(Tail{}, one, kt + 5u, A_AT[1], A_AT[0], B_AT[2], B_AT[0], B_AT[1]);
+            }
+            const uint32_t rem = numStages - kt;
+            if(rem > 0u)
+            {
+                stageBody(Tail{}, one, kt, A_AT[0], A_AT[1], B_AT[0], B_AT[1], B_AT[2]);
+                if(rem > 1u)
+                {
+                    stageBody(Tail{}, one, kt + 1u, A_AT[1], A_AT[0], B_AT[1], B_AT[2], B_AT[0]);
+                    if(rem > 2u)
+                    {
+                        stageBody(Tail{}, one, kt + 2u, A_AT[0], A_AT[1], B_AT[2], B_AT[0], B_AT[1]);
+                        if(rem > 3u)
+                        {
+                            stageBody(Tail{}, one, kt + 3u, A_AT[1], A_AT[0], B_AT[0], B_AT[1], B_AT[2]);
+                            if(rem > 4u)
+                                stageBody(Tail{}, one, kt + 4u, A_AT[0], A_AT[1], B_AT[1], B_AT[2], B_AT[0]);
+                        }
                     }
                 }
             }
-        }
+        };
+        if constexpr(TRIANGLE)
+            tm == tn ? multiply(std::true_type{}) : multiply(std::false_type{});
+        else
+            multiply(std::false_type{});
 
         R355_STAMP(2);
         // the loads past the last stage (zeros) are still landing in buffers the epilogue reuses, and the
