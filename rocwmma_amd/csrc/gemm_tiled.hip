@@ -1668,12 +1668,12 @@ namespace
     //     elements each (the M-contiguous image, transposing reads): the same 16-byte pieces at unaligned addresses either way,
     //     through registers into the image.  A stage of the diagonal tile is both images of its pieces left of the diagonal (16-bit;
     //     f32 gathers it element by element).
-    //   * two buffers per operand; the loads of stage kt + 1 are in flight under the matrix instructions of stage kt, and what
-    //     that leaves exposed other workgroups of the CU cover (two of the 128 x 128 tile, four of the 64 x 64 one: 80 and 40 KiB of LDS).
+    //   * the loads of stage kt + 1 are in flight under the matrix instructions of stage kt (16-bit: of stage kt - 1), and what that leaves exposed
+    //     other workgroups of the CU cover (two of the 128 x 128 tile, four of the 64 x 64 one: 64 and 32 KiB of LDS).
     // S holds zeros only on its diagonal and beyond row or column m, as the products of the [m][m] matrix have them.  Few stages bound
     // the small shapes (latency of one stage's loads each), the matrix instructions and the loads' distance the large ones:
-    // f16 1024 x 1024 x 64 232 us, bf16 320 x 192 x 96 13.6, bf16 64 x 400 x 1011 25.9, f32 224 x 384 x 213 97.  (Gathered element by element,
-    // eight 2-byte loads for each 16 bytes, the diagonal stages took the 16-bit ones to 250, 16.7 and 39.5; without the matrix instructions the
+    // f16 1024 x 1024 x 64 223 us, bf16 320 x 192 x 96 13.1, bf16 64 x 400 x 1011 25.9, f32 224 x 384 x 213 97.  (Gathered element by element,
+    // eight 2-byte loads for each 16 bytes, the diagonal stages took the 16-bit ones from 232, 13.7 and 25.9 to 250, 16.7 and 39.5; without the matrix instructions the
     // times do not change, so multiplying by a diagonal stage twice costs nothing there.)
     using BwdParams = r355::DlrmBwdParams;
 
@@ -1685,8 +1685,8 @@ namespace
         using Word            = std::conditional_t<ES == 2, uint16_t, uint32_t>;
         typedef int i32x4u __attribute__((ext_vector_type(4), aligned(2)));
         constexpr bool     ACROSS = ES == 2; // a diagonal stage's mirrored elements are an image of their own (f32: gathered)
-        constexpr uint32_t B_AT = 2u * OPER, ACROSS_AT = 4u * OPER; // two buffers of A, two of B, that image
-        __shared__ __attribute__((aligned(1024))) char lds[(ACROSS ? 5u : 4u) * OPER];
+        constexpr uint32_t B_AT = 2u * OPER, ACROSS_AT = OPER; // a buffer of A and that image (f32: two of A), two of B
+        __shared__ __attribute__((aligned(1024))) char lds[4u * OPER];
 
         // all workgroups of an XCD walk one contiguous run of (sample, tile): the tiles of a sample share its X and T in one L2
         const uint32_t perXcd = (p.total + 7u) / 8u, slotX = blockIdx.x / 8u, local = (blockIdx.x % 8u) * perXcd + slotX;
@@ -1847,19 +1847,27 @@ namespace
                 }
             }
         };
-        auto compute = [&](auto aK, uint32_t aAt, uint32_t bAt) {
+        i32x4 fa[2][WB], fb[2][WB];
+        auto  readA = [&](auto aK, uint32_t at) {
             constexpr bool AK = decltype(aK)::value;
-            i32x4          fa[2][WB], fb[2][WB];
 #pragma unroll
             for(uint32_t s = 0; s < 2; ++s)
 #pragma unroll
                 for(uint32_t i = 0; i < WB; ++i)
 #pragma unroll
                     for(uint32_t part = 0; part < 2; ++part)
-                    {
-                        readBlock8<AK, WB, ES>(lds + aAt, AK ? rdAK : rdAM, i, s, part, fa[s][i], 0u);
-                        readBlock8<false, WB, ES>(lds + bAt, rdB, i, s, part, fb[s][i], 0u);
-                    }
+                        readBlock8<AK, WB, ES>(lds + at, AK ? rdAK : rdAM, i, s, part, fa[s][i], 0u);
+        };
+        auto readB = [&](uint32_t at) {
+#pragma unroll
+            for(uint32_t s = 0; s < 2; ++s)
+#pragma unroll
+                for(uint32_t i = 0; i < WB; ++i)
+#pragma unroll
+                    for(uint32_t part = 0; part < 2; ++part)
+                        readBlock8<false, WB, ES>(lds + at, rdB, i, s, part, fb[s][i], 0u);
+        };
+        auto products = [&] {
 #pragma unroll
             for(uint32_t s = 0; s < 2; ++s)
 #pragma unroll
@@ -1871,33 +1879,72 @@ namespace
 
         issueB(0u, B_AT);
         loadA(0u);
+        if constexpr(ACROSS)
+            waitVmcnt<0>();
         writeA(0u, 0u);
-        waitVmcnt<0>();
+        if constexpr(!ACROSS)
+            waitVmcnt<0>();
+        else if(numStages > 1u)
+        {
+            issueB(1u, B_AT + OPER);
+            loadA(1u);
+        }
         ldsBarrier();
-        auto stageBody = [&](auto aK, uint32_t st) {
+        // 16-bit, bound by its loads: a stage is read into registers whole, and while it is multiplied the next, requested a stage before, takes
+        // its place in LDS and the one after that is requested (requested and awaited around the same multiplications: f16 1024 x 1024 x 64 234 us
+        // for 223, 1024 x 256 x 4 13.3 for 12.1, bf16 320 x 192 x 96 13.7 for 13.1).
+        auto stageAhead = [&](auto aK, uint32_t st) {
+            const uint32_t bAt = B_AT + (st & 1u) * OPER;
+            readA(aK, 0u);
+            readB(bAt);
+            if constexpr(decltype(aK)::value)
+                if(inDiag(st))
+                {
+                    products();
+                    readA(std::false_type{}, ACROSS_AT);
+                }
+            ldsBarrier(); // every wave has this stage in registers
+            if(st + 1u < numStages) // (uniform)
+            {
+                waitVmcnt<0>();
+                writeA(0u, st + 1u);
+                if(st + 2u < numStages)
+                {
+                    issueB(st + 2u, bAt);
+                    loadA(st + 2u);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            products();
+            if(st + 1u < numStages)
+                ldsBarrier();
+        };
+        // f32, bound by the matrix instructions: one barrier a stage (as above 1024 x 1024 x 64 1077 -> 1163 us, 112 x 48 x 847 24.5 -> 26.5)
+        auto stageNext = [&](auto aK, uint32_t st) {
             const uint32_t cur = (st & 1u) * OPER, nxt = OPER - cur;
             const bool     more = st + 1u < numStages; // (uniform)
             if(more)
             {
                 issueB(st + 1u, B_AT + nxt);
-                if constexpr(!ACROSS && !decltype(aK)::value)
-                    loadRight(st + 1u);
-                else
+                if constexpr(decltype(aK)::value)
                     loadA(st + 1u);
+                else
+                    loadRight(st + 1u);
             }
-            compute(aK, cur, B_AT + cur);
-            if constexpr(ACROSS && decltype(aK)::value)
-                if(inDiag(st))
-                    compute(std::false_type{}, ACROSS_AT, B_AT + cur);
+            readA(aK, cur);
+            readB(B_AT + cur);
+            products();
             if(more)
-            {
-                if(ACROSS && decltype(aK)::value && inDiag(st) && inDiag(st + 1u))
-                    ldsBarrier(); // the mirrored image is being read until every wave has multiplied by it
                 writeA(nxt, st + 1u);
-            }
             // the direct loads of the next stage have landed, and every wave has read this one
             waitVmcnt<0>();
             ldsBarrier();
+        };
+        auto stageBody = [&](auto aK, uint32_t st) {
+            if constexpr(ACROSS)
+                stageAhead(aK, st);
+            else
+                stageNext(aK, st);
         };
         uint32_t st = 0;
         for(; st < diagEnd; ++st)
