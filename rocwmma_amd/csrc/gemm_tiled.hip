@@ -586,6 +586,46 @@ namespace
         }
     }
 
+    // The same for a whole macro tile left of the diagonal tile, its rows (256 bytes; 16-bit 64 x 64 tile: 128) as one run each instead
+    // of one per wave tile: all four waves stage the tile in LDS, and each stores a quarter of its rows.  Bound by the L2, which puts a
+    // run's partial lines together with the neighbouring tile's; whole runs, and not kept afterwards (nontemporal): f16 512 x 256 x 200,
+    // 12 us of it stores, 35.4 -> 34.9 as rows, 29.9 nontemporal too; 512 x 512 x 120 32.6 -> 27.9, 256 x 112 x 756
+    // 31.7 -> 27.7, f32 1024 x 64 x 64 66.7 -> 58.8, f16 1024 x 1024 x 64 89.6 -> 88 - 89.  Stored per wave tile, nontemporal runs of 128 bytes
+    // were slower (1024 x 64 x 64 24.4 -> 35), and so are those of the diagonal tiles, which stay ordinary stores (24.2 -> 27.8).
+    template <typename OutT, uint32_t WB>
+    __device__ __forceinline__ void storeTriangleRows(f32x4 (&acc)[WB][WB], OutT* d, uint32_t m, uint32_t row0, uint32_t col0, uint32_t wave, uint32_t lane,
+                                                      char* scratch)
+    {
+        constexpr uint32_t OS = sizeof(OutT), TILE = 32u * WB, WT = 16u * WB, ROW_BYTES = TILE * OS, ROW_CHUNKS = ROW_BYTES / CHUNK;
+        constexpr uint32_t SWZ = ROW_CHUNKS < 16u ? ROW_CHUNKS - 1u : 15u, EPC = CHUNK / OS, RPI = 64u / ROW_CHUNKS;
+        using OutV = OutT __attribute__((ext_vector_type(4)));
+        typedef int i32x4u __attribute__((ext_vector_type(4), aligned(2)));
+        const uint32_t r16 = lane & 15u, g = lane >> 4;
+#pragma unroll
+        for(uint32_t i = 0; i < WB; ++i)
+#pragma unroll
+            for(uint32_t j = 0; j < WB; ++j)
+            {
+                OutV out;
+#pragma unroll
+                for(uint32_t e = 0; e < 4; ++e)
+                    out[e] = static_cast<OutT>(acc[i][j][e]);
+                const uint32_t row = (wave >> 1) * WT + 16u * i + r16, byteInRow = ((wave & 1u) * WT + 16u * j + 4u * g) * OS;
+                *reinterpret_cast<OutV*>(scratch + row * ROW_BYTES + (((byteInRow / CHUNK) ^ (row & SWZ)) * CHUNK) + byteInRow % CHUNK) = out;
+            }
+        r355::ldsBarrier();
+        const uint32_t c = lane % ROW_CHUNKS;
+#pragma unroll
+        for(uint32_t it = 0; it < TILE / 4u / RPI; ++it)
+        {
+            const uint32_t row = wave * (TILE / 4u) + it * RPI + lane / ROW_CHUNKS;
+            const i32x4    v   = *reinterpret_cast<const i32x4*>(scratch + row * ROW_BYTES + ((c ^ (row & SWZ)) * CHUNK));
+            const uint64_t gi  = row0 + row;
+            if(gi < m)
+                __builtin_nontemporal_store(v, reinterpret_cast<i32x4u*>(d + (gi * (gi - 1u) / 2u + col0 + c * EPC)));
+        }
+    }
+
     //
     // WB is the number of accumulator blocks per wave tile edge: 8 (wave tile 128 x 128, macro tile
     // 256 x 256, one workgroup per CU).  The body also works with 4 (wave tile 64 x 64, macro tile
@@ -1323,6 +1363,12 @@ namespace
         asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
         waitVmcnt<0>();
         ldsBarrier();
+        if constexpr(TRIANGLE)
+            if(tm != tn)
+            {
+                storeTriangleRows<OutT, WB>(acc, reinterpret_cast<OutT*>(p.d), p.m, tm * TILE, tn * TILE, wave, lane, lds);
+                return;
+            }
         if constexpr(TRIANGLE)
             storeTriangle<OutT, WB>(acc, reinterpret_cast<OutT*>(p.d), p.m, tm * TILE + wm * WT, tn * TILE + wn * WT, lane, lds + wave * (WB * 4096u));
         else
