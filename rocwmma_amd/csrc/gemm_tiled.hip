@@ -1712,15 +1712,15 @@ namespace
     //   * A = S lies in memory as rows of T that start at any element.  Left of the diagonal tile a stage is TILE rows x 128 bytes
     //     of T (the K-contiguous image); right of it S(i, j) = T(j, i), so a stage is 128 bytes' worth of rows of T, TILE
     //     elements each (the M-contiguous image, transposing reads): the same 16-byte pieces at unaligned addresses either way,
-    //     through registers into the image.  A stage of the diagonal tile is both images of its pieces left of the diagonal (16-bit;
-    //     f32 gathers it element by element).
+    //     through registers into the image.  A stage of the diagonal tile is both images of its pieces left of the diagonal, put together
+    //     in registers (16-bit; f32 gathers it element by element).
     //   * the loads of stage kt + 1 are in flight under the matrix instructions of stage kt (16-bit: of stage kt - 1), and what that leaves exposed
     //     other workgroups of the CU cover (two of the 128 x 128 tile, four of the 64 x 64 one: 64 and 32 KiB of LDS).
-    // S holds zeros only on its diagonal and beyond row or column m, as the products of the [m][m] matrix have them.  Few stages bound
-    // the small shapes (latency of one stage's loads each), the matrix instructions and the loads' distance the large ones:
-    // f16 1024 x 1024 x 64 223 us, bf16 320 x 192 x 96 13.1, bf16 64 x 400 x 1011 25.9, f32 224 x 384 x 213 97.  (Gathered element by element,
-    // eight 2-byte loads for each 16 bytes, the diagonal stages took the 16-bit ones from 232, 13.7 and 25.9 to 250, 16.7 and 39.5; without the matrix instructions the
-    // times do not change, so multiplying by a diagonal stage twice costs nothing there.)
+    // S holds zeros only on its diagonal and beyond row or column m, as the products of the [m][m] matrix have them: an infinite feature is NaN
+    // in its own row of the gradient and nowhere else.  Few stages bound the small shapes (latency of one stage's loads each), the matrix
+    // instructions and the loads' distance the large ones: f16 1024 x 1024 x 64 219 us, bf16 320 x 192 x 96 12.9, bf16 64 x 400 x 1011 25.5, f32
+    // 224 x 384 x 213 96.  (The 16-bit ones 225, 13.0 and 25.8 with a diagonal stage's images multiplied one after the other; 250, 16.7 and 39.5
+    // gathered element by element, eight 2-byte loads for each 16 bytes, and every stage requested one ahead.)
     using BwdParams = r355::DlrmBwdParams;
 
     template <Elem E, typename T, uint32_t WB>
@@ -1773,10 +1773,10 @@ namespace
         const uint32_t diagFirst = row0 / TK, diagEnd = diagFirst + TILE / TK < numStages ? diagFirst + TILE / TK : numStages;
         const uint32_t rK = tid >> 3, cK = ((tid & 7u) ^ swzK8(tid >> 3)) * EPC; // K-contiguous image: row rK + 32 j, first column of the piece
         // A stage of the diagonal tile.  16-bit: two images, T's rows left of the diagonal (K-contiguous), and the stage's rows of T within
-        // the tile's columns (M-contiguous, in a buffer of its own), multiplied one after the other.  A piece that the diagonal cuts is
-        // read as the row's last EPC elements and moved down, which puts zeros in the place of the rest (a row shorter than that
-        // reads into the k elements before the triangle).  f32: gathered element by element, a quarter as many loads per byte, where the
-        // second multiplication would cost more (224 x 384 x 213 96 us gathered, 113 as two images).
+        // the tile's columns (M-contiguous, in a buffer of its own).  A piece that the diagonal cuts is read as the row's last EPC
+        // elements and moved down, which puts zeros in the place of the rest (a row shorter than that reads into the k elements before the
+        // triangle).  f32: gathered element by element, a quarter as many loads per byte (as two images, multiplied one after the other,
+        // 224 x 384 x 213 took 113 us for 96).
         i32x4 aNext[WB], aAcross[WB];
         auto  cutBy   = [](uint32_t row, uint32_t col) { return row < col + EPC ? col + EPC - row : 0u; }; // elements from the diagonal on
         auto  loadCut = [&](uint32_t row, uint32_t col) {
@@ -1904,6 +1904,18 @@ namespace
                     for(uint32_t part = 0; part < 2; ++part)
                         readBlock8<AK, WB, ES>(lds + at, AK ? rdAK : rdAM, i, s, part, fa[s][i], 0u);
         };
+        auto addAcross = [&] { // (both images come in the same register layout, and where one holds an element of S the other holds zero bits)
+#pragma unroll
+            for(uint32_t s = 0; s < 2; ++s)
+#pragma unroll
+                for(uint32_t i = 0; i < WB; ++i)
+                {
+                    i32x4 across;
+                    readBlock8<false, WB, ES>(lds + ACROSS_AT, rdAM, i, s, 0u, across, 0u);
+                    readBlock8<false, WB, ES>(lds + ACROSS_AT, rdAM, i, s, 1u, across, 0u);
+                    fa[s][i] |= across;
+                }
+        };
         auto readB = [&](uint32_t at) {
 #pragma unroll
             for(uint32_t s = 0; s < 2; ++s)
@@ -1942,13 +1954,10 @@ namespace
         auto stageAhead = [&](auto aK, uint32_t st) {
             const uint32_t bAt = B_AT + (st & 1u) * OPER;
             readA(aK, 0u);
-            readB(bAt);
             if constexpr(decltype(aK)::value)
-                if(inDiag(st))
-                {
-                    products();
-                    readA(std::false_type{}, ACROSS_AT);
-                }
+                if(inDiag(st)) // S whole before it is multiplied: a zero of one image times an infinite feature would be NaN
+                    addAcross();
+            readB(bAt);
             ldsBarrier(); // every wave has this stage in registers
             if(st + 1u < numStages) // (uniform)
             {
