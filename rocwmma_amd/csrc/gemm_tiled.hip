@@ -1255,8 +1255,14 @@ namespace
                 }
         };
 
-        auto multiply = [&](auto one) {
-            constexpr bool ONE = decltype(one)::value;
+        using Main = std::true_type;
+        using Tail = std::false_type;
+        // The K loop stands here twice.  Once, in a generic lambda called for either kind of tile, it cost 39 of GEMM's kernels scalars that were kept in
+        // vector registers and read back in the loop (up to 31 in six stages; col-col products 1 - 2 % longer, int8 4096^3 56.5 -> 57.6 us); as
+        // two instantiations of this body it cost the triangle's small launches up to 5 % (320 x 192 x 96 8.9 -> 9.3).
+        constexpr std::false_type both;
+        if(!TRIANGLE || tm != tn)
+        {
             // prologue: stages 0 and 1 (and, where B runs three stages ahead, B of stage 2) requested in the order the
             // loop keeps; stage 0 published
             if constexpr(SPREAD)
@@ -1266,13 +1272,6 @@ namespace
                 issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, 1u), gOffB, gStepB, kByteB, p.ldb, validOf(1u), B_AT[1]);
                 issueHalf(LA, A_KCONTIG, stageAddr(gA, gStageA, 1u), gOffA, gStepA, kByteA, p.lda, validOf(1u), A_AT[1]);
                 waitVmcnt<LA + LB>();
-            }
-            else if constexpr(ONE)
-            {
-#pragma unroll
-                for(uint32_t stage = 0; stage < 3u; ++stage)
-                    issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, stage), gOffB, gStepB, kByteB, p.ldb, validOf(stage), B_AT[stage]);
-                waitVmcnt<2u * WB>();
             }
             else
             {
@@ -1286,22 +1285,11 @@ namespace
             refillA = stageAddr(gA, gStageA, 2u), refillB = stageAddr(gB, gStageB, B_AHEAD);
             ldsBarrier();
             R355_STAMP(1);
-            if constexpr(ONE)
-                if(wm < wn) // (uniform) the wave tile above the diagonal: nothing to multiply, its share of the loads
-                {
-                    for(uint32_t kt = 0, at = B_AT[0]; kt < numStages; ++kt, at = at == B_AT[2] ? B_AT[0] : at + OPER)
-                    {
-                        waitVmcnt<LB>();
-                        ldsBarrier();
-                        issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, kt + 3u), gOffB, gStepB, kByteB, p.ldb, validOf(kt + 3u), at);
-                    }
-                    return;
-                }
 #pragma unroll
             for(uint32_t x = 0; x < XS; ++x)
             {
-                readAt(ONE ? B_AT[0] : A_AT[0], B_AT[0], 0, x, 0);
-                readAt(ONE ? B_AT[0] : A_AT[0], B_AT[0], 0, x, 1);
+                readAt(A_AT[0], B_AT[0], 0, x, 0);
+                readAt(A_AT[0], B_AT[0], 0, x, 1);
             }
 
             // six stages per trip bring every buffer back to its role; single-exit loops, then the remainder.  The main part
@@ -1311,51 +1299,112 @@ namespace
             const uint32_t     wholeStages = (A_KCONTIG || B_KCONTIG) ? p.k / TK : 0u;
             constexpr uint32_t REACH       = 5u + B_AHEAD;
             const uint32_t     mainTrips   = wholeStages > REACH ? (wholeStages - REACH + 5u) / 6u : 0u;
-            using Main = std::true_type;
-            using Tail = std::false_type;
-            uint32_t kt = 0;
+            uint32_t           kt = 0;
             for(uint32_t trips = mainTrips; trips > 0; --trips, kt += 6u)
             {
-                stageBody(Main{}, one, kt, A_AT[0], A_AT[1], B_AT[0], B_AT[1], B_AT[2]);
-                stageBody(Main{}, one, kt + 1u, A_AT[1], A_AT[0], B_AT[1], B_AT[2], B_AT[0]);
-                stageBody(Main{}, one, kt + 2u, A_AT[0], A_AT[1], B_AT[2], B_AT[0], B_AT[1]);
-                stageBody(Main{}, one, kt + 3u, A_AT[1], A_AT[0], B_AT[0], B_AT[1], B_AT[2]);
-                stageBody(Main{}, one, kt + 4u, A_AT[0], A_AT[1], B_AT[1], B_AT[2], B_AT[0]);
-                stageBody(Main{}, one, kt + 5u, A_AT[1], A_AT[0], B_AT[2], B_AT[0], B_AT[1]);
+                stageBody(Main{}, both, kt, A_AT[0], A_AT[1], B_AT[0], B_AT[1], B_AT[2]);
+                stageBody(Main{}, both, kt + 1u, A_AT[1], A_AT[0], B_AT[1], B_AT[2], B_AT[0]);
+                stageBody(Main{}, both, kt + 2u, A_AT[0], A_AT[1], B_AT[2], B_AT[0], B_AT[1]);
+                stageBody(Main{}, both, kt + 3u, A_AT[1], A_AT[0], B_AT[0], B_AT[1], B_AT[2]);
+                stageBody(Main{}, both, kt + 4u, A_AT[0], A_AT[1], B_AT[1], B_AT[2], B_AT[0]);
+                stageBody(Main{}, both, kt + 5u, A_AT[1], A_AT[0], B_AT[2], B_AT[0], B_AT[1]);
             }
             for(uint32_t trips = numStages / 6u - mainTrips; trips > 0; --trips, kt += 6u)
             {
-                stageBody(Tail{}, one, kt, A_AT[0], A_AT[1], B_AT[0], B_AT[1], B_AT[2]);
-                stageBody(Tail{}, one, kt + 1u, A_AT[1], A_AT[0], B_AT[1], B_AT[2], B_AT[0]);
-                stageBody(Tail{}, one, kt + 2u, A_AT[0], A_AT[1], B_AT[2], B_AT[0], B_AT[1]);
-                stageBody(Tail{}, one, kt + 3u, A_AT[1], A_AT[0], B_AT[0], B_AT[1], B_AT[2]);
-                stageBody(Tail{}, one, kt + 4u, A_AT[0], A_AT[1], B_AT[1], B_AT[2], B_AT[0]);
-                stageBody(Tail{}, one, kt + 5u, A_AT[1], A_AT[0], B_AT[2], B_AT[0], B_AT[1]);
+                stageBody(Tail{}, both, kt, A_AT[0], A_AT[1], B_AT[0], B_AT[1], B_AT[2]);
+                stageBody(Tail{}, both, kt + 1u, A_AT[1], A_AT[0], B_AT[1], B_AT[2], B_AT[0]);
+                stageBody(Tail{}, both, kt + 2u, A_AT[0], A_AT[1], B_AT[2], B_AT[0], B_AT[1]);
+                stageBody(Tail{}, both, kt + 3u, A_AT[1], A_AT[0], B_AT[0], B_AT[1], B_AT[2]);
+                stageBody(Tail{}, both, kt + 4u, A_AT[0], A_AT[1], B_AT[1], B_AT[2], B_AT[0]);
+                stageBody(Tail{}, both, kt + 5u, A_AT[1], A_AT[0], B_AT[2], B_AT[0], B_AT[1]);
             }
             const uint32_t rem = numStages - kt;
             if(rem > 0u)
             {
-                stageBody(Tail{}, one, kt, A_AT[0], A_AT[1], B_AT[0], B_AT[1], B_AT[2]);
+                stageBody(Tail{}, both, kt, A_AT[0], A_AT[1], B_AT[0], B_AT[1], B_AT[2]);
                 if(rem > 1u)
                 {
-                    stageBody(Tail{}, one, kt + 1u, A_AT[1], A_AT[0], B_AT[1], B_AT[2], B_AT[0]);
+                    stageBody(Tail{}, both, kt + 1u, A_AT[1], A_AT[0], B_AT[1], B_AT[2], B_AT[0]);
                     if(rem > 2u)
                     {
-                        stageBody(Tail{}, one, kt + 2u, A_AT[0], A_AT[1], B_AT[2], B_AT[0], B_AT[1]);
+                        stageBody(Tail{}, both, kt + 2u, A_AT[0], A_AT[1], B_AT[2], B_AT[0], B_AT[1]);
                         if(rem > 3u)
                         {
-                            stageBody(Tail{}, one, kt + 3u, A_AT[1], A_AT[0], B_AT[0], B_AT[1], B_AT[2]);
+                            stageBody(Tail{}, both, kt + 3u, A_AT[1], A_AT[0], B_AT[0], B_AT[1], B_AT[2]);
                             if(rem > 4u)
-                                stageBody(Tail{}, one, kt + 4u, A_AT[0], A_AT[1], B_AT[1], B_AT[2], B_AT[0]);
+                                stageBody(Tail{}, both, kt + 4u, A_AT[0], A_AT[1], B_AT[1], B_AT[2], B_AT[0]);
                         }
                     }
                 }
             }
-        };
-        if constexpr(TRIANGLE)
-            tm == tn ? multiply(std::true_type{}) : multiply(std::false_type{});
-        else
-            multiply(std::false_type{});
+        }
+        else if constexpr(TRIANGLE) // a diagonal tile
+        {
+#pragma unroll
+            for(uint32_t stage = 0; stage < 3u; ++stage)
+                issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, stage), gOffB, gStepB, kByteB, p.ldb, validOf(stage), B_AT[stage]);
+            waitVmcnt<2u * WB>();
+            refillA = 0u, refillB = stageAddr(gB, gStageB, B_AHEAD);
+            ldsBarrier();
+            R355_STAMP(1);
+            if(wm < wn) // (uniform) the wave tile above the diagonal: nothing to multiply, its share of the loads
+                for(uint32_t kt = 0, at = B_AT[0]; kt < numStages; ++kt, at = at == B_AT[2] ? B_AT[0] : at + OPER)
+                {
+                    waitVmcnt<LB>();
+                    ldsBarrier();
+                    issueHalf(LB, B_KCONTIG, stageAddr(gB, gStageB, kt + 3u), gOffB, gStepB, kByteB, p.ldb, validOf(kt + 3u), at);
+                }
+            else
+            {
+                constexpr std::true_type one; // (the buffers of A hold nothing)
+#pragma unroll
+                for(uint32_t x = 0; x < XS; ++x)
+                {
+                    readAt(B_AT[0], B_AT[0], 0, x, 0);
+                    readAt(B_AT[0], B_AT[0], 0, x, 1);
+                }
+                constexpr uint32_t REACH       = 5u + B_AHEAD;
+                const uint32_t     wholeStages = p.k / TK, mainTrips = wholeStages > REACH ? (wholeStages - REACH + 5u) / 6u : 0u;
+                uint32_t           kt = 0;
+                for(uint32_t trips = mainTrips; trips > 0; --trips, kt += 6u)
+                {
+                    stageBody(Main{}, one, kt, 0u, 0u, B_AT[0], B_AT[1], B_AT[2]);
+                    stageBody(Main{}, one, kt + 1u, 0u, 0u, B_AT[1], B_AT[2], B_AT[0]);
+                    stageBody(Main{}, one, kt + 2u, 0u, 0u, B_AT[2], B_AT[0], B_AT[1]);
+                    stageBody(Main{}, one, kt + 3u, 0u, 0u, B_AT[0], B_AT[1], B_AT[2]);
+                    stageBody(Main{}, one, kt + 4u, 0u, 0u, B_AT[1], B_AT[2], B_AT[0]);
+                    stageBody(Main{}, one, kt + 5u, 0u, 0u, B_AT[2], B_AT[0], B_AT[1]);
+                }
+                for(uint32_t trips = numStages / 6u - mainTrips; trips > 0; --trips, kt += 6u)
+                {
+                    stageBody(Tail{}, one, kt, 0u, 0u, B_AT[0], B_AT[1], B_AT[2]);
+                    stageBody(Tail{}, one, kt + 1u, 0u, 0u, B_AT[1], B_AT[2], B_AT[0]);
+                    stageBody(Tail{}, one, kt + 2u, 0u, 0u, B_AT[2], B_AT[0], B_AT[1]);
+                    stageBody(Tail{}, one, kt + 3u, 0u, 0u, B_AT[0], B_AT[1], B_AT[2]);
+                    stageBody(Tail{}, one, kt + 4u, 0u, 0u, B_AT[1], B_AT[2], B_AT[0]);
+                    stageBody(Tail{}, one, kt + 5u, 0u, 0u, B_AT[2], B_AT[0], B_AT[1]);
+                }
+                const uint32_t rem = numStages - kt;
+                if(rem > 0u)
+                {
+                    stageBody(Tail{}, one, kt, 0u, 0u, B_AT[0], B_AT[1], B_AT[2]);
+                    if(rem > 1u)
+                    {
+                        stageBody(Tail{}, one, kt + 1u, 0u, 0u, B_AT[1], B_AT[2], B_AT[0]);
+                        if(rem > 2u)
+                        {
+                            stageBody(Tail{}, one, kt + 2u, 0u, 0u, B_AT[2], B_AT[0], B_AT[1]);
+                            if(rem > 3u)
+                            {
+                                stageBody(Tail{}, one, kt + 3u, 0u, 0u, B_AT[0], B_AT[1], B_AT[2]);
+                                if(rem > 4u)
+                                    stageBody(Tail{}, one, kt + 4u, 0u, 0u, B_AT[1], B_AT[2], B_AT[0]);
+                            }
+                        }
+                    }
+                }
+            }
+        }
 
         R355_STAMP(2);
         // the loads past the last stage (zeros) are still landing in buffers the epilogue reuses, and the
@@ -1367,6 +1416,7 @@ namespace
             if(tm != tn)
             {
                 storeTriangleRows<OutT, WB>(acc, reinterpret_cast<OutT*>(p.d), p.m, tm * TILE, tn * TILE, wave, lane, lds);
+                R355_STAMP_END();
                 return;
             }
         if constexpr(TRIANGLE)
