@@ -144,9 +144,9 @@ namespace r355
     int gemmTiledPart2(const r355_gemm_args& g, bool aK, bool bK, uint32_t tile, const GemmTileParams& p, hipStream_t s);
     int gemmTiledPart3(const r355_gemm_args& g, bool aK, bool bK, uint32_t tile, const GemmTileParams& p, hipStream_t s);
     // DLRM forward on macro tiles of X X^T (dlrmFwdTiled below), one per element type
-    int dlrmFwdTiledPart0(const GemmTileParams& p, uint32_t tile, uint32_t groups, hipStream_t s);
-    int dlrmFwdTiledPart1(const GemmTileParams& p, uint32_t tile, uint32_t groups, hipStream_t s);
-    int dlrmFwdTiledPart3(const GemmTileParams& p, uint32_t tile, uint32_t groups, hipStream_t s);
+    int dlrmFwdTiledPart0(const GemmTileParams& p, uint32_t tile, uint32_t groups, bool nontemporal, hipStream_t s);
+    int dlrmFwdTiledPart1(const GemmTileParams& p, uint32_t tile, uint32_t groups, bool nontemporal, hipStream_t s);
+    int dlrmFwdTiledPart3(const GemmTileParams& p, uint32_t tile, uint32_t groups, bool nontemporal, hipStream_t s);
     // DLRM backward on macro tiles of S X (dlrmBwdTile below), one per element type
     struct DlrmBwdParams
     {
@@ -586,13 +586,14 @@ namespace
         }
     }
 
-    // The same for a whole macro tile left of the diagonal tile, its rows (256 bytes; 16-bit 64 x 64 tile: 128) as one run each instead
-    // of one per wave tile: all four waves stage the tile in LDS, and each stores a quarter of its rows.  Bound by the L2, which puts a
-    // run's partial lines together with the neighbouring tile's; whole runs, and not kept afterwards (nontemporal): f16 512 x 256 x 200,
-    // 12 us of it stores, 35.4 -> 34.9 as rows, 29.9 nontemporal too; 512 x 512 x 120 32.6 -> 27.9, 256 x 112 x 756
-    // 31.7 -> 27.7, f32 1024 x 64 x 64 66.7 -> 58.8, f16 1024 x 1024 x 64 89.6 -> 88 - 89.  Stored per wave tile, nontemporal runs of 128 bytes
-    // were slower (1024 x 64 x 64 24.4 -> 35), and so are those of the diagonal tiles, which stay ordinary stores (24.2 -> 27.8).
-    template <typename OutT, uint32_t WB>
+    // The same for a whole macro tile left of the diagonal tile, its rows (128 bytes of the 16-bit 64 x 64 tile to 512 of the f32
+    // 128 x 128 one) as one run each instead of one per wave tile: all four waves stage the tile in LDS, and each stores a quarter of its
+    // rows.  Bound by the L2, which puts a run's partial lines together with the neighbouring tile's.  NONTEMPORAL for launches that do not
+    // fit the L2 (dlrmFwdTiled): f16 512 x 256 x 200, 12 us of it stores, 35.4 -> 34.9 as rows, 28.4 nontemporal too; 512 x 512 x 120
+    // 31.6 -> 30.8 -> 27.2, 256 x 112 x 756 31.4 -> 31.1 -> 26.6, f32 1024 x 64 x 64 63.4 -> 63.2 -> 54.5, f16 1024 x 1024 x 64 the same
+    // throughout, 1024 x 64 x 64 23.3 -> 22.5 -> 23.7.  Stored per wave tile, nontemporal runs of 128 bytes were slower (24.4 -> 35), and so are
+    // those of the diagonal tiles, which stay ordinary stores (24.2 -> 27.8).
+    template <typename OutT, uint32_t WB, bool NONTEMPORAL>
     __device__ __forceinline__ void storeTriangleRows(f32x4 (&acc)[WB][WB], OutT* d, uint32_t m, uint32_t row0, uint32_t col0, uint32_t wave, uint32_t lane,
                                                       char* scratch)
     {
@@ -621,8 +622,14 @@ namespace
             const uint32_t row = wave * (TILE / 4u) + it * RPI + lane / ROW_CHUNKS;
             const i32x4    v   = *reinterpret_cast<const i32x4*>(scratch + row * ROW_BYTES + ((c ^ (row & SWZ)) * CHUNK));
             const uint64_t gi  = row0 + row;
+            i32x4u* const  to  = reinterpret_cast<i32x4u*>(d + (gi * (gi - 1u) / 2u + col0 + c * EPC));
             if(gi < m)
-                __builtin_nontemporal_store(v, reinterpret_cast<i32x4u*>(d + (gi * (gi - 1u) / 2u + col0 + c * EPC)));
+            {
+                if constexpr(NONTEMPORAL)
+                    __builtin_nontemporal_store(v, to);
+                else
+                    *to = v;
+            }
         }
     }
 
@@ -1050,7 +1057,7 @@ namespace
     // stages ahead, and its wave tile above the diagonal is left out: f16 1024 x 1024 x 64 (8 of a sample's 36 tiles) 96.3 -> 87 - 91 us,
     // 96 x 576 x 1116 (all of them) 41.4 -> 36.8, 64 x 1024 x 200 on 64 x 64 tiles 7.5 -> 6.9.  (Into A's two buffers, two
     // stages ahead: 94, 37.6 and 9.1.)
-    template <Elem E, typename OutT, bool A_KCONTIG, bool B_KCONTIG, uint32_t WB, bool TRIANGLE = false, uint32_t WM = WB>
+    template <Elem E, typename OutT, bool A_KCONTIG, bool B_KCONTIG, uint32_t WB, bool TRIANGLE = false, uint32_t WM = WB, bool NONTEMPORAL = false>
     __device__ __forceinline__ void gemmTiled5(const Params& whole)
     {
         static_assert(WB == 8 || WB == 4 || WB == 2, "wave tile of 8 x 8, 4 x 4 or 2 x 2 blocks");
@@ -1415,7 +1422,7 @@ namespace
         if constexpr(TRIANGLE)
             if(tm != tn)
             {
-                storeTriangleRows<OutT, WB>(acc, reinterpret_cast<OutT*>(p.d), p.m, tm * TILE, tn * TILE, wave, lane, lds);
+                storeTriangleRows<OutT, WB, NONTEMPORAL>(acc, reinterpret_cast<OutT*>(p.d), p.m, tm * TILE, tn * TILE, wave, lane, lds);
                 R355_STAMP_END();
                 return;
             }
@@ -1741,18 +1748,17 @@ namespace
     {
         gemmTiled5<Elem::F64, double, A_KCONTIG, B_KCONTIG, 4>(p);
     }
-    template <Elem E, typename T, uint32_t WB>
+    template <Elem E, typename T, uint32_t WB, bool NONTEMPORAL>
     __global__ void __launch_bounds__(THREADS) dlrmFwdTiled(Params p)
     {
-        gemmTiled5<E, T, true, true, WB, true>(p);
+        gemmTiled5<E, T, true, true, WB, true, WB, NONTEMPORAL>(p);
     }
     template <Elem E, typename T>
-    int launchTriangle(const Params& p, uint32_t tile, uint32_t groups, hipStream_t stream)
+    int launchTriangle(const Params& p, uint32_t tile, uint32_t groups, bool nontemporal, hipStream_t stream)
     {
-        if(tile == 128u)
-            hipLaunchKernelGGL((dlrmFwdTiled<E, T, 4>), dim3(groups), dim3(THREADS), 0, stream, p);
-        else
-            hipLaunchKernelGGL((dlrmFwdTiled<E, T, 2>), dim3(groups), dim3(THREADS), 0, stream, p);
+        const auto kernel = tile == 128u ? (nontemporal ? dlrmFwdTiled<E, T, 4, true> : dlrmFwdTiled<E, T, 4, false>)
+                                         : (nontemporal ? dlrmFwdTiled<E, T, 2, true> : dlrmFwdTiled<E, T, 2, false>);
+        hipLaunchKernelGGL(kernel, dim3(groups), dim3(THREADS), 0, stream, p);
         return r355::checkLaunch("dlrm_fwd (macro tile)");
     }
     // ------------------------------------------------------------------------------------------
@@ -2823,10 +2829,14 @@ namespace r355
             p.a = p.b   = static_cast<const char*>(in) + (uint64_t)first * m * k * es;
             p.d         = static_cast<char*>(out) + (uint64_t)first * stride * es;
             p.tileCount = count * pairs;
-            const uint32_t groups = (p.tileCount + 7u) / 8u * 8u;
-            const int      rc     = dtype == R355_F16    ? dlrmFwdTiledPart0(p, tile, groups, stream)
-                                    : dtype == R355_BF16 ? dlrmFwdTiledPart1(p, tile, groups, stream)
-                                                         : dlrmFwdTiledPart3(p, tile, groups, stream);
+            // Nontemporal stores of the triangle's rows where input and result go beyond some 14 MB, not half of the 32 MiB of L2.  Below that they cost up
+            // to 7 % (bf16 176 x 48 x 37 3.60 us for 3.37 kept, f16 480 x 192 x 22 5.95 for 5.65, f32 976 x 32 x 6 7.77 for 7.36, 640 x 80 x 7 7.18 for
+            // 6.76), above they save up to 18 % (f16 928 x 656 x 10 14.5 for 15.0, 272 x 80 x 144 9.8 for 10.1, f32 688 x 96 x 13 10.7 for 11.1).
+            const bool     nontemporal = count * ((uint64_t)m * k + stride) * es > 14000000u;
+            const uint32_t groups      = (p.tileCount + 7u) / 8u * 8u;
+            const int      rc          = dtype == R355_F16    ? dlrmFwdTiledPart0(p, tile, groups, nontemporal, stream)
+                                         : dtype == R355_BF16 ? dlrmFwdTiledPart1(p, tile, groups, nontemporal, stream)
+                                                              : dlrmFwdTiledPart3(p, tile, groups, nontemporal, stream);
             if(rc != R355_OK || batch - first <= most) // (first + most may pass 2^32)
                 return rc;
         }
@@ -3023,9 +3033,9 @@ namespace r355
 #endif // part 0
 
 #if R355_TILED_HAS(0)
-    int dlrmFwdTiledPart0(const GemmTileParams& p, uint32_t tile, uint32_t groups, hipStream_t stream)
+    int dlrmFwdTiledPart0(const GemmTileParams& p, uint32_t tile, uint32_t groups, bool nontemporal, hipStream_t stream)
     {
-        return launchTriangle<Elem::F16, _Float16>(p, tile, groups, stream);
+        return launchTriangle<Elem::F16, _Float16>(p, tile, groups, nontemporal, stream);
     }
     int dlrmBwdTiledPart0(const DlrmBwdParams& p, uint32_t tile, hipStream_t stream)
     {
@@ -3038,9 +3048,9 @@ namespace r355
     }
 #endif
 #if R355_TILED_HAS(1)
-    int dlrmFwdTiledPart1(const GemmTileParams& p, uint32_t tile, uint32_t groups, hipStream_t stream)
+    int dlrmFwdTiledPart1(const GemmTileParams& p, uint32_t tile, uint32_t groups, bool nontemporal, hipStream_t stream)
     {
-        return launchTriangle<Elem::BF16, __bf16>(p, tile, groups, stream);
+        return launchTriangle<Elem::BF16, __bf16>(p, tile, groups, nontemporal, stream);
     }
     int dlrmBwdTiledPart1(const DlrmBwdParams& p, uint32_t tile, hipStream_t stream)
     {
@@ -3064,9 +3074,9 @@ namespace r355
     }
 #endif
 #if R355_TILED_HAS(3)
-    int dlrmFwdTiledPart3(const GemmTileParams& p, uint32_t tile, uint32_t groups, hipStream_t stream)
+    int dlrmFwdTiledPart3(const GemmTileParams& p, uint32_t tile, uint32_t groups, bool nontemporal, hipStream_t stream)
     {
-        return launchTriangle<Elem::F32, float>(p, tile, groups, stream);
+        return launchTriangle<Elem::F32, float>(p, tile, groups, nontemporal, stream);
     }
     int dlrmBwdTiledPart3(const DlrmBwdParams& p, uint32_t tile, hipStream_t stream)
     {
