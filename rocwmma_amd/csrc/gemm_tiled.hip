@@ -1779,7 +1779,19 @@ namespace
     // gathered element by element, eight 2-byte loads for each 16 bytes, and every stage requested one ahead.)
     using BwdParams = r355::DlrmBwdParams;
 
-    template <Elem E, typename T, uint32_t WB>
+    // f(0), f(1), ...: compile-time arguments
+    template <typename F, uint32_t... J>
+    __device__ __forceinline__ void forEach(std::integer_sequence<uint32_t, J...>, F f)
+    {
+        (f(std::integral_constant<uint32_t, J>{}), ...);
+    }
+
+    // ALONE (16-bit, 64 x 64 tiles): at most one workgroup a CU, with no other to issue while it works out its addresses, which is then what a
+    // stage waits for.  Stages off the diagonal tile have code of their own, without the tests and shifts of pieces that the diagonal
+    // cuts: f16 1024 x 16 x 1 11.5 -> 10.1 us, 784 x 48 x 4 10.0 -> 9.0, 512 x 240 x 2 7.4 -> 6.9 (10.1, 9.1 and 7.4 with the diagonal stages gathered).
+    // Where several share a CU that is slower (128 x 64 x 1689 17.7 -> 19.4, 320 x 192 x 96 13.1 -> 14.3, 1024 x 1024 x 64 on 128 x 128 tiles
+    // 218 -> 233), and it is for samples of few tiles, most of whose stages are diagonal ones (128 x 192 x 12 4.03 -> 4.16, 256 x 16 x 1 4.79 -> 4.83).
+    template <Elem E, typename T, uint32_t WB, bool ALONE = false>
     __device__ __forceinline__ void dlrmBwdTile(const BwdParams& p)
     {
         constexpr uint32_t ES = ElemTraits<E>::Bytes, TILE = 32u * WB, WT = 16u * WB, OPER = TILE * STAGE_KB;
@@ -1892,12 +1904,31 @@ namespace
             }
         };
         // 16-bit (one place for every kind of stage: with a loop for each the compiler kept the pieces in scratch memory)
-        auto loadA = [&](uint32_t st) {
-            const bool     right = st >= diagEnd; // (uniform)
+        using Pieces = std::make_integer_sequence<uint32_t, WB>;
+        auto loadA   = [&](auto aK, uint32_t st) {
+            constexpr bool AK    = decltype(aK)::value; // (else the stages before were right of the diagonal tile already)
+            const bool     right = (ALONE && !AK) || st >= diagEnd; // (uniform)
             const uint32_t k0    = st * TK;
             if constexpr(!ACROSS)
             {
                 loadGathered(st);
+                return;
+            }
+            if constexpr(ALONE)
+            {
+                if(AK && inDiag(st))
+                    forEach(Pieces{}, [&](auto j) {
+                        aNext[j]   = loadCut(row0 + rK + 32u * j, k0 + cK);
+                        aAcross[j] = loadCut(k0 + rowM(j), row0 + colM(j));
+                    });
+                else
+                    forEach(Pieces{}, [&](auto j) { // (every column of the piece lies left of the diagonal)
+                        const uint64_t row = right ? k0 + rowM(j) : row0 + rK + 32u * j;
+                        const uint32_t col = right ? row0 + colM(j) : k0 + cK;
+                        aNext[j]           = i32x4{0, 0, 0, 0};
+                        if(row < p.m)
+                            aNext[j] = *reinterpret_cast<const i32x4u*>(tril + (row * (row - 1u) / 2u + col));
+                    });
                 return;
             }
 #pragma unroll
@@ -1908,7 +1939,20 @@ namespace
                 for(uint32_t j = 0; j < WB; ++j)
                     aAcross[j] = loadCut(k0 + rowM(j), row0 + colM(j));
         };
-        auto writeA = [&](uint32_t at, uint32_t st) { // (every image takes piece j * 256 + tid at byte 16 of that)
+        auto writeA = [&](auto aK, uint32_t at, uint32_t st) { // (every image takes piece j * 256 + tid at byte 16 of that)
+            if constexpr(ALONE)
+            {
+                if(decltype(aK)::value && inDiag(st))
+                    forEach(Pieces{}, [&](auto j) {
+                        *reinterpret_cast<i32x4*>(lds + at + (j * THREADS + tid) * CHUNK)
+                            = shiftDown(aNext[j], cutBy(row0 + rK + 32u * j, st * TK + cK));
+                        *reinterpret_cast<i32x4*>(lds + ACROSS_AT + (j * THREADS + tid) * CHUNK)
+                            = shiftDown(aAcross[j], cutBy(st * TK + rowM(j), row0 + colM(j)));
+                    });
+                else
+                    forEach(Pieces{}, [&](auto j) { *reinterpret_cast<i32x4*>(lds + at + (j * THREADS + tid) * CHUNK) = aNext[j]; });
+                return;
+            }
 #pragma unroll
             for(uint32_t j = 0; j < WB; ++j)
             {
@@ -1992,16 +2036,16 @@ namespace
         };
 
         issueB(0u, B_AT);
-        loadA(0u);
+        loadA(std::true_type{}, 0u);
         if constexpr(ACROSS)
             waitVmcnt<0>();
-        writeA(0u, 0u);
+        writeA(std::true_type{}, 0u, 0u);
         if constexpr(!ACROSS)
             waitVmcnt<0>();
         else if(numStages > 1u)
         {
             issueB(1u, B_AT + OPER);
-            loadA(1u);
+            loadA(std::true_type{}, 1u);
         }
         ldsBarrier();
         // 16-bit, bound by its loads: a stage is read into registers whole, and while it is multiplied the next, requested a stage before, takes
@@ -2018,11 +2062,11 @@ namespace
             if(st + 1u < numStages) // (uniform)
             {
                 waitVmcnt<0>();
-                writeA(0u, st + 1u);
+                writeA(aK, 0u, st + 1u);
                 if(st + 2u < numStages)
                 {
                     issueB(st + 2u, bAt);
-                    loadA(st + 2u);
+                    loadA(aK, st + 2u);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -2038,7 +2082,7 @@ namespace
             {
                 issueB(st + 1u, B_AT + nxt);
                 if constexpr(decltype(aK)::value)
-                    loadA(st + 1u);
+                    loadA(aK, st + 1u);
                 else
                     loadRight(st + 1u);
             }
@@ -2046,7 +2090,7 @@ namespace
             readB(B_AT + cur);
             products();
             if(more)
-                writeA(nxt, st + 1u);
+                writeA(aK, nxt, st + 1u);
             // the direct loads of the next stage have landed, and every wave has read this one
             waitVmcnt<0>();
             ldsBarrier();
@@ -2079,11 +2123,21 @@ namespace
         dlrmBwdTile<E, T, 2>(p);
     }
     template <Elem E, typename T>
+    __global__ void __launch_bounds__(THREADS, 4) dlrmBwdTiled64Alone(BwdParams p)
+    {
+        dlrmBwdTile<E, T, 2, true>(p);
+    }
+    template <Elem E, typename T>
     int launchBwdTiled(const BwdParams& p, uint32_t tile, hipStream_t stream)
     {
         const uint32_t groups = (p.total + 7u) / 8u * 8u;
         if(tile == 128u)
             hipLaunchKernelGGL((dlrmBwdTiled128<E, T>), dim3(groups), dim3(THREADS), 0, stream, p);
+        else if(ElemTraits<E>::Bytes == 2 && p.tilesM >= 6u && p.total <= r355::computeUnits()) // (384 x 16 x 1 5.95 -> 5.73 us, 1024 x 64 x 16 12.7 -> 12.5)
+        {
+            if constexpr(ElemTraits<E>::Bytes == 2)
+                hipLaunchKernelGGL((dlrmBwdTiled64Alone<E, T>), dim3(groups), dim3(THREADS), 0, stream, p);
+        }
         else
             hipLaunchKernelGGL((dlrmBwdTiled64<E, T>), dim3(groups), dim3(THREADS), 0, stream, p);
         return r355::checkLaunch("dlrm_bwd (macro tiles)");
