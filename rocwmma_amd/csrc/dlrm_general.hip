@@ -322,7 +322,9 @@ namespace
     // Which kernel a launch runs is the cheapest by a timing model: microseconds as a linear function of the launch's workgroups
     // (or waves; `groups` in thousands on 256 CUs), their steps along K and one more term.  Fitted by least squares of the relative
     // error to launches of every kernel on the same random shapes, m from 32 to 1024, k from 16 to 1024, up to 12000 samples
-    // (profiles/tile_choice_survey.md: how well the models do, and what the choices give on further shapes).
+    // (profiles/tile_choice_survey.md: how well the models do, and what the choices give on further shapes).  The tiles' constants of the 16-bit types were
+    // fitted when their diagonal stages, and the forward's stores, took up to 1.5 times as long as now: on 665 further 16-bit shapes the choice takes
+    // 1.010 (forward) and 1.033 (backward) times as long as the fastest of itself and the two tiles, 87 of them more than 3 % longer.
     struct LaunchTime
     {
         double fixed, step, group, groupStep, more;
@@ -347,10 +349,10 @@ namespace
     // Forward.  A block per wave (steps of one matrix instruction) has the shortest launch, pads nothing, and re-reads every row of X for
     // each block of the sample, from lines that collide in the caches where rows are multiples of 128 bytes (the last term: waves times
     // steps again).  Macro tiles (steps: stages of 128 bytes; the last term: megabytes of input and output) read a row once per 64 or 128
-    // others but pad m to the tile's edge: with few features or a short K most of a tile is padding and fixed cost.  bf16 32 x 48 x 7174: 9.4 us a block
-    // per wave, 22 on 64 x 64 tiles, 51 on 128 x 128 ones; f16 64 x 112 x 2687: 28, 15 and 27; bf16 176 x 576 x 428: 227, 25 and 30; f16
-    // 1024 x 1024 x 64: 96 on 128 x 128 tiles.  Beyond 160 features only small launches run a block per wave: its reads of the
-    // rows of X then cost more than the model says (bf16 192 x 16 x 505: 15.6 us, modelled 11, 13.1 on 64 x 64 tiles).
+    // others but pad m to the tile's edge: with few features or a short K most of a tile is padding and fixed cost.  bf16 32 x 48 x 7174: 10.3 us a block
+    // per wave, 21 on 64 x 64 tiles, 48 on 128 x 128 ones; f16 64 x 112 x 2687: 28, 13.3 and 24; bf16 176 x 576 x 428: 227, 28 and 32; f16
+    // 1024 x 1024 x 64: 136 and 88 on tiles.  Beyond 160 features only small launches run a block per wave: its reads of the
+    // rows of X then cost more than the model says (bf16 192 x 16 x 505: 15.6 us, modelled 11, 12.0 on 64 x 64 tiles).
     constexpr LaunchTime FWD_WAVE[2]  = {{2.70, 0.0415, 0.104, 0.124, 0.104}, {2.48, 0.0954, 0.135, 0.225, 0.00649}}; // 16-bit, f32
     constexpr LaunchTime FWD_64[2]    = {{3.38, 0.00367, 2.13, 0.564, 0.0370}, {3.49, 0.227, 1.95, 1.62, 0.0517}};
     constexpr LaunchTime FWD_128      = {3.88, 0.124, 5.27, 0.804, 0.0816}; // 16-bit: f32, bound by its matrix instructions, is faster on 64 x 64 throughout
@@ -377,9 +379,9 @@ namespace
     }
 
     // Backward.  The fragment-API kernels are a block per wave and 2 x 4 blocks per wave (the register-blocked kernel; waves of 32 x 64 of the
-    // gradient, workgroups of 32 x 256 that form S once); macro tiles pad m and the K of the product, which is m again, to 64 or 128.  f16 32 x 208 x 4021: 23 us register-blocked, 56 on 64 x 64 tiles; f16 80 x 208 x 1410: 34 and 57;
-    // f16 112 x 48 x 1612: 44 and 22; f16 1024 x 256 x 4: 96 a block per wave, 10.5 on 64 x 64; f16 992 x 464 x 27: 117 register-blocked, 72 on 64 x 64,
-    // 58 on 128 x 128 tiles; f16 1024 x 1024 x 64: 473, 295 and 214.
+    // gradient, workgroups of 32 x 256 that form S once); macro tiles pad m and the K of the product, which is m again, to 64 or 128.  f16 32 x 208 x 4021: 33 us register-blocked,
+    // 45 on 64 x 64 tiles; f16 80 x 208 x 1410: 38 and 42; f16 112 x 48 x 1612: 44 and 15.5; f16 1024 x 256 x 4: 96 a block per wave, 11.8 on
+    // 64 x 64; f16 992 x 464 x 27: 117 register-blocked, 69 on 64 x 64, 52 on 128 x 128 tiles; f16 1024 x 1024 x 64: 473, 328 and 222.
     // By f16, bf16, f32.  Steps: blocks of 16 rows (fragments), stages of 128 bytes of K (tiles); the last term: megabytes, for the
     // register-blocked kernel thousands of block products.
     constexpr LaunchTime BWD_WAVE[3]    = {{1.71, 0.538, 0.0, 0.195, 0.305}, {1.97, 0.543, 0.0, 0.187, 0.296}, {1.77, 0.735, 0.0, 0.303, 0.124}};
