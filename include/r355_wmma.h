@@ -121,7 +121,10 @@ typedef struct
     uint64_t    workspace_bytes;
 } r355_gemm_args;
 
-/* Replaces: hipExtLaunchKernelGGL(gemm_rocwmma_d, ...) in samples/perf_hgemm.cpp:820-842 and
+/* R355_F32: launches of many 64 x 64 tiles multiply on the bf16 matrix instructions, every operand as the sum of three bf16, summed in f32
+ * (closer to the exact result than the f32 instructions' sums); a tile that meets an infinity, a NaN, an overflow or operands with bits
+ * below 2^-133 is multiplied with the f32 instructions.
+ * Replaces: hipExtLaunchKernelGGL(gemm_rocwmma_d, ...) in samples/perf_hgemm.cpp:820-842 and
  * test/gemm/gemm_kernel_base_impl.hpp:622-645. */
 int r355_gemm(const r355_gemm_args* args, void* stream);
 

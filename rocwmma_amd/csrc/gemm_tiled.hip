@@ -46,6 +46,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "gemm_params.hpp"
 #include "lds_dma.hpp"
 #include "operand_tile.hpp"
 #include "tile_map.hpp"
@@ -99,30 +100,6 @@ extern "C" int R355_TL_PASTE(r355_timeline_read_p, R355_TILED_PART)(void* host, 
 
 namespace r355
 {
-    struct GemmTileParams
-    {
-        uint32_t    m, n, k;
-        const char* a;
-        const char* b;
-        const char* c;
-        char*       d;
-        uint32_t    lda, ldb, ldc, ldd; // elements
-        double      alpha, beta; // narrowed to the accumulator type in the epilogue
-        uint32_t    tilesM, tilesN;
-        // the launch covers tile indices [tileFirst, tileFirst + tileCount) of the tilesM x tilesN walk; with
-        // tileQuad the walk is over tiles of twice the kernel's edge, four workgroups each (tile_map.hpp)
-        uint32_t tileFirst, tileCount, tileQuad;
-        // split-K (128 x 128 tile kernels): workgroup row blockIdx.y multiplies K stages [y * splitStages, (y + 1) * splitStages)
-        // and writes its partial D (in the accumulator type) at d + y * splitStrideD bytes; 0 = the whole K in one workgroup
-        uint32_t splitStages;
-        uint64_t splitStrideD;
-        // host side only: 16-bit operands on the 256 x 256 tile take the five-buffer K loop instead of the two-buffer one
-        uint32_t deepPipeline;
-        // experiment (R355_STAGGER_TICKS in the environment, 10 ns units; 0 = off): the first staggerBlocks workgroups - the
-        // first round over the CUs - start 0, 1, 2 or 3 x stagger ticks late, by groups of CUs within each XCD, so that
-        // the rounds' epilogues do not all store at once
-        uint32_t stagger, staggerBlocks;
-    };
     // K stages of 128 bytes of a problem.  k in bytes need not fit 32 bits: 16 rows of 2^29 doubles are 64 GiB
     inline uint32_t stagesOfK(uint32_t k, uint32_t elemBytes)
     {
@@ -2488,7 +2465,9 @@ namespace
             }
             else if constexpr(E == Elem::F32)
             {
-                if(tile == 64u)
+                if(tile == 64u && r355::f32TilesOnBf16((uint64_t)whole.tileCount * splits, p.splitStages ? p.splitStages : r355::stagesOfK(p.k, 4u)))
+                    r355::gemmF32Tiles(AK, BK, splits, p, stream);
+                else if(tile == 64u)
                     hipLaunchKernelGGL((gemmTiledKernelF32Tiny<AK, BK>), grid, block, 0, stream, p);
                 else if(tile == 128u)
                     hipLaunchKernelGGL((gemmTiledKernelF32Small<AK, BK>), grid, block, 0, stream, p);
@@ -2653,11 +2632,11 @@ namespace
     //            fixed   latency   per workgroup    fixed   latency   per workgroup
     //   8-bit     3.9     0.46        0.46           2.6     0.28        0.27
     //   16-bit    2.9     0.46        0.46           1.2     0.32        0.236
-    //   f32       0.8     1.80        1.80           0.0     0.48        0.4575
+    //   f32       0.8     1.80        1.80           0.0     0.48        0.4575   (two together on the bf16 instructions, f32TilesOnBf16: 1.5, 0.45, 0.385)
     //   f64       1.6     1.834       1.834          0.0     0.48        0.458
     // Bound by the matrix instructions' rate, f32 and f64 run four small tiles in the time of a large one: they take the small
-    // tile nearly everywhere (f32 2560^3 284 -> 253 us, 720 x 832 x 784 48.7 -> 15.5; f64 1584 x 608 x 672 81 -> 24) and keep the
-    // large one where it fills whole rounds (f32 8192^3, 4096^3: the small tile would be 1 % slower).  16- and 8-bit problems
+    // tile nearly everywhere (720 x 832 x 784 48.7 -> 15.5; f64 1584 x 608 x 672 81 -> 24), and on the bf16 instructions, which only the
+    // small f32 tile has, it is the faster one everywhere (f32 2560^3 252 -> 205 us beside 284 on large tiles).  16- and 8-bit problems
     // take it for few tiles and short K (bf16 608 x 896 x 1680 12.3 -> 7.4 us, int8 1024 x 688 x 2896 11.7 -> 8.6).
     struct TileWork
     {
@@ -2669,6 +2648,7 @@ namespace
     };
     constexpr TileTimes TIMES_128[4] = {{3.9, 0.46, 0.46}, {2.9, 0.46, 0.46}, {0.8, 1.80, 1.80}, {1.6, 1.834, 1.834}}; // by log2(element size)
     constexpr TileTimes TIMES_64[4]  = {{2.6, 0.28, 0.27}, {1.2, 0.32, 0.236}, {0.0, 0.48, 0.4575}, {0.0, 0.48, 0.458}};
+    constexpr TileTimes TIMES_F32_BF16 = {1.5, 0.45, 0.385};
     constexpr double    REDUCE_FIXED = 3.5, REDUCE_PER_MB = 0.3; // the reduction's launch, and its share per MB of partial results
     TileWork tileWork(const r355_gemm_args& g)
     {
@@ -2683,14 +2663,15 @@ namespace
         double         bestTime = 0.0, plannedTime = 0.0;
         for(const uint32_t edge : {128u, 64u})
         {
-            const TileTimes& t        = edge == 128u ? TIMES_128[cls] : TIMES_64[cls];
-            const uint64_t   together = edge == 128u ? 2u : 4u;
-            const uint64_t   tiles    = (uint64_t)r355::tilesOf(g.m, edge) * r355::tilesOf(g.n, edge);
+            const uint64_t tiles = (uint64_t)r355::tilesOf(g.m, edge) * r355::tilesOf(g.n, edge);
             for(uint32_t s = 1u; s <= splits; ++s)
             {
                 const uint32_t share = (stages + s - 1u) / s;
                 if((stages + share - 1u) / share != s)
                     continue; // a share would be empty
+                const bool       onBf16   = g.in_type == R355_F32 && edge == 64u && r355::f32TilesOnBf16(tiles * s, share);
+                const TileTimes& t        = edge == 128u ? TIMES_128[cls] : onBf16 ? TIMES_F32_BF16 : TIMES_64[cls];
+                const uint64_t   together = edge == 128u || onBf16 ? 2u : 4u;
                 // (an XCD's share of the tiles, times the splits, over its CUs: 84 tiles x 3 are 33 on the first seven XCDs of 32 CUs)
                 const uint64_t perXcd = (tiles + 7u) / 8u * s, perCu = (perXcd * 8u + cus - 1u) / cus, rest = perCu % together;
                 auto           round = [&](uint64_t count) {

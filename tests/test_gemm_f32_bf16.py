@@ -1,0 +1,102 @@
+"""f32 GEMM on the bf16 matrix instructions (gemm_f32.hip): launches of more workgroups of 64 x 64 tiles than CUs, with K shares of 512
+elements and more.  Partial tiles and K tails, values that three bf16 do not hold, infinities, and the error against float64."""
+import numpy as np
+import pytest
+
+import oraclelib as O
+import rocwmma_amd as R
+from gpuutil import device_filled, to_device, to_host
+
+pytestmark = pytest.mark.gpu
+LAYOUTS = [(O.ROW, O.COL), (O.COL, O.ROW), (O.ROW, O.ROW), (O.COL, O.COL)]
+
+
+def _flat(x, layout):
+    return np.ascontiguousarray(x if layout == O.ROW else x.T).ravel()
+
+
+def _run(A, B, la, lb, C=None, alpha=1.0, beta=0.0, ldl=O.ROW, workspace=0, splits=1):
+    (m, k), n = A.shape, B.shape[1]
+    d = device_filled(m * n, np.float32, 0xFF)
+    c = None if C is None else to_device(_flat(C, ldl))
+    ws = device_filled(workspace, np.uint8, 0xFF) if workspace else None
+    g = R.gemm_args(R.F32, R.F32, m, n, k, to_device(_flat(A, la)), to_device(_flat(B, lb)), c, d, alpha, beta, la, lb, ldl, ldl, workspace=ws,
+                    workspace_bytes=workspace)
+    plan = R.gemm_launch_plan(g)
+    assert (plan.macro_tile_m, plan.split_k) == (64, splits) and plan.grid_x * splits > R.device_info().compute_units
+    R._check(R.lib().r355_gemm(R.ctypes.byref(g), None))
+    got = to_host(d, np.float32)
+    return got.reshape(m, n) if ldl == O.ROW else got.reshape(n, m).T
+
+
+def _uniform(seed, *shape):
+    return np.random.default_rng(seed).uniform(-1, 1, shape).astype(np.float32)
+
+
+# (k + 4) u (|alpha| |A| |B| + |beta| |C|): the forward bound of any order of f32 sums; the norm: half of what such sums of 512 and more products
+# show on uniform operands (4.0e-7), three times what these kernels do (0.8e-7)
+@pytest.mark.parametrize("la,lb", LAYOUTS)
+@pytest.mark.parametrize("ldl", [O.ROW, O.COL])
+@pytest.mark.parametrize("m,n,k", [(1040, 1072, 516), (1104, 1008, 636), (1024, 1088, 544)])
+def test_orientations_partial_tiles_and_k_tails(la, lb, ldl, m, n, k):
+    A, B, C = _uniform(1, m, k), _uniform(2, k, n), _uniform(3, m, n)
+    got = _run(A, B, la, lb, C, 2.0, -0.5, ldl).astype(np.float64)
+    exact = 2.0 * (A.astype(np.float64) @ B) - 0.5 * C
+    bound = (k + 4) * 2.0 ** -24 * (2.0 * (np.abs(A).astype(np.float64) @ np.abs(B)) + 0.5 * np.abs(C))
+    assert np.all(np.abs(got - exact) <= bound)
+    assert np.linalg.norm(got - exact) <= 2e-7 * np.linalg.norm(exact)
+
+
+@pytest.mark.parametrize("la,lb", LAYOUTS)
+def test_every_bit_of_an_operand(la, lb):
+    # one product a row: every bit of the other operand, from the largest exponents to the smallest
+    m, n, k = 1056, 1056, 1056
+    rng = np.random.default_rng(4)
+    bits = rng.integers(0, 2 ** 32, (k, n), dtype=np.uint32)
+    bits = np.where((bits >> 23 & 0xFF) == 0xFF, bits & 0x807FFFFF, bits)  # finite
+    values = bits.view(np.float32)
+    pick = np.zeros((m, k), np.float32)
+    pick[np.arange(m), rng.permutation(k)[:m]] = 1.0
+    want = values[pick.argmax(axis=1)]
+    assert np.array_equal(_run(pick, values, la, lb), want)
+    assert np.array_equal(_run(np.ascontiguousarray(values.T), np.ascontiguousarray(pick.T), la, lb), want.T)
+
+
+@pytest.mark.parametrize("ea,eb", [(-125, 100), (100, -125), (-60, -70), (55, 60)])
+def test_operands_of_extreme_size(ea, eb):
+    # results keep their precision where the operands' last pieces would lie below the range of bf16
+    m, n, k = 1040, 1040, 528
+    A, B = np.ldexp(_uniform(5, m, k), ea), np.ldexp(_uniform(6, k, n), eb)
+    got = _run(A, B, O.ROW, O.COL).astype(np.float64)
+    exact = A.astype(np.float64) @ B
+    # (operands and results below 2^-126 are rounded to multiples of 2^-149)
+    bound = (k + 4) * (2.0 ** -24 * (np.abs(A).astype(np.float64) @ np.abs(B)) + 2.0 ** -149)
+    assert np.all(np.abs(got - exact) <= bound)
+
+
+@pytest.mark.parametrize("la,lb", [(O.ROW, O.COL), (O.COL, O.ROW)])
+def test_infinities_and_nan(la, lb):
+    m, n, k = 1040, 1072, 520
+    A, B = _uniform(7, m, k), _uniform(8, k, n)
+    A[3, 17], A[130, 519], B[200, 70], A[1039, 0] = np.inf, -np.inf, np.nan, 3e38
+    B[17, 1000] = 0.0  # infinity times zero
+    B[0, 5] = 3e38  # an overflow
+    got = _run(A, B, la, lb)
+    with np.errstate(all="ignore"):
+        want = (A.astype(np.float64) @ B.astype(np.float64)).astype(np.float32)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isinf(got), np.isinf(want)) and np.array_equal(got[np.isinf(got)], want[np.isinf(want)])
+    fin = np.isfinite(want)
+    scale = np.abs(np.where(np.isfinite(A), A, 0)).astype(np.float64) @ np.abs(np.where(np.isfinite(B), B, 0))
+    assert np.all(np.abs(got[fin].astype(np.float64) - want[fin]) <= ((k + 4) * 2.0 ** -24 * scale)[fin] + np.abs(want[fin]) * 2.0 ** -24)
+
+
+def test_shares_of_k():
+    # 16 x 17 tiles, three shares of 22 stages, the last of 21 and one 16-byte chunk
+    m, n, k = 1024, 1040, 2084
+    A, B, C = _uniform(9, m, k), _uniform(10, k, n), _uniform(11, m, n)
+    need = int(R.gemm_query(R.gemm_args(R.F32, R.F32, m, n, k, 0x1000, 0x2000, 0x3000, 0x4000, 1.5, 1.0, O.ROW, O.COL, O.ROW, O.ROW,
+                                        workspace_bytes=2 ** 62)).workspace_bytes)
+    got = _run(A, B, O.ROW, O.COL, C, 1.5, 1.0, workspace=need, splits=3)
+    exact = 1.5 * (A.astype(np.float64) @ B) + C
+    assert np.linalg.norm(got - exact) <= 2e-7 * np.linalg.norm(exact)
