@@ -28,7 +28,12 @@ namespace
     // on scheduling.  STREAM as in the row-major kernel.
     // SPLIT: workgroup (b, s) of a two-dimensional grid sums columns [s kPer, (s + 1) kPer) only and leaves its rows' sums,
     // unscaled, in an array of partial sums (yOut; element (row, s) at row * partRow + s * partSplit) for gemvAddSplits.
-    template <typename T, uint32_t RL, uint32_t COL_WAVES, bool STREAM, bool SPLIT = false>
+    // BY_XCD: columns that do not start on 128-byte boundaries, where the runs of neighbouring blocks of rows share cache lines.  A grid of one
+    // dimension, whose workgroups every XCD takes as one contiguous stretch of (split, block), blocks first: the two owners of a line then ask
+    // one L2 for it at about the same time, instead of two L2s (runs of 1 KiB, 6152 x 11012: 47.2 -> 42.2 us; 64 bytes, 1164 x 940: 5.5 -> 4.5; of
+    // matrices whose columns are aligned 8192^2 would take 51 us instead of 44).  The last, partial trip is requested at once as well (f64 3896 x 472, all
+    // of it a partial trip: 7.1 -> 5.7), and the wave's number is a scalar, which lets the 1 KiB runs read x as scalars.
+    template <typename T, uint32_t RL, uint32_t COL_WAVES, bool STREAM, bool SPLIT = false, bool BY_XCD = false>
     __global__ void __launch_bounds__(COL_WAVES * 64) gemvColMajor(uint32_t m,
                                                                   uint32_t k,
                                                                   const T* a,
@@ -40,14 +45,24 @@ namespace
                                                                   T        beta,
                                                                   uint32_t kPer,
                                                                   uint32_t partRow,
-                                                                  uint32_t partSplit)
+                                                                  uint32_t partSplit,
+                                                                  uint32_t blocks,
+                                                                  uint32_t groups)
     {
         constexpr uint32_t V = 16u / sizeof(T), ROWS = RL * V, CL = 64u / RL, COLS = COL_WAVES * CL, DEPTH = 8;
+        uint32_t           block = blockIdx.x, part = blockIdx.y; // of the rows, of K
+        if constexpr(BY_XCD) // `groups` workgroups with work: `blocks` of each split
+        {
+            const uint32_t perXcd = (groups + 7u) / 8u, id = (block % 8u) * perXcd + block / 8u;
+            if(block / 8u >= perXcd || id >= groups)
+                return;
+            block = SPLIT ? id % blocks : id, part = SPLIT ? id / blocks : 0u;
+        }
         using VecT = T __attribute__((ext_vector_type(V)));
         __shared__ T   partial[COLS][ROWS];
-        const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+        const uint32_t lane = threadIdx.x & 63u, wave = BY_XCD ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
         const uint32_t r = lane % RL, c = lane / RL;
-        const uint32_t row0 = blockIdx.x * ROWS + r * V; // (m is a multiple of V: a lane's rows are inside or outside together)
+        const uint32_t row0 = block * ROWS + r * V; // (m is a multiple of V: a lane's rows are inside or outside together)
         T              acc[V];
 #pragma unroll
         for(uint32_t e = 0; e < V; ++e)
@@ -61,8 +76,8 @@ namespace
                 else
                     return *reinterpret_cast<const VecT*>(at);
             };
-            const uint32_t kEnd = SPLIT ? (k - blockIdx.y * kPer < kPer ? k : (blockIdx.y + 1u) * kPer) : k;
-            uint32_t       kk   = (SPLIT ? blockIdx.y * kPer : 0u) + wave * CL + c;
+            const uint32_t kEnd = SPLIT ? (k - part * kPer < kPer ? k : (part + 1u) * kPer) : k;
+            uint32_t       kk   = (SPLIT ? part * kPer : 0u) + wave * CL + c;
             for(; kk + (DEPTH - 1u) * COLS < kEnd; kk += DEPTH * COLS)
             {
                 VecT v[DEPTH];
@@ -79,30 +94,71 @@ namespace
                     for(uint32_t e = 0; e < V; ++e)
                         acc[e] += v[u][e] * xv[u];
             }
-            for(; kk < kEnd; kk += COLS)
+            if constexpr(BY_XCD)
             {
-                const VecT v  = fetch(p + (uint64_t)kk * lda);
-                const T    xv = x[kk];
+                // fewer than DEPTH columns: requested together as well (those past the end: the first of them again, taken as zero)
+                if(kk < kEnd)
+                {
+                    VecT v[DEPTH];
+                    T    xv[DEPTH];
 #pragma unroll
-                for(uint32_t e = 0; e < V; ++e)
-                    acc[e] += v[e] * xv;
+                    for(uint32_t u = 0; u < DEPTH; ++u)
+                        v[u] = fetch(p + (uint64_t)(u * COLS < kEnd - kk ? kk + u * COLS : kk) * lda);
+#pragma unroll
+                    for(uint32_t u = 0; u < DEPTH; ++u)
+                        xv[u] = x[u * COLS < kEnd - kk ? kk + u * COLS : kk];
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for(uint32_t u = 0; u < DEPTH; ++u)
+#pragma unroll
+                        for(uint32_t e = 0; e < V; ++e)
+                            acc[e] = u * COLS < kEnd - kk ? acc[e] + v[u][e] * xv[u] : acc[e];
+                }
             }
+            else
+                for(; kk < kEnd; kk += COLS)
+                {
+                    const VecT v  = fetch(p + (uint64_t)kk * lda);
+                    const T    xv = x[kk];
+#pragma unroll
+                    for(uint32_t e = 0; e < V; ++e)
+                        acc[e] += v[e] * xv;
+                }
         }
 #pragma unroll
         for(uint32_t e = 0; e < V; ++e)
             partial[wave * CL + c][r * V + e] = acc[e];
         __syncthreads();
+        // (with 32 lane groups and more, eighths of them first, a thread each)
+        constexpr bool EIGHTHS = BY_XCD && COLS >= 32u;
+        constexpr uint32_t TERMS = EIGHTHS ? 8u : COLS;
+        if constexpr(EIGHTHS)
+        {
+            static_assert(8u * ROWS <= COL_WAVES * 64u, "a thread for every eighth of a row's sum");
+            const uint32_t eighth = threadIdx.x / ROWS, mine = threadIdx.x % ROWS;
+            T              sum    = T(0);
+            if(eighth < 8u)
+            {
+#pragma unroll
+                for(uint32_t w = 0; w < COLS / 8u; ++w)
+                    sum += partial[eighth * (COLS / 8u) + w][mine];
+            }
+            __syncthreads();
+            if(eighth < 8u)
+                partial[eighth][mine] = sum;
+            __syncthreads();
+        }
         if(threadIdx.x < ROWS)
         {
-            const uint32_t row = blockIdx.x * ROWS + threadIdx.x;
+            const uint32_t row = block * ROWS + threadIdx.x;
             if(row < m)
             {
                 T sum = T(0);
 #pragma unroll
-                for(uint32_t w = 0; w < COLS; ++w)
+                for(uint32_t w = 0; w < TERMS; ++w)
                     sum += partial[w][threadIdx.x];
                 if constexpr(SPLIT)
-                    yOut[(uint64_t)row * partRow + (uint64_t)blockIdx.y * partSplit] = sum;
+                    yOut[(uint64_t)row * partRow + (uint64_t)part * partSplit] = sum;
                 else
                     yOut[row] = beta != T(0) ? alpha * sum + beta * yIn[row] : alpha * sum;
             }
@@ -480,6 +536,51 @@ namespace
         return best;
     }
 
+    // Col-major A whose columns do not start on 128-byte boundaries: 16-byte pieces of a run, splits of K (`most` at most) and columns per split, the
+    // cheapest by a timing model of a launch.  Its workgroups go round the CUs, 32 of an XCD at a time; one streams at most 42 GB/s, all together
+    // 9.1 TB/s, and beyond 86 MB, where A does not come from the caches, short runs cost again as much as the lines they share; every row's sum ends with
+    // an addition per lane group, and a split launch with a second kernel.  Splits: none, as many as make a round of workgroups, or all.  Runs of up to 256
+    // bytes on eight waves, longer ones on four.  On 85 random shapes from 256 to 16384 rows and columns, A in the memory-side cache or not, the choice
+    // takes 1.03 times as long as the best of 5 runs x 3 numbers of waves x every number of splits; on 62 further ones from HBM 1 / 1.18 of the time that
+    // blocks of rows over all XCDs took (f32 6152 x 11012 51.6 -> 43.5 us, 13012 x 7684 78.8 -> 60.2, 8244 x 864 13.1 -> 9.2, 2300 x 3896 23.0 -> 12.1;
+    // f64 13276 x 8072 152 -> 124), none of them more than 3 % longer.
+    struct AskewPlan
+    {
+        uint32_t lanes, splits, kPer;
+    };
+    constexpr uint32_t askewWaves(uint32_t lanes)
+    {
+        return lanes <= 16u ? 8u : 4u;
+    }
+    template <typename T>
+    AskewPlan askewPlan(uint32_t m, uint32_t k, uint32_t most)
+    {
+        constexpr uint32_t V = 16u / sizeof(T);
+        const uint32_t     cus = r355::computeUnits(), perXcd = cus / 8u ? cus / 8u : 1u;
+        const bool         cold = static_cast<double>(m) * k * sizeof(T) > 86.0e6;
+        AskewPlan          best{};
+        double             bestTime = 0.0;
+        for(uint32_t lanes = 4u; lanes <= 64u; lanes *= 2u)
+        {
+            const uint32_t blocks = (m + lanes * V - 1u) / (lanes * V), columns = askewWaves(lanes) * 64u / lanes;
+            const uint32_t round  = cus / blocks < 1u ? 1u : cus / blocks < most ? cus / blocks : most;
+            for(const uint32_t want : {1u, round, most})
+            {
+                const uint64_t kPer = ((uint64_t)(k - 1u) / want / columns + 1u) * columns; // (k itself may lie just below 2^32)
+                const uint32_t splits = static_cast<uint32_t>((k - 1u) / kPer) + 1u;
+                const uint64_t groups = (uint64_t)blocks * splits, rounds = ((groups + 7u) / 8u + perXcd - 1u) / perXcd;
+                if((groups + 8u) * askewWaves(lanes) * 64u >> 32)
+                    continue; // a launch's threads are counted in 32 bits (runs of 64 lanes: one or two of them a row)
+                const double   active = groups < cus ? static_cast<double>(groups) : cus, rate = 9.1e6 / active < 42.0e3 ? 9.1e6 / active : 42.0e3;
+                const double   bytes = lanes * 16.0 * static_cast<double>(kPer) * static_cast<double>(rounds); // of a CU
+                const double   time  = bytes * (1.0 + (cold ? 3.0 : 0.3) / lanes) / rate + 0.0086 * (columns >= 32u ? columns / 8u + 8u : columns) + (splits > 1u ? 2.0 : 0.0);
+                if(best.lanes == 0u || time < bestTime)
+                    best = {lanes, splits, splits > 1u ? static_cast<uint32_t>(kPer) : k}, bestTime = time;
+            }
+        }
+        return best;
+    }
+
     // Rows per workgroup of the batched shared-row kernel for a streamed row-major A with long rows and fewer than 2048
     // of them, 0 = another kernel serves it.  Four or two rows, the larger count whose workgroups load the CUs evenly:
     // at least five eighths of them in a single round, at least 80 % of the slots of several rounds (f32, rows of 512 KiB
@@ -518,10 +619,19 @@ namespace
         hipStream_t s = static_cast<hipStream_t>(stream);
         r355::beginCall();
         // K split over several workgroups per block of rows when the shape calls for it and the workspace holds the partial sums
-        uint32_t       kPer   = k;
-        const uint32_t splits = (layout_a == R355_COL_MAJOR || layout_a == R355_ROW_MAJOR) && workspace ? gemvSplits<T>(layout_a, m, k, lda, kPer) : 1u;
-        const bool     split  = splits > 1u && (uint64_t)splits * m * sizeof(T) <= workspaceBytes;
-        T*             parts  = static_cast<T*>(workspace);
+        uint32_t kPer = k, splits = (layout_a == R355_COL_MAJOR || layout_a == R355_ROW_MAJOR) && workspace ? gemvSplits<T>(layout_a, m, k, lda, kPer) : 1u;
+        if((uint64_t)splits * m * sizeof(T) > workspaceBytes)
+            splits = 1u;
+        T* parts = static_cast<T*>(workspace);
+        // columns off 128-byte boundaries
+        const bool askew = layout_a == R355_COL_MAJOR && lda >= m && ((uint64_t)lda * sizeof(T) % 128u != 0u || !r355::aligned(a, 128)) && m < (1u << 30);
+        AskewPlan  plan{};
+        if(askew)
+        {
+            plan   = askewPlan<T>(m, k, splits);
+            splits = plan.splits, kPer = plan.kPer;
+        }
+        const bool     split  = splits > 1u;
         const bool     byWave = splits >= 32u; // layout of the partial sums: [m][splits] for the wave-per-row reduction, else [splits][m]
         const uint32_t partRow = byWave ? splits : 1u, partSplit = byWave ? 1u : m;
         if(layout_a == R355_COL_MAJOR)
@@ -529,33 +639,49 @@ namespace
             if(lda < m)
                 return r355::fail(R355_ERR_BAD_ARG, "gemv: lda < m");
             const bool stream = (uint64_t)k * lda * sizeof(T) > (256ull << 20);
-            auto       go     = [&](auto rl, auto waves) {
+            auto       go     = [&](auto rl, auto waves, auto byXcd) {
                 constexpr uint32_t RL = decltype(rl)::value, ROWS = RL * V, WAVES = decltype(waves)::value;
-                const dim3         grid((m + ROWS - 1u) / ROWS, split ? splits : 1u), block(WAVES * 64);
+                constexpr bool     BY_XCD = decltype(byXcd)::value;
+                const uint32_t     blocks = (m + ROWS - 1u) / ROWS, groups = blocks * splits;
+                const dim3         grid   = BY_XCD ? dim3((groups + 7u) / 8u * 8u) : dim3(blocks, splits), block(WAVES * 64);
+                T* const           out    = split ? parts : y_out;
                 if(split && stream)
-                    hipLaunchKernelGGL((gemvColMajor<T, RL, WAVES, true, true>), grid, block, 0, s, m, k, a, lda, x, y_in, parts, alpha, beta, kPer, partRow, partSplit);
+                    hipLaunchKernelGGL((gemvColMajor<T, RL, WAVES, true, true, BY_XCD>), grid, block, 0, s, m, k, a, lda, x, y_in, out, alpha, beta, kPer, partRow, partSplit, blocks, groups);
                 else if(split)
-                    hipLaunchKernelGGL((gemvColMajor<T, RL, WAVES, false, true>), grid, block, 0, s, m, k, a, lda, x, y_in, parts, alpha, beta, kPer, partRow, partSplit);
+                    hipLaunchKernelGGL((gemvColMajor<T, RL, WAVES, false, true, BY_XCD>), grid, block, 0, s, m, k, a, lda, x, y_in, out, alpha, beta, kPer, partRow, partSplit, blocks, groups);
                 else if(stream)
-                    hipLaunchKernelGGL((gemvColMajor<T, RL, WAVES, true>), grid, block, 0, s, m, k, a, lda, x, y_in, y_out, alpha, beta, k, 0u, 0u);
+                    hipLaunchKernelGGL((gemvColMajor<T, RL, WAVES, true, false, BY_XCD>), grid, block, 0, s, m, k, a, lda, x, y_in, out, alpha, beta, k, 0u, 0u, blocks, groups);
                 else
-                    hipLaunchKernelGGL((gemvColMajor<T, RL, WAVES, false>), grid, block, 0, s, m, k, a, lda, x, y_in, y_out, alpha, beta, k, 0u, 0u);
+                    hipLaunchKernelGGL((gemvColMajor<T, RL, WAVES, false, false, BY_XCD>), grid, block, 0, s, m, k, a, lda, x, y_in, out, alpha, beta, k, 0u, 0u, blocks, groups);
             };
+            using std::integral_constant;
+            constexpr std::true_type  byXcd;
+            constexpr std::false_type plain;
             // 256-byte runs once the rows give every CU a workgroup with them (8192^2 f32: 0.0415 ms against 0.0374 with
             // 128-byte runs and twice the workgroups; 16384^2: 0.151 against 0.161); sixteen waves per workgroup either way
             // (four: 0.0399 and 0.163)
-            if(split && splitRunLanes<T>(m, k) == 32u)
-                go(std::integral_constant<uint32_t, 32>{}, std::integral_constant<uint32_t, 16>{});
+            if(askew && plan.lanes == 4u)
+                go(integral_constant<uint32_t, 4>{}, integral_constant<uint32_t, askewWaves(4)>{}, byXcd);
+            else if(askew && plan.lanes == 8u)
+                go(integral_constant<uint32_t, 8>{}, integral_constant<uint32_t, askewWaves(8)>{}, byXcd);
+            else if(askew && plan.lanes == 16u)
+                go(integral_constant<uint32_t, 16>{}, integral_constant<uint32_t, askewWaves(16)>{}, byXcd);
+            else if(askew && plan.lanes == 32u)
+                go(integral_constant<uint32_t, 32>{}, integral_constant<uint32_t, askewWaves(32)>{}, byXcd);
+            else if(askew)
+                go(integral_constant<uint32_t, 64>{}, integral_constant<uint32_t, askewWaves(64)>{}, byXcd);
+            else if(split && splitRunLanes<T>(m, k) == 32u)
+                go(integral_constant<uint32_t, 32>{}, integral_constant<uint32_t, 16>{}, plain);
             else if(split && splitRunLanes<T>(m, k) == 64u)
-                go(std::integral_constant<uint32_t, 64>{}, std::integral_constant<uint32_t, 8>{});
+                go(integral_constant<uint32_t, 64>{}, integral_constant<uint32_t, 8>{}, plain);
             else if(split && splitRunLanes<T>(m, k) == 16u)
-                go(std::integral_constant<uint32_t, 16>{}, std::integral_constant<uint32_t, 8>{});
+                go(integral_constant<uint32_t, 16>{}, integral_constant<uint32_t, 8>{}, plain);
             else if(split)
-                go(std::integral_constant<uint32_t, 8>{}, std::integral_constant<uint32_t, 16>{});
+                go(integral_constant<uint32_t, 8>{}, integral_constant<uint32_t, 16>{}, plain);
             else if(m >= 16u * V * 256u)
-                go(std::integral_constant<uint32_t, 16>{}, std::integral_constant<uint32_t, 16>{});
+                go(integral_constant<uint32_t, 16>{}, integral_constant<uint32_t, 16>{}, plain);
             else
-                go(std::integral_constant<uint32_t, 8>{}, std::integral_constant<uint32_t, 16>{});
+                go(integral_constant<uint32_t, 8>{}, integral_constant<uint32_t, 16>{}, plain);
         }
         else if(layout_a == R355_ROW_MAJOR)
         {
