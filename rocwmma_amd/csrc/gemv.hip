@@ -282,8 +282,8 @@ namespace
     // after the other with that piece of x held in registers, and only then moves on along k.  Each wave waits for its
     // load before it asks for the next row: variants with two or four loads per row under way, or with the next row's
     // requested ahead, were slower the more they had in flight (16384^2 f32: 0.77, 0.67, 0.64 of the peak against 0.86),
-    // and so were 8 and 16 rows per workgroup.  Eight waves are ahead for rows below 128 KiB, sixteen from there on
-    // (16384^2: 0.887 / 0.844; 8192 x 32768: 0.818 / 0.882; 32768^2: 0.842 / 0.895; one row per wave: 0.82, 0.79, 0.82).
+    // and so were 8 and 16 rows per workgroup.  Sixteen waves, for rows of 128 KiB and more (8192 x 32768: 0.882, with eight 0.818; 32768^2: 0.895
+    // and 0.842; one row per wave: 0.79, 0.82); shorter ones go by rowGroup.
     // STREAM: A lies beyond the memory-side cache and is read with nontemporal loads; a smaller one (few very long rows
     // of a matrix that is multiplied again and again) keeps ordinary loads so that the next call finds it there, as in
     // gemvRowMajor / gemvColMajor.
@@ -601,6 +601,32 @@ namespace
         return 0u;
     }
 
+    // Waves and rows of a workgroup for a row-major A with rows below 128 KiB, {0, 0}: a wave per row, four to a workgroup (gemvRowMajor).  A row of a
+    // few KiB wants as many waves as make one or two trips of it, so that its loads are all under way at once; a matrix from HBM wants two rows a workgroup,
+    // which share x and keep as many loads more in flight; short rows by the ten thousands want four rows a wave.  168 random shapes from 256 to 16384
+    // rows and columns, A in the memory-side cache or not: 1.03 times as long as the best of 13 combinations, where a wave per row takes 1.15 times
+    // (f32 576 x 1780 from HBM 3.40 -> 2.81 us, 380 x 11964 10.9 -> 6.0, 8920 x 3796 26.4 -> 22.6, 9496 x 12800 87 -> 70; f64 2052 x 5680 25.7 -> 18.7), and
+    // 1.02 on most shapes outside (f32 88 x 27708 18.2 -> 6.5, 390884 x 16 64 -> 35, 16384^2 160 -> 150).
+    struct RowGroup
+    {
+        uint32_t waves, rows;
+    };
+    inline RowGroup rowGroup(uint32_t m, uint64_t rowBytes, uint32_t elemBytes)
+    {
+        const uint64_t bytes = rowBytes * m;
+        if(rowBytes <= 2048u && m >= 16384u)
+            return elemBytes == 8u && rowBytes < 256u ? RowGroup{0u, 0u} : RowGroup{1u, 4u}; // (f64 25772 x 24 5.0 -> 5.7)
+        if(rowBytes <= 1024u)
+            return {0u, 0u};
+        if(rowBytes <= 5632u)
+            return {1u, 1u};
+        if(rowBytes <= 9344u)
+            return {2u, 1u};
+        if(bytes <= 23000000u)
+            return {rowBytes < (64u << 10) ? 4u : 8u, 1u};
+        return {bytes <= 165000000u ? 4u : 8u, 2u};
+    }
+
     template <typename T>
     int gemvLaunch(int32_t layout_a, uint32_t m, uint32_t k, const T* a, uint32_t lda, const T* x, const T* y_in, T* y_out,
                    T alpha, T beta, void* stream, void* workspace = nullptr, size_t workspaceBytes = 0)
@@ -690,9 +716,8 @@ namespace
             const dim3 grid((m + THREADS / 64 - 1) / (THREADS / 64));
             const bool     stream   = (uint64_t)m * lda * sizeof(T) > (256ull << 20);
             const uint64_t rowBytes = (uint64_t)k * sizeof(T);
-            // rows of 16 KiB and more (f32, 1 GiB of A, against a wave per row: +1..2 % at 16 KiB, +4 % at 24 KiB, none at
-            // 32 KiB, +5 % at 40 KiB, +7..11 % from 64 KiB on; 8 KiB rows lose 6 %), short enough for a 32-bit buffer
-            // offset, and enough of them for two workgroups per CU
+            // rows of 128 KiB and more of a streamed matrix share the loads of x (gemvRowMajorShared), short enough for a 32-bit buffer offset, and
+            // enough of them for two workgroups per CU
             // Few and very long rows leave a wave per row with a handful of waves on the whole chip: a workgroup of sixteen
             // waves per row instead (f32, 512 MiB of A: 512 rows 0.42 -> 0.64 of the HBM peak, 256 rows 0.23 -> 0.77, 128 rows
             // 0.12 -> 0.43; rows of 512 KiB: 640 rows 0.52 -> 0.67, 768 rows 0.61 -> 0.76, 896 rows even; a wave per row is
@@ -720,13 +745,33 @@ namespace
                 else
                     hipLaunchKernelGGL((gemvRowMajorShared<T, 16, 1, false>), dim3(m), dim3(16 * 64), 0, s, m, k, a, lda, x, y_in, y_out, alpha, beta, k, 0u, 0u);
             }
-            else if(stream && rowBytes >= (16u << 10) && rowBytes < (1ull << 31) && m >= SHARED_ROWS * 512u)
+            else if(stream && rowBytes >= (128u << 10) && rowBytes < (1ull << 31) && m >= SHARED_ROWS * 512u)
+                hipLaunchKernelGGL((gemvRowMajorShared<T, 16>), dim3((m + SHARED_ROWS - 1u) / SHARED_ROWS), dim3(16 * 64), 0, s, m, k, a, lda, x, y_in, y_out, alpha, beta, k, 0u, 0u);
+            else if(const RowGroup group = rowBytes < (128u << 10) ? rowGroup(m, rowBytes, sizeof(T)) : RowGroup{}; group.waves != 0u)
             {
-                const dim3 blocks((m + SHARED_ROWS - 1u) / SHARED_ROWS);
-                if(rowBytes < (128u << 10))
-                    hipLaunchKernelGGL((gemvRowMajorShared<T, 8>), blocks, dim3(8 * 64), 0, s, m, k, a, lda, x, y_in, y_out, alpha, beta, k, 0u, 0u);
+                auto shared = [&](auto waves, auto rows) {
+                    constexpr uint32_t W = decltype(waves)::value, RB = decltype(rows)::value;
+                    const dim3         blocks((m + RB - 1u) / RB), threads(W * 64u);
+                    if(stream)
+                        hipLaunchKernelGGL((gemvRowMajorShared<T, W, RB, true, false, (RB > 1u)>), blocks, threads, 0, s, m, k, a, lda, x, y_in, y_out, alpha, beta, k, 0u, 0u);
+                    else
+                        hipLaunchKernelGGL((gemvRowMajorShared<T, W, RB, false, false, (RB > 1u)>), blocks, threads, 0, s, m, k, a, lda, x, y_in, y_out, alpha, beta, k, 0u, 0u);
+                };
+                using std::integral_constant;
+                if(group.rows == 4u)
+                    shared(integral_constant<uint32_t, 1>{}, integral_constant<uint32_t, 4>{});
+                else if(group.rows == 2u && group.waves == 4u)
+                    shared(integral_constant<uint32_t, 4>{}, integral_constant<uint32_t, 2>{});
+                else if(group.rows == 2u)
+                    shared(integral_constant<uint32_t, 8>{}, integral_constant<uint32_t, 2>{});
+                else if(group.waves == 1u)
+                    shared(integral_constant<uint32_t, 1>{}, integral_constant<uint32_t, 1>{});
+                else if(group.waves == 2u)
+                    shared(integral_constant<uint32_t, 2>{}, integral_constant<uint32_t, 1>{});
+                else if(group.waves == 4u)
+                    shared(integral_constant<uint32_t, 4>{}, integral_constant<uint32_t, 1>{});
                 else
-                    hipLaunchKernelGGL((gemvRowMajorShared<T, 16>), blocks, dim3(16 * 64), 0, s, m, k, a, lda, x, y_in, y_out, alpha, beta, k, 0u, 0u);
+                    shared(integral_constant<uint32_t, 8>{}, integral_constant<uint32_t, 1>{});
             }
             else if(stream)
                 hipLaunchKernelGGL((gemvRowMajor<T, true>), grid, dim3(THREADS), 0, s, m, k, a, lda, x, y_in, y_out, alpha, beta);
