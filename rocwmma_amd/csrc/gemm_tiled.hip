@@ -127,7 +127,8 @@ namespace r355
     // DLRM backward on macro tiles of S X (dlrmBwdTile below), one per element type
     struct DlrmBwdParams
     {
-        uint32_t    m, k, tilesM, tilesN, total; // total: tiles of all samples of the launch
+        uint32_t    m, k, tilesM, tilesN, total; // total: workgroups of the launch, tilesM * tilesN a sample
+        uint32_t    together;                    // tiles of a row of tiles that a workgroup takes: 1, 2 or 3
         const char *x, *up;
         char *      mlp, *grad;
     };
@@ -1748,10 +1749,10 @@ namespace
     //     through registers into the image.  A stage of the diagonal tile is both images of its pieces left of the diagonal, put together
     //     in registers (16-bit; f32 gathers it element by element).
     //   * the loads of stage kt + 1 are in flight under the matrix instructions of stage kt (16-bit: of stage kt - 1), and what that leaves exposed
-    //     other workgroups of the CU cover (two of the 128 x 128 tile, four of the 64 x 64 one: 64 and 32 KiB of LDS).
+    //     other workgroups of the CU cover (two of the 128 x 128 tile, four of the 64 x 64 one, two or three of the 64 x 64 ones below: 32 to 64 KiB of LDS).
     // S holds zeros only on its diagonal and beyond row or column m, as the products of the [m][m] matrix have them: an infinite feature is NaN
     // in its own row of the gradient and nowhere else.  Few stages bound the small shapes (latency of one stage's loads each), the matrix
-    // instructions and the loads' distance the large ones: f16 1024 x 1024 x 64 219 us, bf16 320 x 192 x 96 12.9, bf16 64 x 400 x 1011 25.5, f32
+    // instructions and the loads' distance the large ones: f16 1024 x 1024 x 64 219 us, bf16 320 x 192 x 96 9.6 (12.9 with one tile a workgroup), bf16 64 x 400 x 1011 25.5, f32
     // 224 x 384 x 213 96.  (The 16-bit ones 225, 13.0 and 25.8 with a diagonal stage's images multiplied one after the other; 250, 16.7 and 39.5
     // gathered element by element, eight 2-byte loads for each 16 bytes, and every stage requested one ahead.)
     using BwdParams = r355::DlrmBwdParams;
@@ -1768,18 +1769,23 @@ namespace
     // cuts: f16 1024 x 16 x 1 11.5 -> 10.1 us, 784 x 48 x 4 10.0 -> 9.0, 512 x 240 x 2 7.4 -> 6.9 (10.1, 9.1 and 7.4 with the diagonal stages gathered).
     // Where several share a CU that is slower (128 x 64 x 1689 17.7 -> 19.4, 320 x 192 x 96 13.1 -> 14.3, 1024 x 1024 x 64 on 128 x 128 tiles
     // 218 -> 233), and it is for samples of few tiles, most of whose stages are diagonal ones (128 x 192 x 12 4.03 -> 4.16, 256 x 16 x 1 4.79 -> 4.83).
-    template <Elem E, typename T, uint32_t WB, bool ALONE = false>
+    // NT (16-bit, 64 x 64 tiles): tiles of a row of tiles that a workgroup takes, one image of S with NT of X.  A stage's image of S goes through
+    // registers, in up to 8-byte parts, with a shift and tests on the diagonal tile; it and the waits weigh as much as the rest of a stage.  48
+    // KiB of LDS and three workgroups a CU with two, 64 KiB and two with three: six tiles at a time in place of four, in the time of four
+    // (bf16 320 x 192 x 96 12.9 -> 9.6 us, f16 688 x 480 x 16 22.7 -> 16.2, bf16 384 x 656 x 85 50.7 -> 39.4).  Where: bwdTogether.
+    template <Elem E, typename T, uint32_t WB, bool ALONE = false, uint32_t NT = 1>
     __device__ __forceinline__ void dlrmBwdTile(const BwdParams& p)
     {
+        static_assert(NT == 1 || ElemTraits<E>::Bytes == 2, "several tiles of 16-bit elements");
         constexpr uint32_t ES = ElemTraits<E>::Bytes, TILE = 32u * WB, WT = 16u * WB, OPER = TILE * STAGE_KB;
         constexpr uint32_t TK = STAGE_KB / ES, EPC = CHUNK / ES; // K elements per stage, elements per 16-byte piece
         using Word            = std::conditional_t<ES == 2, uint16_t, uint32_t>;
         typedef int i32x4u __attribute__((ext_vector_type(4), aligned(2)));
         constexpr bool     ACROSS = ES == 2; // a diagonal stage's mirrored elements are an image of their own (f32: gathered)
-        constexpr uint32_t B_AT = 2u * OPER, ACROSS_AT = OPER; // a buffer of A and that image (f32: two of A), two of B
-        __shared__ __attribute__((aligned(1024))) char lds[4u * OPER];
+        constexpr uint32_t B_AT = 2u * OPER, ACROSS_AT = OPER, B_BYTES = NT * OPER; // a buffer of A and that image (f32: two of A), two of B
+        __shared__ __attribute__((aligned(1024))) char lds[2u * OPER + 2u * B_BYTES];
 
-        // all workgroups of an XCD walk one contiguous run of (sample, tile): the tiles of a sample share its X and T in one L2
+        // all workgroups of an XCD walk one contiguous run of (sample, tiles): the tiles of a sample share its X and T in one L2
         const uint32_t perXcd = (p.total + 7u) / 8u, slotX = blockIdx.x / 8u, local = (blockIdx.x % 8u) * perXcd + slotX;
         if(slotX >= perXcd || local >= p.total)
             return;
@@ -1789,10 +1795,10 @@ namespace
         const char*    up  = p.up + (uint64_t)sample * ((uint64_t)p.k + (uint64_t)p.m * (p.m - 1u) / 2u) * ES;
         const uint32_t tid = threadIdx.x, lane = tid & 63u;
         const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1u;
-        const uint32_t row0 = tm * TILE, col0 = tn * TILE;
+        const uint32_t row0 = tm * TILE, col0 = tn * (NT * TILE);
         if(tm == 0u) // bottom-MLP gradient: the first k values of the upstream row, this tile's columns of them
         {
-            const uint32_t bytes = (p.k - col0 < TILE ? p.k - col0 : TILE) * ES, at = tid * CHUNK;
+            const uint32_t bytes = (p.k - col0 < NT * TILE ? p.k - col0 : NT * TILE) * ES, at = tid * CHUNK;
             if(at < bytes)
                 *reinterpret_cast<i32x4*>(p.mlp + ((uint64_t)sample * p.k + col0) * ES + at)
                     = *reinterpret_cast<const i32x4*>(up + (uint64_t)col0 * ES + at);
@@ -1801,17 +1807,29 @@ namespace
 
         const uint32_t ldsBase = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds));
         const uint32_t dmaDst  = ldsBase + wave * 64u * CHUNK;
-        uint32_t       gOffB[WB], gStepB, kByteB;
+        uint32_t       gOffB[NT][WB], gStepB, kByteB;
         uint64_t       gStageB;
-        laneOffsets8<false, WB, ES>(tid, p.k, p.k - col0 < TILE ? p.k - col0 : TILE, gOffB, gStepB, gStageB, kByteB);
+#pragma unroll
+        for(uint32_t t = 0; t < NT; ++t)
+        {
+            // (a tile past the last column reads the first tile's)
+            const bool     inside = col0 + t * TILE < p.k;
+            const uint32_t first = inside ? t * TILE : 0u, left = p.k - col0 - first;
+            laneOffsets8<false, WB, ES>(tid, p.k, left < TILE ? left : TILE, gOffB[t], gStepB, gStageB, kByteB);
+#pragma unroll
+            for(uint32_t j = 0; j < WB; ++j)
+                gOffB[t][j] += first * ES;
+        }
         const uint64_t gB        = r355::uniformAddress(p.x + xAt + (uint64_t)col0 * ES);
         const uint32_t numStages = (p.m + TK - 1u) / TK;
         auto           issueB    = [&](uint32_t st, uint32_t at) { // rows of X past the last one arrive as zeros
             const uint32_t left = (p.m - st * TK) * ES;
             const i32x4    rsrc = stageRsrc8(false, gB + st * gStageB, left < STAGE_KB ? left : STAGE_KB, p.k);
 #pragma unroll
-            for(uint32_t j = 0; j < WB; ++j)
-                loadToLds(rsrc, gOffB[j], j * gStepB, dmaDst + at + j * THREADS * CHUNK);
+            for(uint32_t t = 0; t < NT; ++t)
+#pragma unroll
+                for(uint32_t j = 0; j < WB; ++j)
+                    loadToLds(rsrc, gOffB[t][j], j * gStepB, dmaDst + at + t * OPER + j * THREADS * CHUNK);
         };
 
         // A: stages [0, diagFirst) left of the diagonal tile, [diagFirst, diagEnd) in it, [diagEnd, numStages) right of it
@@ -1948,12 +1966,14 @@ namespace
         readOffsets8<true, WB, ES>(wm, lane, rdAK);
         readOffsets8<false, WB, ES>(wm, lane, rdAM);
         readOffsets8<false, WB, ES>(wn, lane, rdB);
-        f32x4 acc[WB][WB];
+        f32x4 acc[NT][WB][WB];
 #pragma unroll
-        for(uint32_t i = 0; i < WB; ++i)
+        for(uint32_t t = 0; t < NT; ++t)
 #pragma unroll
-            for(uint32_t j = 0; j < WB; ++j)
-                acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            for(uint32_t i = 0; i < WB; ++i)
+#pragma unroll
+                for(uint32_t j = 0; j < WB; ++j)
+                    acc[t][i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         // Builtins, not inline assembly: between its loops the compiler may copy accumulators, and it has to know that the last
         // instructions' results are late.
         auto multiply = [](f32x4& c, i32x4 x, i32x4 y) {
@@ -1971,7 +1991,7 @@ namespace
                 }
             }
         };
-        i32x4 fa[2][WB], fb[2][WB];
+        i32x4 fa[2][WB], fb[NT][2][WB];
         auto  readA = [&](auto aK, uint32_t at) {
             constexpr bool AK = decltype(aK)::value;
 #pragma unroll
@@ -1996,21 +2016,25 @@ namespace
         };
         auto readB = [&](uint32_t at) {
 #pragma unroll
-            for(uint32_t s = 0; s < 2; ++s)
+            for(uint32_t t = 0; t < NT; ++t)
 #pragma unroll
-                for(uint32_t i = 0; i < WB; ++i)
+                for(uint32_t s = 0; s < 2; ++s)
 #pragma unroll
-                    for(uint32_t part = 0; part < 2; ++part)
-                        readBlock8<false, WB, ES>(lds + at, rdB, i, s, part, fb[s][i], 0u);
+                    for(uint32_t i = 0; i < WB; ++i)
+#pragma unroll
+                        for(uint32_t part = 0; part < 2; ++part)
+                            readBlock8<false, WB, ES>(lds + at + t * OPER, rdB, i, s, part, fb[t][s][i], 0u);
         };
         auto products = [&] {
 #pragma unroll
-            for(uint32_t s = 0; s < 2; ++s)
+            for(uint32_t t = 0; t < NT; ++t)
 #pragma unroll
-                for(uint32_t i = 0; i < WB; ++i)
+                for(uint32_t s = 0; s < 2; ++s)
 #pragma unroll
-                    for(uint32_t j = 0; j < WB; ++j)
-                        multiply(acc[i][j], fb[s][j], fa[s][i]); // (operands swapped, as everywhere here)
+                    for(uint32_t i = 0; i < WB; ++i)
+#pragma unroll
+                        for(uint32_t j = 0; j < WB; ++j)
+                            multiply(acc[t][i][j], fb[t][s][j], fa[s][i]); // (operands swapped, as everywhere here)
         };
 
         issueB(0u, B_AT);
@@ -2022,7 +2046,7 @@ namespace
             waitVmcnt<0>();
         else if(numStages > 1u)
         {
-            issueB(1u, B_AT + OPER);
+            issueB(1u, B_AT + B_BYTES);
             loadA(std::true_type{}, 1u);
         }
         ldsBarrier();
@@ -2030,7 +2054,7 @@ namespace
         // its place in LDS and the one after that is requested (requested and awaited around the same multiplications: f16 1024 x 1024 x 64 234 us
         // for 223, 1024 x 256 x 4 13.3 for 12.1, bf16 320 x 192 x 96 13.7 for 13.1).
         auto stageAhead = [&](auto aK, uint32_t st) {
-            const uint32_t bAt = B_AT + (st & 1u) * OPER;
+            const uint32_t bAt = B_AT + (st & 1u) * B_BYTES;
             readA(aK, 0u);
             if constexpr(decltype(aK)::value)
                 if(inDiag(st)) // S whole before it is multiplied: a zero of one image times an infinite feature would be NaN
@@ -2088,7 +2112,9 @@ namespace
         d.m = p.m, d.n = p.k, d.ldd = p.k;
         d.d     = p.grad + xAt;
         d.alpha = 1.0;
-        storeTileStaged<T, false, f32x4, T, WB, WB, WB * 4096u>(acc, d, row0 + wm * WT, col0 + wn * WT, lane, lds + wave * (WB * 4096u));
+#pragma unroll
+        for(uint32_t t = 0; t < NT; ++t) // (nothing of a tile past the last column)
+            storeTileStaged<T, false, f32x4, T, WB, WB, WB * 4096u>(acc[t], d, row0 + wm * WT, col0 + t * TILE + wn * WT, lane, lds + wave * (WB * 4096u));
     }
     template <Elem E, typename T>
     __global__ void __launch_bounds__(THREADS, 2) dlrmBwdTiled128(BwdParams p)
@@ -2107,9 +2133,26 @@ namespace
         dlrmBwdTile<E, T, 2, true>(p);
     }
     template <Elem E, typename T>
+    __global__ void __launch_bounds__(THREADS, 3) dlrmBwdTiled64x2(BwdParams p)
+    {
+        dlrmBwdTile<E, T, 2, false, 2>(p);
+    }
+    template <Elem E, typename T>
+    __global__ void __launch_bounds__(THREADS, 2) dlrmBwdTiled64x3(BwdParams p)
+    {
+        dlrmBwdTile<E, T, 2, false, 3>(p);
+    }
+    template <Elem E, typename T>
     int launchBwdTiled(const BwdParams& p, uint32_t tile, hipStream_t stream)
     {
         const uint32_t groups = (p.total + 7u) / 8u * 8u;
+        if constexpr(ElemTraits<E>::Bytes == 2)
+            if(p.together > 1u)
+            {
+                const auto kernel = p.together == 2u ? dlrmBwdTiled64x2<E, T> : dlrmBwdTiled64x3<E, T>;
+                hipLaunchKernelGGL(kernel, dim3(groups), dim3(THREADS), 0, stream, p);
+                return r355::checkLaunch("dlrm_bwd (macro tiles)");
+            }
         if(tile == 128u)
             hipLaunchKernelGGL((dlrmBwdTiled128<E, T>), dim3(groups), dim3(THREADS), 0, stream, p);
         else if(ElemTraits<E>::Bytes == 2 && p.tilesM >= 6u && p.total <= r355::computeUnits()) // (384 x 16 x 1 5.95 -> 5.73 us, 1024 x 64 x 16 12.7 -> 12.5)
@@ -2879,12 +2922,47 @@ namespace r355
         }
     }
 
+    // 64 x 64 tiles of a row of tiles that a workgroup of the 16-bit backward takes.  One below four workgroups a CU, where the CUs are not
+    // full with single tiles (f16 592 x 160 x 23, 690 of them: 11.5 us with one, 11.5 with two, 11.3 with three; 864 x 80 x 9, 252: 9.9, 12.4,
+    // 14.1), of one column of tiles, and of one K stage, which has next to nothing to share (64 x 400 x 1011 25.9, 27.3, 29.4).  Else what a CU
+    // takes: `at once` workgroups make a round; a round costs what it waits for, each workgroup what it issues, both per launch and stage.  us,
+    // fitted over 160 shapes (within 5 %; the choice takes 93 % of what the best of the three would gain, at most 5 % lost to one tile):
+    //                at once   launch   round   workgroup   round's stage   workgroup's stage
+    //   one tile        4       2.51     0.58      0.23          0.27             0.18
+    //   two             3       2.14     0.43      0.67          0.48             0.16
+    //   three           2       1.83     0.65      0.97          0.57             0.19
+    // e.g. bf16 320 x 192 x 96 13.8, 13.3, 9.4 us; 240 x 528 x 43 12.6, 12.1, 13.8; f16 224 x 208 x 302 30.8, 25.1, 33.5; 688 x 960 x 9 23.2,
+    // 22.9, 15.4.  More than one has to promise 5 %.
+    inline uint32_t bwdTogether(uint32_t tilesM, uint32_t tilesN, uint32_t batch)
+    {
+        const uint64_t cus = r355::computeUnits();
+        if(tilesM < 2u || tilesN < 2u || (uint64_t)tilesM * tilesN * batch <= 3u * cus)
+            return 1u;
+        static constexpr double US[3][5] = {{2.51, 0.58, 0.23, 0.27, 0.18}, {2.14, 0.43, 0.67, 0.48, 0.16}, {1.83, 0.65, 0.97, 0.57, 0.19}};
+        uint32_t best = 1u;
+        double   least = 0.0;
+        for(uint32_t n = 1u; n <= 3u; ++n)
+        {
+            const uint64_t groups = (uint64_t)tilesM * ((tilesN + n - 1u) / n) * batch;
+            const uint64_t perCu = (groups + cus - 1u) / cus, atOnce = 5u - n;
+            const double   each = static_cast<double>(perCu), rounds = static_cast<double>((perCu + atOnce - 1u) / atOnce);
+            const double*  c    = US[n - 1u];
+            const double   time = c[0] + rounds * (c[1] + c[3] * tilesM) + each * (c[2] + c[4] * tilesM);
+            if(n == 1u)
+                least = 0.95 * time;
+            else if(time < least)
+                least = time, best = n;
+        }
+        return best;
+    }
+
     int dlrmBwdTiled(int32_t dtype, const void* in, const void* upstream, void* mlpGrad, void* inGrad, uint32_t m, uint32_t k, uint32_t batch,
                      uint32_t tile, hipStream_t stream)
     {
         DlrmBwdParams p{};
         p.m = m, p.k = k;
-        p.tilesM = tilesOf(m, tile), p.tilesN = tilesOf(k, tile);
+        p.together = tile == 64u && dtype != R355_F32 ? bwdTogether(tilesOf(m, tile), tilesOf(k, tile), batch) : 1u;
+        p.tilesM = tilesOf(m, tile), p.tilesN = tilesOf(k, tile * p.together);
         const uint64_t es = dtypeBytes(dtype), stride = (uint64_t)k + (uint64_t)m * (m - 1u) / 2u;
         const uint64_t tiles = (uint64_t)p.tilesM * p.tilesN;
         if(tiles > MAX_GROUPS)
