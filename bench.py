@@ -23,6 +23,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 sys.path.insert(0, os.path.join(ROOT, "tests"))
 
+# (f32: of the f32 matrix instructions.  Launches of many tiles sum six bf16 products instead, at most 2500 / 6 = 417: fractions above 1)
 PEAK_TFLOPS = {"f16": 2500.0, "bf16": 2500.0, "e4m3": 5000.0, "i8": 5000.0, "f32": 157.3, "f64": 78.6}
 HBM_PEAK_GBPS = 8000.0
 # rocprofv3 --pmc results per benchmark case (MFMA busy, LDS bank conflicts, bytes across the L2 <-> fabric
@@ -30,7 +31,7 @@ HBM_PEAK_GBPS = 8000.0
 # was measured on; a row whose digest differs from the sources of this tree is reported as null, so a counter
 # can never outlive the kernel it belongs to.
 COUNTERS_FILE = os.path.join(ROOT, "profiles", "bench_counters.md")
-KERNEL_SOURCES = {"gemm": ["gemm_tiled.hip", "tile_map.hpp", "lds_dma.hpp", "operand_tile.hpp"],
+KERNEL_SOURCES = {"gemm": ["gemm_tiled.hip", "gemm_f32.hip", "gemm_params.hpp", "tile_map.hpp", "lds_dma.hpp", "operand_tile.hpp"],
                   "sparse": ["sparse.hip", "tile_map.hpp", "lds_dma.hpp", "operand_tile.hpp"],
                   "dlrm": ["dlrm.hip"]}
 

@@ -1770,7 +1770,7 @@ namespace
     // Where several share a CU that is slower (128 x 64 x 1689 17.7 -> 19.4, 320 x 192 x 96 13.1 -> 14.3, 1024 x 1024 x 64 on 128 x 128 tiles
     // 218 -> 233), and it is for samples of few tiles, most of whose stages are diagonal ones (128 x 192 x 12 4.03 -> 4.16, 256 x 16 x 1 4.79 -> 4.83).
     // NT (16-bit, 64 x 64 tiles): tiles of a row of tiles that a workgroup takes, one image of S with NT of X.  A stage's image of S goes through
-    // registers, in up to 8-byte parts, with a shift and tests on the diagonal tile; it and the waits weigh as much as the rest of a stage.  48
+    // registers, with a shift and tests on the diagonal tile; it and the waits weigh as much as the rest of a stage.  48
     // KiB of LDS and three workgroups a CU with two, 64 KiB and two with three: six tiles at a time in place of four, in the time of four
     // (bf16 320 x 192 x 96 12.9 -> 9.6 us, f16 688 x 480 x 16 22.7 -> 16.2, bf16 384 x 656 x 85 50.7 -> 39.4).  Where: bwdTogether.
     template <Elem E, typename T, uint32_t WB, bool ALONE = false, uint32_t NT = 1>
@@ -2965,7 +2965,7 @@ namespace r355
         p.tilesM = tilesOf(m, tile), p.tilesN = tilesOf(k, tile * p.together);
         const uint64_t es = dtypeBytes(dtype), stride = (uint64_t)k + (uint64_t)m * (m - 1u) / 2u;
         const uint64_t tiles = (uint64_t)p.tilesM * p.tilesN;
-        if(tiles > MAX_GROUPS)
+        if((uint64_t)p.tilesM * tilesOf(k, tile) > MAX_GROUPS)
             return fail(R355_ERR_BAD_SIZE, "dlrm_bwd: m=%u, k=%u: too many tiles of a sample", m, k);
         const uint32_t most = MAX_GROUPS / static_cast<uint32_t>(tiles); // samples per launch
         for(uint32_t first = 0;; first += most)

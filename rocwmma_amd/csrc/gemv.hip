@@ -7,7 +7,7 @@
 // the matrix core contributes nothing; the kernel is organised for memory bandwidth.
 //   col-major A (the sample's layout): a workgroup of sixteen waves owns 32 or 64 rows (f64: 16 or 32); its lanes split
 //     the columns and combine their partial sums through LDS in a fixed order.
-//   row-major A: one wave per row, lanes stride k in 16-byte pieces, then a wave reduction.
+//   row-major A: one wave per row or several, lanes stride k in 16-byte pieces, then a reduction over the row's waves.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
