@@ -536,7 +536,7 @@ namespace
         return best;
     }
 
-    // Col-major A whose columns do not start on 128-byte boundaries: 16-byte pieces of a run, splits of K (`most` at most) and columns per split, the
+    // Col-major A whose columns do not start on 128-byte boundaries, or that leaves CUs idle (leavesCusIdle): 16-byte pieces of a run, splits of K (`most` at most) and columns per split, the
     // cheapest by a timing model of a launch.  Its workgroups go round the CUs, 32 of an XCD at a time; one streams at most 42 GB/s, all together
     // 9.1 TB/s, and beyond 86 MB, where A does not come from the caches, short runs cost again as much as the lines they share; every row's sum ends with
     // an addition per lane group, and a split launch with a second kernel.  Splits: none, as many as make a round of workgroups, or all.  Runs of up to 256
@@ -564,8 +564,12 @@ namespace
         {
             const uint32_t blocks = (m + lanes * V - 1u) / (lanes * V), columns = askewWaves(lanes) * 64u / lanes;
             const uint32_t round  = cus / blocks < 1u ? 1u : cus / blocks < most ? cus / blocks : most;
+            uint32_t       before = 0;
             for(const uint32_t want : {1u, round, most})
             {
+                if(want == before)
+                    continue;
+                before = want;
                 const uint64_t kPer = ((uint64_t)(k - 1u) / want / columns + 1u) * columns; // (k itself may lie just below 2^32)
                 const uint32_t splits = static_cast<uint32_t>((k - 1u) / kPer) + 1u;
                 const uint64_t groups = (uint64_t)blocks * splits, rounds = ((groups + 7u) / 8u + perXcd - 1u) / perXcd;
@@ -581,6 +585,20 @@ namespace
         return best;
     }
 
+    // Whether an aligned col-major A goes by askewPlan too, whose shorter or longer runs and smaller workgroups reach all CUs: where the plain launch has blocks of
+    // rows for three quarters of the CUs at most, and A is of 64 MB at most, or 200 where K may be split.  Different matrices one after another / one repeated:
+    // f32 2048^2 7.4 -> 6.2 us / 5.1 -> 4.6, 3712 x 3048 15.4 -> 12.8 / 10.3 -> 9.7, f64 1840 x 2868 15.2 -> 10.9 / 10.2 -> 8.1; split f32
+    // 2240 x 2504 15.9 -> 7.9 / 11.6 -> 5.5, 1344 x 9192 18.3 -> 12.4 / 11.9 -> 10.4, f64 1360 x 11088 25.4 -> 23.9 / 21.8 -> 20.3, f32 3584 x 9464 even.  Full
+    // rounds are better off as they are (f32 8192^2 44 -> 55, 8192 x 2048 13.3 -> 15.4, f64 4096^2 23.3 -> 27.2), many second rounds too (f64 5696 x 1236
+    // 13.9 -> 17.3, f32 8608 x 2244 19.7 -> 22.4), and larger matrices when repeated (f32 4096 x 11008 49.0 -> 44.7 / 29.2 -> 33.6, 2048 x 32768 48.1 -> 46.2 / 39.5 -> 41.2).
+    template <typename T>
+    bool leavesCusIdle(uint32_t m, uint32_t k, bool maySplit)
+    {
+        constexpr uint32_t V = 16u / sizeof(T);
+        const uint32_t     rows = (m >= 16u * V * 256u ? 16u : 8u) * V;
+        const uint64_t     blocks = ((uint64_t)m + rows - 1u) / rows;
+        return 4u * blocks <= 3u * r355::computeUnits() && (uint64_t)m * k * sizeof(T) <= (maySplit ? 200000000u : 64000000u);
+    }
     // Rows per workgroup of the batched shared-row kernel for a streamed row-major A with long rows and fewer than 2048
     // of them, 0 = another kernel serves it.  Four or two rows, the larger count whose workgroups load the CUs evenly:
     // at least five eighths of them in a single round, at least 80 % of the slots of several rounds (f32, rows of 512 KiB
@@ -649,8 +667,9 @@ namespace
         if((uint64_t)splits * m * sizeof(T) > workspaceBytes)
             splits = 1u;
         T* parts = static_cast<T*>(workspace);
-        // columns off 128-byte boundaries
-        const bool askew = layout_a == R355_COL_MAJOR && lda >= m && ((uint64_t)lda * sizeof(T) % 128u != 0u || !r355::aligned(a, 128)) && m < (1u << 30);
+        // columns off 128-byte boundaries, and aligned ones of which the plain launch has few blocks
+        const bool askew = layout_a == R355_COL_MAJOR && lda >= m && m < (1u << 30)
+                           && ((uint64_t)lda * sizeof(T) % 128u != 0u || !r355::aligned(a, 128) || leavesCusIdle<T>(m, k, splits > 1u));
         AskewPlan  plan{};
         if(askew)
         {
