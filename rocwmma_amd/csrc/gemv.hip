@@ -591,13 +591,20 @@ namespace
     // 2240 x 2504 15.9 -> 7.9 / 11.6 -> 5.5, 1344 x 9192 18.3 -> 12.4 / 11.9 -> 10.4, f64 1360 x 11088 25.4 -> 23.9 / 21.8 -> 20.3, f32 3584 x 9464 even.  Full
     // rounds are better off as they are (f32 8192^2 44 -> 55, 8192 x 2048 13.3 -> 15.4, f64 4096^2 23.3 -> 27.2), many second rounds too (f64 5696 x 1236
     // 13.9 -> 17.3, f32 8608 x 2244 19.7 -> 22.4), and larger matrices when repeated (f32 4096 x 11008 49.0 -> 44.7 / 29.2 -> 33.6, 2048 x 32768 48.1 -> 46.2 / 39.5 -> 41.2).
+    // A matrix of more blocks beyond the memory-side cache, K split, goes by the plan where that is one round of workgroups: f32 8416 x 10936 64.1 -> 54.5 us,
+    // 17000 x 16384 195 -> 163, 26272 x 3000 52.3 -> 45.8, f64 14144 x 4748 85.5 -> 77.4; 23 shapes 1.02 - 1.19, repeated or not.  Of several rounds 16640 x 16384
+    // took 170 for 161; matrices within the cache lose up to 4 % repeated (f64 4272 x 3680 20.8 -> 21.7).
     template <typename T>
-    bool leavesCusIdle(uint32_t m, uint32_t k, bool maySplit)
+    bool fewBlocks(uint32_t m)
     {
         constexpr uint32_t V = 16u / sizeof(T);
         const uint32_t     rows = (m >= 16u * V * 256u ? 16u : 8u) * V;
-        const uint64_t     blocks = ((uint64_t)m + rows - 1u) / rows;
-        return 4u * blocks <= 3u * r355::computeUnits() && (uint64_t)m * k * sizeof(T) <= (maySplit ? 200000000u : 64000000u);
+        return 4u * (((uint64_t)m + rows - 1u) / rows) <= 3u * r355::computeUnits();
+    }
+    template <typename T>
+    bool leavesCusIdle(uint32_t m, uint32_t k, bool maySplit)
+    {
+        return fewBlocks<T>(m) && (uint64_t)m * k * sizeof(T) <= (maySplit ? 200000000u : 64000000u);
     }
     // Rows per workgroup of the batched shared-row kernel for a streamed row-major A with long rows and fewer than 2048
     // of them, 0 = another kernel serves it.  Four or two rows, the larger count whose workgroups load the CUs evenly:
@@ -667,14 +674,20 @@ namespace
         if((uint64_t)splits * m * sizeof(T) > workspaceBytes)
             splits = 1u;
         T* parts = static_cast<T*>(workspace);
-        // columns off 128-byte boundaries, and aligned ones of which the plain launch has few blocks
-        const bool askew = layout_a == R355_COL_MAJOR && lda >= m && m < (1u << 30)
-                           && ((uint64_t)lda * sizeof(T) % 128u != 0u || !r355::aligned(a, 128) || leavesCusIdle<T>(m, k, splits > 1u));
+        // columns off 128-byte boundaries, and aligned ones that the plain launch or the splits above leave CUs idle with
+        const bool colPlan  = layout_a == R355_COL_MAJOR && lda >= m && m < (1u << 30);
+        const bool offLines = (uint64_t)lda * sizeof(T) % 128u != 0u || !r355::aligned(a, 128);
+        const bool streamed = splits > 1u && (uint64_t)m * k * sizeof(T) > (256ull << 20) && !fewBlocks<T>(m);
+        bool       askew    = colPlan && (offLines || streamed || leavesCusIdle<T>(m, k, splits > 1u));
         AskewPlan  plan{};
         if(askew)
         {
-            plan   = askewPlan<T>(m, k, splits);
-            splits = plan.splits, kPer = plan.kPer;
+            plan = askewPlan<T>(m, k, splits);
+            // (a streamed matrix of several rounds of blocks: where the plan is a single round of workgroups)
+            if(!offLines && streamed && (uint64_t)plan.splits * ((m + plan.lanes * (16u / sizeof(T)) - 1u) / (plan.lanes * (16u / sizeof(T)))) > r355::computeUnits())
+                askew = false;
+            else
+                splits = plan.splits, kPer = plan.kPer;
         }
         const bool     split  = splits > 1u;
         const bool     byWave = splits >= 32u; // layout of the partial sums: [m][splits] for the wave-per-row reduction, else [splits][m]
