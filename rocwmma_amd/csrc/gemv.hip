@@ -78,6 +78,13 @@ namespace
             };
             const uint32_t kEnd = SPLIT ? (k - part * kPer < kPer ? k : (part + 1u) * kPer) : k;
             uint32_t       kk   = (SPLIT ? part * kPer : 0u) + wave * CL + c;
+            // BY_XCD: a lane may add a thousand columns and more; those of a trip, sixteen trips and all of them are three sums, so that no chain of roundings is
+            // as long (norm of the error, f32 6152 x 11012 3.2e-7 as one sum, 1.2e-7 as three, as fast; 17000 x 16384 6.6e-7 and 1.3e-7; sixteen waves of 32 to 128 columns each, before: 1.6e-7 and 1.7e-7)
+            [[maybe_unused]] T        near[V];
+            [[maybe_unused]] uint32_t trips = 0;
+#pragma unroll
+            for(uint32_t e = 0; e < V; ++e)
+                near[e] = T(0);
             for(; kk + (DEPTH - 1u) * COLS < kEnd; kk += DEPTH * COLS)
             {
                 VecT v[DEPTH];
@@ -88,11 +95,32 @@ namespace
 #pragma unroll
                 for(uint32_t u = 0; u < DEPTH; ++u)
                     xv[u] = x[kk + u * COLS];
+                if constexpr(BY_XCD)
+                {
+                    T sum[V];
 #pragma unroll
-                for(uint32_t u = 0; u < DEPTH; ++u)
+                    for(uint32_t u = 0; u < DEPTH; ++u)
+#pragma unroll
+                        for(uint32_t e = 0; e < V; ++e)
+                            sum[e] = u == 0u ? v[u][e] * xv[u] : sum[e] + v[u][e] * xv[u];
 #pragma unroll
                     for(uint32_t e = 0; e < V; ++e)
-                        acc[e] += v[u][e] * xv[u];
+                        near[e] += sum[e];
+                    if(++trips % 16u == 0u)
+                    {
+#pragma unroll
+                        for(uint32_t e = 0; e < V; ++e)
+                            acc[e] += near[e], near[e] = T(0);
+                    }
+                }
+                else
+                {
+#pragma unroll
+                    for(uint32_t u = 0; u < DEPTH; ++u)
+#pragma unroll
+                        for(uint32_t e = 0; e < V; ++e)
+                            acc[e] += v[u][e] * xv[u];
+                }
             }
             if constexpr(BY_XCD)
             {
@@ -112,8 +140,11 @@ namespace
                     for(uint32_t u = 0; u < DEPTH; ++u)
 #pragma unroll
                         for(uint32_t e = 0; e < V; ++e)
-                            acc[e] = u * COLS < kEnd - kk ? acc[e] + v[u][e] * xv[u] : acc[e];
+                            near[e] = u * COLS < kEnd - kk ? near[e] + v[u][e] * xv[u] : near[e];
                 }
+#pragma unroll
+                for(uint32_t e = 0; e < V; ++e)
+                    acc[e] += near[e];
             }
             else
                 for(; kk < kEnd; kk += COLS)
@@ -683,8 +714,11 @@ namespace
         if(askew)
         {
             plan = askewPlan<T>(m, k, splits);
-            // (a streamed matrix of several rounds of blocks: where the plan is a single round of workgroups)
-            if(!offLines && streamed && (uint64_t)plan.splits * ((m + plan.lanes * (16u / sizeof(T)) - 1u) / (plan.lanes * (16u / sizeof(T)))) > r355::computeUnits())
+            // (a streamed matrix of several rounds of blocks: where the plan is a single round of workgroups; aligned columns otherwise split: not in runs of 64 bytes
+            // over many columns, f32 864 x 13476, 3456 of them, 12.3 -> 14.4 us, 576 x 10216, 2048 of them, 12.0 -> 9.8)
+            if(!offLines && splits > 1u && plan.lanes == 4u && plan.kPer > 2700u)
+                askew = false;
+            else if(!offLines && streamed && (uint64_t)plan.splits * ((m + plan.lanes * (16u / sizeof(T)) - 1u) / (plan.lanes * (16u / sizeof(T)))) > r355::computeUnits())
                 askew = false;
             else
                 splits = plan.splits, kPer = plan.kPer;
