@@ -13,6 +13,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "gemv_rows.hpp"
 
 namespace
 {
@@ -314,7 +315,7 @@ namespace
     // load before it asks for the next row: variants with two or four loads per row under way, or with the next row's
     // requested ahead, were slower the more they had in flight (16384^2 f32: 0.77, 0.67, 0.64 of the peak against 0.86),
     // and so were 8 and 16 rows per workgroup.  Sixteen waves, for rows of 128 KiB and more (8192 x 32768: 0.882, with eight 0.818; 32768^2: 0.895
-    // and 0.842; one row per wave: 0.79, 0.82); shorter ones go by rowGroup.
+    // and 0.842; one row per wave: 0.79, 0.82); shorter ones go by rowGroup (gemv_rows.hpp).
     // STREAM: A lies beyond the memory-side cache and is read with nontemporal loads; a smaller one (few very long rows
     // of a matrix that is multiplied again and again) keeps ordinary loads so that the next call finds it there, as in
     // gemvRowMajor / gemvColMajor.
@@ -657,56 +658,19 @@ namespace
         return 0u;
     }
 
-    // Waves and rows of a workgroup for a row-major A with rows below 128 KiB, {0, 0}: a wave per row, four to a workgroup (gemvRowMajor).  A row of a
-    // few KiB wants as many waves as make one or two trips of it, so that its loads are all under way at once; a matrix from HBM wants two rows a workgroup,
-    // which share x and keep as many loads more in flight; short rows by the ten thousands want four rows a wave.  168 random shapes from 256 to 16384
-    // rows and columns, A in the memory-side cache or not: 1.03 times as long as the best of 13 combinations, where a wave per row takes 1.15 times
-    // (f32 576 x 1780 from HBM 3.40 -> 2.81 us, 380 x 11964 10.9 -> 6.0, 8920 x 3796 26.4 -> 22.6, 9496 x 12800 87 -> 70; f64 2052 x 5680 25.7 -> 18.7), and
-    // 1.02 on most shapes outside (f32 88 x 27708 18.2 -> 6.5, 390884 x 16 64 -> 35, 16384^2 160 -> 150).
-    struct RowGroup
-    {
-        uint32_t waves, rows;
-    };
-    inline RowGroup rowGroup(uint32_t m, uint64_t rowBytes, uint32_t elemBytes)
-    {
-        const uint64_t bytes = rowBytes * m;
-        if(rowBytes <= 2048u && m >= 16384u)
-            return elemBytes == 8u && rowBytes < 256u ? RowGroup{0u, 0u} : RowGroup{1u, 4u}; // (f64 25772 x 24 5.0 -> 5.7)
-        if(rowBytes <= 1024u)
-            return {0u, 0u};
-        if(rowBytes <= 5632u)
-            return {1u, 1u};
-        if(rowBytes <= 9344u)
-            return {2u, 1u};
-        if(bytes <= 23000000u)
-            return {rowBytes < (64u << 10) ? 4u : 8u, 1u};
-        return {bytes <= 165000000u ? 4u : 8u, 2u};
-    }
-
+    // One launch (two with K split) of m rows; arguments as gemvLaunch has checked them
     template <typename T>
-    int gemvLaunch(int32_t layout_a, uint32_t m, uint32_t k, const T* a, uint32_t lda, const T* x, const T* y_in, T* y_out,
-                   T alpha, T beta, void* stream, void* workspace = nullptr, size_t workspaceBytes = 0)
+    void gemvRows(int32_t layout_a, uint32_t m, uint32_t k, const T* a, uint32_t lda, const T* x, const T* y_in, T* y_out,
+                  T alpha, T beta, hipStream_t s, void* workspace, size_t workspaceBytes)
     {
         constexpr uint32_t V = 16u / sizeof(T);
-        if(!a || !x || !y_out || (beta != T(0) && !y_in))
-            return r355::fail(R355_ERR_BAD_ARG, "gemv: null pointer");
-        if(m == 0 || k == 0)
-            return r355::fail(R355_ERR_BAD_ARG, "gemv: m and k must be non-zero");
-        if(m % V || k % V)
-            return r355::fail(R355_ERR_BAD_SIZE, "gemv: m=%u and k=%u must be multiples of %u", m, k, V);
-        if(!r355::aligned(a, 16) || lda % V || !r355::aligned(x, 16) || !r355::aligned(y_out, 16))
-            return r355::fail(R355_ERR_MISALIGNED, "gemv: a, x, y need 16-byte alignment and lda %% %u == 0", V);
-        if(workspace && !r355::aligned(workspace, 16))
-            return r355::fail(R355_ERR_MISALIGNED, "gemv: the workspace needs 16-byte alignment");
-        hipStream_t s = static_cast<hipStream_t>(stream);
-        r355::beginCall();
         // K split over several workgroups per block of rows when the shape calls for it and the workspace holds the partial sums
-        uint32_t kPer = k, splits = (layout_a == R355_COL_MAJOR || layout_a == R355_ROW_MAJOR) && workspace ? gemvSplits<T>(layout_a, m, k, lda, kPer) : 1u;
+        uint32_t kPer = k, splits = workspace ? gemvSplits<T>(layout_a, m, k, lda, kPer) : 1u;
         if((uint64_t)splits * m * sizeof(T) > workspaceBytes)
             splits = 1u;
         T* parts = static_cast<T*>(workspace);
         // columns off 128-byte boundaries, and aligned ones that the plain launch or the splits above leave CUs idle with
-        const bool colPlan  = layout_a == R355_COL_MAJOR && lda >= m && m < (1u << 30);
+        const bool colPlan  = layout_a == R355_COL_MAJOR;
         const bool offLines = (uint64_t)lda * sizeof(T) % 128u != 0u || !r355::aligned(a, 128);
         const bool streamed = splits > 1u && (uint64_t)m * k * sizeof(T) > (256ull << 20) && !fewBlocks<T>(m);
         bool       askew    = colPlan && (offLines || streamed || leavesCusIdle<T>(m, k, splits > 1u));
@@ -728,8 +692,6 @@ namespace
         const uint32_t partRow = byWave ? splits : 1u, partSplit = byWave ? 1u : m;
         if(layout_a == R355_COL_MAJOR)
         {
-            if(lda < m)
-                return r355::fail(R355_ERR_BAD_ARG, "gemv: lda < m");
             const bool stream = (uint64_t)k * lda * sizeof(T) > (256ull << 20);
             auto       go     = [&](auto rl, auto waves, auto byXcd) {
                 constexpr uint32_t RL = decltype(rl)::value, ROWS = RL * V, WAVES = decltype(waves)::value;
@@ -775,10 +737,8 @@ namespace
             else
                 go(integral_constant<uint32_t, 8>{}, integral_constant<uint32_t, 16>{}, plain);
         }
-        else if(layout_a == R355_ROW_MAJOR)
+        else
         {
-            if(lda < k)
-                return r355::fail(R355_ERR_BAD_ARG, "gemv: lda < k");
             const dim3 grid((m + THREADS / 64 - 1) / (THREADS / 64));
             const bool     stream   = (uint64_t)m * lda * sizeof(T) > (256ull << 20);
             const uint64_t rowBytes = (uint64_t)k * sizeof(T);
@@ -813,7 +773,7 @@ namespace
             }
             else if(stream && rowBytes >= (128u << 10) && rowBytes < (1ull << 31) && m >= SHARED_ROWS * 512u)
                 hipLaunchKernelGGL((gemvRowMajorShared<T, 16>), dim3((m + SHARED_ROWS - 1u) / SHARED_ROWS), dim3(16 * 64), 0, s, m, k, a, lda, x, y_in, y_out, alpha, beta, k, 0u, 0u);
-            else if(const RowGroup group = rowBytes < (128u << 10) ? rowGroup(m, rowBytes, sizeof(T)) : RowGroup{}; group.waves != 0u)
+            else if(const r355::RowGroup group = rowBytes < (128u << 10) ? r355::rowGroup(m, rowBytes, sizeof(T)) : r355::RowGroup{}; group.waves != 0u)
             {
                 auto shared = [&](auto waves, auto rows) {
                     constexpr uint32_t W = decltype(waves)::value, RB = decltype(rows)::value;
@@ -844,12 +804,40 @@ namespace
             else
                 hipLaunchKernelGGL((gemvRowMajor<T, false>), grid, dim3(THREADS), 0, s, m, k, a, lda, x, y_in, y_out, alpha, beta);
         }
-        else
-            return r355::fail(R355_ERR_BAD_ARG, "gemv: unknown layout");
         if(split && byWave)
             hipLaunchKernelGGL(gemvAddSplitsByWave<T>, dim3((m + THREADS / 64u - 1u) / (THREADS / 64u)), dim3(THREADS), 0, s, m, splits, parts, y_in, y_out, alpha, beta);
         else if(split)
             hipLaunchKernelGGL(gemvAddSplits<T>, dim3((m + THREADS - 1u) / THREADS), dim3(THREADS), 0, s, m, splits, parts, y_in, y_out, alpha, beta);
+    }
+
+    template <typename T>
+    int gemvLaunch(int32_t layout_a, uint32_t m, uint32_t k, const T* a, uint32_t lda, const T* x, const T* y_in, T* y_out,
+                   T alpha, T beta, void* stream, void* workspace = nullptr, size_t workspaceBytes = 0)
+    {
+        constexpr uint32_t V = 16u / sizeof(T);
+        if(!a || !x || !y_out || (beta != T(0) && !y_in))
+            return r355::fail(R355_ERR_BAD_ARG, "gemv: null pointer");
+        if(m == 0 || k == 0)
+            return r355::fail(R355_ERR_BAD_ARG, "gemv: m and k must be non-zero");
+        if(m % V || k % V)
+            return r355::fail(R355_ERR_BAD_SIZE, "gemv: m=%u and k=%u must be multiples of %u", m, k, V);
+        if(!r355::aligned(a, 16) || lda % V || !r355::aligned(x, 16) || !r355::aligned(y_out, 16))
+            return r355::fail(R355_ERR_MISALIGNED, "gemv: a, x, y need 16-byte alignment and lda %% %u == 0", V);
+        if(workspace && !r355::aligned(workspace, 16))
+            return r355::fail(R355_ERR_MISALIGNED, "gemv: the workspace needs 16-byte alignment");
+        const bool colMajor = layout_a == R355_COL_MAJOR;
+        if(!colMajor && layout_a != R355_ROW_MAJOR)
+            return r355::fail(R355_ERR_BAD_ARG, "gemv: unknown layout");
+        if(lda < (colMajor ? m : k))
+            return r355::fail(R355_ERR_BAD_ARG, colMajor ? "gemv: lda < m" : "gemv: lda < k");
+        r355::beginCall();
+        const uint32_t most = r355::gemvLaunchRows(colMajor, m, (uint64_t)k * sizeof(T), sizeof(T));
+        for(uint32_t first = 0, rows = 0; first < m; first += rows)
+        {
+            rows = m - first < most ? m - first : most;
+            gemvRows<T>(layout_a, rows, k, a + (colMajor ? (uint64_t)first : (uint64_t)first * lda), lda, x, y_in ? y_in + first : nullptr,
+                        y_out + first, alpha, beta, static_cast<hipStream_t>(stream), workspace, workspaceBytes);
+        }
         return r355::checkLaunch("gemv");
     }
 } // namespace
