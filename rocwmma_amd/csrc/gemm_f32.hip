@@ -1,13 +1,13 @@
 // f32 GEMM on the bf16 matrix instructions, 64 x 64 macro tiles.
 //
 // v_mfma_f32_16x16x4_f32 runs at a sixteenth of the rate of v_mfma_f32_16x16x32_bf16.  An f32 has 24 significant bits, a bf16
-// eight: x = h + m + l with three bf16, each the rounded value of what the ones before it leave, holds every f32 exactly
-// (bits below 2^-133 apart, see Pieces).  Of the nine products of two such sums the six down to 2^-18 of the whole are multiplied,
+// eight: 2^16 x = h + m + l with three bf16, each the rounded value of what the ones before it leave, holds every f32 below 2^112 exactly (the smallest,
+// 2^-149, becomes 2^-133, the last bit of a bf16).  Of the nine products of two such sums the six down to 2^-17 of the whole are multiplied,
 //     h h'   and   h m' + m h' + m m' + h l' + l h',
-// which leaves out less than 2^-25 of a product, and summed in f32 accumulators, the first one in one of its own, so that the long chain
-// of roundings is that of one product in 32 instead of one in one.  Against 64 bits the result is closer than with the f32 instructions
-// (norm of the difference, uniform operands, every orientation alike): K = 64 1.45e-7 -> 0.45e-7, 512 4.0e-7 -> 0.71e-7, 2560 9.1e-7 -> 1.36e-7,
-// 3584 10.7e-7 -> 1.6e-7; positive operands, K = 2560, 7.8e-7 -> 0.8e-7.
+// which leaves out up to 2^-24 of a product (|m| is up to 2^-8 of x, |l| 2^-17: m l' + l m'), and summed in f32 accumulators, the first one in one of its
+// own, so that the long chain of roundings is that of one product in 32 instead of one in one.  Against 64 bits such a sum is closer than with the f32
+// instructions (norm of the difference, uniform operands, every orientation alike): K = 512 4.0e-7 -> 0.71e-7, 2560 9.1e-7 -> 1.36e-7, 3584 10.7e-7 -> 1.6e-7;
+// positive operands, K = 2560, 7.8e-7 -> 0.8e-7.
 //
 //   workgroup    four waves, two workgroups a CU.  Each wave multiplies the whole tile over its own slices of K (32 wide, every fourth one),
 //                so that an operand element is taken apart once in a workgroup and no wave waits for another before the end
@@ -15,14 +15,17 @@
 //                B's under the last block's matrix instructions
 //   registers    2 x 64 of accumulators, 48 of A's pieces, 12 of a block of B's
 //   end          the four partial tiles meet in LDS and are added in the order of the waves
-//   not a number An infinite or missing value anywhere in a tile makes the sum of the products that is not finite (l of an infinity is NaN).
-//                Such a tile, and one whose operands have bits below 2^-133, is multiplied again with the f32 instructions, as
-//                all of them were before: their results are what they were.
+//   not a number An infinite or missing value anywhere in a tile makes the sum of the products that is not finite (l of an infinity is NaN), and so
+//                does an operand from 2^112 (5e33) or a sum from 2^96 (8e28) on.  Such a tile is multiplied again with the f32 instructions, each wave
+//                its own slices of K (the kernel of fewer tiles sums K in one chain: other roundings, the same infinities and NaN but where a sum
+//                overflows in between).  It costs both: 2560^3 210 us, 390 with one infinity in A, 480 with one in every row, 250 with f32 instructions alone.
 //
-// What bounds it: the board's power, then the vector instructions that take the operands apart (384 per 96 matrix instructions, which
-// hide two each).  2560^3: 252 us with f32 instructions -> 205 (184 with all-zero operands; 120 of it with the pieces not formed,
-// 107 the forming alone, 102 the direct loads alone).  Tried: the same with v_mfma_f32_32x32x16_bf16, 227; the pieces by v_dot2c_f32_bf16
-// subtractions, 207 (a dot product takes the matrix pipe); the forming dealt out between the matrix instructions, 211 (173 with zeros).
+// What bounds it: the board's power, then the vector instructions that take the operands apart (416 per 96 matrix instructions, which
+// hide two each).  2560^3: 255 us with f32 instructions -> 210 (188 with all-zero operands, 211 with a softmax of wide logits, a quarter of whose values are below
+// 2^-110; without the factor 2^16, whose multiplications are two of every thirteen vector instructions, 206, but 475 where tiles with such values were multiplied again).
+// Tried: the same with v_mfma_f32_32x32x16_bf16, 1.1 times as long; the pieces by v_dot2c_f32_bf16 subtractions, 1.01 (a dot product takes the matrix
+// pipe); the forming dealt out between the matrix instructions, 1.03; all eight products but l l' 1.15 to 1.18, no faster than the f32 instructions on
+// most shapes; the waves of a SIMD at different priorities, 0.96 to 1.01.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -41,6 +44,7 @@ namespace
     using Params = r355::GemmTileParams;
     using r355::loadToLds;
 
+    constexpr float    SCALE = 65536.0f; // no f32 has bits that are below the last one of bf16 after it
     constexpr uint32_t TILE = 64, WAVES = 4, THREADS = 256;
     constexpr uint32_t SLICE = 32, SLICE_BYTES = 128; // K of a slice: elements, bytes
     constexpr uint32_t CHUNK = 16, OPER = TILE * SLICE_BYTES; // 8 KiB of an operand per slice
@@ -57,8 +61,7 @@ namespace
         asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
     }
 
-    // Eight f32 as three bf16 each.  What is left after the third is zero but for operands with bits below 2^-133, the last of bf16: those
-    // bits stand in the lower half of the last remainder and are noted in `lost`.
+    // Eight f32 times SCALE as three bf16 each
     struct Pieces
     {
         i32x4 h, m, l;
@@ -69,18 +72,17 @@ namespace
         asm volatile("" : "+v"(w)); // (a word like any other: its halves are taken apart by a shift and a mask, not rounded once more)
         return w;
     }
-    __device__ __forceinline__ Pieces split(const float (&in)[8], uint32_t& lost)
+    __device__ __forceinline__ Pieces split(const float (&in)[8])
     {
         Pieces p;
 #pragma unroll
         for(uint32_t e = 0; e < 4; ++e)
         {
-            float          x0 = in[2u * e], x1 = in[2u * e + 1u];
+            float          x0 = in[2u * e] * SCALE, x1 = in[2u * e + 1u] * SCALE;
             const uint32_t h = pack(x0, x1);
             x0 -= __builtin_bit_cast(float, h << 16), x1 -= __builtin_bit_cast(float, h & 0xFFFF0000u);
             const uint32_t m = pack(x0, x1);
             x0 -= __builtin_bit_cast(float, m << 16), x1 -= __builtin_bit_cast(float, m & 0xFFFF0000u);
-            asm volatile("v_or3_b32 %0, %0, %1, %2" : "+v"(lost) : "v"(x0), "v"(x1));
             p.h[e] = static_cast<int>(h), p.m[e] = static_cast<int>(m), p.l[e] = static_cast<int>(pack(x0, x1));
         }
         return p;
@@ -203,7 +205,6 @@ namespace
         const uint32_t dstA = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds)) + wave * 2u * OPER;
         const uint32_t dstB = dstA + OPER;
         auto validOf = [&](uint32_t s) { return s + 1u < total ? SLICE_BYTES : lastBytes; };
-        uint32_t lost = 0u; // bits of an operand that its three pieces do not hold
 
         f32x4 hi[BLOCKS][BLOCKS], lo[BLOCKS][BLOCKS];
         bool  exact = false;
@@ -232,7 +233,7 @@ namespace
                     {
                         float x[8];
                         a.read(mine, i, x);
-                        pa[i] = split(x, lost);
+                        pa[i] = split(x);
                         __builtin_amdgcn_sched_barrier(0);
                     }
                     waitReads(); // the reads of A are done, its place may be filled again
@@ -248,7 +249,7 @@ namespace
                     {
                         float x[8];
                         b.read(mine + OPER, j, x);
-                        const Pieces pb = split(x, lost);
+                        const Pieces pb = split(x);
                         if(j + 1u == BLOCKS)
                         {
                             waitReads();
@@ -331,19 +332,19 @@ namespace
                 for(uint32_t e = 0; e < 4; ++e)
                     finite = finite && __builtin_isfinite(sum[it][e]);
             }
-            if(!exact && __syncthreads_or(!finite || (lost & 0xFFFFu) != 0u))
+            if(!exact && __syncthreads_or(!finite))
             {
                 exact = true;
                 continue;
             }
-            const float alpha = static_cast<float>(p.alpha), beta = static_cast<float>(p.beta);
+            const float alpha = static_cast<float>(p.alpha), beta = static_cast<float>(p.beta), unscale = exact ? 1.0f : 1.0f / (SCALE * SCALE);
 #pragma unroll
             for(uint32_t it = 0; it < 4; ++it)
             {
                 const uint32_t row = m0 + 16u * it + (tid >> 4), col = n0 + (tid & 15u) * 4u;
                 if(row < p.m && col < p.n)
                 {
-                    f32x4 out = sum[it] * alpha;
+                    f32x4 out = sum[it] * unscale * alpha;
                     if(beta != 0.0f)
                         out += beta * *reinterpret_cast<const f32x4*>(p.c + ((uint64_t)row * p.ldc + col) * 4u);
                     __builtin_nontemporal_store(out, reinterpret_cast<f32x4*>(d + ((uint64_t)row * p.ldd + col) * 4u));

@@ -1,5 +1,5 @@
 """f32 GEMM on the bf16 matrix instructions (gemm_f32.hip): launches of more workgroups of 64 x 64 tiles than CUs, with K shares of 512
-elements and more.  Partial tiles and K tails, values that three bf16 do not hold, infinities, and the error against float64."""
+elements and more.  Partial tiles and K tails, operands from the smallest f32 to the largest, infinities, and the error against float64."""
 import numpy as np
 import pytest
 
@@ -49,7 +49,8 @@ def test_orientations_partial_tiles_and_k_tails(la, lb, ldl, m, n, k):
 
 @pytest.mark.parametrize("la,lb", LAYOUTS)
 def test_every_bit_of_an_operand(la, lb):
-    # one product a row: every bit of the other operand, from the largest exponents to the smallest
+    # one product a row: every bit of the other operand, from the largest exponents to the smallest (every tile meets some of 2^112 and more,
+    # so that all of it is the second pass, on the f32 instructions)
     m, n, k = 1056, 1056, 1056
     rng = np.random.default_rng(4)
     bits = rng.integers(0, 2 ** 32, (k, n), dtype=np.uint32)
@@ -60,6 +61,43 @@ def test_every_bit_of_an_operand(la, lb):
     want = values[pick.argmax(axis=1)]
     assert np.array_equal(_run(pick, values, la, lb), want)
     assert np.array_equal(_run(np.ascontiguousarray(values.T), np.ascontiguousarray(pick.T), la, lb), want.T)
+
+
+@pytest.mark.parametrize("la,lb", LAYOUTS)
+def test_every_bit_of_the_pieces(la, lb):
+    # the same for all f32 below 2^95, the denormal ones among them: no piece and no sum (2^32 times the result) overflows, so that no tile is
+    # multiplied again
+    m, n, k = 1056, 1056, 1056
+    rng = np.random.default_rng(14)
+    values = (rng.integers(0, 222 << 23, (k, n), dtype=np.uint32) | rng.integers(0, 2, (k, n), dtype=np.uint32) << 31).view(np.float32)
+    pick = np.zeros((m, k), np.float32)
+    pick[np.arange(m), rng.permutation(k)[:m]] = 1.0
+    want = values[pick.argmax(axis=1)]
+    assert np.array_equal(_run(pick, values, la, lb), want)
+    assert np.array_equal(_run(np.ascontiguousarray(values.T), np.ascontiguousarray(pick.T), la, lb), want.T)
+
+
+@pytest.mark.parametrize("la,lb", LAYOUTS)
+def test_tiny_values_take_no_second_pass(la, lb):
+    # values below 2^-110 in every row and column, and operands of nothing else: the error is that of the bf16 instructions (0.7e-7 of the norm), not of a
+    # second pass with the f32 ones (2.1e-7)
+    m, n, k = 1040, 1056, 528
+    A, B = _uniform(15, m, k), _uniform(16, k, n)
+    A[np.arange(m), np.arange(m) % k] *= np.float32(2.0 ** -120)
+    B[np.arange(n) % k, np.arange(n)] *= np.float32(2.0 ** -125)
+    for scale in (0, -110):
+        got = _run(np.ldexp(A, scale), np.ldexp(B, -scale - 20), la, lb).astype(np.float64)
+        exact = np.ldexp(A, scale).astype(np.float64) @ np.ldexp(B, -scale - 20).astype(np.float64)
+        assert np.linalg.norm(got - exact) <= 1.2e-7 * np.linalg.norm(exact)
+
+
+def test_one_product_below_the_normal_numbers():
+    # rounded to 2^-149 once: products of the pieces are not rounded there one by one
+    m, n, k = 1040, 1040, 528
+    A, B = np.zeros((m, k), np.float32), np.ldexp(_uniform(17, k, n), -70)
+    A[np.arange(m), np.arange(m) % k] = np.ldexp(_uniform(18, m), -60)
+    got = _run(A, B, O.ROW, O.COL).astype(np.float64)
+    assert np.all(np.abs(got - A.astype(np.float64) @ B) <= 0.6 * 2.0 ** -149)
 
 
 @pytest.mark.parametrize("ea,eb", [(-125, 100), (100, -125), (-60, -70), (55, 60)])
