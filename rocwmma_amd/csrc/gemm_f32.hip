@@ -7,22 +7,25 @@
 // which leaves out up to 2^-24 of a product (|m| is up to 2^-8 of x, |l| 2^-17: m l' + l m'), and summed in f32 accumulators, the first one in one of its
 // own, so that the long chain of roundings is that of one product in 32 instead of one in one.  Against 64 bits such a sum is closer than with the f32
 // instructions (norm of the difference, uniform operands, every orientation alike): K = 512 4.0e-7 -> 0.71e-7, 2560 9.1e-7 -> 1.36e-7, 3584 10.7e-7 -> 1.6e-7;
-// positive operands, K = 2560, 7.8e-7 -> 0.8e-7.
+// positive operands, K = 2560, 7.8e-7 -> 0.85e-7; two products other than zero 3.1e-8 -> 2.6e-8, four 4.0e-8 -> 2.7e-8.  One product, correctly rounded by the
+// f32 instructions, 2.53e-8 -> 2.60e-8: within 0.96 ulp instead of 0.5, 4 % of them the neighbouring f32.
 //
 //   workgroup    four waves, two workgroups a CU.  Each wave multiplies the whole tile over its own slices of K (32 wide, every fourth one),
 //                so that an operand element is taken apart once in a workgroup and no wave waits for another before the end
 //   global->LDS  direct loads into the wave's own 16 KiB, one slice ahead: A's half is filled again as soon as A's pieces are in registers,
 //                B's under the last block's matrix instructions
 //   registers    2 x 64 of accumulators, 48 of A's pieces, 12 of a block of B's
-//   end          the four partial tiles meet in LDS and are added in the order of the waves
+//   end          the four partial tiles meet in LDS and are added in the order of the waves: first the sums of h h' alone, then those of the rest, so that no wave
+//                rounds one to the other (sums of two products: 3.5e-8 with one rounding a wave).  It costs 0.5 us per round, 2560^3 210 -> 213 us,
+//                2048 x 2048 x 640 37.0 -> 39.0 (40.4 with f32 instructions); each wave adding up a quarter in its registers takes as long.
 //   not a number An infinite or missing value anywhere in a tile makes the sum of the products that is not finite (l of an infinity is NaN), and so
 //                does an operand from 2^112 (5e33) or a sum from 2^96 (8e28) on.  Such a tile is multiplied again with the f32 instructions, each wave
 //                its own slices of K (the kernel of fewer tiles sums K in one chain: other roundings, the same infinities and NaN but where a sum
-//                overflows in between).  It costs both: 2560^3 210 us, 390 with one infinity in A, 480 with one in every row, 250 with f32 instructions alone.
+//                overflows in between).  It costs both: 2560^3 213 us, 390 with one infinity in A, 480 with one in every row, 250 with f32 instructions alone.
 //
 // What bounds it: the board's power, then the vector instructions that take the operands apart (416 per 96 matrix instructions, which
-// hide two each).  2560^3: 255 us with f32 instructions -> 210 (188 with all-zero operands, 211 with a softmax of wide logits, a quarter of whose values are below
-// 2^-110; without the factor 2^16, whose multiplications are two of every thirteen vector instructions, 206, but 475 where tiles with such values were multiplied again).
+// hide two each).  2560^3: 254 us with f32 instructions -> 213 (191 with all-zero operands, 213 with a softmax of wide logits, a quarter of whose values are below
+// 2^-110; without the factor 2^16, whose multiplications are two of every thirteen vector instructions, 209, but 475 where tiles with such values were multiplied again).
 // Tried: the same with v_mfma_f32_32x32x16_bf16, 1.1 times as long; the pieces by v_dot2c_f32_bf16 subtractions, 1.01 (a dot product takes the matrix
 // pipe); the forming dealt out between the matrix instructions, 1.03; all eight products but l l' 1.15 to 1.18, no faster than the f32 instructions on
 // most shapes; the waves of a SIMD at different priorities, 0.96 to 1.01.
@@ -306,32 +309,42 @@ namespace
                     }
                 }
             }
-            // the waves' partial tiles, 16 KiB each in the place of the wave's operands, chunk c of row r in slot c ^ r ^ (r >> 2)
-#pragma unroll
-            for(uint32_t i = 0; i < BLOCKS; ++i)
-#pragma unroll
-                for(uint32_t j = 0; j < BLOCKS; ++j)
-                {
-                    const uint32_t row = 16u * i + t, c = 4u * j + g;
-                    *reinterpret_cast<f32x4*>(mine + row * (TILE * 4u) + ((c ^ (row & 15u)) * CHUNK)) = hi[i][j] + lo[i][j];
-                }
-            __syncthreads();
+            // the waves' partial tiles, 16 KiB each in the place of the wave's operands, chunk c of row r in slot c ^ r; the leading products first,
+            // so that no wave rounds them to the rest of its own
             f32x4 sum[4];
             bool  finite = true;
 #pragma unroll
-            for(uint32_t it = 0; it < 4; ++it)
+            for(uint32_t part = 0; part < 2; ++part)
             {
-                const uint32_t row = 16u * it + (tid >> 4), c = tid & 15u;
-                const char*    q = lds + row * (TILE * 4u) + ((c ^ (row & 15u)) * CHUNK);
-                f32x4          v[WAVES];
+                if(part != 0u)
+                    __syncthreads();
 #pragma unroll
-                for(uint32_t w = 0; w < WAVES; ++w)
-                    v[w] = *reinterpret_cast<const f32x4*>(q + w * 2u * OPER);
-                sum[it] = (v[0] + v[1]) + (v[2] + v[3]);
+                for(uint32_t i = 0; i < BLOCKS; ++i)
+#pragma unroll
+                    for(uint32_t j = 0; j < BLOCKS; ++j)
+                    {
+                        const uint32_t row = 16u * i + t, c = 4u * j + g;
+                        *reinterpret_cast<f32x4*>(mine + row * (TILE * 4u) + ((c ^ (row & 15u)) * CHUNK)) = part == 0u ? hi[i][j] : lo[i][j];
+                    }
+                __syncthreads();
+#pragma unroll
+                for(uint32_t it = 0; it < 4; ++it)
+                {
+                    const uint32_t row = 16u * it + (tid >> 4), c = tid & 15u;
+                    const char*    q = lds + row * (TILE * 4u) + ((c ^ (row & 15u)) * CHUNK);
+                    f32x4          v[WAVES];
+#pragma unroll
+                    for(uint32_t w = 0; w < WAVES; ++w)
+                        v[w] = *reinterpret_cast<const f32x4*>(q + w * 2u * OPER);
+                    const f32x4 whole = (v[0] + v[1]) + (v[2] + v[3]);
+                    sum[it]           = part == 0u ? whole : sum[it] + whole;
+                }
+            }
+#pragma unroll
+            for(uint32_t it = 0; it < 4; ++it)
 #pragma unroll
                 for(uint32_t e = 0; e < 4; ++e)
                     finite = finite && __builtin_isfinite(sum[it][e]);
-            }
             if(!exact && __syncthreads_or(!finite))
             {
                 exact = true;

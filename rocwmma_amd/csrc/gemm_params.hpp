@@ -33,12 +33,15 @@ namespace r355
     // f32 GEMM on the bf16 matrix instructions, 64 x 64 tiles (gemm_f32.hip): a launch of p.tileCount tiles x `splits` shares of K
     void gemmF32Tiles(bool aK, bool bK, uint32_t splits, const GemmTileParams& p, hipStream_t stream);
     // Whether an f32 launch of 64 x 64 tiles takes that kernel: more workgroups than CUs, K shares of 16 stages (512 elements) at least.
-    // 100 random shapes of 260 to 3000 tiles and K from 512 to 3584: 1.03 to 1.41 times as fast, 1.17 in the geometric mean (260 tiles x 2496
-    // 74.8 -> 54.0 us, 1521 x 1856 166 -> 142); 143 tiles x 2512 in three shares 30.1 -> 27.6.  A CU's only workgroup has nothing that covers its loads: 207 tiles x 2128 36.3 -> 35.9, 132 x 1024
-    // 18.6 -> 19.5, 24 x 272 7.1 -> 9.3; short K is latency and the partial tiles' meeting: 1024 x 64 8.0 -> 12.3.
-    inline bool f32TilesOnBf16(uint64_t workgroups, uint32_t stages)
+    // 70 random shapes of 260 to 2900 workgroups and K from 512 to 3640: 0.98 to 1.30 times as fast, 1.11 in the geometric mean (493 tiles x 3080
+    // 93.0 -> 79.3 us, 1521 x 1856 165 -> 140, 294 x 3632 in three shares 75.0 -> 67.4; below K = 640, 0.98 to 1.05: 510 x 548 19.7 -> 20.1, 896 x 512 31.9 -> 31.0).  A CU's
+    // only workgroup has nothing that covers its loads: 207 tiles x 2128 36.3 -> 35.9, 132 x 1024 18.6 -> 19.5, 24 x 272 7.1 -> 9.3; short K is
+    // latency and the partial tiles' meeting: 1024 x 64 8.0 -> 12.3.
+    // Shares of K want 22: they are for few tiles, and one or two rounds of short ones are the partial tiles' meeting: 48 tiles x 5168 in ten shares of 17 stages
+    // 22.2 -> 25.1, 27 x 7924 in sixteen of 16 21.6 -> 25.5, 186 x 2364 in four of 19 33.7 -> 34.9; 108 x 2868 in four of 23 27.8 -> 27.2.
+    inline bool f32TilesOnBf16(uint64_t tiles, uint32_t splits, uint32_t stages)
     {
-        return workgroups > computeUnits() && stages >= 16u;
+        return tiles * splits > computeUnits() && stages >= (splits > 1u ? 22u : 16u);
     }
 } // namespace r355
 

@@ -2508,7 +2508,7 @@ namespace
             }
             else if constexpr(E == Elem::F32)
             {
-                if(tile == 64u && r355::f32TilesOnBf16((uint64_t)whole.tileCount * splits, p.splitStages ? p.splitStages : r355::stagesOfK(p.k, 4u)))
+                if(tile == 64u && r355::f32TilesOnBf16(whole.tileCount, splits, p.splitStages ? p.splitStages : r355::stagesOfK(p.k, 4u)))
                     r355::gemmF32Tiles(AK, BK, splits, p, stream);
                 else if(tile == 64u)
                     hipLaunchKernelGGL((gemmTiledKernelF32Tiny<AK, BK>), grid, block, 0, stream, p);
@@ -2675,11 +2675,11 @@ namespace
     //            fixed   latency   per workgroup    fixed   latency   per workgroup
     //   8-bit     3.9     0.46        0.46           2.6     0.28        0.27
     //   16-bit    2.9     0.46        0.46           1.2     0.32        0.236
-    //   f32       0.8     1.80        1.80           0.0     0.48        0.4575   (two together on the bf16 instructions, f32TilesOnBf16: 1.5, 0.45, 0.385)
+    //   f32       0.8     1.80        1.80           0.0     0.48        0.4575   (two together on the bf16 instructions, f32TilesOnBf16: 2.0, 0.45, 0.385)
     //   f64       1.6     1.834       1.834          0.0     0.48        0.458
     // Bound by the matrix instructions' rate, f32 and f64 run four small tiles in the time of a large one: they take the small
     // tile nearly everywhere (720 x 832 x 784 48.7 -> 15.5; f64 1584 x 608 x 672 81 -> 24), and on the bf16 instructions, which only the
-    // small f32 tile has, it is the faster one everywhere (f32 2560^3 252 -> 205 us beside 284 on large tiles).  16- and 8-bit problems
+    // small f32 tile has, it is the faster one everywhere (f32 2560^3 254 -> 213 us beside 284 on large tiles).  16- and 8-bit problems
     // take it for few tiles and short K (bf16 608 x 896 x 1680 12.3 -> 7.4 us, int8 1024 x 688 x 2896 11.7 -> 8.6).
     struct TileWork
     {
@@ -2691,7 +2691,7 @@ namespace
     };
     constexpr TileTimes TIMES_128[4] = {{3.9, 0.46, 0.46}, {2.9, 0.46, 0.46}, {0.8, 1.80, 1.80}, {1.6, 1.834, 1.834}}; // by log2(element size)
     constexpr TileTimes TIMES_64[4]  = {{2.6, 0.28, 0.27}, {1.2, 0.32, 0.236}, {0.0, 0.48, 0.4575}, {0.0, 0.48, 0.458}};
-    constexpr TileTimes TIMES_F32_BF16 = {1.5, 0.45, 0.385};
+    constexpr TileTimes TIMES_F32_BF16 = {2.0, 0.45, 0.385};
     constexpr double    REDUCE_FIXED = 3.5, REDUCE_PER_MB = 0.3; // the reduction's launch, and its share per MB of partial results
     TileWork tileWork(const r355_gemm_args& g)
     {
@@ -2712,7 +2712,7 @@ namespace
                 const uint32_t share = (stages + s - 1u) / s;
                 if((stages + share - 1u) / share != s)
                     continue; // a share would be empty
-                const bool       onBf16   = g.in_type == R355_F32 && edge == 64u && r355::f32TilesOnBf16(tiles * s, share);
+                const bool       onBf16   = g.in_type == R355_F32 && edge == 64u && r355::f32TilesOnBf16(tiles, s, share);
                 const TileTimes& t        = edge == 128u ? TIMES_128[cls] : onBf16 ? TIMES_F32_BF16 : TIMES_64[cls];
                 const uint64_t   together = edge == 128u || onBf16 ? 2u : 4u;
                 // (an XCD's share of the tiles, times the splits, over its CUs: 84 tiles x 3 are 33 on the first seven XCDs of 32 CUs)

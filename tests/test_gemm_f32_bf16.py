@@ -91,6 +91,23 @@ def test_tiny_values_take_no_second_pass(la, lb):
         assert np.linalg.norm(got - exact) <= 1.2e-7 * np.linalg.norm(exact)
 
 
+@pytest.mark.parametrize("la,lb", [(O.ROW, O.COL), (O.COL, O.ROW)])
+@pytest.mark.parametrize("count", [1, 2, 3, 4])
+def test_few_products(la, lb, count):
+    # 2^-24 of each product is left out at most, and the leading sums of all waves are rounded to the rest once.  One product: 2^-24 for that rounding and
+    # 2^-29 for those of the rest, itself 2^-7 of the whole.  More: three additions of leading sums and one of the rest, and in the norm less than the
+    # f32 instructions' sums of two products and more show on such operands (3.1e-8; these 2.6e-8 to 2.7e-8, 3.5e-8 with a rounding in every wave)
+    m, n, k = 1056, 1072, 1052
+    rng = np.random.default_rng(19)
+    A, B = np.zeros((m, k), np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    for _ in range(count):
+        A[np.arange(m), rng.integers(0, k, m)] = rng.standard_normal(m)
+    got = _run(A, B, la, lb).astype(np.float64)
+    exact, size = A.astype(np.float64) @ B, np.abs(A).astype(np.float64) @ np.abs(B)
+    assert np.all(np.abs(got - exact) <= (2.0 ** -23 + 2.0 ** -29 if count == 1 else 5 * 2.0 ** -24) * size)
+    assert np.linalg.norm(got - exact) <= 2.9e-8 * np.linalg.norm(exact)
+
+
 def test_one_product_below_the_normal_numbers():
     # rounded to 2^-149 once: products of the pieces are not rounded there one by one
     m, n, k = 1040, 1040, 528
