@@ -188,6 +188,7 @@ namespace
     __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) gemmF32Kernel(Params p)
     {
         __shared__ __attribute__((aligned(1024))) char lds[WAVES * 2u * OPER];
+        static_assert(sizeof(lds) == r355::F32_TILES_LDS, "what a launch plan reports");
         uint32_t tm, tn;
         if(!r355::tileCoordRange(blockIdx.x, p.tilesM, p.tilesN, p.tileFirst, p.tileCount, false, tm, tn))
             return;

@@ -30,6 +30,7 @@ namespace r355
         // the rounds' epilogues do not all store at once
         uint32_t stagger, staggerBlocks;
     };
+    constexpr uint32_t F32_TILES_LDS = 65536; // bytes of a workgroup of the following
     // f32 GEMM on the bf16 matrix instructions, 64 x 64 tiles (gemm_f32.hip): a launch of p.tileCount tiles x `splits` shares of K
     void gemmF32Tiles(bool aK, bool bK, uint32_t splits, const GemmTileParams& p, hipStream_t stream);
     // Whether an f32 launch of 64 x 64 tiles takes that kernel: more workgroups than CUs, K shares of 16 stages (512 elements) at least.

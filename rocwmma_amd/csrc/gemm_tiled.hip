@@ -2692,6 +2692,11 @@ namespace
     constexpr TileTimes TIMES_128[4] = {{3.9, 0.46, 0.46}, {2.9, 0.46, 0.46}, {0.8, 1.80, 1.80}, {1.6, 1.834, 1.834}}; // by log2(element size)
     constexpr TileTimes TIMES_64[4]  = {{2.6, 0.28, 0.27}, {1.2, 0.32, 0.236}, {0.0, 0.48, 0.4575}, {0.0, 0.48, 0.458}};
     constexpr TileTimes TIMES_F32_BF16 = {2.0, 0.45, 0.385};
+    // Whether a launch of `tile` x `tile` macro tiles and `splits` shares of K multiplies f32 on the bf16 instructions
+    bool onBf16Instructions(const r355_gemm_args& g, uint32_t tile, uint32_t splits)
+    {
+        return g.in_type == R355_F32 && tile == 64u && r355::f32TilesOnBf16((uint64_t)r355::tilesOf(g.m, tile) * r355::tilesOf(g.n, tile), splits, splitStagesOf(g, splits));
+    }
     constexpr double    REDUCE_FIXED = 3.5, REDUCE_PER_MB = 0.3; // the reduction's launch, and its share per MB of partial results
     TileWork tileWork(const r355_gemm_args& g)
     {
@@ -2712,7 +2717,7 @@ namespace
                 const uint32_t share = (stages + s - 1u) / s;
                 if((stages + share - 1u) / share != s)
                     continue; // a share would be empty
-                const bool       onBf16   = g.in_type == R355_F32 && edge == 64u && r355::f32TilesOnBf16(tiles, s, share);
+                const bool       onBf16   = onBf16Instructions(g, edge, s);
                 const TileTimes& t        = edge == 128u ? TIMES_128[cls] : onBf16 ? TIMES_F32_BF16 : TIMES_64[cls];
                 const uint64_t   together = edge == 128u || onBf16 ? 2u : 4u;
                 // (an XCD's share of the tiles, times the splits, over its CUs: 84 tiles x 3 are 33 on the first seven XCDs of 32 CUs)
@@ -3027,6 +3032,8 @@ namespace r355
             plan->block_x      = THREADS;
             plan->block_y      = 1;
             plan->lds_bytes    = (fiveBuffers || tile != 256u ? 5u * OPER_BYTES : NUM_STAGES * STAGE_BYTES) * tile / 256u;
+            if(onBf16Instructions(g, tile, 1u))
+                plan->lds_bytes = F32_TILES_LDS;
             const uint32_t splits = tile == 128u ? splitCount(g, true) : 1u;
             plan->split_k         = splits;
             plan->grid_y          = splits;
@@ -3053,7 +3060,7 @@ namespace r355
         plan->grid_y            = shape.splits;
         plan->block_x           = THREADS;
         plan->block_y           = 1;
-        plan->lds_bytes         = (fiveBuffers ? 5u * OPER_BYTES : NUM_STAGES * STAGE_BYTES) * tile / 256u;
+        plan->lds_bytes         = onBf16Instructions(g, tile, shape.splits) ? F32_TILES_LDS : (fiveBuffers ? 5u * OPER_BYTES : NUM_STAGES * STAGE_BYTES) * tile / 256u;
         plan->split_k           = shape.splits;
         plan->workspace_bytes   = shape.splits > 1u ? (uint64_t)shape.splits * g.m * g.n * accBytes(g.in_type) : 0u;
     }

@@ -68,3 +68,16 @@ def test_other_kernel_families():
 def test_a_lead_within_the_models_error_does_not_move_a_call(in_t, out_t, m, n, k, tile, splits):
     plan = R.gemm_launch_plan(_args(in_t, out_t, m, n, k, need=R.gemm_query(_args(in_t, out_t, m, n, k, need=2 ** 64 - 1)).workspace_bytes))
     assert ((plan.macro_tile_m, plan.macro_tile_n), plan.split_k) == (tile, splits)
+
+
+# f32 on 64 x 64 tiles: four waves with 16 KiB each on the bf16 instructions (more workgroups than CUs, K of 16 stages of 128 bytes, shares of 22), five
+# buffers of 8 KiB on the f32 ones
+@pytest.mark.parametrize("m,n,k,splits,lds", [(2560, 2560, 2560, 1, 65536), (1040, 1072, 484, 1, 65536), (1040, 1072, 480, 1, 40960), (1024, 1024, 2560, 1, 40960),
+                                              (1024, 1040, 2084, 3, 65536), (560, 160, 7924, 8, 40960)])
+def test_lds_of_f32_tiles(m, n, k, splits, lds):
+    need = R.gemm_query(_args(R.F32, R.F32, m, n, k, need=2 ** 64 - 1)).workspace_bytes if splits > 1 else 0
+    plan = R.gemm_launch_plan(_args(R.F32, R.F32, m, n, k, need=need))
+    assert (plan.macro_tile_m, plan.split_k, plan.lds_bytes) == (64, splits, lds)
+    if splits == 1:
+        for query in (R.gemm_query, R.gemm_launch_plan):
+            assert query(_args(R.F32, R.F32, m, n, k, kernel=R.KERNEL_TILED_64)).lds_bytes == lds
