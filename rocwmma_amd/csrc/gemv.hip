@@ -681,9 +681,11 @@ namespace
         if(askew)
         {
             plan = askewPlan<T>(m, k, splits);
-            // (a streamed matrix of several rounds of blocks: where the plan is a single round of workgroups; aligned columns otherwise split: not in runs of 64 bytes
-            // over many columns, f32 864 x 13476, 3456 of them, 12.3 -> 14.4 us, 576 x 10216, 2048 of them, 12.0 -> 9.8)
-            if(!offLines && splits > 1u && plan.lanes == 4u && plan.kPer > 2700u)
+            // (a streamed matrix of several rounds of blocks: where the plan is a single round of workgroups; aligned columns otherwise split: not in split runs of 64 bytes
+            // over many columns, f32 864 x 13476, 3456 of them, 12.3 -> 14.4 us, 768 x 14480 14.8 -> 17.0, 576 x 10216, 2048 of them, 12.0 -> 9.8, f64 352 x 14812 14.1 -> 15.6,
+            // 384 x 15084 15.9 -> 18.0, 272 x 19872 14.6 -> 15.1; in one piece they are the faster ones, f32 2016 x 2708 19.7 -> 9.6, 2752 x 4352 19.7 -> 15.5, f64 1216 x 2792
+            // 22.8 -> 12.6, 1280 x 3172 20.8 -> 17.3)
+            if(!offLines && splits > 1u && plan.splits > 1u && plan.lanes == 4u && plan.kPer > 2700u)
                 askew = false;
             else if(!offLines && streamed && (uint64_t)plan.splits * ((m + plan.lanes * (16u / sizeof(T)) - 1u) / (plan.lanes * (16u / sizeof(T)))) > r355::computeUnits())
                 askew = false;
