@@ -155,3 +155,47 @@ def test_shares_of_k():
     got = _run(A, B, O.ROW, O.COL, C, 1.5, 1.0, workspace=need, splits=3)
     exact = 1.5 * (A.astype(np.float64) @ B) + C
     assert np.linalg.norm(got - exact) <= 2e-7 * np.linalg.norm(exact)
+
+
+@pytest.mark.parametrize("k", [484, 512])
+def test_the_shortest_k(k):
+    # sixteen stages of 128 bytes, the last of one 16-byte chunk or whole: four slices a wave
+    m, n = 1040, 1072
+    A, B = _uniform(20, m, k), _uniform(21, k, n)
+    got = _run(A, B, O.ROW, O.ROW)
+    exact = A.astype(np.float64) @ B
+    assert np.linalg.norm(got - exact) <= 1.2e-7 * np.linalg.norm(exact)
+
+
+def test_second_pass_in_one_share_of_k():
+    # an overflow and an infinity that only the second of three shares meets: its tiles of that row and column are multiplied again, the other shares' are not
+    m, n, k = 1024, 1040, 2084
+    A, B, C = _uniform(22, m, k), _uniform(23, k, n), _uniform(24, m, n)
+    A[100, 1000], B[900, 700] = np.float32(1e34), np.inf
+    need = int(R.gemm_query(R.gemm_args(R.F32, R.F32, m, n, k, 0x1000, 0x2000, 0x3000, 0x4000, 1.5, 1.0, O.ROW, O.COL, O.ROW, O.ROW,
+                                        workspace_bytes=2 ** 62)).workspace_bytes)
+    got = _run(A, B, O.ROW, O.COL, C, 1.5, 1.0, workspace=need, splits=3).astype(np.float64)
+    with np.errstate(all="ignore"):
+        exact = 1.5 * (A.astype(np.float64) @ B.astype(np.float64)) + C
+    assert np.array_equal(np.isinf(got), np.isinf(exact)) and np.array_equal(got[np.isinf(got)], exact[np.isinf(exact)]) and not np.isnan(got).any()
+    fin = np.isfinite(exact)
+    scale = 1.5 * np.abs(A).astype(np.float64) @ np.abs(np.where(np.isfinite(B), B, 0)) + np.abs(C)
+    assert np.all(np.abs(got - exact)[fin] <= ((k + 8) * 2.0 ** -24 * scale)[fin])
+
+
+@pytest.mark.parametrize("la,lb", [(O.ROW, O.COL), (O.COL, O.ROW)])
+@pytest.mark.parametrize("ldl", [O.ROW, O.COL])
+def test_result_in_the_place_of_c(la, lb, ldl):
+    m, n, k = 1072, 1040, 636
+    A, B, C = _uniform(25, m, k), _uniform(26, k, n), _uniform(27, m, n)
+    A[77, 300] = np.inf  # (a row of tiles that is multiplied again adds C once as well)
+    B[300, :] = np.abs(B[300, :]) + np.float32(0.5)
+    d = to_device(_flat(C, ldl))
+    R.gemm(R.F32, R.F32, m, n, k, to_device(_flat(A, la)), to_device(_flat(B, lb)), d, d, 2.0, -0.5, la, lb, ldl, ldl)
+    got = to_host(d, np.float32)
+    got = (got.reshape(m, n) if ldl == O.ROW else got.reshape(n, m).T).astype(np.float64)
+    assert np.all(got[77] == np.inf)
+    rows = np.arange(m) != 77
+    exact = 2.0 * (A[rows].astype(np.float64) @ B) - 0.5 * C[rows]
+    bound = (k + 4) * 2.0 ** -24 * (2.0 * (np.abs(A[rows]).astype(np.float64) @ np.abs(B)) + 0.5 * np.abs(C[rows]))
+    assert np.all(np.abs(got[rows] - exact) <= bound)
