@@ -23,8 +23,8 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 sys.path.insert(0, os.path.join(ROOT, "tests"))
 
-# (f32: of the f32 matrix instructions.  Launches of many tiles sum six bf16 products instead, at most 2500 / 6 = 417: fractions above 1)
-PEAK_TFLOPS = {"f16": 2500.0, "bf16": 2500.0, "e4m3": 5000.0, "i8": 5000.0, "f32": 157.3, "f64": 78.6}
+# f32: of the f32 matrix instructions, or of six bf16 products for one (launches of many tiles, on_bf16 below)
+PEAK_TFLOPS = {"f16": 2500.0, "bf16": 2500.0, "e4m3": 5000.0, "i8": 5000.0, "f32": 157.3, "f32_on_bf16": round(2500.0 / 6, 1), "f64": 78.6}
 HBM_PEAK_GBPS = 8000.0
 # rocprofv3 --pmc results per benchmark case (MFMA busy, LDS bank conflicts, bytes across the L2 <-> fabric
 # boundary), one table row per case.  Each row carries the SHA-256 (first 16 hex digits) of the kernel sources it
@@ -38,7 +38,13 @@ KERNEL_SOURCES = {"gemm": ["gemm_tiled.hip", "gemm_f32.hip", "gemm_params.hpp", 
 
 # Matrix-core operations per CU and clock of gfx950, dense (the Multiplier of the reference's peak model,
 # test/performance.hpp:435-442: peak = Multiplier x CUs x clock; 2:4 sparse doubles it): published peak / (256 CUs x 2.4 GHz)
-MULTIPLIER = {"f16": 4096, "bf16": 4096, "e4m3": 8192, "i8": 8192, "f32": 256, "f64": 128}
+MULTIPLIER = {"f16": 4096, "bf16": 4096, "e4m3": 8192, "i8": 8192, "f32": 256, "f32_on_bf16": 4096 / 6, "f64": 128}
+
+
+def on_bf16(R, g):
+    """Whether an f32 GEMM runs on the bf16 matrix instructions: 64 x 64 tiles with 16 KiB of LDS for each of four waves"""
+    plan = R.gemm_launch_plan(g)
+    return g.in_type == R.F32 and plan.macro_tile_m == 64 and plan.lds_bytes == 65536
 
 
 class ClockSampler:
@@ -391,6 +397,9 @@ def run_extras(R, O, np, torch, args, counters, clocks, cus):
         d = torch.empty(mm * nn * R.DTYPE_BYTES[out_t], dtype=torch.uint8, device="cuda")
         g = R.gemm_args(in_t, out_t, mm, nn, kk, a, b, None, d, 1.0, 0.0, la, lb, R.ROW_MAJOR, R.ROW_MAJOR,
                         a_meta=sparse_meta, workspace=workspace)
+        kind = KIND[in_t]
+        if on_bf16(R, g):
+            kind, peak = "f32_on_bf16", PEAK_TFLOPS["f32_on_bf16"]
         settle(torch, lambda: R.lib().r355_gemm(ctypes.byref(g), None))
         # event-timed launches with the engine clock read meanwhile; short kernels run more launches so that the
         # sampler sees at least ~60 ms of them
@@ -401,7 +410,9 @@ def run_extras(R, O, np, torch, args, counters, clocks, cus):
         rec = {"ms": round(ms, 4), "value": round(tf, 2), "unit": unit, "peak": peak * peak_scale,
                "frac": round(tf / (peak * peak_scale), 4), "launches_timed": steps,
                "validated": sampled_ok(in_t, out_t, la, lb, mm, nn, kk, a, b, d, sparse_rows)}
-        rec.update(clock_fields(KIND[in_t], tf, mhz, cus, sparse=sparse_meta is not None))
+        if kind == "f32_on_bf16":
+            rec["peak_of"] = "six bf16 products for one f32 product (f32 matrix instructions: %.1f)" % PEAK_TFLOPS["f32"]
+        rec.update(clock_fields(kind, tf, mhz, cus, sparse=sparse_meta is not None))
         out[name] = with_counters(name, rec)
         if workspace is not None:  # split-K: the same problem with one workgroup per tile beside it
             out[name]["split_k"] = R.gemm_query(g).split_k
