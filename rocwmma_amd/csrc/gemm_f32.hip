@@ -27,7 +27,7 @@
 // hide two each).  2560^3: 254 us with f32 instructions -> 213 (191 with all-zero operands, 213 with a softmax of wide logits, a quarter of whose values are below
 // 2^-110; without the factor 2^16, whose multiplications are two of every thirteen vector instructions, 209, but 475 where tiles with such values were multiplied again).
 // Tried: the same with v_mfma_f32_32x32x16_bf16, 1.1 times as long; the pieces by v_dot2c_f32_bf16 subtractions, 1.01 (a dot product takes the matrix
-// pipe); the forming dealt out between the matrix instructions, 1.03; all eight products but l l' 1.15 to 1.18, no faster than the f32 instructions on
+// pipe); the forming dealt out between the matrix instructions, 1.03; all eight products but l l' 1.11 to 1.18, no faster than the f32 instructions on
 // most shapes; the waves of a SIMD at different priorities, 0.96 to 1.01.
 #include <hip/hip_runtime.h>
 
